@@ -35,8 +35,15 @@ typedef enum npbcg_status {
  * (npbcg_opts.cg_form) and keep every scalar on the GPU; the reference issues
  * 6 launches and 2 blocking copies per CG step (cg.cu:814-837). */
 enum {
-    NPBCG_ENGINE_AUTO = 0,        /* KERNELS (measured faster: 8.5 ms against 14.6 ms for
-                                     10 outer iterations at n = 75000) */
+    NPBCG_ENGINE_AUTO = 0,        /* up to n = 19152, with the layout and step form left
+                                     to the library too (spmv_variant, cg_form,
+                                     dot_pass, fuse_p_update, tile and sort options 0)
+                                     and no row of more than some thousand entries: the
+                                     resident engine, one launch per call that keeps
+                                     vectors and matrix on chip (plain FP64 solves with
+                                     solve_batch 0 too).  Else KERNELS (8.5 ms against
+                                     14.6 ms of PERSISTENT for 10 outer iterations at
+                                     n = 75000) */
     NPBCG_ENGINE_KERNELS = 1,     /* fused per-phase kernels (two a CG step), replayed
                                      from a captured HIP graph per outer iteration */
     NPBCG_ENGINE_PERSISTENT = 2   /* one cooperative kernel runs whole outer iterations
@@ -107,7 +114,8 @@ typedef struct npbcg_timing {
     int launches;           /* kernel launches (or graph launches) issued */
     long long nnz;          /* rowstr[n] of the context's matrix */
     int n;
-    int engine;             /* engine actually used */
+    int engine;             /* engine actually used (PERSISTENT for the resident
+                               engine too: one kernel ran whole outer iterations) */
 } npbcg_timing;
 
 void npbcg_default_opts(npbcg_opts *opts);
@@ -206,7 +214,9 @@ typedef struct {
  * count returns NPBCG_ERR_INVALID).  Replaces the reference's PROFILING build
  * (cg.cu:83-94 timers around each launch, table printed at cg.cu:565-589).
  * Library calls also open roctx ranges named after the call
- * ("npbcg_power", "npbcg_solve", ...) for rocprofv3 --marker-trace. */
+ * ("npbcg_power", "npbcg_solve", ...) for rocprofv3 --marker-trace.  A context
+ * on the resident engine lists its three kernels; NPBCG_ENGINE_KERNELS gives
+ * the table phase by phase. */
 int npbcg_profile_kernels(npbcg_ctx *ctx, int niter, double shift, double *zeta_out,
                           npbcg_kernel_time *out, int max_kinds, int *nkinds,
                           double *total_ms);

@@ -81,6 +81,11 @@ struct npbcg_ctx {
     // persistent engine: partials, barrier words, argument block (lazy)
     npbcg_dev::PersistentState ps{};
 
+    // resident engine (small orders): launch shape (grid 0: not used) and
+    // buffers, allocated by the first call that runs on it
+    npbcg_dev::ResidentShape rshape;
+    npbcg_dev::ResidentState rstate;
+
     // Captured outer iterations: [0] first (x used as is), [1] later ones
     // (x = z/||z|| of the previous iteration applied first).
     hipGraphExec_t outer_graph[2] = {nullptr, nullptr};
@@ -170,6 +175,11 @@ constexpr int kNumVectors = 8;
 constexpr int kDotApartBlocks = 24;
 // Widest default sort window of the SELL copy (npbcg_opts.sort_window = 0).
 constexpr int kMaxSortWindow = 8192;
+// Exchange buffers of one resident launch at most (npbcg_power runs more outer
+// iterations in several launches).
+constexpr size_t kResidentWords = (size_t)8 << 20;
+// Steps of a resident solve launch at most.
+constexpr int kResidentSolveSteps = 64;
 constexpr int kVecPAlt = 5, kVecB = 6, kVecXsol = 7;
 
 namespace {
@@ -450,6 +460,74 @@ int run_persistent(npbcg_ctx *c, int niter, int scale_first, int record, int fin
     return NPBCG_OK;
 }
 
+// Whether calls of this context run on the resident engine; one outer
+// iteration of `steps` CG steps has to fit the exchange workspace.
+bool use_resident(const npbcg_ctx *c, int steps) {
+    return c->rshape.grid > 0 &&
+           (size_t)(steps + 1) * (size_t)c->rshape.stride <= kResidentWords;
+}
+
+// Buffers of a resident launch of niter outer iterations of `steps` steps.
+int ensure_resident(npbcg_ctx *c, int steps, int niter) {
+    auto &rs = c->rstate;
+    const auto &sh = c->rshape;
+    if (!rs.val) {
+        const size_t entries = (size_t)std::max(1, sh.wave_off.back()) * npbcg_dev::kWave;
+        std::vector<int> maps(sh.wave_off);
+        maps.insert(maps.end(), sh.word_row.begin(), sh.word_row.end());
+        maps.insert(maps.end(), sh.row_word.begin(), sh.row_word.end());
+        NPBCG_HIP(hipMalloc(&rs.wave_off, sizeof(int) * maps.size()));
+        rs.word_row = rs.wave_off + sh.wave_off.size();
+        rs.row_word = rs.word_row + sh.word_row.size();
+        NPBCG_HIP(hipMalloc(&rs.abort_word, sizeof(unsigned)));
+        NPBCG_HIP(hipMalloc(&rs.col, sizeof(uint16_t) * entries));
+        NPBCG_HIP(hipMalloc(&rs.val, sizeof(double) * entries));
+        NPBCG_HIP(hipMemcpyAsync(rs.wave_off, maps.data(), sizeof(int) * maps.size(),
+                                 hipMemcpyHostToDevice, c->stream));
+        NPBCG_HIP(hipStreamSynchronize(c->stream));  // maps goes out of scope
+        NPBCG_HIP(npbcg_dev::launch_resident_fill(c->pb, sh, rs, c->stream));
+    }
+    const size_t words = (size_t)niter * (steps + 1) * sh.stride;
+    const size_t part = npbcg_dev::resident_partials(sh, niter);
+    if (words > rs.xchg_words || part > rs.part_words) {
+        NPBCG_HIP(hipStreamSynchronize(c->stream));
+        (void)hipFree(rs.xchg);
+        (void)hipFree(rs.part);
+        rs.xchg = nullptr;
+        rs.part = nullptr;
+        rs.xchg_words = rs.part_words = 0;
+        NPBCG_HIP(hipMalloc(&rs.xchg, sizeof(double) * words));
+        NPBCG_HIP(hipMalloc(&rs.part, sizeof(double) * part));
+        rs.xchg_words = words;
+        rs.part_words = part;
+    }
+    return NPBCG_OK;
+}
+
+// Held from a resident launch until its results are on the host: the
+// workgroups of two such launches could each take part of the CUs and wait for
+// the rest.
+std::mutex &resident_turn(int device) {
+    static std::mutex turn[64];
+    return turn[device & 63];
+}
+
+// niter outer iterations on the resident engine, in launches whose exchange
+// buffers fit the workspace; the caller holds resident_turn.
+int run_resident(npbcg_ctx *c, const Fp64Problem &pb, int niter, int record, int *launches) {
+    const size_t per = (size_t)(c->cgitmax + 1) * c->rshape.stride;
+    const int chunk = std::min(niter, (int)std::max<size_t>(1, kResidentWords / per));
+    int rc = ensure_resident(c, c->cgitmax, chunk);
+    if (rc != NPBCG_OK) return rc;
+    for (int done = 0; done < niter; done += chunk) {
+        NPBCG_HIP(npbcg_dev::launch_resident(pb, c->rshape, c->rstate, c->cgitmax,
+                                             std::min(chunk, niter - done), done > 0, done,
+                                             record, 0, 0.0, c->stream));
+        *launches += 3;
+    }
+    return NPBCG_OK;
+}
+
 int read_scalars(npbcg_ctx *c, Scalars *out) {
     NPBCG_HIP(hipMemcpyAsync(c->h_stage, c->d_sc, sizeof(Scalars), hipMemcpyDeviceToHost,
                              c->stream));
@@ -534,7 +612,8 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
         return set_error(NPBCG_ERR_INVALID,
                          "npbcg_create: sort_window must be 0 or a positive multiple of 64");
     }
-    // AUTO takes the graph-replayed kernels: 8.5 ms against 14.6 ms for the
+    // AUTO takes the resident engine at small orders (below), else the
+    // graph-replayed kernels: 8.5 ms against 14.6 ms for the
     // persistent kernel over 10 outer iterations at n = 75000, whose grid
     // barriers each write back and invalidate every XCD's L2
     c->engine = c->opts.engine == NPBCG_ENGINE_PERSISTENT ? NPBCG_ENGINE_PERSISTENT
@@ -773,6 +852,27 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
         c->ps.spin_limit = (long long)std::max(clock_khz, 1000) * 2000;
         c->ps.cgitmax = c->cgitmax;
     }
+    // Resident engine: the engine, layout and step form all left to the
+    // library, and an order its kernels take.  Microseconds a CG step, resident
+    // against the kernels this context would launch (CSR below n = 16384,
+    // LDS-staged above): 2.2 / 8.8 at n = 1400, 3.8 / 10.9 at 7000, 7.1 / 16.2
+    // at 14000, 7.2 / 17.8 at 16000, 11.9 / 27.5 at 19000, where the LDS ends.
+    if (c->opts.engine == NPBCG_ENGINE_AUTO && c->opts.spmv_variant == 0 &&
+        c->opts.cg_form == 0 && c->opts.dot_pass == 0 && !c->opts.fuse_p_update &&
+        c->opts.tile_rows <= 0 && c->opts.tile_width <= 0 && c->opts.sort_window == 0) {
+        int lds_cap = 0, per_cu = 0, clock_khz = 0;
+        if (hipDeviceGetAttribute(&lds_cap, hipDeviceAttributeSharedMemPerBlockOptin,
+                                  c->device) != hipSuccess || lds_cap <= 0)
+            lds_cap = 64 * 1024;
+        if (npbcg_dev::resident_shape(n, rowstr, cus, lds_cap, &c->rshape)) {
+            CREATE_HIP(npbcg_dev::resident_capacity(c->rshape, &per_cu));
+            CREATE_HIP(hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate,
+                                             c->device));
+            // a read that waits 1 s has lost a workgroup: the launch gives up
+            c->rstate.spin_limit = (long long)std::max(clock_khz, 1000) * 1000;
+        }
+        if (per_cu < 1) c->rshape = npbcg_dev::ResidentShape{};
+    }
     CREATE_HIP(npbcg_dev::launch_fill(c->pb.x, n + 1, 1.0, vec_blocks, c->stream));
     CREATE_HIP(hipStreamSynchronize(c->stream));
 #undef CREATE_HIP
@@ -832,6 +932,12 @@ void npbcg_destroy(npbcg_ctx *c) {
     (void)hipFree(c->ps.part);
     (void)hipFree(c->ps.bar);
     (void)hipFree(c->ps.args);
+    (void)hipFree(c->rstate.val);
+    (void)hipFree(c->rstate.col);
+    (void)hipFree(c->rstate.wave_off);
+    (void)hipFree(c->rstate.xchg);
+    (void)hipFree(c->rstate.part);
+    (void)hipFree(c->rstate.abort_word);
     if (c->h_stage) (void)hipHostFree(c->h_stage);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -842,7 +948,14 @@ int npbcg_conj_grad_device(npbcg_ctx *c, double *rnorm) {
     if (!c) return set_error(NPBCG_ERR_INVALID, "npbcg_conj_grad_device: NULL context");
     NPBCG_HIP(hipSetDevice(c->device));
     NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
-    if (c->engine == NPBCG_ENGINE_PERSISTENT) {
+    bool resident = use_resident(c, c->cgitmax);
+    int launches = 0;
+    std::unique_lock<std::mutex> turn;
+    if (resident) {
+        turn = std::unique_lock<std::mutex>(resident_turn(c->device));
+        int rc = run_resident(c, c->pb, 1, 0, &launches);
+        if (rc != NPBCG_OK) return rc;
+    } else if (c->engine == NPBCG_ENGINE_PERSISTENT) {
         int rc = run_persistent(c, 1, 0, 0, 0);
         if (rc != NPBCG_OK) return rc;
     } else {
@@ -852,15 +965,25 @@ int npbcg_conj_grad_device(npbcg_ctx *c, double *rnorm) {
     Scalars s;
     int rc = read_scalars(c, &s);
     if (rc != NPBCG_OK) return rc;
+    if (resident && s.aborted) {  // x is untouched: the multi-kernel engine takes over
+        c->rshape.grid = 0;
+        resident = false;
+        turn.unlock();
+        NPBCG_HIP(npbcg_dev::enqueue_conj_grad(c->pb, c->cgitmax, 0, 0, c->stream, nullptr));
+        NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
+        rc = read_scalars(c, &s);
+        if (rc != NPBCG_OK) return rc;
+    }
     float ms = 0.f;
     NPBCG_HIP(hipEventElapsedTime(&ms, c->ev_start, c->ev_stop));
     c->timing.total_ms = ms;
     c->timing.spmv_samples = 0;
     c->timing.spmv_avg_ms = 0.0;
-    c->timing.launches = c->engine == NPBCG_ENGINE_PERSISTENT
+    c->timing.launches = resident ? launches
+                         : c->engine == NPBCG_ENGINE_PERSISTENT
                              ? 2
                              : npbcg_dev::conj_grad_launches(c->pb, c->cgitmax);
-    c->timing.engine = c->engine;
+    c->timing.engine = resident ? NPBCG_ENGINE_PERSISTENT : c->engine;
     if (rnorm) *rnorm = s.rnorm;
     clear_error();
     return NPBCG_OK;
@@ -948,13 +1071,48 @@ int npbcg_power(npbcg_ctx *c, int niter, double shift, double *zeta_out,
         clear_error();
         return NPBCG_OK;
     }
+    const bool sample = c->sample_every > 0 && (c->device_calls % c->sample_every) == 0;
+    c->device_calls++;
+    if (niter > 0 && !sample && use_resident(c, c->cgitmax)) {
+        int launches = 2;
+        std::unique_lock<std::mutex> turn(resident_turn(c->device));
+        NPBCG_HIP(npbcg_dev::launch_reset_scalars(c->pb, shift, c->stream));
+        NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
+        rc = run_resident(c, c->pb, niter, 1, &launches);
+        if (rc != NPBCG_OK) return rc;
+        NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
+        Scalars s;
+        rc = read_scalars(c, &s);
+        turn.unlock();
+        if (rc != NPBCG_OK) return rc;
+        if (!s.aborted) {
+            NPBCG_HIP(npbcg_dev::launch_scale_x(c->pb, 0.0, 1, c->stream));
+            NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
+            if (zeta_out)
+                NPBCG_HIP(hipMemcpyAsync(zeta_out, c->d_hist, sizeof(double) * niter,
+                                         hipMemcpyDeviceToHost, c->stream));
+            if (rnorm_out)
+                NPBCG_HIP(hipMemcpyAsync(rnorm_out, c->d_hist + c->hist_cap,
+                                         sizeof(double) * niter, hipMemcpyDeviceToHost,
+                                         c->stream));
+            NPBCG_HIP(hipStreamSynchronize(c->stream));
+            float ms = 0.f;
+            NPBCG_HIP(hipEventElapsedTime(&ms, c->ev_start, c->ev_stop));
+            c->timing.total_ms = ms;
+            c->timing.launches = launches;
+            c->timing.engine = NPBCG_ENGINE_PERSISTENT;
+            c->timing.spmv_samples = 0;
+            c->timing.spmv_avg_ms = 0.0;
+            clear_error();
+            return NPBCG_OK;
+        }
+        c->rshape.grid = 0;  // x is untouched: the multi-kernel engine takes over
+    }
     const bool use_graph = c->opts.use_graph != 0;
     if (use_graph) {
         rc = ensure_graph(c);
         if (rc != NPBCG_OK) return rc;
     }
-    const bool sample = c->sample_every > 0 && (c->device_calls % c->sample_every) == 0;
-    c->device_calls++;
     npbcg_dev::SpmvProbe probe{nullptr, nullptr, 0};
     if (sample) {
         rc = ensure_probes(c);
@@ -1025,7 +1183,21 @@ int npbcg_profile_kernels(npbcg_ctx *c, int niter, double shift, double *zeta_ou
     pb.marks = &marks;
     marks.stamp(c->stream);
     hipError_t e = marks.err;
-    for (int it = 0; it < niter && e == hipSuccess; it++)
+    bool resident = use_resident(c, c->cgitmax);
+    if (resident) {
+        int launches = 0;
+        std::unique_lock<std::mutex> turn(resident_turn(c->device));
+        rc = run_resident(c, pb, niter, 1, &launches);
+        Scalars s;
+        if (rc == NPBCG_OK) rc = read_scalars(c, &s);
+        if (rc != NPBCG_OK) return rc;
+        if (s.aborted) {
+            c->rshape.grid = 0;
+            return npbcg_profile_kernels(c, niter, shift, zeta_out, out, max_kinds, nkinds,
+                                         total_ms);
+        }
+    }
+    for (int it = 0; it < niter && e == hipSuccess && !resident; it++)
         e = npbcg_dev::enqueue_conj_grad(pb, c->cgitmax, it > 0 ? 1 : 0, 1, c->stream, nullptr);
     if (e == hipSuccess) e = npbcg_dev::launch_scale_x(pb, 0.0, 1, c->stream);
     if (e == hipSuccess) e = marks.err;
@@ -1702,7 +1874,12 @@ int npbcg_log_pairs(npbcg_ctx *c, int pairs, float *r, float *e) {
     const int kind = c->precond;
     c->precond = NPBCG_PRECOND_NONE;
     npbcg_solve_stats st{};
+    // by the kernels that log the pairs below: the last corrections x* - x_k
+    // are a few digits above x*'s own rounding
+    const int resident_grid = c->rshape.grid;
+    c->rshape.grid = 0;
     rc = npbcg_solve(c, NPBCG_SOLVE_FP64, 1e-12, 5000, &st);
+    c->rshape.grid = resident_grid;
     c->precond = kind;
     if (rc != NPBCG_OK) return rc;
     auto &pr = c->pairs;
@@ -1890,6 +2067,11 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
         // but still cost a launch each)
         int *bud = c->budget[0][c->active_precond];
         int batch = std::min(bud[0] > 0 ? bud[0] : batch0, maxit);
+        // plain CG on the resident engine: one launch runs until the stop
+        // test passes; a solve it leaves unfinished goes on below
+        const int res_steps = std::min(maxit, kResidentSolveSteps);
+        const bool resident = c->active_precond == NPBCG_PRECOND_NONE &&
+                              c->opts.solve_batch <= 0 && use_resident(c, res_steps);
         // first batch: reset, init, `batch` steps, residual (captured once per key)
         auto first_batch = [&]() -> hipError_t {
             hipError_t e = npbcg_dev::launch_reset_scalars(pbs, 0.0, c->stream, rtol, 1);
@@ -1899,9 +2081,19 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
             return e;
         };
         NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
-        int rc = run_solve_sequence(c, 0, rtol, maxit, batch, first_batch);
-        if (rc != NPBCG_OK) return rc;
         bool first = true;
+        std::unique_lock<std::mutex> turn;
+        if (resident) {
+            turn = std::unique_lock<std::mutex>(resident_turn(c->device));
+            int rc = ensure_resident(c, res_steps, 1);
+            if (rc != NPBCG_OK) return rc;
+            NPBCG_HIP(npbcg_dev::launch_reset_scalars(pbs, 0.0, c->stream, rtol, 1));
+            NPBCG_HIP(npbcg_dev::launch_resident(pbs, c->rshape, c->rstate, res_steps, 1, 0, 0, 0,
+                                                 1, rtol, c->stream));
+        } else {
+            int rc = run_solve_sequence(c, 0, rtol, maxit, batch, first_batch);
+            if (rc != NPBCG_OK) return rc;
+        }
         for (;;) {
             if (!first) {
                 NPBCG_HIP(npbcg_dev::enqueue_solve_steps(pbs, batch, 0, c->stream));
@@ -1909,7 +2101,16 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
             }
             NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
             int rc = read_scalars_from(c, pbs.sc, &sc);
+            if (turn.owns_lock()) turn.unlock();
             if (rc != NPBCG_OK) return rc;
+            if (first && resident && sc.aborted) {  // b is untouched: start over without it
+                c->rshape.grid = 0;
+                rc = run_solve_sequence(c, 0, rtol, maxit, batch, first_batch);
+                if (rc != NPBCG_OK) return rc;
+                NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
+                rc = read_scalars_from(c, pbs.sc, &sc);
+                if (rc != NPBCG_OK) return rc;
+            }
             s.sweeps++;
             s.fp64_spmvs = sc.steps + s.sweeps;
             relres = sc.rnorm / c->rhs_norm;

@@ -176,7 +176,7 @@ struct Scalars {
     int inner_total; // mixed solve: inner steps of the finished sweeps
     int sweep1_steps;  // mixed solve: inner steps of the first two sweeps
     int sweep2_steps;
-    int pad;
+    int aborted;     // a resident launch gave up waiting (its results are not valid)
     // one-reduction CG form: rho and alpha of CG step k in slot k & 1 (a step
     // reads the previous step's slot while its workgroup 0 writes its own)
     double cg_rho[2];

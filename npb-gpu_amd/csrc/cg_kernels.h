@@ -235,6 +235,52 @@ long long persistent_barriers(int cgitmax);
 hipError_t launch_persistent(const Fp64Problem &pb, const PersistentState &ps, int niter,
                              int scale_first, int record, int final_scale, hipStream_t st);
 
+// Resident CG for small orders (cg_resident.hip): the launch shape of a matrix
+// and its device buffers.
+constexpr int kResidentMaxEntries = 128;  // matrix entries of one lane at most
+struct ResidentShape {
+    int kernel = 0;     // which of the engine's kernels
+    int lpr = 0;        // lanes per row
+    int chunk = 0;      // words of a chunk: chunk - 1 rows and a partial sum
+    int words_wg = 0;   // words of a workgroup
+    int grid = 0;
+    int words = 0;      // grid * words_wg
+    int lds_bytes = 0;
+    int stride = 0;     // words of one exchange buffer
+    std::vector<int> word_row;  // row of each word, -1: none
+    std::vector<int> row_word;  // word of each row
+    std::vector<int> wave_off;  // first entry (64 lanes each) of each wavefront, and the end
+};
+struct ResidentState {
+    double *val = nullptr;
+    uint16_t *col = nullptr;
+    int *wave_off = nullptr;       // wave_off | word_row | row_word of the shape
+    int *word_row = nullptr, *row_word = nullptr;
+    double *xchg = nullptr;        // exchange buffers of one launch
+    size_t xchg_words = 0;
+    double *part = nullptr;        // resident_partials(shape, niter) doubles
+    size_t part_words = 0;
+    unsigned *abort_word = nullptr;
+    long long spin_limit = 0;      // wall-clock ticks one exchange may wait
+};
+// The shape for order n on `cus` CUs with lds_cap bytes of LDS per workgroup;
+// false where the engine does not apply (the vector does not fit the LDS, or
+// a row is longer than its lanes take).
+bool resident_shape(int n, const int *rowstr, int cus, int lds_cap, ResidentShape *out);
+hipError_t resident_capacity(const ResidentShape &s, int *per_cu);
+size_t resident_partials(const ResidentShape &s, int niter);
+// Copies the CSR into the shape's register order.
+hipError_t launch_resident_fill(const Fp64Problem &pb, const ResidentShape &s,
+                                const ResidentState &rs, hipStream_t st);
+// niter outer iterations {conj_grad of `steps` steps; rnorm, zeta, xscale} from
+// pb.x (scale_first: from xscale z of the previous call), recorded as history
+// entries first, first + 1, ... with `record`; pb.x is not written.  With
+// `solve` (niter 1) pb.x is the right-hand side and the steps stop once
+// r.r <= rtol^2 r0.r0.  sc->aborted is set if a wait ran out.
+hipError_t launch_resident(const Fp64Problem &pb, const ResidentShape &s, const ResidentState &rs,
+                           int steps, int niter, int scale_first, int first, int record,
+                           int solve, double rtol, hipStream_t st);
+
 }  // namespace npbcg_dev
 
 #endif
