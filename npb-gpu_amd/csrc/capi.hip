@@ -246,24 +246,16 @@ void drop_graph(npbcg_ctx *c) {
     }
 }
 
-int check_csr(int n, const int *rowstr, const int *colidx, long long *nnz_out,
-              bool *sorted_out) {
+int check_rowstr(int n, const int *rowstr, long long *nnz_out) {
     if (rowstr[0] != 0) return set_error(NPBCG_ERR_INVALID, "rowstr[0] must be 0");
     for (int j = 0; j < n; j++)
         if (rowstr[j + 1] < rowstr[j])
             return set_error(NPBCG_ERR_INVALID, "rowstr must be non-decreasing");
-    const long long nnz = rowstr[n];
-    bool sorted = true;
-    for (int j = 0; j < n; j++)
-        for (long long k = rowstr[j]; k < rowstr[j + 1]; k++) {
-            if (colidx[k] < 0 || colidx[k] >= n)
-                return set_error(NPBCG_ERR_INVALID, "colidx entry outside [0, n)");
-            if (k > rowstr[j] && colidx[k] <= colidx[k - 1]) sorted = false;
-        }
-    *nnz_out = nnz;
-    *sorted_out = sorted;
+    *nnz_out = rowstr[n];
     return NPBCG_OK;
 }
+
+int bad_column() { return set_error(NPBCG_ERR_INVALID, "colidx entry outside [0, n)"); }
 
 // Digest of `bytes` bytes at p (whole 8-byte words, then the tail): four
 // independent lanes h = ((h ^ w) * K) ^ (h >> 29) over the words i = lane
@@ -536,6 +528,128 @@ int read_scalars(npbcg_ctx *c, Scalars *out) {
     return NPBCG_OK;
 }
 
+// Device arrays of a SELL copy: wg_slice | slice_off | slice_row | row_slot in
+// one allocation (with room for `extra` more ints), and the block sums.
+hipError_t alloc_sell(npbcg_ctx *c, npbcg_dev::SellDev *sd, int slices, size_t extra) {
+    const size_t nwg1 = (size_t)sd->grid + 1, nsl1 = (size_t)slices + 1;
+    const size_t nrow = (size_t)slices * npbcg_detail::kSliceRows;
+    hipError_t e = hipMalloc(&c->d_sell_idx,
+                             sizeof(int) * (nwg1 + nsl1 + nrow + (size_t)sd->nblk * c->n + extra));
+    // one block sum per slot (64 per slice), stored by slot
+    if (e == hipSuccess)
+        e = hipMalloc(&c->d_rows_part, sizeof(double) * std::max<size_t>(1, nrow));
+    if (e != hipSuccess) return e;
+    sd->wg_slice = c->d_sell_idx;
+    sd->slice_off = c->d_sell_idx + nwg1;
+    sd->slice_row = c->d_sell_idx + nwg1 + nsl1;
+    sd->row_slot = c->d_sell_idx + nwg1 + nsl1 + nrow;
+    sd->slots = (long long)nrow;
+    sd->rows_part = c->d_rows_part;
+    return hipSuccess;
+}
+
+hipError_t alloc_sell_entries(npbcg_ctx *c, npbcg_dev::SellDev *sd, long long stored) {
+    const size_t count = (size_t)std::max<long long>(1, stored);
+    hipError_t e = hipMalloc(&c->d_sell_val, sizeof(double) * count);
+    if (e == hipSuccess) e = hipMalloc(&c->d_sell_col, sizeof(uint16_t) * count);
+    sd->val = c->d_sell_val;
+    sd->col = c->d_sell_col;
+    c->sell_stored = stored;
+    return e;
+}
+
+int alloc_error(hipError_t e, const char *what) {
+    return set_error(e == hipErrorOutOfMemory ? NPBCG_ERR_NOMEM : NPBCG_ERR_DEVICE,
+                     std::string(what) + ": " + hipGetErrorString(e));
+}
+
+// The SELL copy of shape *sd from the context's device CSR; sm->wg_slice is
+// set.  *ok = false if it does not fit 32-bit offsets.
+int build_sell_device(npbcg_ctx *c, npbcg_detail::SellBlocks<double> *sm,
+                      npbcg_dev::SellDev *sd, int window, int waves, bool *ok) {
+    const int n = c->n, slices = sm->wg_slice.back();
+    const size_t rows = (size_t)sd->nblk * n;
+    hipError_t e = alloc_sell(c, sd, slices, (size_t)slices);
+    if (e != hipSuccess) return alloc_error(e, "npbcg_create: SELL index");
+    int *const idx = c->d_sell_idx;
+    int *const slice_off = idx + (sd->slice_off - idx), *const slice_row = idx + (sd->slice_row - idx);
+    int *const row_slot = idx + (sd->row_slot - idx), *const src = row_slot + rows;
+    npbcg_dev::SellBuild sb;
+    sb.n = n;
+    sb.W = sd->W;
+    sb.nblk = sd->nblk;
+    sb.R = sd->R;
+    sb.nrange = sd->nrange;
+    sb.window = std::min(window, (sd->R + npbcg_detail::kSliceRows - 1) /
+                                     npbcg_detail::kSliceRows * npbcg_detail::kSliceRows);
+    sb.rowstr = c->d_rowstr;
+    sb.colidx = c->d_colidx;
+    sb.a = c->d_a;
+    sb.wg_slice = sd->wg_slice;
+    // scratch in arrays that are written last: 2 nblk - 1 ints a row fit the
+    // block sums' 2 nblk, the widths the lane rows they turn into
+    sb.order = reinterpret_cast<int *>(c->d_rows_part);
+    sb.seg = sb.order + rows;
+    sb.width = slice_row;
+    NPBCG_HIP(hipMemcpyAsync(idx, sm->wg_slice.data(), sizeof(int) * sm->wg_slice.size(),
+                             hipMemcpyHostToDevice, c->stream));
+    NPBCG_HIP(npbcg_dev::launch_sell_order(sb, c->stream));
+    std::vector<int> width((size_t)slices), place, off;
+    NPBCG_HIP(hipMemcpyAsync(width.data(), sb.width, sizeof(int) * (size_t)slices,
+                             hipMemcpyDeviceToHost, c->stream));
+    NPBCG_HIP(hipStreamSynchronize(c->stream));
+    const long long stored =
+        npbcg_detail::place_sell_slices(sm->wg_slice, width.data(), waves, &place, &off);
+    if (stored < 0) {
+        (void)hipFree(c->d_sell_idx);
+        (void)hipFree(c->d_rows_part);
+        c->d_sell_idx = nullptr;
+        c->d_rows_part = nullptr;
+        *ok = false;
+        return NPBCG_OK;
+    }
+    // sorted slice i of a workgroup -> its first row's place in `order`
+    for (int wg = 0; wg < sd->grid; wg++) {
+        const int s0 = sm->wg_slice[wg], b = wg / sd->nrange, r0 = wg % sd->nrange * sd->R;
+        for (int s = s0; s < sm->wg_slice[wg + 1]; s++)
+            place[s] = b * n + r0 + (place[s] - s0) * npbcg_detail::kSliceRows;
+    }
+    e = alloc_sell_entries(c, sd, stored);
+    if (e != hipSuccess) return alloc_error(e, "npbcg_create: SELL entries");
+    NPBCG_HIP(hipMemcpyAsync(src, place.data(), sizeof(int) * place.size(), hipMemcpyHostToDevice,
+                             c->stream));
+    NPBCG_HIP(hipMemcpyAsync(slice_off, off.data(), sizeof(int) * off.size(),
+                             hipMemcpyHostToDevice, c->stream));
+    NPBCG_HIP(npbcg_dev::launch_sell_fill(sb, src, slice_off, slices, slice_row, row_slot,
+                                          c->d_sell_val, c->d_sell_col, c->stream));
+    NPBCG_HIP(hipStreamSynchronize(c->stream));  // place and off go out of scope
+    return NPBCG_OK;
+}
+
+// A copy built on the host.
+int upload_sell(npbcg_ctx *c, const npbcg_detail::SellBlocks<double> &sm,
+                npbcg_dev::SellDev *sd) {
+    const int slices = (int)sm.slice_off.size() - 1;
+    hipError_t e = alloc_sell(c, sd, slices, 0);
+    if (e == hipSuccess) e = alloc_sell_entries(c, sd, sm.stored);
+    if (e != hipSuccess) return alloc_error(e, "npbcg_create: SELL copy");
+    auto put = [&](const int *dst, const std::vector<int> &v) {
+        return hipMemcpy(const_cast<int *>(dst), v.data(), sizeof(int) * v.size(),
+                         hipMemcpyHostToDevice);
+    };
+    NPBCG_HIP(put(sd->wg_slice, sm.wg_slice));
+    NPBCG_HIP(put(sd->slice_off, sm.slice_off));
+    NPBCG_HIP(put(sd->slice_row, sm.slice_row));
+    NPBCG_HIP(put(sd->row_slot, sm.row_slot));
+    if (!sm.val.empty()) {
+        NPBCG_HIP(hipMemcpy(c->d_sell_val, sm.val.data(), sizeof(double) * sm.val.size(),
+                            hipMemcpyHostToDevice));
+        NPBCG_HIP(hipMemcpy(c->d_sell_col, sm.col.data(), sizeof(uint16_t) * sm.col.size(),
+                            hipMemcpyHostToDevice));
+    }
+    return NPBCG_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -586,12 +700,15 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
         return set_error(NPBCG_ERR_INVALID, "npbcg_create: invalid argument");
     long long nnz = 0;
     bool sorted = true;
-    int rc = check_csr(n, rowstr, colidx, &nnz, &sorted);
+    int rc = check_rowstr(n, rowstr, &nnz);
     if (rc != NPBCG_OK) return rc;
 
     int ndev = 0;
-    if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0)
+    if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) {
+        for (long long k = 0; k < nnz; k++)
+            if (colidx[k] < 0 || colidx[k] >= n) return bad_column();
         return set_error(NPBCG_ERR_NODEVICE, "npbcg_create: no GPU device visible");
+    }
 
     npbcg_ctx *c = new (std::nothrow) npbcg_ctx();
     if (!c) return set_error(NPBCG_ERR_NOMEM, "npbcg_create: host allocation");
@@ -620,7 +737,6 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
                                                           : NPBCG_ENGINE_KERNELS;
     c->n = n;
     c->nnz = nnz;
-    c->cols_sorted = sorted;
 
     auto fail = [&](int code) {
         npbcg_destroy(c);
@@ -643,6 +759,33 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
     hipDeviceProp_t prop;
     CREATE_HIP(hipGetDeviceProperties(&prop, c->device));
     const int cus = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
+
+    // The CSR, and the check of its columns: nothing else reads them before.
+    CREATE_HIP(hipMalloc(&c->d_rowstr, sizeof(int) * ((size_t)n + 1)));
+    CREATE_HIP(hipMalloc(&c->d_colidx, sizeof(int) * std::max<long long>(1, nnz)));
+    CREATE_HIP(hipMalloc(&c->d_a, sizeof(double) * std::max<long long>(1, nnz)));
+    CREATE_HIP(hipMalloc(&c->d_sc, npbcg_dev::scalars_bytes()));
+    CREATE_HIP(hipHostMalloc(&c->h_stage,
+                             sizeof(double) * (5 * ((size_t)n + 1)) + 4096));
+    CREATE_HIP(hipMemcpyAsync(c->d_rowstr, rowstr, sizeof(int) * ((size_t)n + 1),
+                              hipMemcpyHostToDevice, c->stream));
+    if (nnz > 0) {
+        int *flags = reinterpret_cast<int *>(c->d_sc);  // scratch until the scalars are cleared
+        CREATE_HIP(hipMemcpyAsync(c->d_colidx, colidx, sizeof(int) * nnz, hipMemcpyHostToDevice,
+                                  c->stream));
+        CREATE_HIP(hipMemsetAsync(flags, 0, 2 * sizeof(int), c->stream));
+        CREATE_HIP(npbcg_dev::launch_csr_check(c->d_rowstr, c->d_colidx, n, flags, c->stream));
+        CREATE_HIP(hipMemcpyAsync(c->h_stage, flags, 2 * sizeof(int), hipMemcpyDeviceToHost,
+                                  c->stream));
+        CREATE_HIP(hipMemcpyAsync(c->d_a, a, sizeof(double) * nnz, hipMemcpyHostToDevice,
+                                  c->stream));
+        CREATE_HIP(hipStreamSynchronize(c->stream));
+        int got[2];
+        std::memcpy(got, c->h_stage, sizeof(got));
+        if (got[0]) return fail(bad_column());
+        sorted = !got[1];
+    }
+    c->cols_sorted = sorted;
 
     int variant = pick_variant(c->opts.spmv_variant, n, nnz, sorted);
     const int rpb = npbcg_dev::spmv_rows_per_block(variant);
@@ -732,30 +875,54 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
                 ? c->opts.sort_window
                 : std::min(kMaxSortWindow, std::max(npbcg_detail::kSortWindow,
                                                     (R + kSlice - 1) / kSlice * kSlice));
-        if (W * 8 > lds_budget || !sorted ||
-            !npbcg_detail::build_sell_blocks(n, rowstr, colidx, a, W, R, &sm, window,
-                                             block / 64)) {
-            variant = pick_variant(npbcg_dev::kSpmvSeg64, n, nnz, false);
-        } else {
+        const int kept_blocks = (n + W - 1) / W, kept_ranges = (n + R - 1) / R;
+        // windows the device's sort takes (in range of its keys); wider ones,
+        // which only sort_window asks for, are built on the host
+        const bool on_device = std::min(window, R) <= npbcg_dev::kSellSortRows;
+        bool built = W * 8 <= lds_budget && W <= 65536 && sorted;
+        if (built && on_device) {
+            // slices of every workgroup follow from the sizes
+            const long long slices_ll = (long long)kept_blocks *
+                                        ((long long)(kept_ranges - 1) * ((R + kSlice - 1) / kSlice) +
+                                         (n - (long long)(kept_ranges - 1) * R + kSlice - 1) / kSlice);
+            built = slices_ll * kSlice <= (long long)INT32_MAX;
+            if (built) {
+                sm.wg_slice.assign((size_t)kept_blocks * kept_ranges + 1, 0);
+                for (int wg = 0; wg < kept_blocks * kept_ranges; wg++) {
+                    const int r0 = wg % kept_ranges * R, rows = std::min(n, r0 + R) - r0;
+                    sm.wg_slice[wg + 1] = sm.wg_slice[wg] + (rows + kSlice - 1) / kSlice;
+                }
+            }
+        } else if (built) {
+            built = npbcg_detail::build_sell_blocks(n, rowstr, colidx, a, W, R, &sm, window,
+                                                    block / 64);
+        }
+        if (built) {
             c->sort_window = window;
-            sd.W = sm.W;
-            sd.nblk = sm.nblk;
-            sd.R = sm.R;
-            sd.nrange = sm.nrange;
-            sd.grid = sm.nblk * sm.nrange;
+            sd.W = W;
+            sd.nblk = kept_blocks;
+            sd.R = R;
+            sd.nrange = kept_ranges;
+            sd.grid = kept_blocks * kept_ranges;
             sd.block = block;
             int max_slices = 0;
             for (size_t w = 0; w + 1 < sm.wg_slice.size(); w++)
                 max_slices = std::max(max_slices, sm.wg_slice[w + 1] - sm.wg_slice[w]);
-            sd.lds_bytes = (sm.W + max_slices) * 8;
-            if (sd.lds_bytes > lds_budget) variant = pick_variant(npbcg_dev::kSpmvSeg64, n, nnz, false);
+            sd.lds_bytes = (W + max_slices) * 8;
+            built = sd.lds_bytes <= lds_budget;
+        }
+        if (built && on_device) {
+            rc = build_sell_device(c, &sm, &sd, window, block / 64, &built);
+            if (rc != NPBCG_OK) return fail(rc);
+        }
+        if (!built) {
+            variant = pick_variant(npbcg_dev::kSpmvSeg64, n, nnz, false);
+            sd = npbcg_dev::SellDev{};
+            sm = npbcg_detail::SellBlocks<double>{};
         }
     }
 
     c->vstride = ((size_t)n + 2 + 63) & ~(size_t)63;
-    CREATE_HIP(hipMalloc(&c->d_rowstr, sizeof(int) * ((size_t)n + 1)));
-    CREATE_HIP(hipMalloc(&c->d_colidx, sizeof(int) * std::max<long long>(1, nnz)));
-    CREATE_HIP(hipMalloc(&c->d_a, sizeof(double) * std::max<long long>(1, nnz)));
     CREATE_HIP(hipMalloc(&c->d_vec, sizeof(double) * kNumVectors * c->vstride));
     c->part_vec = vec_blocks;
     c->part_spmv = variant == npbcg_dev::kSpmvTiled ? std::max(sd.grid, vec_blocks)
@@ -764,50 +931,10 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
                          sizeof(double) * (7 * (size_t)c->part_vec + 4 * (size_t)c->part_spmv)));
     if (variant == npbcg_dev::kSpmvTiled) {
         CREATE_HIP(npbcg_dev::prepare_sell_kernels(sd.lds_bytes));
-        const size_t nwg1 = sm.wg_slice.size(), nsl1 = sm.slice_off.size();
-        const size_t nrow = sm.slice_row.size();
-        const size_t idx = nwg1 + nsl1 + nrow + sm.row_slot.size();
-        CREATE_HIP(hipMalloc(&c->d_sell_idx, sizeof(int) * idx));
-        CREATE_HIP(hipMalloc(&c->d_sell_val, sizeof(double) * std::max<size_t>(1, sm.val.size())));
-        CREATE_HIP(hipMalloc(&c->d_sell_col,
-                             sizeof(uint16_t) * std::max<size_t>(1, sm.col.size())));
-        // one block sum per slot (64 per slice), stored by slot
-        CREATE_HIP(hipMalloc(&c->d_rows_part, sizeof(double) * std::max<size_t>(1, nrow)));
-        CREATE_HIP(hipMemcpy(c->d_sell_idx, sm.wg_slice.data(), sizeof(int) * nwg1,
-                             hipMemcpyHostToDevice));
-        CREATE_HIP(hipMemcpy(c->d_sell_idx + nwg1, sm.slice_off.data(), sizeof(int) * nsl1,
-                             hipMemcpyHostToDevice));
-        CREATE_HIP(hipMemcpy(c->d_sell_idx + nwg1 + nsl1, sm.slice_row.data(),
-                             sizeof(int) * nrow, hipMemcpyHostToDevice));
-        CREATE_HIP(hipMemcpy(c->d_sell_idx + nwg1 + nsl1 + nrow, sm.row_slot.data(),
-                             sizeof(int) * sm.row_slot.size(), hipMemcpyHostToDevice));
-        if (!sm.val.empty()) {
-            CREATE_HIP(hipMemcpy(c->d_sell_val, sm.val.data(), sizeof(double) * sm.val.size(),
-                                 hipMemcpyHostToDevice));
-            CREATE_HIP(hipMemcpy(c->d_sell_col, sm.col.data(),
-                                 sizeof(uint16_t) * sm.col.size(), hipMemcpyHostToDevice));
+        if (!c->d_sell_idx) {  // built on the host
+            rc = upload_sell(c, sm, &sd);
+            if (rc != NPBCG_OK) return fail(rc);
         }
-        sd.wg_slice = c->d_sell_idx;
-        sd.slice_off = c->d_sell_idx + nwg1;
-        sd.slice_row = c->d_sell_idx + nwg1 + nsl1;
-        sd.row_slot = c->d_sell_idx + nwg1 + nsl1 + nrow;
-        sd.slots = (long long)nrow;
-        sd.val = c->d_sell_val;
-        sd.col = c->d_sell_col;
-        sd.rows_part = c->d_rows_part;
-        c->sell_stored = sm.stored;
-    }
-    CREATE_HIP(hipMalloc(&c->d_sc, npbcg_dev::scalars_bytes()));
-    CREATE_HIP(hipHostMalloc(&c->h_stage,
-                             sizeof(double) * (5 * ((size_t)n + 1)) + 4096));
-
-    CREATE_HIP(hipMemcpyAsync(c->d_rowstr, rowstr, sizeof(int) * ((size_t)n + 1),
-                              hipMemcpyHostToDevice, c->stream));
-    if (nnz > 0) {
-        CREATE_HIP(hipMemcpyAsync(c->d_colidx, colidx, sizeof(int) * nnz,
-                                  hipMemcpyHostToDevice, c->stream));
-        CREATE_HIP(hipMemcpyAsync(c->d_a, a, sizeof(double) * nnz, hipMemcpyHostToDevice,
-                                  c->stream));
     }
     CREATE_HIP(hipMemsetAsync(c->d_vec, 0, sizeof(double) * kNumVectors * c->vstride, c->stream));
     CREATE_HIP(hipMemsetAsync(c->d_sc, 0, npbcg_dev::scalars_bytes(), c->stream));

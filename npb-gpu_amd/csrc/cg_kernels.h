@@ -39,6 +39,30 @@ struct SellDev {
     int lds_bytes = 0;  // dynamic LDS: W vector entries + one double per slice
 };
 
+// Device construction of the SELL copy (sell_build.hip).
+constexpr int kSellSortBits = 13;
+constexpr int kSellSortRows = 1 << kSellSortBits;  // widest sort window it takes
+struct SellBuild {
+    int n = 0, W = 0, nblk = 0, R = 0, nrange = 0;
+    int window = 0;                 // rows sorted together, at most kSellSortRows
+    const int *rowstr = nullptr, *colidx = nullptr;  // CSR, columns ascending
+    const double *a = nullptr;
+    const int *wg_slice = nullptr;  // [nblk * nrange + 1]
+    int *seg = nullptr;             // [(nblk - 1) * n] bounds between blocks, by row
+    int *order = nullptr;           // [nblk * n] rows of each window, longest first
+    int *width = nullptr;           // [slices] in that order
+};
+// flags (two ints, zero before): [0] set if a column lies outside [0, n),
+// [1] if a row's columns do not ascend.
+hipError_t launch_csr_check(const int *rowstr, const int *colidx, int n, int *flags,
+                            hipStream_t st);
+// seg, order and width; then, with the slices placed (slice s at slice_off[s],
+// its rows from order[src[s]] on), the copy itself.
+hipError_t launch_sell_order(const SellBuild &sb, hipStream_t st);
+hipError_t launch_sell_fill(const SellBuild &sb, const int *src, const int *slice_off, int slices,
+                            int *slice_row, int *row_slot, double *val, uint16_t *col,
+                            hipStream_t st);
+
 // Per-workgroup partial sums handed from one kernel to the next.
 struct Partials {
     double *xx;      // x.x of cg_init            [vec_blocks]

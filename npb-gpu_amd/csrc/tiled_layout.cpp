@@ -91,6 +91,35 @@ void place_slices(const std::vector<int> &width, int waves, std::vector<int> *po
     }
 }
 
+}  // namespace
+
+long long place_sell_slices(const std::vector<int> &wg_slice, const int *width, int waves,
+                            std::vector<int> *src, std::vector<int> *slice_off) {
+    const int nwg = (int)wg_slice.size() - 1, slices = wg_slice[nwg];
+    src->resize((size_t)slices);
+    slice_off->assign((size_t)slices + 1, 0);
+    auto place = [&](int wg) {
+        const int s0 = wg_slice[wg], nsl = wg_slice[wg + 1] - s0;
+        std::vector<int> w(width + s0, width + s0 + nsl), pos;
+        place_slices(w, waves, &pos);
+        for (int i = 0; i < nsl; i++) (*src)[(size_t)s0 + pos[i]] = s0 + i;
+    };
+    if (slices < 32768) {  // not worth starting threads for
+        for (int wg = 0; wg < nwg; wg++) place(wg);
+    } else {
+        parallel_items(nwg, place);
+    }
+    long long off = 0;
+    for (int s = 0; s < slices; s++) {
+        off += (long long)kSliceRows * width[(*src)[s]];
+        if (off > (long long)INT32_MAX) return -1;
+        (*slice_off)[(size_t)s + 1] = (int)off;
+    }
+    return off;
+}
+
+namespace {
+
 template <class V>
 bool build_impl(int n, const int *rowstr, const int *colidx, const double *a, int W, int R,
                 int window, int waves, SellBlocks<V> *out) {

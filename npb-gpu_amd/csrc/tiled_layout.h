@@ -59,6 +59,13 @@ bool build_sell_blocks(int n, const int *rowstr, const int *colidx, const double
                        int W, int R, SellBlocks<float> *out, int window = kSortWindow,
                        int waves = 0);
 
+// Places the slices of a copy whose widths are known (wg_slice as above,
+// width[s] of the slices in sorted order): src[s] is the sorted slice at
+// position s of its workgroup, slice_off its offset (one more than slices).
+// Returns the entries stored, padding included, or -1 past 32-bit offsets.
+long long place_sell_slices(const std::vector<int> &wg_slice, const int *width, int waves,
+                            std::vector<int> *src, std::vector<int> *slice_off);
+
 }  // namespace npbcg_detail
 
 #endif
