@@ -793,10 +793,23 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
     const int spmv_blocks = std::max(1, std::min((n + rpb - 1) / rpb, 4 * cus));
 
     // Column-blocked SELL copy for the LDS-staged SpMV.  One column block of
-    // the vector must fit the CU's LDS: the widest blocks (fewest partial
-    // sums) take one 1024-thread workgroup per CU; blocks that fit twice use
-    // 512-thread workgroups, two per CU.  Row ranges spread the
+    // the vector must fit the CU's LDS: past 6 of the widest blocks (fewest
+    // partial sums) one 1024-thread workgroup per CU, or, for blocks given so
+    // narrow that they fit twice, two of 512 threads.  Row ranges spread the
     // nblk * nrange workgroups evenly over the CUs.
+    //
+    // Up to 6 of the widest blocks (n <= 121344 with 160 KB) 6 blocks are
+    // taken all the same, and ranges of whole 64-row slices, one workgroup per
+    // CU: fewer blocks mean shorter ranges, whose last slice is mostly padding
+    // (1.99 entries stored per nonzero in 79-row ranges at n = 20000), and a
+    // longer block for every workgroup to stage.  FP64 step of the power loop /
+    // FP32 product, us, before and with 6 blocks: n = 8009 25.7 / 20.0 and
+    // 11.3 / 7.0, 20000 27.0 / 22.0 and 15.4 / 8.2, 30011 19.1 / 10.7 and 15.3 /
+    // 7.9, 60013 26.4 / 15.9 and 25.1 / 13.1, 75000 32.0 / 17.9 and 31.9 / 16.5;
+    // 4, 5, 7 and 8 blocks are within 5 % of 6 and better at some orders only;
+    // two workgroups per CU are 5 to 15 % slower.  Up to 16 slices 8 wavefronts
+    // take two each (15.3 us at 30011, 16.4 with 16 wavefronts); past that 16
+    // wavefronts share the rest better (21.5 against 22.5 us at 45000).
     npbcg_detail::SellBlocks<double> sm;
     npbcg_dev::SellDev sd;
     if (variant == npbcg_dev::kSpmvTiled) {
@@ -805,12 +818,16 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
                                   c->device) != hipSuccess || lds_cap <= 0)
             lds_cap = 64 * 1024;
         const int lds_budget = lds_cap - 2048;  // static LDS of the reduction epilogue
+        constexpr int kMidBlocks = 6;
         int W;
+        bool mid = false;
         if (c->opts.tile_width > 0) {
             W = c->opts.tile_width;
         } else {
             const int wmax = std::min(65536, lds_budget / 8);
-            const int nblk = (n + wmax - 1) / wmax;
+            int nblk = (n + wmax - 1) / wmax;
+            mid = nblk <= kMidBlocks && c->opts.tile_rows <= 0 && cus >= kMidBlocks;
+            if (mid) nblk = kMidBlocks;
             W = (n + nblk - 1) / nblk;
         }
         W = std::max(2, (W + 1) & ~1);
@@ -823,12 +840,18 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
             return (int)(((long long)n + nrange - 1) / nrange);
         };
         int R = c->opts.tile_rows > 0 ? c->opts.tile_rows : default_rows();
+        const int kSlice = npbcg_detail::kSliceRows;
+        if (mid) {
+            const int nrange = cus / kMidBlocks;
+            const int slices = ((n + nrange - 1) / nrange + kSlice - 1) / kSlice;
+            R = slices * kSlice;
+            block = slices <= 16 ? 512 : 1024;
+        }
         // The per-slice p.q slots (one double per 64-row slice of a workgroup)
         // share the LDS with the vector block.  When the range's slices do not
         // fit beside the block (large n: few ranges of many rows), the block
         // is narrowed to 7/8 of the LDS and the range capped at the slices
         // the rest holds: more, shorter workgroups instead of the CSR kernel.
-        const int kSlice = npbcg_detail::kSliceRows;
         if ((long long)(W + (R + kSlice - 1) / kSlice) * 8 > lds_budget) {
             if (c->opts.tile_width <= 0) {
                 const int wcap = (lds_budget / 8) * 7 / 8;
