@@ -6,7 +6,6 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
-#include <functional>
 #include <limits>
 #include <mutex>
 #include <string>
@@ -151,14 +150,6 @@ struct npbcg_ctx {
     // batch; mixed inner steps of sweeps 1, 2
     int budget[2][4][2] = {};
 
-    // captured solve sequences, one per mode; replayed while the key matches
-    struct SolveGraph {
-        hipGraph_t g = nullptr;
-        hipGraphExec_t ex = nullptr;
-        int kind = -1, maxit = 0, batch = 0;
-        double rtol = 0.0, rhs = 0.0;
-    } solve_graph[2];
-
     // residual/correction pairs (lazy)
     struct Pairs {
         int count = 0;
@@ -180,6 +171,8 @@ constexpr int kMaxSortWindow = 8192;
 constexpr size_t kResidentWords = (size_t)8 << 20;
 // Steps of a resident solve launch at most.
 constexpr int kResidentSolveSteps = 64;
+// Entries of a right-hand side copied and sent at a time.
+constexpr int kRhsPiece = 32768;
 constexpr int kVecPAlt = 5, kVecB = 6, kVecXsol = 7;
 
 namespace {
@@ -1045,10 +1038,6 @@ void npbcg_destroy(npbcg_ctx *c) {
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     drop_graph(c);
-    for (auto &sg : c->solve_graph) {
-        if (sg.ex) (void)hipGraphExecDestroy(sg.ex);
-        if (sg.g) (void)hipGraphDestroy(sg.g);
-    }
     for (auto e : c->probe_start) (void)hipEventDestroy(e);
     for (auto e : c->probe_stop) (void)hipEventDestroy(e);
     if (c->ev_start) (void)hipEventDestroy(c->ev_start);
@@ -1720,11 +1709,17 @@ int ensure_mixed(npbcg_ctx *c) {
     return NPBCG_OK;
 }
 
-int read_scalars_from(npbcg_ctx *c, const Scalars *dev, Scalars *out) {
-    NPBCG_HIP(hipMemcpyAsync(c->h_stage, dev, sizeof(Scalars), hipMemcpyDeviceToHost,
-                             c->stream));
+// One or two sets of device scalars, once the stream has run what it holds.
+int read_scalars_from(npbcg_ctx *c, const Scalars *dev, Scalars *out,
+                      const Scalars *dev2 = nullptr, Scalars *out2 = nullptr) {
+    Scalars *stage = reinterpret_cast<Scalars *>(c->h_stage);
+    NPBCG_HIP(hipMemcpyAsync(stage, dev, sizeof(Scalars), hipMemcpyDeviceToHost, c->stream));
+    if (dev2)
+        NPBCG_HIP(hipMemcpyAsync(stage + 1, dev2, sizeof(Scalars), hipMemcpyDeviceToHost,
+                                 c->stream));
     NPBCG_HIP(hipStreamSynchronize(c->stream));
-    std::memcpy(out, c->h_stage, sizeof(Scalars));
+    std::memcpy(out, stage, sizeof(Scalars));
+    if (dev2) std::memcpy(out2, stage + 1, sizeof(Scalars));
     return NPBCG_OK;
 }
 
@@ -1733,12 +1728,27 @@ int read_scalars_from(npbcg_ctx *c, const Scalars *dev, Scalars *out) {
 int npbcg_set_rhs(npbcg_ctx *c, const double *b) {
     if (!c || !b) return set_error(NPBCG_ERR_INVALID, "npbcg_set_rhs: NULL argument");
     NPBCG_HIP(hipSetDevice(c->device));
-    double s = 0.0;
-    for (int j = 0; j < c->n; j++) s += b[j] * b[j];
-    c->rhs_norm = std::sqrt(s);
-    const size_t bytes = sizeof(double) * (size_t)c->n;
-    std::memcpy(c->h_stage, b, bytes);
-    NPBCG_HIP(hipMemcpyAsync(c->pbs.x, c->h_stage, bytes, hipMemcpyHostToDevice, c->stream));
+    // Staged and sent in pieces, the next one squared and copied while the last
+    // one is on its way; eight sums, so that no addition waits for the last.
+    double s[8] = {};
+    for (int j0 = 0; j0 < c->n; j0 += kRhsPiece) {
+        const int count = std::min(kRhsPiece, c->n - j0);
+        const double *from = b + j0;
+        double *to = c->h_stage + j0;
+        int j = 0;
+        for (; j + 8 <= count; j += 8)
+            for (int u = 0; u < 8; u++) {
+                to[j + u] = from[j + u];
+                s[u] += from[j + u] * from[j + u];
+            }
+        for (; j < count; j++) {
+            to[j] = from[j];
+            s[0] += from[j] * from[j];
+        }
+        NPBCG_HIP(hipMemcpyAsync(c->pbs.x + j0, to, sizeof(double) * (size_t)count,
+                                 hipMemcpyHostToDevice, c->stream));
+    }
+    c->rhs_norm = std::sqrt(((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7])));
     NPBCG_HIP(hipStreamSynchronize(c->stream));
     clear_error();
     return NPBCG_OK;
@@ -2121,9 +2131,7 @@ int npbcg_solve(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stat
     if (c->precond == NPBCG_PRECOND_LEARNED &&
         (rc == NPBCG_ERR_NOCONV || !(s.relres == s.relres))) {
         // The learned operator did not get there: Jacobi-CG redoes the solve
-        // from x = 0.  The solve views now point at the Jacobi diagonal, and the
-        // captured solve sequences are keyed by the preconditioner in effect,
-        // so nothing of the learned sequence is replayed.
+        // from x = 0.
         const double first_ms = s.time_ms;
         rc = select_precond(c, NPBCG_PRECOND_JACOBI);
         if (rc != NPBCG_OK) return rc;
@@ -2137,51 +2145,6 @@ int npbcg_solve(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stat
 }
 
 namespace {
-
-// Runs the first stretch of a solve: replays its captured graph when the
-// key (mode, preconditioner in effect, rtol, maxit, batch, ||b||) matches the
-// last capture, else captures `enqueue` anew (or, with use_graph = 0,
-// launches it directly).  The preconditioner in effect decides which
-// buffers the captured kernels read (Jacobi diagonal or sparse operator).
-int run_solve_sequence(npbcg_ctx *c, int mode, double rtol, int maxit, int batch,
-                       const std::function<hipError_t()> &enqueue) {
-    if (!c->opts.use_graph) {
-        NPBCG_HIP(enqueue());
-        return NPBCG_OK;
-    }
-    auto &sg = c->solve_graph[mode];
-    if (!(sg.ex && sg.kind == c->active_precond && sg.rtol == rtol && sg.maxit == maxit &&
-          sg.batch == batch && sg.rhs == c->rhs_norm)) {
-        if (sg.ex) (void)hipGraphExecDestroy(sg.ex);
-        if (sg.g) (void)hipGraphDestroy(sg.g);
-        sg = npbcg_ctx::SolveGraph{};
-        NPBCG_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        hipError_t e = enqueue();
-        hipGraph_t g = nullptr;
-        hipError_t e2 = hipStreamEndCapture(c->stream, &g);
-        if (e != hipSuccess || e2 != hipSuccess) {
-            if (g) (void)hipGraphDestroy(g);
-            return set_error(NPBCG_ERR_DEVICE, std::string("solve graph capture failed: ") +
-                                                   hipGetErrorString(e != hipSuccess ? e : e2));
-        }
-        hipGraphExec_t ex = nullptr;
-        hipError_t e3 = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-        if (e3 != hipSuccess) {
-            (void)hipGraphDestroy(g);
-            return set_error(NPBCG_ERR_DEVICE, std::string("hipGraphInstantiate: ") +
-                                                   hipGetErrorString(e3));
-        }
-        sg.g = g;
-        sg.ex = ex;
-        sg.kind = c->active_precond;
-        sg.rtol = rtol;
-        sg.maxit = maxit;
-        sg.batch = batch;
-        sg.rhs = c->rhs_norm;
-    }
-    NPBCG_HIP(hipGraphLaunch(sg.ex, c->stream));
-    return NPBCG_OK;
-}
 
 int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats *st) {
     if (!c || !(rtol > 0.0) || maxit < 1 ||
@@ -2222,7 +2185,9 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
         const int res_steps = std::min(maxit, kResidentSolveSteps);
         const bool resident = c->active_precond == NPBCG_PRECOND_NONE &&
                               c->opts.solve_batch <= 0 && use_resident(c, res_steps);
-        // first batch: reset, init, `batch` steps, residual (captured once per key)
+        // First batch: reset, init, `batch` steps, residual.  Launched as they
+        // are: a captured graph of them replays no faster (n = 150000: 653
+        // against 645 us, 17003: 191 against 194) and costs 150 us to make.
         auto first_batch = [&]() -> hipError_t {
             hipError_t e = npbcg_dev::launch_reset_scalars(pbs, 0.0, c->stream, rtol, 1);
             if (e == hipSuccess) e = npbcg_dev::launch_cg_init(pbs, 0, c->stream);
@@ -2241,8 +2206,7 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
             NPBCG_HIP(npbcg_dev::launch_resident(pbs, c->rshape, c->rstate, res_steps, 1, 0, 0, 0,
                                                  1, rtol, c->stream));
         } else {
-            int rc = run_solve_sequence(c, 0, rtol, maxit, batch, first_batch);
-            if (rc != NPBCG_OK) return rc;
+            NPBCG_HIP(first_batch());
         }
         for (;;) {
             if (!first) {
@@ -2255,8 +2219,7 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
             if (rc != NPBCG_OK) return rc;
             if (first && resident && sc.aborted) {  // b is untouched: start over without it
                 c->rshape.grid = 0;
-                rc = run_solve_sequence(c, 0, rtol, maxit, batch, first_batch);
-                if (rc != NPBCG_OK) return rc;
+                NPBCG_HIP(first_batch());
                 NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
                 rc = read_scalars_from(c, pbs.sc, &sc);
                 if (rc != NPBCG_OK) return rc;
@@ -2307,16 +2270,13 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
             return e;
         };
         NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
-        int rc0 = run_solve_sequence(c, 1, rtol, maxit, b1 * 1000 + b2, first_two);
-        if (rc0 != NPBCG_OK) return rc0;
+        NPBCG_HIP(first_two());
         int enqueued = 2, inner_steps = 0, si_last_steps = 0;
         for (bool first = true;; first = false) {
             if (!first) NPBCG_HIP(sweep(enqueued++));
             NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
             Scalars si{};
-            int rc = read_scalars_from(c, mp.sc, &si);
-            if (rc != NPBCG_OK) return rc;
-            rc = read_scalars_from(c, pbs.sc, &sc);
+            int rc = read_scalars_from(c, pbs.sc, &sc, mp.sc, &si);
             if (rc != NPBCG_OK) return rc;
             inner_steps = sc.inner_total + si.steps;
             si_last_steps = si.steps;
