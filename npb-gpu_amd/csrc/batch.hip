@@ -7,7 +7,10 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
+#include <queue>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "batch_kernels.h"
@@ -33,12 +36,10 @@ using npbcg_detail::set_error;
 // Host metadata of one SELL copy of the batch.
 struct SellHost {
     int W = 0;                          // column block width
+    int split = 0;                      // windows of kSellWindow >> split rows
     std::vector<int> nb;                // blocks per system
     std::vector<std::vector<int>> wg;   // per system: global first slice of each
                                         // (block, window), block-major, + end
-    std::vector<int> nrange;            // windows per system
-    std::vector<long long> part;        // per system: first row partial (elements)
-    long long part_total = 0;
     std::vector<int> off;               // [slices + 1] first entry of each slice
 };
 
@@ -76,10 +77,8 @@ struct npbcg_batch {
     void *d_sell_val = nullptr;
     uint16_t *d_sell_col = nullptr;
     int *d_sell_off = nullptr, *d_sell_row = nullptr;
-    int *d_block_item = nullptr;     // workgroup lists of the SELL SpMM (sell_wg_lists)
+    int *d_block_item = nullptr;     // workgroup lists and items of the SELL SpMM (sell_plan)
     size_t block_item_cap = 0;
-    int *d_item_sl = nullptr;        // slice ranges of the SELL items (make_sell_items)
-    size_t item_sl_cap = 0;
     // FP64 SELL copy of the true residual: in FP64 mode the inner copy itself
     // (aliased), in MIXED mode a copy of its own with blocks sized for FP64
     // vectors.  Items are one sorting window each.
@@ -88,12 +87,9 @@ struct npbcg_batch {
     double *d_res_val = nullptr;
     uint16_t *d_res_col = nullptr;
     int *d_res_off = nullptr, *d_res_row = nullptr;
-    int *d_res_items = nullptr;      // [items][4]
-    int *d_res_sys = nullptr;        // sys_item | sys_row | sys_nb
-    long long *d_res_part = nullptr; // sys_part
+    int *d_res_sys = nullptr;        // sys_item
     int *d_res_block_item = nullptr;
-    int *d_res_item_sl = nullptr;
-    int res_items = 0, res_item_blocks = 0;
+    int res_item_blocks = 0;
     int *d_flags = nullptr;          // done
     BatchScalars *d_sc = nullptr;
     double *d_b = nullptr, *d_x = nullptr, *d_res = nullptr;   // [rows][nr]
@@ -185,101 +181,165 @@ int upload_order(npbcg_batch *b, const std::vector<int> &order, int **buf, size_
 // Rows per tile of the vector kernels under the SELL layout.
 constexpr int kSellTileRows = 256;
 
-// SELL items, one per sorting window: (system, first local row, rows, offset
-// into *item_sl), in system order, and the first item of each system.
-// item_sl holds, for each item, the window's slice range [first, end) in
-// each column block of its system.
-void make_sell_items(const SellHost &h, const std::vector<int> &n, std::vector<int> *items,
-                     std::vector<int> *sys_item, std::vector<int> *item_sl) {
-    const int nsys = (int)n.size();
-    items->clear();
-    item_sl->clear();
-    sys_item->assign(nsys + 1, 0);
-    for (int s = 0; s < nsys; s++) {
-        (*sys_item)[s] = (int)(items->size() / 4);
-        const int nw = h.nrange[s];
-        const std::vector<int> &wg = h.wg[s];
-        for (int r = 0; r < nw; r++) {
-            items->push_back(s);
-            items->push_back(r * kSellWindow);
-            items->push_back(std::min(kSellWindow, n[s] - r * kSellWindow));
-            items->push_back((int)item_sl->size());
-            for (int blk = 0; blk < h.nb[s]; blk++) {
-                item_sl->push_back(wg[(size_t)blk * nw + r]);
-                item_sl->push_back(wg[(size_t)blk * nw + r + 1]);
+// Workgroup lists of the SELL SpMM.  The launch has one workgroup per CU
+// (each holds a vector block and a window's row sums), kXcds * per_xcd in all;
+// workgroup g walks its list (backwards when the launch reverses its order),
+// so no workgroup is dispatched per item and no dispatch slot is left empty.
+// The items go, heaviest first, to the least loaded workgroup (longest
+// processing time first): over all workgroups, or, when that ends no later and
+// there are at least kXcds systems, with whole systems on one XCD (greedy by
+// cost, largest first; workgroup g runs on XCD g % kXcds), so a system's vector
+// blocks are read through one XCD's L2.  (176000 rows in 8 systems from 4000 to
+// 40000, four FP64 right-hand sides: 169 us on XCDs, 94 us over all.)
+// Returns the load of the fullest workgroup; lists[g] are indices into cost.
+double sell_wg_lists(const npbcg_batch *b, const std::vector<int> &sys_item,
+                     const std::vector<double> &cost, std::vector<std::vector<int>> *lists) {
+    const int nsys = b->nsys, per_xcd = std::max(1, b->cus / kXcds), G = kXcds * per_xcd;
+    double best = 0.0;
+    for (int pools : {1, kXcds}) {
+        if (pools > 1 && nsys < kXcds) continue;
+        std::vector<std::pair<double, int>> sys(nsys);  // (-cost, system)
+        for (int s = 0; s < nsys; s++) {
+            sys[s] = {0.0, s};
+            for (int it = sys_item[s]; it < sys_item[s + 1]; it++) sys[s].first -= cost[it];
+        }
+        std::sort(sys.begin(), sys.end());
+        std::vector<std::vector<int>> pool(pools);
+        std::vector<double> xload(pools, 0.0);
+        for (const auto &[negative, s] : sys) {
+            const int x = (int)(std::min_element(xload.begin(), xload.end()) - xload.begin());
+            xload[x] -= negative;
+            for (int it = sys_item[s]; it < sys_item[s + 1]; it++) pool[x].push_back(it);
+        }
+        std::vector<std::vector<int>> out(G);
+        double fullest = 0.0;
+        for (int x = 0; x < pools; x++) {
+            std::stable_sort(pool[x].begin(), pool[x].end(),
+                             [&](int p, int q) { return cost[p] > cost[q]; });
+            typedef std::pair<double, int> Load;  // (load, workgroup), least first
+            std::priority_queue<Load, std::vector<Load>, std::greater<Load>> heap;
+            for (int g = x; g < G; g += pools) heap.push({0.0, g});
+            for (int it : pool[x]) {
+                Load l = heap.top();
+                heap.pop();
+                l.first += cost[it];
+                out[l.second].push_back(it);
+                fullest = std::max(fullest, l.first);
+                heap.push(l);
             }
         }
+        if (pools == 1 || fullest <= best) {
+            best = fullest;
+            lists->swap(out);
+        }
     }
-    (*sys_item)[nsys] = (int)(items->size() / 4);
+    return best;
 }
 
-// Workgroup lists of the SELL SpMM.  The launch has one workgroup per CU
-// (each holds a vector block and a window's row sums), kXcds * per_xcd in all; workgroup g
-// walks the items first[g] .. first[g + 1] - 1 of the list (backwards when
-// the launch reverses its order), so no workgroup is dispatched per item and
-// no dispatch slot is left empty.  With at least kXcds systems, whole
-// systems go to XCDs (greedy by cost, largest first; workgroup g runs on XCD
-// g % kXcds), so a system's vector blocks are read through one XCD's L2.
-// Inside an XCD (over all workgroups with fewer systems) the items go,
-// heaviest first, to the least loaded workgroup (longest processing time
-// first).  An item costs its stored entries (value and 16-bit column), the
-// vector blocks it stages, its rows' q and p, and a fixed 16 KB per block for
-// the fill and the start of the block's pipeline.
-// *out = first[0 .. G] | items.
-void sell_wg_lists(const npbcg_batch *b, const SellHost &h, const std::vector<int> &items,
-                   const std::vector<int> &sys_item, const std::vector<int> &item_sl, int elem,
-                   std::vector<int> *out) {
-    const int nsys = b->nsys, per_xcd = std::max(1, b->cus / kXcds), G = kXcds * per_xcd;
-    const int ni = sys_item[nsys];
-    std::vector<double> cost(ni), sys_cost(nsys, 0.0);
-    for (int s = 0; s < nsys; s++)
-        for (int it = sys_item[s]; it < sys_item[s + 1]; it++) {
-            const int nrows = items[4 * it + 2], so = items[4 * it + 3];
+// What an item costs, in bytes streamed by one CU: its stored entries (value and
+// 16-bit column), the vector blocks it stages, its rows' q and p, and 48 KB per
+// block for the fill and the start of the block's pipeline (fitted to launches
+// of 15 to 5000 items; 25 to 28 KB take a microsecond).
+double item_cost(const npbcg_batch *b, double stored, int n, int nrows, int W, int elem) {
+    return stored * (elem + 2.0) + (double)(n + 2 * nrows) * b->nr * elem +
+           49152.0 * ((n + W - 1) / W);
+}
+
+// First item of each system when every window of kSellWindow >> split rows is one.
+std::vector<int> first_items(const npbcg_batch *b, int split) {
+    const int H = kSellWindow >> split;
+    std::vector<int> first(b->nsys + 1, 0);
+    for (int s = 0; s < b->nsys; s++) first[s + 1] = first[s] + (b->n[s] + H - 1) / H;
+    return first;
+}
+
+// The split of a SELL copy of W-column blocks: windows of kSellWindow >> split
+// rows, whose slices' entries are cut into 1 << split parts so that 16
+// wavefronts share 32 units of work either way.  Whole windows are the least work
+// (every window stages the system's vector, and few rows sort into slices with
+// more padding), but a batch of few rows leaves most CUs without one: the split
+// taken is the one whose fullest workgroup has the least to do.  SpMM, whole
+// windows and as chosen: 30000 rows in 6 systems, one FP64 right-hand side
+// 62.8 and 14.4 us; 11000 rows in 2, four FP32 ones 37.6 and 11.7; 176000 in 8,
+// four FP64 ones 137 and 90; 336000 in 16, four FP32 ones 65.8 and 58.4 us (whole
+// windows are 172 items for 256 CUs).
+int sell_split(const npbcg_batch *b, int W, int elem, const std::vector<int> &rp) {
+    const double padded[] = {1.03, 1.04, 1.06, 1.09, 1.15, 1.25};
+    const int G = kXcds * std::max(1, b->cus / kXcds);
+    int best = 0;
+    double best_load = 0.0;
+    for (int split = 0; split < 6; split++) {
+        const int H = kSellWindow >> split;
+        const std::vector<int> first = first_items(b, split);
+        if (split > 0 && first[b->nsys] > 16 * G) break;  // enough for every CU
+        std::vector<double> cost;
+        for (int s = 0; s < b->nsys; s++)
+            for (int r = 0; r < b->n[s]; r += H) {
+                const int rows = std::min(H, b->n[s] - r), at = b->row_off[s] + r;
+                cost.push_back(item_cost(b, padded[split] * (rp[at + rows] - rp[at]), b->n[s],
+                                         rows, W, elem));
+            }
+        std::vector<std::vector<int>> lists;
+        const double load = sell_wg_lists(b, first, cost, &lists);
+        if (split == 0 || load < best_load) {
+            best_load = load;
+            best = split;
+        }
+    }
+    return best;
+}
+
+// Items of a SELL copy and their workgroup lists, as the kernel reads them: the
+// list offsets (padded to whole items), then the lists.  *sys_item: first item
+// of each system; *blocks: workgroups.
+void sell_plan(const npbcg_batch *b, const SellHost &h, int elem, std::vector<int> *sys_item,
+               std::vector<int> *plan, int *blocks) {
+    const int H = kSellWindow >> h.split;
+    *sys_item = first_items(b, h.split);
+    std::vector<SellItem> items;
+    std::vector<double> cost;
+    for (int s = 0; s < b->nsys; s++) {
+        const std::vector<int> &wg = h.wg[s];
+        const int nw = (b->n[s] + H - 1) / H;
+        for (int r = 0; r < nw; r++) {
+            SellItem it;
+            it.sys = s;
+            it.index = (int)items.size();
+            it.row = b->row_off[s] + r * H;
+            it.rows = std::min(H, b->n[s] - r * H);
+            it.sys_row = b->row_off[s];
+            it.n = b->n[s];
+            it.first = wg[r];
+            it.stride = wg[nw] - wg[0];
             double stored = 0.0;
             for (int blk = 0; blk < h.nb[s]; blk++)
-                stored += (double)h.off[item_sl[so + 2 * blk + 1]] - (double)h.off[item_sl[so + 2 * blk]];
-            cost[it] = stored * (elem + 2.0) + (double)(b->n[s] + 2 * nrows) * b->nr * elem +
-                       16384.0 * h.nb[s];
-            sys_cost[s] += cost[it];
-        }
-    std::vector<int> order(nsys);
-    for (int s = 0; s < nsys; s++) order[s] = s;
-    std::stable_sort(order.begin(), order.end(),
-                     [&](int x, int y) { return sys_cost[x] > sys_cost[y]; });
-    // items of each XCD (one pool over all workgroups with fewer systems)
-    const int pools = nsys >= kXcds ? kXcds : 1;
-    std::vector<std::vector<int>> pool(pools);
-    std::vector<double> xload(kXcds, 0.0);
-    for (int s : order) {
-        int x = 0;
-        if (pools > 1) {
-            x = (int)(std::min_element(xload.begin(), xload.end()) - xload.begin());
-            xload[x] += sys_cost[s];
-        }
-        for (int it = sys_item[s]; it < sys_item[s + 1]; it++) pool[x].push_back(it);
-    }
-    std::vector<std::vector<int>> lists(G);
-    std::vector<double> load(G, 0.0);
-    const int stride = pools > 1 ? kXcds : 1, count = pools > 1 ? per_xcd : G;
-    for (int x = 0; x < pools; x++) {
-        std::vector<int> &its = pool[x];
-        std::stable_sort(its.begin(), its.end(), [&](int a, int c) { return cost[a] > cost[c]; });
-        for (int it : its) {
-            int best = x;
-            for (int j = 1; j < count; j++) {
-                const int g = x + j * stride;
-                if (load[g] < load[best]) best = g;
-            }
-            load[best] += cost[it];
-            lists[best].push_back(it);
+                stored += (double)h.off[wg[(size_t)blk * nw + r + 1]] -
+                          (double)h.off[wg[(size_t)blk * nw + r]];
+            cost.push_back(item_cost(b, stored, it.n, it.rows, h.W, elem));
+            items.push_back(it);
         }
     }
-    out->assign((size_t)G + 1, 0);
-    out->reserve((size_t)G + 1 + ni);
-    for (int g = 0; g < G; g++) {
-        (*out)[g + 1] = (*out)[g] + (int)lists[g].size();
-        out->insert(out->end(), lists[g].begin(), lists[g].end());
+    std::vector<std::vector<int>> lists;
+    sell_wg_lists(b, *sys_item, cost, &lists);
+    *blocks = (int)lists.size();
+    constexpr int kInts = sizeof(SellItem) / sizeof(int);
+    const size_t head = ((size_t)*blocks + kInts) / kInts * kInts;  // blocks + 1 offsets
+    plan->assign(head + items.size() * kInts, 0);
+    int at = 0;
+    for (int g = 0; g < *blocks; g++) {
+        (*plan)[g] = at;
+        for (int it : lists[g])
+            std::memcpy(plan->data() + head + (size_t)(at++) * kInts, &items[it], sizeof(SellItem));
     }
+    (*plan)[*blocks] = at;
+}
+
+// Points bd at an uploaded plan.
+void use_plan(BatchDev *bd, const int *plan, int blocks) {
+    constexpr int kInts = sizeof(SellItem) / sizeof(int);
+    bd->item_blocks = blocks;
+    bd->block_item = plan;
+    bd->wg_item = reinterpret_cast<const SellItem *>(plan + ((size_t)blocks + kInts) / kInts * kInts);
 }
 
 int apply_shape(npbcg_batch *b, int lpr, int rt, int layout) {
@@ -289,26 +349,17 @@ int apply_shape(npbcg_batch *b, int lpr, int rt, int layout) {
     make_tiles(b, layout == 3 ? kSellTileRows : rt, ts, tr, st);
     if (layout == 3) {  // items: one sorting window each, in system order
         rt = kSellWindow;
-        std::vector<int> items, sys_item, item_sl;
-        make_sell_items(b->sell_h, b->n, &items, &sys_item, &item_sl);
-        const int ni = sys_item[b->nsys];
-        if (ni > b->items_cap) return set_error(NPBCG_ERR_INTERNAL, "batch: item capacity");
-        B_HIP(hipMemcpyAsync(b->d_items, items.data(), sizeof(int) * items.size(),
-                             hipMemcpyHostToDevice, b->stream));
+        std::vector<int> sys_item, plan;
+        int blocks = 0;
+        sell_plan(b, b->sell_h, b->opts.mode == NPBCG_SOLVE_MIXED ? 4 : 8, &sys_item, &plan, &blocks);
         B_HIP(hipMemcpyAsync(b->d_sysinfo, sys_item.data(), sizeof(int) * (b->nsys + 1),
                              hipMemcpyHostToDevice, b->stream));
         B_HIP(hipStreamSynchronize(b->stream));
-        int rc = upload_order(b, item_sl, &b->d_item_sl, &b->item_sl_cap);
+        int rc = upload_order(b, plan, &b->d_block_item, &b->block_item_cap);
         if (rc != NPBCG_OK) return rc;
-        std::vector<int> wl;
-        sell_wg_lists(b, b->sell_h, items, sys_item, item_sl,
-                      b->opts.mode == NPBCG_SOLVE_MIXED ? 4 : 8, &wl);
-        rc = upload_order(b, wl, &b->d_block_item, &b->block_item_cap);
-        if (rc != NPBCG_OK) return rc;
-        b->bd.items = ni;
-        b->bd.item_blocks = (int)wl.size() - ni - 1;
-        b->bd.block_item = b->d_block_item;
-        b->bd.item_sl = b->d_item_sl;
+        b->bd.items = sys_item[b->nsys];
+        b->bd.split = b->sell_h.split;
+        use_plan(&b->bd, b->d_block_item, blocks);
     }
     if (layout == 2) {  // items: (system, column block, row range) in system order
         std::vector<int> items, sys_item(b->nsys + 1, 0);
@@ -393,13 +444,8 @@ bool build_batch_sell(const npbcg_batch *b, int W, const std::vector<int> &rp,
     h->W = W;
     h->nb.assign(b->nsys, 0);
     h->wg.assign(b->nsys, {});
-    h->nrange.assign(b->nsys, 0);
-    h->part.assign(b->nsys, 0);
-    h->part_total = 0;
     for (int s = 0; s < b->nsys; s++) {
         h->nb[s] = (b->n[s] + W - 1) / W;
-        h->part[s] = h->part_total;
-        h->part_total += (long long)b->n[s] * h->nb[s] * b->nr;
     }
     std::vector<int> lrs, lci;
     for (int s = 0; s < b->nsys; s++) {
@@ -410,10 +456,10 @@ bool build_batch_sell(const npbcg_batch *b, int W, const std::vector<int> &rp,
         for (int j = 0; j <= ns; j++) lrs[j] = rp[off + j] - e0;
         for (int k = 0; k < nnz_s; k++) lci[k] = col[(size_t)e0 + k] - off;
         SellBlocks<V> sb;
-        if (!build_sell_blocks(ns, lrs.data(), lci.data(), val.data() + e0, W, kSellWindow, &sb) ||
+        if (!build_sell_blocks(ns, lrs.data(), lci.data(), val.data() + e0, W, kSellWindow >> h->split,
+                               &sb) ||
             sb.nblk != h->nb[s] || entries + sb.stored > (long long)INT32_MAX)
             return false;
-        h->nrange[s] = sb.nrange;
         std::vector<int> &wg = h->wg[s];
         wg.resize(sb.wg_slice.size());
         for (size_t i = 0; i < wg.size(); i++) wg[i] = slices + sb.wg_slice[i];
@@ -458,22 +504,15 @@ BatchVecs<T> inner_vecs(const npbcg_batch *b) {
 // items and partial offsets; rows, tiles and flags of the batch.
 BatchDev resid_dev(const npbcg_batch *b) {
     BatchDev d = b->bd;
-    const int ns = b->nsys;
     d.cb = 1;
     d.sell = 1;
     d.cbw = b->res_h.W;
-    d.items = b->res_items;
-    d.item = b->d_res_items;
+    d.split = b->res_h.split;
     d.sys_item = b->d_res_sys;
-    d.sys_row = b->d_res_sys + ns + 1;
-    d.sys_nb = b->d_res_sys + 2 * ns + 2;
-    d.sys_part = b->d_res_part;
-    d.item_blocks = b->res_item_blocks;
-    d.block_item = b->d_res_block_item;
+    use_plan(&d, b->d_res_block_item, b->res_item_blocks);
     d.sell_off = b->d_res_off;
     d.sell_row = b->d_res_row;
     d.sell_col = b->d_res_col;
-    d.item_sl = b->d_res_item_sl;
     return d;
 }
 
@@ -555,18 +594,32 @@ template <typename T>
 int run_inner(npbcg_batch *b, int maxsteps) {
     const BatchVecs<T> v = inner_vecs<T>(b);
     B_HIP(batch_init<T>(b->bd, v, b->d_res, b->stream));
-    const int chunk = 8;
+    std::vector<int> done(b->nsys * b->nr);
+    std::vector<BatchScalars> sc(done.size());
+    int chunk = 8;
     for (int step = 0; step < maxsteps;) {
         const int end = std::min(maxsteps, step + chunk);
         for (; step < end; step++) B_HIP(batch_cg_step<T>(b->bd, v, step, step == 0, b->stream));
         // stop early when every solve has finished
-        std::vector<int> done(b->nsys * b->nr);
         B_HIP(hipMemcpyAsync(done.data(), b->bd.done, sizeof(int) * done.size(),
                              hipMemcpyDeviceToHost, b->stream));
+        B_HIP(hipMemcpyAsync(sc.data(), b->d_sc, sizeof(BatchScalars) * sc.size(),
+                             hipMemcpyDeviceToHost, b->stream));
         B_HIP(hipStreamSynchronize(b->stream));
-        bool all = true;
-        for (int f : done) all = all && f;
-        if (all) break;
+        // The next chunk: the steps the slowest solve still needs at the rate
+        // it went so far (rho is the r.r of the step before the last), at most
+        // 8; a step past the end costs three launches that do nothing.
+        chunk = 0;
+        for (size_t i = 0; i < done.size(); i++) {
+            if (done[i]) continue;
+            const double start = sc[i].tol2 / sc[i].rtol2;
+            const double rate = std::log(start / sc[i].rho) / (sc[i].sweep_steps - 1);
+            const double left = std::log(sc[i].rho / sc[i].tol2) / rate - 1.0;
+            chunk = std::max(chunk, left >= 1.0 && left <= 8.0 ? (int)std::ceil(left)
+                                    : left < 1.0               ? 1
+                                                               : 8);
+        }
+        if (chunk == 0) break;
     }
     B_HIP(batch_refine<T>(b->bd, b->d_x, v.d, b->stream));
     return NPBCG_OK;
@@ -591,11 +644,9 @@ void npbcg_batch_destroy(npbcg_batch *b) {
         for (void *p : {(void *)b->d_res_val, (void *)b->d_res_col, (void *)b->d_res_off,
                         (void *)b->d_res_row})
             (void)hipFree(p);
-    for (void *p : {(void *)b->d_res_items, (void *)b->d_res_sys, (void *)b->d_res_part,
-                    (void *)b->d_res_block_item, (void *)b->d_res_item_sl})
-        (void)hipFree(p);
+    for (void *p : {(void *)b->d_res_sys, (void *)b->d_res_block_item}) (void)hipFree(p);
     for (void *p : {b->d_sell_val, (void *)b->d_sell_col, (void *)b->d_sell_off,
-                    (void *)b->d_sell_row, (void *)b->d_block_item, (void *)b->d_item_sl,
+                    (void *)b->d_sell_row, (void *)b->d_block_item,
                     (void *)b->d_items, (void *)b->d_sysinfo, (void *)b->d_sys64, (void *)b->d_seg,
                     b->d_rows_part, (void *)b->d_rowptr, (void *)b->d_col, (void *)b->d_val,
                     (void *)b->d_val32,
@@ -696,8 +747,9 @@ int npbcg_batch_create(npbcg_batch **out, int nsys, const int *n, const int *con
             const int k0 = rowstr[s][j], k1 = rowstr[s][j + 1];
             order.resize(k1 - k0);
             for (int k = k0; k < k1; k++) order[k - k0] = k;
-            std::stable_sort(order.begin(), order.end(),
-                             [&](int x, int y) { return colidx[s][x] < colidx[s][y]; });
+            if (!std::is_sorted(colidx[s] + k0, colidx[s] + k1))
+                std::stable_sort(order.begin(), order.end(),
+                                 [&](int x, int y) { return colidx[s][x] < colidx[s][y]; });
             int* sg = &seg[(size_t)(sys_seg[s] + (long long)j * (nb + 1))];
             int blk = 0;
             for (int k : order) {
@@ -712,6 +764,9 @@ int npbcg_batch_create(npbcg_batch **out, int nsys, const int *n, const int *con
         }
     }
     rp[rows] = (int)e;
+    b->sell_h.split = sell_split(b, b->cbw, o.mode == NPBCG_SOLVE_MIXED ? 4 : 8, rp);
+    if (o.mode == NPBCG_SOLVE_MIXED)
+        b->res_h.split = sell_split(b, res_width(b, b->device), 8, rp);
     // SELL copy in the inner type (layout 3)
     std::vector<float> sval32;
     std::vector<double> sval64;
@@ -815,33 +870,15 @@ int npbcg_batch_create(npbcg_batch **out, int nsys, const int *n, const int *con
             b->d_res_off = b->d_sell_off;
             b->d_res_row = b->d_sell_row;
         }
-        std::vector<int> items, sys_item, item_sl;
-        make_sell_items(b->res_h, b->n, &items, &sys_item, &item_sl);
-        b->res_items = sys_item[nsys];
-        std::vector<int> sys(3 * (size_t)nsys + 2);
-        for (int s = 0; s <= nsys; s++) {
-            sys[s] = sys_item[s];
-            sys[nsys + 1 + s] = b->row_off[s];
-        }
-        for (int s = 0; s < nsys; s++) sys[2 * nsys + 2 + s] = b->res_h.nb[s];
-        std::vector<int> order;
-        sell_wg_lists(b, b->res_h, items, sys_item, item_sl, 8, &order);
-        b->res_item_blocks = (int)order.size() - b->res_items - 1;
-        TRY(hipMalloc(&b->d_res_items, sizeof(int) * std::max<size_t>(items.size(), 4)));
-        TRY(hipMalloc(&b->d_res_sys, sizeof(int) * sys.size()));
-        TRY(hipMalloc(&b->d_res_part, sizeof(long long) * nsys));
-        TRY(hipMalloc(&b->d_res_block_item, sizeof(int) * std::max<size_t>(order.size(), 1)));
-        TRY(hipMalloc(&b->d_res_item_sl, sizeof(int) * std::max<size_t>(item_sl.size(), 1)));
-        TRY(hipMemcpyAsync(b->d_res_item_sl, item_sl.data(), sizeof(int) * item_sl.size(),
+        std::vector<int> sys_item, plan;
+        sell_plan(b, b->res_h, 8, &sys_item, &plan, &b->res_item_blocks);
+        TRY(hipMalloc(&b->d_res_sys, sizeof(int) * sys_item.size()));
+        TRY(hipMalloc(&b->d_res_block_item, sizeof(int) * plan.size()));
+        TRY(hipMemcpyAsync(b->d_res_sys, sys_item.data(), sizeof(int) * sys_item.size(),
                            hipMemcpyHostToDevice, b->stream));
-        TRY(hipMemcpyAsync(b->d_res_items, items.data(), sizeof(int) * items.size(),
+        TRY(hipMemcpyAsync(b->d_res_block_item, plan.data(), sizeof(int) * plan.size(),
                            hipMemcpyHostToDevice, b->stream));
-        TRY(hipMemcpyAsync(b->d_res_sys, sys.data(), sizeof(int) * sys.size(),
-                           hipMemcpyHostToDevice, b->stream));
-        TRY(hipMemcpyAsync(b->d_res_part, b->res_h.part.data(), sizeof(long long) * nsys,
-                           hipMemcpyHostToDevice, b->stream));
-        TRY(hipMemcpyAsync(b->d_res_block_item, order.data(), sizeof(int) * order.size(),
-                           hipMemcpyHostToDevice, b->stream));
+        TRY(hipStreamSynchronize(b->stream));  // sys_item and plan go out of scope
         const hipError_t e3 =
             batch_prepare_resid((int)sell_lds_bytes(b->res_h.W, b->nr, sizeof(double)));
         if (e3 != hipSuccess)

@@ -9,9 +9,20 @@
 
 namespace npbcg_dev {
 
-// Rows of a SELL sorting window (layout 3): a system's rows are sorted by
-// their segment length inside windows of this many rows.
+// Rows of a SELL sorting window (layout 3) at most: a system's rows are sorted
+// by their segment length inside windows of H rows, H = kSellWindow >> split
+// (sell_split).
 constexpr int kSellWindow = 2048;
+
+// One sorting window of a system, the work item of the SELL SpMM: everything a
+// workgroup needs to start on it, in one load.  Column block b of the window
+// has the slices first + b * stride .. + (rows + 63) / 64.
+struct SellItem {
+    int sys, index;     // system; item (in system order), where its partials go
+    int row, rows;      // first row (global) and rows of the window
+    int sys_row, n;     // first row and order of the system
+    int first, stride;
+};
 
 // Per (system, right-hand side) scalars of the inner CG.
 struct BatchScalars {
@@ -57,16 +68,14 @@ struct BatchDev {
                                     // are [seg[b], seg[b+1]) (columns sorted in a row)
     // SELL SpMM (sell = 1, also cb = 1): a column-blocked SELL copy of every
     // system (blocks of cbw columns, rows sorted by segment length inside
-    // kSellWindow-row windows, 64-row slices stored column-major, 16-bit
-    // columns inside the block).  Item = one window: (system, first local row,
-    // rows, offset into item_sl), where item_sl holds the window's slice range
-    // [first, end) in each of the system's blocks.  The SpMM writes q (not
-    // block partials) and one p.q partial per item.
+    // windows of kSellWindow >> split rows, 64-row slices stored column-major,
+    // 16-bit columns inside the block).  Item = one window.  The SpMM writes q
+    // (not block partials) and one p.q partial per item.
     int sell = 0;
-    const int *item_sl = nullptr;
+    int split = 0;                     // log2 of the parts a slice's entries are cut into
     int item_blocks = 0;               // workgroups of the SELL SpMM (one per CU)
-    const int *block_item = nullptr;   // [item_blocks + 1] list offsets, then the lists:
-                                       // workgroup g runs items list[first[g] .. first[g+1])
+    const int *block_item = nullptr;   // [item_blocks + 1] workgroup g runs
+    const SellItem *wg_item = nullptr; // wg_item[block_item[g] .. block_item[g + 1])
     const int *sell_off = nullptr;     // [slices + 1] first entry of each slice
     const int *sell_row = nullptr;     // [slices * 64] global row of each lane, -1: padding
     const uint16_t *sell_col = nullptr;  // [stored] column inside the block

@@ -277,8 +277,8 @@ __global__ __launch_bounds__(kBlock) void batch_spmm_cb_kernel(BatchDev bd,
     block_sum_store<NR>(dot, pq_part + (size_t)it * NR);
 }
 
-// SELL SpMM over one 2048-row sorting window per item (system s, window
-// rows [r0, r0 + nrows)).  For each column block of the system in turn, the
+// SELL SpMM over one sorting window per item (SellItem; kSellWindow >> split
+// rows).  For each column block of the system in turn, the
 // block's vector entries (cbw rows of p, NR values each) are staged in LDS
 // and each wavefront streams whole slices of the window's block, one row per
 // lane, so the (value, 16-bit column) loads are contiguous across the
@@ -290,6 +290,15 @@ __global__ __launch_bounds__(kBlock) void batch_spmm_cb_kernel(BatchDev bd,
 // written once, with the p.q partial of the item.  No block partials go
 // through memory.  Slices go to wavefronts in a fixed snake order, so the
 // sums are reproducible.
+//
+// A short window has too few slices for the 16 wavefronts, so the entries of a
+// slice are cut into 1 << split parts at chunk borders, a unit of work each,
+// which keep row sums of their own (1 << split times H rows of them, the LDS of
+// one whole window); the parts of a row are added in order at the end.  What
+// bounds short windows is the staging (the whole vector of the system for each,
+// about 2 us and 28 KB/us a block) and, for an item or two per workgroup, the
+// chain of loads before the first entries: list, item, slice bounds, entries;
+// the stop flags are tested once those are on their way.
 //
 // RESID = true computes the FP64 true residual instead: res = b - A x for the
 // window's rows and the partials of |res|^2.
@@ -314,7 +323,8 @@ __global__ __launch_bounds__(BLOCK) void batch_spmm_sell_kernel(BatchDev bd,
                                                                 int rev) {
     extern __shared__ double2 lds_sell[];  // 16-byte aligned
     T *vlds = reinterpret_cast<T *>(lds_sell);
-    T *acc_lds = vlds + (size_t)bd.cbw * NR;  // [kSellWindow][NR] row sums of the window
+    T *acc_lds = vlds + (size_t)bd.cbw * NR;  // [parts][H][NR] row sums of the window
+    const int split = bd.split, H = kSellWindow >> split;
     constexpr int kWaves = BLOCK / kWave;
     const int lane = threadIdx.x & (kWave - 1);
     // wave-uniform (scalar) index: every branch on the slice loop is scalar
@@ -322,36 +332,44 @@ __global__ __launch_bounds__(BLOCK) void batch_spmm_sell_kernel(BatchDev bd,
     const int *__restrict__ off = bd.sell_off;
     const uint16_t *__restrict__ col = bd.sell_col;
     const int *__restrict__ lane_row = bd.sell_row;
-    const int *__restrict__ wl = bd.block_item + bd.item_blocks + 1;
     const int k0 = bd.block_item[blockIdx.x], k1 = bd.block_item[blockIdx.x + 1];
     for (int li = k0; li < k1; li++) {
-        const int it = wl[rev ? k0 + k1 - 1 - li : li];
-        const int s = bd.item[4 * it];
-        if (!RESID && system_done<NR>(bd.done, s)) continue;  // the same for every thread
-        const int r0 = bd.item[4 * it + 1], nrows = bd.item[4 * it + 2];
-        const int *__restrict__ ranges = bd.item_sl + bd.item[4 * it + 3];
-        const int srow = bd.sys_row[s], ns = bd.sys_row[s + 1] - srow, nb = bd.sys_nb[s];
-        const int wrow = srow + r0;  // first global row of the window
-        for (int b = 0; b < nb; b++) {
-            const int sl0 = ranges[2 * b], nsl = ranges[2 * b + 1] - sl0;
-            const int c0 = b * bd.cbw;
-            const int w = min(bd.cbw, ns - c0);
-            // Slice of round rd for this wave (snake order: slices of a window
-            // are sorted widest first, and alternating the direction of each
-            // round evens out the width per wavefront), or -1.  Rounds are
-            // increasing in k, so after the first -1 there is none.
-            auto slice_of = [&](int rd) {
+        const SellItem item = bd.wg_item[rev ? k0 + k1 - 1 - li : li];
+        const int s = item.sys, nrows = item.rows, wrow = item.row, srow = item.sys_row;
+        const int nsl = (nrows + kWave - 1) / kWave;
+        bool finished = false;
+        for (int c0 = 0, sl0 = item.first; c0 < item.n; c0 += bd.cbw, sl0 += item.stride) {
+            const int w = min(bd.cbw, item.n - c0);
+            // Unit (slice << split) + part of round rd for this wave (snake
+            // order: slices of a window are sorted widest first, and
+            // alternating the direction of each round evens out the width per
+            // wavefront), or -1.  Rounds are increasing in k, so after the
+            // first -1 there is none.
+            auto unit_of = [&](int rd) {
                 const int k = rd * kWaves + ((rd & 1) ? kWaves - 1 - wave : wave);
-                return k < nsl ? sl0 + k : -1;
+                return k < nsl << split ? k : -1;
+            };
+            // A unit's entries, whole chunks of its slice but the last.
+            auto bounds = [&](int k, int &base, int &width) {
+                const int sl = sl0 + (k >> split), part = k & ((1 << split) - 1);
+                base = off[sl];
+                width = (off[sl + 1] - base) / kWave;
+                const int chunks = (width + UNR - 1) / UNR;
+                const int j0 = ((chunks * part) >> split) * UNR;
+                width = min(width, ((chunks * (part + 1)) >> split) * UNR) - j0;
+                base += j0 * kWave;
             };
             T na[UNR];
             int nc[UNR];
-            int cur = slice_of(0), cbase = 0, cwidth = 0, nrow = -1;
+            int cur = unit_of(0), cbase = 0, cwidth = 0, nrow = -1;
             if (cur >= 0) {
-                cbase = off[cur];
-                cwidth = (off[cur + 1] - cbase) / kWave;
-                nrow = lane_row[(size_t)cur * kWave + lane];
+                bounds(cur, cbase, cwidth);
+                nrow = lane_row[(size_t)(sl0 + (cur >> split)) * kWave + lane];
                 if (cwidth > 0) sell_chunk<T, UNR>(sval, col, cbase, cwidth, 0, lane, na, nc);
+            }
+            if (!RESID && c0 == 0) {  // (the first loads are on their way)
+                finished = system_done<NR>(bd.done, s);  // the same for every thread
+                if (finished) break;
             }
             if constexpr (NR * sizeof(T) % 16 == 0) {  // rows of whole 16-byte units, aligned
                 constexpr int kUnits = NR * (int)sizeof(T) / 16;
@@ -365,12 +383,9 @@ __global__ __launch_bounds__(BLOCK) void batch_spmm_sell_kernel(BatchDev bd,
             __syncthreads();
             for (int rd = 0; cur >= 0; rd++) {
                 const int width = cwidth, base = cbase, row = nrow;
-                const int nxt = slice_of(rd + 1);
+                const int nxt = unit_of(rd + 1);
                 int xbase = 0, xwidth = 0;
-                if (nxt >= 0) {
-                    xbase = off[nxt];
-                    xwidth = (off[nxt + 1] - xbase) / kWave;
-                }
+                if (nxt >= 0) bounds(nxt, xbase, xwidth);
                 T acc[NR];
 #pragma unroll
                 for (int q = 0; q < NR; q++) acc[q] = T(0);
@@ -387,7 +402,7 @@ __global__ __launch_bounds__(BLOCK) void batch_spmm_sell_kernel(BatchDev bd,
                     if (ch + 1 < nch) {
                         sell_chunk<T, UNR>(sval, col, base, width, (ch + 1) * UNR, lane, na, nc);
                     } else if (nxt >= 0) {
-                        nrow = lane_row[(size_t)nxt * kWave + lane];
+                        nrow = lane_row[(size_t)(sl0 + (nxt >> split)) * kWave + lane];
                         if (xwidth > 0) sell_chunk<T, UNR>(sval, col, xbase, xwidth, 0, lane, na, nc);
                     }
 #pragma unroll
@@ -398,13 +413,14 @@ __global__ __launch_bounds__(BLOCK) void batch_spmm_sell_kernel(BatchDev bd,
                     }
                 }
                 if (nch == 0 && nxt >= 0) {
-                    nrow = lane_row[(size_t)nxt * kWave + lane];
+                    nrow = lane_row[(size_t)(sl0 + (nxt >> split)) * kWave + lane];
                     if (xwidth > 0) sell_chunk<T, UNR>(sval, col, xbase, xwidth, 0, lane, na, nc);
                 }
                 if (row >= 0) {  // every row of the window is in one slice of each block
-                    T *dst = acc_lds + (size_t)(row - wrow) * NR;
+                    T *dst = acc_lds +
+                             ((size_t)(cur & ((1 << split) - 1)) * H + (size_t)(row - wrow)) * NR;
                     VecT<T, NR> sum;
-                    if (b == 0) {
+                    if (c0 == 0) {
 #pragma unroll
                         for (int q = 0; q < NR; q++) sum.v[q] = acc[q];
                     } else {
@@ -420,11 +436,17 @@ __global__ __launch_bounds__(BLOCK) void batch_spmm_sell_kernel(BatchDev bd,
             }
             __syncthreads();  // the vector block is free again; the row sums are visible
         }
+        if (finished) continue;
         double dot[NR];
 #pragma unroll
         for (int q = 0; q < NR; q++) dot[q] = 0.0;
         for (int i = threadIdx.x; i < nrows; i += BLOCK) {
-            const VecT<T, NR> sum = load_vec<T, NR>(acc_lds + (size_t)i * NR);
+            VecT<T, NR> sum = load_vec<T, NR>(acc_lds + (size_t)i * NR);
+            for (int k = 1; k < 1 << split; k++) {  // the parts in order
+                const VecT<T, NR> more = load_vec<T, NR>(acc_lds + ((size_t)k * H + i) * NR);
+#pragma unroll
+                for (int q = 0; q < NR; q++) sum.v[q] += more.v[q];
+            }
             const size_t at = (size_t)(wrow + i) * NR;
             if constexpr (RESID) {
 #pragma unroll
@@ -440,7 +462,7 @@ __global__ __launch_bounds__(BLOCK) void batch_spmm_sell_kernel(BatchDev bd,
                 for (int q = 0; q < NR; q++) dot[q] += (double)pv.v[q] * (double)sum.v[q];
             }
         }
-        block_sum_store<NR, BLOCK>(dot, part + (size_t)it * NR);
+        block_sum_store<NR, BLOCK>(dot, part + (size_t)item.index * NR);
         __syncthreads();  // the row sums and the reduction slots are free again
     }
 }
