@@ -23,6 +23,8 @@ constexpr int kHid = 64;      // hidden width
 constexpr int kXW = 2 * kHid; // [H | aggregated H] input of a message-passing layer
 constexpr int kLayers = 3;    // message-passing layers
 constexpr int kPairs = 8;     // residual/correction pairs per training system
+constexpr int kWeightParts = 256;   // workgroups of the weight-gradient GEMMs at most
+constexpr int kReadoutParts = 512;  // workgroups of the readout's backward at most
 
 // FP32 master parameters (one array).
 constexpr int kOffW0 = 0;                          // [kK0][kHid]
@@ -72,13 +74,13 @@ struct NetBuffers {
     float *dx = nullptr;         // [cap][kXW]
     float *gh = nullptr;         // g [cap], h [cap]
     float *dgh = nullptr;        // dL/dg [cap], dL/dh [cap]
-    float *pw = nullptr;         // loss forward: (N + N^T) Q r_p per pair [kPairs][cap]
-    float *pd = nullptr;         // loss forward: dL/dy per pair [kPairs][cap]
+    float *pw = nullptr;         // loss forward: (N + N^T) Q r_p per pair [cap][kPairs]
+    float *pd = nullptr;         // loss forward: dL/dy per pair [cap][kPairs]
     const float *norm = nullptr; // feature mean [kFeat], std [kFeat]
-    float *wpart = nullptr;      // weight-gradient partials [wparts][kXW*kHid + kHid]
-    int wparts = 0;
-    float *rpart = nullptr;      // readout-gradient partials [row blocks][kReadout]
-    double *loss_part = nullptr; // loss partials [row blocks]
+    float *wpart = nullptr;      // weight-gradient partials, layers 1 to 3, then 0:
+                                 // [kLayers + 1][kWeightParts][kXW*kHid + kHid]
+    float *rpart = nullptr;      // readout-gradient partials [kReadoutParts][kReadout]
+    double *loss_part = nullptr; // loss partials [pair blocks]
 };
 
 // Graph, features and transpose (once per matrix).  cnt is n ints of scratch.
@@ -107,6 +109,7 @@ hipError_t launch_pair_weights(const double *part, int parts, int pairs, float *
                                hipStream_t st);
 hipError_t launch_random_rhs(double *b, int n, unsigned long long seed, hipStream_t st);
 int row_blocks(int n);   // workgroups of the 16-lanes-per-row kernels
+int pair_blocks(int n);  // workgroups of the pair-loss kernels
 
 // Forward through the readout: gh = (g, h).
 hipError_t launch_net_forward(const NetBuffers &nb, const NetSystem &sys, const float *params,

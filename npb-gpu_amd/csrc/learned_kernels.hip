@@ -46,6 +46,7 @@ int exact_blocks(long long items, int per_block) {
 }  // namespace
 
 int row_blocks(int n) { return exact_blocks((long long)n * 16, kBlock); }
+int pair_blocks(int n) { return exact_blocks((long long)n * kPairs, kBlock); }
 
 // ---------------------------------------------------------------------------
 // Graph and features (once per matrix)
@@ -501,28 +502,61 @@ __global__ __launch_bounds__(kBlock) void aggregate_kernel(__bf16 *__restrict__ 
     *reinterpret_cast<bf16x4 *>(x + (size_t)j * kXW + kHid + f) = o;
 }
 
-// g = G tanh(ug . H3 + cg), h = G tanh(uh . H3 + ch): 16 lanes per row.
+// The readout's sums ug . H3 + cg and uh . H3 + ch of kReadRows rows from j0 for a
+// group of 16 lanes, four columns a lane: lane t of the group keeps row j0 + t's
+// sums (lanes past kReadRows: the last row's), so that one tanh serves kReadRows
+// rows; hv holds the lane's columns of every row.  FP64 tanh is most of the
+// readout kernels (a row per group: 11.0 us forward, 11.1 backward at n = 40009; now
+// 5.7 and 7.5).
+constexpr int kReadRows = 4;
+__device__ __forceinline__ void readout_sums(const __bf16 *__restrict__ h3,
+                                             const float (&ug)[4], const float (&uh)[4],
+                                             double cg, double ch, long long j0, int n,
+                                             bf16x4 (&hv)[kReadRows], double &sg, double &sh) {
+    const int sub = threadIdx.x & 15;
+#pragma unroll
+    for (int t = 0; t < kReadRows; t++) {
+        hv[t] = bf16x4{};
+        if (j0 + t < n)
+            hv[t] = *reinterpret_cast<const bf16x4 *>(h3 + (size_t)(j0 + t) * kHid + sub * 4);
+    }
+    sg = sh = 0.0;
+#pragma unroll
+    for (int t = 0; t < kReadRows; t++) {
+        double a = 0.0, b = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            a += (double)((float)hv[t][q] * ug[q]);
+            b += (double)((float)hv[t][q] * uh[q]);
+        }
+        a = segment_sum<16>(a) + cg;
+        b = segment_sum<16>(b) + ch;
+        if (sub >= t) {
+            sg = a;
+            sh = b;
+        }
+    }
+}
+
+// g = G tanh(ug . H3 + cg), h = G tanh(uh . H3 + ch).
 __global__ __launch_bounds__(kBlock) void readout_fwd_kernel(const __bf16 *__restrict__ h3,
                                                              const float *__restrict__ ro,
                                                              float gmax, int n,
                                                              float *__restrict__ gh) {
-    const long long gid = blockIdx.x * (long long)kBlock + threadIdx.x;
-    const int j = (int)(gid / 16), f = (int)(gid % 16) * 4;
-    const bool valid = j < n;
-    double sg = 0.0, sh = 0.0;
-    if (valid) {
-        const bf16x4 hv = *reinterpret_cast<const bf16x4 *>(h3 + (size_t)j * kHid + f);
+    const long long j0 = (blockIdx.x * (long long)kBlock + threadIdx.x) / 16 * kReadRows;
+    const int sub = threadIdx.x & 15, f = sub * 4;
+    float ug[4], uh[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            sg += (double)((float)hv[q] * ro[f + q]);
-            sh += (double)((float)hv[q] * ro[kHid + 1 + f + q]);
-        }
+    for (int q = 0; q < 4; q++) {
+        ug[q] = ro[f + q];
+        uh[q] = ro[kHid + 1 + f + q];
     }
-    sg = segment_sum<16>(sg) + ro[kHid];
-    sh = segment_sum<16>(sh) + ro[2 * kHid + 1];
-    if (valid && (threadIdx.x & 15) == 0) {
-        gh[j] = (float)(gmax * tanh(sg));
-        gh[n + j] = (float)(gmax * tanh(sh));
+    bf16x4 hv[kReadRows];
+    double sg, sh;
+    readout_sums(h3, ug, uh, ro[kHid], ro[2 * kHid + 1], j0, n, hv, sg, sh);
+    if (sub < kReadRows && j0 + sub < n) {
+        gh[j0 + sub] = (float)(gmax * tanh(sg));
+        gh[n + j0 + sub] = (float)(gmax * tanh(sh));
     }
 }
 
@@ -530,29 +564,52 @@ __global__ __launch_bounds__(kBlock) void readout_fwd_kernel(const __bf16 *__res
 // Pair loss under the preconditioner of (g, h)
 // ---------------------------------------------------------------------------
 
-// out[p] += sum over the symmetric pattern of row j of C_jk q_k v[p][k],
-// C = N + N^T, q_k = exp(g_k + h_k): out-edges of j first, then in-edges.
-__device__ __forceinline__ void gather_sym(const NetSystem &sys, const float *__restrict__ gh,
-                                           int n, int j, const float *__restrict__ v, int pairs,
-                                           float (&out)[kPairs]) {
+// Eight lanes per row, one per pair: 40009 rows are 5000 wavefronts that gather
+// at the same time, where a thread per row left 2.4 of them on a CU, each with 64
+// gathers of its own in turn (forward and backward 56 and 55 us; now 19 and 10).
+static_assert(kPairs == 8, "a row's lanes");
+
+// Sum over the symmetric pattern of row j of C_jk q_k v_k for the lane's pair,
+// C = N + N^T, q_k = exp(g_k + h_k): out-edges of j first, then in-edges, the
+// lanes of the row taking the next eight edges together.  v_k of the lane's pair
+// is v[k * stride].
+__device__ __forceinline__ float gather_sym(const NetSystem &sys, const float *__restrict__ gh,
+                                            int n, int j, const float *__restrict__ v,
+                                            int stride) {
+    const int sub = threadIdx.x & (kPairs - 1);
+    const int t0 = sys.tptr[j] - kNbr, m = sys.tptr[j + 1] - t0;  // edge e >= kNbr at t0 + e
+    float out = 0.0f;
+    for (int e0 = 0; e0 < m; e0 += kPairs) {
+        const int e = e0 + sub;
+        float c = 0.0f;
+        int k = -1;
+        if (e < kNbr) {
+            c = sys.nval[(size_t)j * kNbr + e];
+            k = sys.nbr[(size_t)j * kNbr + e];
+        } else if (e < m) {
+            c = sys.tval[t0 + e];
+            k = sys.tsrc[t0 + e];
+        }
+        if (c == 0.0f) k = -1;
+        const float cq = k >= 0 ? c * expf(gh[k] + gh[n + k]) : 0.0f;
+        float x[kPairs];
+        int kk[kPairs];
 #pragma unroll
-    for (int t = 0; t < kNbr; t++) {
-        const float c = sys.nval[(size_t)j * kNbr + t];
-        if (c == 0.0f) continue;
-        const int k = sys.nbr[(size_t)j * kNbr + t];
-        const float cq = c * expf(gh[k] + gh[n + k]);
-        for (int p = 0; p < pairs; p++) out[p] = fmaf(cq, v[(size_t)p * n + k], out[p]);
+        for (int t = 0; t < kPairs; t++) {
+            kk[t] = __shfl(k, t, kPairs);
+            x[t] = v[(size_t)max(kk[t], 0) * stride];
+        }
+#pragma unroll
+        for (int t = 0; t < kPairs; t++) {
+            const float ct = __shfl(cq, t, kPairs);
+            if (kk[t] >= 0) out = fmaf(ct, x[t], out);
+        }
     }
-    for (int e = sys.tptr[j]; e < sys.tptr[j + 1]; e++) {
-        const float c = sys.tval[e];
-        if (c == 0.0f) continue;
-        const int k = sys.tsrc[e];
-        const float cq = c * expf(gh[k] + gh[n + k]);
-        for (int p = 0; p < pairs; p++) out[p] = fmaf(cq, v[(size_t)p * n + k], out[p]);
-    }
+    return out;
 }
 
-// y_p = s2_j r_p - q_j w_p, w_p = (C Q r_p)_j; loss partials; pw = w, pd = dL/dy.
+// y_p = s2_j r_p - q_j w_p, w_p = (C Q r_p)_j; loss partials; pw = w, pd = dL/dy
+// ([row][kPairs]).
 __global__ __launch_bounds__(kBlock) void pair_loss_fwd_kernel(NetSystem sys,
                                                                const float *__restrict__ gh,
                                                                PairSet ps,
@@ -560,27 +617,28 @@ __global__ __launch_bounds__(kBlock) void pair_loss_fwd_kernel(NetSystem sys,
                                                                float *__restrict__ pd,
                                                                double *__restrict__ loss_part) {
     const int n = sys.n;
+    const long long gid = blockIdx.x * (long long)kBlock + threadIdx.x;
+    const int j = (int)(gid / kPairs), p = (int)(gid % kPairs);
     double acc = 0.0;
-    for (int j = blockIdx.x * kBlock + threadIdx.x; j < n; j += gridDim.x * kBlock) {
-        const float g = gh[j], h = gh[n + j];
-        const float s2 = (float)(exp(2.0 * g) / sys.adiag[j]);
-        const float q = expf(g + h);
-        float w[kPairs] = {};
-        gather_sym(sys, gh, n, j, ps.r, ps.count, w);
-        for (int p = 0; p < ps.count; p++) {
-            const size_t at = (size_t)p * n + j;
-            const float y = s2 * ps.r[at] - q * w[p];
-            const float diff = y - ps.e[at];
-            acc += (double)ps.omega[p] * (double)diff * (double)diff;
-            pw[at] = w[p];
-            pd[at] = 2.0f * ps.omega[p] * diff;
+    if (j < n) {
+        const size_t column = (size_t)min(p, ps.count - 1) * n;
+        const float w = gather_sym(sys, gh, n, j, ps.r + column, 1);
+        if (p < ps.count) {
+            const float g = gh[j], h = gh[n + j];
+            const float s2 = (float)(exp(2.0 * g) / sys.adiag[j]);
+            const float q = expf(g + h);
+            const float y = s2 * ps.r[column + j] - q * w;
+            const float diff = y - ps.e[column + j];
+            acc = (double)ps.omega[p] * (double)diff * (double)diff;
+            pw[gid] = w;
+            pd[gid] = 2.0f * ps.omega[p] * diff;
         }
     }
     store_block_partial<kBlock>(acc, loss_part);
 }
 
 // dL/dq_j = sum_p (-d_pj w_pj - r_pj (C Q d_p)_j); dL/dg = 2 s2 sum_p d r + q dL/dq;
-// dL/dh = q dL/dq.
+// dL/dh = q dL/dq (the pairs in order, in every lane of the row).
 __global__ __launch_bounds__(kBlock) void pair_loss_bwd_kernel(NetSystem sys,
                                                                const float *__restrict__ gh,
                                                                PairSet ps,
@@ -588,18 +646,22 @@ __global__ __launch_bounds__(kBlock) void pair_loss_bwd_kernel(NetSystem sys,
                                                                const float *__restrict__ pd,
                                                                float *__restrict__ dgh) {
     const int n = sys.n;
-    for (int j = blockIdx.x * kBlock + threadIdx.x; j < n; j += gridDim.x * kBlock) {
+    const long long gid = blockIdx.x * (long long)kBlock + threadIdx.x;
+    const int j = (int)(gid / kPairs), p = min((int)(gid % kPairs), ps.count - 1);
+    if (j >= n) return;
+    const float phi = gather_sym(sys, gh, n, j, pd + p, kPairs);
+    const size_t at = (size_t)j * kPairs + p;
+    const float d = pd[at], r = ps.r[(size_t)p * n + j];
+    const float term = d * pw[at] + r * phi;
+    float dq = 0.0f, ds = 0.0f;
+    for (int t = 0; t < ps.count; t++) {
+        dq -= __shfl(term, t, kPairs);
+        ds = fmaf(__shfl(d, t, kPairs), __shfl(r, t, kPairs), ds);
+    }
+    if (gid % kPairs == 0) {
         const float g = gh[j], h = gh[n + j];
         const float s2 = (float)(exp(2.0 * g) / sys.adiag[j]);
         const float q = expf(g + h);
-        float phi[kPairs] = {};
-        gather_sym(sys, gh, n, j, pd, ps.count, phi);
-        float dq = 0.0f, ds = 0.0f;
-        for (int p = 0; p < ps.count; p++) {
-            const size_t at = (size_t)p * n + j;
-            dq -= pd[at] * pw[at] + ps.r[at] * phi[p];
-            ds = fmaf(pd[at], ps.r[at], ds);
-        }
         dgh[j] = 2.0f * s2 * ds + q * dq;
         dgh[n + j] = q * dq;
     }
@@ -610,7 +672,10 @@ __global__ __launch_bounds__(kBlock) void pair_loss_bwd_kernel(NetSystem sys,
 // ---------------------------------------------------------------------------
 
 // From dL/dg, dL/dh: dZ3 = (dtg ug + dth uh) * (H3 > 0) in BF16, and this
-// workgroup's partial readout gradient [ug(64), cg, uh(64), ch].
+// workgroup's partial readout gradient [ug(64), cg, uh(64), ch] over its rows
+// (16 lanes a row, the sums of a lane's rows in registers; as many workgroups
+// as there are parts, kReadoutParts at most: a part for every 16 rows took the
+// reduction 44 us at n = 40009).
 __global__ __launch_bounds__(kBlock) void readout_bwd_kernel(const __bf16 *__restrict__ h3,
                                                              const float *__restrict__ ro,
                                                              float gmax, int n,
@@ -619,42 +684,51 @@ __global__ __launch_bounds__(kBlock) void readout_bwd_kernel(const __bf16 *__res
                                                              float *__restrict__ rpart) {
     constexpr int kRows = kBlock / 16;
     __shared__ float lds[kRows][kReadout];
-    const long long gid = blockIdx.x * (long long)kBlock + threadIdx.x;
-    const int j = (int)(gid / 16), f = (int)(gid % 16) * 4;
+    const int sub = threadIdx.x & 15, f = sub * 4;
     const int grp = threadIdx.x / 16;
-    const bool valid = j < n;
-    float hv[4] = {0.f, 0.f, 0.f, 0.f};
-    double sg = 0.0, sh = 0.0;
-    if (valid) {
-        const bf16x4 h4 = *reinterpret_cast<const bf16x4 *>(h3 + (size_t)j * kHid + f);
+    float ug[4], uh[4], pg[4] = {}, ph[4] = {}, cg = 0.f, ch = 0.f;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            hv[q] = (float)h4[q];
-            sg += (double)(hv[q] * ro[f + q]);
-            sh += (double)(hv[q] * ro[kHid + 1 + f + q]);
-        }
+    for (int q = 0; q < 4; q++) {
+        ug[q] = ro[f + q];
+        uh[q] = ro[kHid + 1 + f + q];
     }
-    sg = segment_sum<16>(sg) + ro[kHid];
-    sh = segment_sum<16>(sh) + ro[2 * kHid + 1];
-    float dtg = 0.f, dth = 0.f;
-    if (valid) {
-        const double tg = tanh(sg), th = tanh(sh);
-        dtg = (float)(dgh[j] * gmax * (1.0 - tg * tg));
-        dth = (float)(dgh[n + j] * gmax * (1.0 - th * th));
-        bf16x4 o;
+    const double cg0 = ro[kHid], ch0 = ro[2 * kHid + 1];
+    for (long long b0 = (long long)blockIdx.x * kRows * kReadRows; b0 < n;
+         b0 += (long long)gridDim.x * kRows * kReadRows) {
+        const long long j0 = b0 + grp * kReadRows;
+        bf16x4 hv[kReadRows];
+        double sg, sh;
+        readout_sums(h3, ug, uh, cg0, ch0, j0, n, hv, sg, sh);
+        float mine_g = 0.f, mine_h = 0.f;
+        if (sub < kReadRows && j0 + sub < n) {
+            const double tg = tanh(sg), th = tanh(sh);
+            mine_g = (float)(dgh[j0 + sub] * gmax * (1.0 - tg * tg));
+            mine_h = (float)(dgh[n + j0 + sub] * gmax * (1.0 - th * th));
+        }
 #pragma unroll
-        for (int q = 0; q < 4; q++)
-            o[q] = (__bf16)(hv[q] > 0.f ? dtg * ro[f + q] + dth * ro[kHid + 1 + f + q] : 0.f);
-        *reinterpret_cast<bf16x4 *>(dz + (size_t)j * kHid + f) = o;
+        for (int t = 0; t < kReadRows; t++) {
+            const float dtg = __shfl(mine_g, t, 16), dth = __shfl(mine_h, t, 16);
+            bf16x4 o;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const float h = (float)hv[t][q];
+                o[q] = (__bf16)(h > 0.f ? dtg * ug[q] + dth * uh[q] : 0.f);
+                pg[q] += dtg * h;
+                ph[q] += dth * h;
+            }
+            if (j0 + t < n) *reinterpret_cast<bf16x4 *>(dz + (size_t)(j0 + t) * kHid + f) = o;
+            cg += dtg;
+            ch += dth;
+        }
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        lds[grp][f + q] = dtg * hv[q];
-        lds[grp][kHid + 1 + f + q] = dth * hv[q];
+        lds[grp][f + q] = pg[q];
+        lds[grp][kHid + 1 + f + q] = ph[q];
     }
     if ((threadIdx.x & 15) == 0) {
-        lds[grp][kHid] = dtg;
-        lds[grp][2 * kHid + 1] = dth;
+        lds[grp][kHid] = cg;
+        lds[grp][2 * kHid + 1] = ch;
     }
     __syncthreads();
     if (threadIdx.x < kReadout) {
@@ -707,14 +781,28 @@ __global__ __launch_bounds__(kBlock) void aggregate_bwd_kernel(
     const long long gid = blockIdx.x * (long long)kBlock + threadIdx.x;
     const int k = (int)(gid / 16), f = (int)(gid % 16) * 4;
     if (k >= n) return;
+    const int e0 = tptr[k], e1 = tptr[k + 1];
     const f32x4 own = *reinterpret_cast<const f32x4 *>(dx + (size_t)k * kXW + f);
     float acc[4] = {own[0], own[1], own[2], own[3]};
-    for (int e = tptr[k]; e < tptr[k + 1]; e++) {
-        const int src = tsrc[e];
-        const float w = tw[e];
-        const f32x4 g = *reinterpret_cast<const f32x4 *>(dx + (size_t)src * kXW + kHid + f);
+    for (int b = e0; b < e1; b += 16) {  // the row's lanes load the next 16 edges
+        const int mine = min(b + (int)(threadIdx.x & 15), e1 - 1);
+        const int src = tsrc[mine];
+        const float w = tw[mine];
+        for (int t = 0; t < 16 && b + t < e1; t += 4) {  // four gathers in flight
+            f32x4 g[4];
+            float wt[4];
 #pragma unroll
-        for (int c = 0; c < 4; c++) acc[c] = fmaf(w, g[c], acc[c]);
+            for (int u = 0; u < 4; u++) {
+                g[u] = *reinterpret_cast<const f32x4 *>(
+                    dx + (size_t)__shfl(src, t + u, 16) * kXW + kHid + f);
+                wt[u] = __shfl(w, t + u, 16);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (b + t + u < e1)
+#pragma unroll
+                    for (int c = 0; c < 4; c++) acc[c] = fmaf(wt[u], g[u][c], acc[c]);
+        }
     }
     const bf16x4 hv = *reinterpret_cast<const bf16x4 *>(x + (size_t)k * kXW + f);
     bf16x4 o;
@@ -724,105 +812,140 @@ __global__ __launch_bounds__(kBlock) void aggregate_bwd_kernel(
 }
 
 // Per-workgroup partial dW[K x 64] = X^T dZ and db[64] = column sums of dZ
-// over this workgroup's rows, in chunks of 32 rows staged in LDS; the MFMA
-// reduction dimension is the row index.  part holds K*64 + 64 floats per
-// workgroup.
+// over this workgroup's rows, in chunks of 64 rows; the MFMA reduction
+// dimension is the row index.  The chunk is stored in LDS by column, so a lane's
+// eight rows of a fragment are one 16-byte read, and the next chunk's loads are
+// on their way while this one is multiplied.  Eight wavefronts, one 16-row block
+// of dW each (K = 128).  part holds K*64 + 64 floats per workgroup; 256 of them
+// (one a CU) instead of 512 halve what the reduction reads.  (32-row chunks read
+// from LDS two bytes at a time, 10.3 us at n = 40009, K = 128; now 7.4.)
+constexpr int kWgBlock = 512;
+constexpr int kWgRows = 64;
 template <int K>
-__global__ __launch_bounds__(kBlock) void gemm_bwd_weight_kernel(const __bf16 *__restrict__ x,
-                                                                 int ldx, int n,
-                                                                 const __bf16 *__restrict__ dz,
-                                                                 float *__restrict__ part) {
-    constexpr int RB = K / 16;  // 16-row blocks of dW
-    constexpr int RBW = (RB + kWavesPerBlock - 1) / kWavesPerBlock;
-    __shared__ __bf16 xs[32][K + 8];
-    __shared__ __bf16 gs[32][kHid + 8];
+__global__ __launch_bounds__(kWgBlock) void gemm_bwd_weight_kernel(const __bf16 *__restrict__ x,
+                                                                   int ldx, int n,
+                                                                   const __bf16 *__restrict__ dz,
+                                                                   float *__restrict__ part) {
+    constexpr int RB = K / 16;                               // 16-row blocks of dW
+    constexpr int XV = kWgRows * K / 8 / kWgBlock;           // vectors of X a thread loads
+    constexpr int XT = XV > 0 ? XV : 1;
+    static_assert(RB <= kWgBlock / kWave && kWgRows * kHid / 8 == kWgBlock, "chunk shape");
+    __shared__ __bf16 xs[K][kWgRows + 8];
+    __shared__ __bf16 gs[kHid][kWgRows + 8];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
-    f32x4 acc[RBW][4] = {};
+    const int rr = lane;  // a wavefront loads 8 columns of the chunk's 64 rows
+    f32x4 acc[4] = {};
     float db = 0.f;
-    for (int r0 = blockIdx.x * 32; r0 < n; r0 += gridDim.x * 32) {
-        __syncthreads();
-        for (int i = threadIdx.x; i < 32 * K / 8; i += kBlock) {
-            const int rr = i / (K / 8), cc = (i % (K / 8)) * 8, row = r0 + rr;
-            bf16x8 v = {};
-            if (row < n) v = *reinterpret_cast<const bf16x8 *>(x + (size_t)row * ldx + cc);
+    bf16x8 xv[XT], gv;
+    auto load = [&](int r0) {
+        const int row = r0 + rr;
 #pragma unroll
-            for (int t = 0; t < 8; t++) xs[rr][cc + t] = v[t];
+        for (int u = 0; u < XT; u++) {
+            const int cc = (wave + u * (kWgBlock / kWave)) * 8;
+            xv[u] = bf16x8{};
+            if (row < n && cc < K)
+                xv[u] = *reinterpret_cast<const bf16x8 *>(x + (size_t)row * ldx + cc);
         }
-        for (int i = threadIdx.x; i < 32 * kHid / 8; i += kBlock) {
-            const int rr = i / (kHid / 8), cc = (i % (kHid / 8)) * 8, row = r0 + rr;
-            bf16x8 v = {};
-            if (row < n) v = *reinterpret_cast<const bf16x8 *>(dz + (size_t)row * kHid + cc);
-#pragma unroll
-            for (int t = 0; t < 8; t++) gs[rr][cc + t] = v[t];
-        }
+        gv = bf16x8{};
+        if (row < n) gv = *reinterpret_cast<const bf16x8 *>(dz + (size_t)row * kHid + wave * 8);
+    };
+    int r0 = blockIdx.x * kWgRows;
+    if (r0 < n) load(r0);
+    for (; r0 < n; r0 += gridDim.x * kWgRows) {
         __syncthreads();
-        if (threadIdx.x < kHid)
-            for (int rr = 0; rr < 32; rr++) db += (float)gs[rr][threadIdx.x];
+#pragma unroll
+        for (int u = 0; u < XT; u++) {
+            const int cc = (wave + u * (kWgBlock / kWave)) * 8;
+            if (cc < K)
+#pragma unroll
+                for (int t = 0; t < 8; t++) xs[cc + t][rr] = xv[u][t];
+        }
+#pragma unroll
+        for (int t = 0; t < 8; t++) gs[wave * 8 + t][rr] = gv[t];
+        __syncthreads();
+        if (r0 + (int)gridDim.x * kWgRows < n) load(r0 + gridDim.x * kWgRows);
         const int kq = 8 * (lane >> 4);
+        if (wave < RB) {
 #pragma unroll
-        for (int q = 0; q < RBW; q++) {
-            const int rb = wave + q * kWavesPerBlock;
-            if (rb < RB) {
-                bf16x8 av;
-#pragma unroll
-                for (int t = 0; t < 8; t++) av[t] = xs[kq + t][rb * 16 + (lane & 15)];
+            for (int ks = 0; ks < kWgRows / 32; ks++) {
+                const bf16x8 av =
+                    *reinterpret_cast<const bf16x8 *>(&xs[wave * 16 + (lane & 15)][ks * 32 + kq]);
 #pragma unroll
                 for (int jb = 0; jb < 4; jb++) {
-                    bf16x8 bv;
-#pragma unroll
-                    for (int t = 0; t < 8; t++) bv[t] = gs[kq + t][jb * 16 + (lane & 15)];
-                    acc[q][jb] =
-                        __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[q][jb], 0, 0, 0);
+                    const bf16x8 bv =
+                        *reinterpret_cast<const bf16x8 *>(&gs[jb * 16 + (lane & 15)][ks * 32 + kq]);
+                    acc[jb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[jb], 0, 0, 0);
                 }
             }
         }
+        if (threadIdx.x < kHid)
+#pragma unroll
+            for (int q = 0; q < kWgRows; q += 8) {
+                const bf16x8 v = *reinterpret_cast<const bf16x8 *>(&gs[threadIdx.x][q]);
+#pragma unroll
+                for (int t = 0; t < 8; t++) db += (float)v[t];
+            }
     }
     float *out = part + (size_t)blockIdx.x * (K * kHid + kHid);
+    if (wave < RB) {
 #pragma unroll
-    for (int q = 0; q < RBW; q++) {
-        const int rb = wave + q * kWavesPerBlock;
-        if (rb < RB) {
+        for (int jb = 0; jb < 4; jb++)
 #pragma unroll
-            for (int jb = 0; jb < 4; jb++)
-#pragma unroll
-                for (int t = 0; t < 4; t++)
-                    out[(size_t)(rb * 16 + 4 * (lane >> 4) + t) * kHid + jb * 16 + (lane & 15)] =
-                        acc[q][jb][t];
-        }
+            for (int t = 0; t < 4; t++)
+                out[(size_t)(wave * 16 + 4 * (lane >> 4) + t) * kHid + jb * 16 + (lane & 15)] =
+                    acc[jb][t];
     }
     if (threadIdx.x < kHid) out[K * kHid + threadIdx.x] = db;
 }
 
 // out[i] = sum over p of part[p * stride + i], i < count, p in increasing
 // order within each of kRedWaves interleaved groups, the groups then added in
-// order (a fixed order: the same bits every run).  A 1024-thread workgroup
-// takes 64 consecutive columns; wavefront w sums the parts p = w, w + 16, ...
-// of its lane's column, so the loads are coalesced and 16 wavefronts share a
-// column's parts.
+// order (a fixed order: the same bits every run), for every gradient of a
+// backward pass in one launch.  A 1024-thread workgroup takes 64 consecutive
+// columns of one of them; wavefront w sums the parts p = w, w + 16, ... of its
+// lane's column, eight loads in flight, so the loads are coalesced and 16
+// wavefronts share a column's parts.  (A launch per gradient, one load in flight:
+// 83 us at n = 40009; now 6.8.)
 constexpr int kRedWaves = 16;
-__global__ __launch_bounds__(kRedWaves * kWave) void reduce_parts_kernel(
-    const float *__restrict__ part, int parts, int stride, int count, float *__restrict__ out) {
+constexpr int kRedSets = kLayers + 2;
+struct RedSet {
+    const float *part;
+    float *out;
+    int parts, stride, first_block;  // columns: stride
+};
+struct RedSets {
+    RedSet set[kRedSets];
+};
+__global__ __launch_bounds__(kRedWaves * kWave) void reduce_parts_kernel(RedSets sets) {
     __shared__ float ws[kRedWaves][kWave];
+    int which = 0;
+#pragma unroll
+    for (int i = 1; i < kRedSets; i++)
+        if ((int)blockIdx.x >= sets.set[i].first_block) which = i;
+    const RedSet rs = sets.set[which];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const int i = blockIdx.x * kWave + lane;
+    const int i = (blockIdx.x - rs.first_block) * kWave + lane;
     float s = 0.f;
-    if (i < count)
-        for (int p = wave; p < parts; p += kRedWaves) s += part[(size_t)p * stride + i];
+    if (i < rs.stride) {
+        const float *from = rs.part + i;
+        int p = wave;
+        for (; p + 7 * kRedWaves < rs.parts; p += 8 * kRedWaves) {
+            float t[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) t[u] = from[(size_t)(p + u * kRedWaves) * rs.stride];
+#pragma unroll
+            for (int u = 0; u < 8; u++) s += t[u];
+        }
+        for (; p < rs.parts; p += kRedWaves) s += from[(size_t)p * rs.stride];
+    }
     ws[wave][lane] = s;
     __syncthreads();
-    if (wave == 0 && i < count) {
+    if (wave == 0 && i < rs.stride) {
         float t = ws[0][lane];
         for (int w = 1; w < kRedWaves; w++) t += ws[w][lane];
-        out[i] = t;
+        rs.out[i] = t;
     }
-}
-
-hipError_t launch_reduce_parts(const float *part, int parts, int stride, int count, float *out,
-                               hipStream_t st) {
-    reduce_parts_kernel<<<(count + kWave - 1) / kWave, kRedWaves * kWave, 0, st>>>(part, parts,
-                                                                                stride, count, out);
-    return hipGetLastError();
 }
 
 // Adam step on the FP32 master parameters (bias-corrected moments).
@@ -877,25 +1000,30 @@ __global__ __launch_bounds__(kBlock) void pack_weights_kernel(const float *__res
 // Preconditioner operator
 // ---------------------------------------------------------------------------
 
-// One thread per row: entry 0 is the diagonal exp(2 g_j) / a_jj, the others
-// -exp(g_j + h_j + g_k + h_k) N (0 for padding).
+// Eight lanes per row (9 entries on average): entry 0 is the diagonal
+// exp(2 g_j) / a_jj, the others -exp(g_j + h_j + g_k + h_k) N (0 for padding).
+// (A thread per row, its entries in turn: 24 us at n = 60013; now 11.8 us.)
 __global__ __launch_bounds__(kBlock) void precond_values_kernel(
     int n, const int *__restrict__ off, const int *__restrict__ col,
     const float *__restrict__ src_val, const double *__restrict__ adiag,
     const float *__restrict__ gh, double *__restrict__ val, float *__restrict__ val32) {
-    for (int j = blockIdx.x * kBlock + threadIdx.x; j < n; j += gridDim.x * kBlock) {
-        const double d = adiag[j];
-        const double gj = (double)gh[j] + gh[n + j];
-        double v = d != 0.0 ? exp(2.0 * (double)gh[j]) / d : 0.0;
-        val[off[j]] = v;
-        val32[off[j]] = (float)v;
-        for (int e = off[j] + 1; e < off[j + 1]; e++) {
+    const long long gid = blockIdx.x * (long long)kBlock + threadIdx.x;
+    const int j = (int)(gid / 8);
+    if (j >= n) return;
+    const int e0 = off[j], e1 = off[j + 1];
+    const double gj = (double)gh[j] + gh[n + j];
+    for (int e = e0 + (int)(gid % 8); e < e1; e += 8) {
+        double v;
+        if (e == e0) {
+            const double d = adiag[j];
+            v = d != 0.0 ? exp(2.0 * (double)gh[j]) / d : 0.0;
+        } else {
             const float sv = src_val[e];
             const int k = col[e];
             v = sv != 0.0f ? -exp(gj + gh[k] + gh[n + k]) * sv : 0.0;
-            val[e] = v;
-            val32[e] = (float)v;
         }
+        val[e] = v;
+        val32[e] = (float)v;
     }
 }
 
@@ -1067,13 +1195,13 @@ hipError_t launch_net_forward(const NetBuffers &nb, const NetSystem &sys, const 
             params + kOffB1 + l * kLayerStride, out, ldy);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    readout_fwd_kernel<<<row_blocks(n), kBlock, 0, st>>>(nb.h3, params + kOffR, gmax, n, nb.gh);
+    readout_fwd_kernel<<<exact_blocks((long long)n * 16, kBlock * kReadRows), kBlock, 0, st>>>(nb.h3, params + kOffR, gmax, n, nb.gh);
     return hipGetLastError();
 }
 
 hipError_t launch_pair_loss(const NetBuffers &nb, const NetSystem &sys, const PairSet &ps,
                             int want_grad, hipStream_t st) {
-    const int blocks = row_blocks(sys.n);
+    const int blocks = pair_blocks(sys.n);
     pair_loss_fwd_kernel<<<blocks, kBlock, 0, st>>>(sys, nb.gh, ps, nb.pw, nb.pd, nb.loss_part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !want_grad) return e;
@@ -1085,20 +1213,24 @@ hipError_t launch_net_backward(const NetBuffers &nb, const NetSystem &sys, const
                                const __bf16 *wb, float gmax, float *grad, hipStream_t st) {
     const int n = sys.n;
     hipError_t e;
-    const int rb = row_blocks(n);
+    const int rb = std::min(kReadoutParts, exact_blocks((long long)n * 16, kBlock * kReadRows));
     readout_bwd_kernel<<<rb, kBlock, 0, st>>>(nb.h3, params + kOffR, gmax, n, nb.dgh, nb.dz,
                                               nb.rpart);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = launch_reduce_parts(nb.rpart, rb, kReadout, kReadout, grad + kOffR, st)) != hipSuccess)
-        return e;
+    RedSets sets;
+    int blocks = 0, used = 0;
+    auto reduce = [&](const float *part, int parts, int columns, float *out) {
+        sets.set[used++] = {part, out, parts, columns, blocks};
+        blocks += (columns + kWave - 1) / kWave;
+    };
+    reduce(nb.rpart, rb, kReadout, grad + kOffR);
     const int gb = exact_blocks(n, 16 * kWavesPerBlock);  // one 16-row tile per wavefront
-    const int wgb = std::min(nb.wparts, blocks_for(n, 32));
+    const int wgb = std::min(kWeightParts, exact_blocks(n, kWgRows));
     for (int l = kLayers - 1; l >= 0; l--) {
-        gemm_bwd_weight_kernel<kXW><<<wgb, kBlock, 0, st>>>(nb.x[l], kXW, n, nb.dz, nb.wpart);
+        float *part = nb.wpart + (size_t)l * kWeightParts * kLayerStride;
+        gemm_bwd_weight_kernel<kXW><<<wgb, kWgBlock, 0, st>>>(nb.x[l], kXW, n, nb.dz, part);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        if ((e = launch_reduce_parts(nb.wpart, wgb, kLayerStride, kLayerStride,
-                                     grad + kOffW1 + l * kLayerStride, st)) != hipSuccess)
-            return e;
+        reduce(part, wgb, kLayerStride, grad + kOffW1 + l * kLayerStride);
         gemm_bwd_data_kernel<<<gb, kBlock, 0, st>>>(
             nb.dz, n, wb + kWtRowMajor + kK0 * kHid + l * kXW * kHid, nb.dx);
         if ((e = hipGetLastError()) != hipSuccess) return e;
@@ -1106,10 +1238,12 @@ hipError_t launch_net_backward(const NetBuffers &nb, const NetSystem &sys, const
                                                                nb.x[l], n, nb.dz);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    gemm_bwd_weight_kernel<kK0><<<wgb, kBlock, 0, st>>>(nb.x0, kK0, n, nb.dz, nb.wpart);
+    float *part = nb.wpart + (size_t)kLayers * kWeightParts * kLayerStride;
+    gemm_bwd_weight_kernel<kK0><<<wgb, kWgBlock, 0, st>>>(nb.x0, kK0, n, nb.dz, part);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    return launch_reduce_parts(nb.wpart, wgb, kK0 * kHid + kHid, kK0 * kHid + kHid, grad + kOffW0,
-                               st);
+    reduce(part, wgb, kK0 * kHid + kHid, grad + kOffW0);
+    reduce_parts_kernel<<<blocks, kRedWaves * kWave, 0, st>>>(sets);
+    return hipGetLastError();
 }
 
 hipError_t launch_adam(float *p, const float *g, float *m1, float *m2, int count, float lr,
@@ -1132,8 +1266,8 @@ hipError_t launch_pack_weights(const float *params, __bf16 *wb, hipStream_t st) 
 
 hipError_t launch_precond_values(const PrecondOp &op, const double *adiag, const float *gh,
                                  hipStream_t st) {
-    precond_values_kernel<<<blocks_for(op.n), kBlock, 0, st>>>(op.n, op.off, op.col, op.src_val,
-                                                               adiag, gh, op.val, op.val32);
+    precond_values_kernel<<<exact_blocks((long long)op.n * 8, kBlock), kBlock, 0, st>>>(
+        op.n, op.off, op.col, op.src_val, adiag, gh, op.val, op.val32);
     return hipGetLastError();
 }
 

@@ -53,7 +53,6 @@ int ctx_n(const npbcg_ctx *c);
 namespace {
 
 constexpr float kGmax = 1.0f;      // |g|, |h| <= 1: scales within [1/e, e]
-constexpr int kWeightParts = 512;  // workgroups of the weight-gradient GEMMs
 
 uint64_t splitmix64(uint64_t &s) {
     uint64_t z = (s += 0x9E3779B97F4A7C15ull);
@@ -107,10 +106,9 @@ int ensure_buffers(npbcg_net *net, int n) {
     NET_HIP(hipMalloc(&nb.dgh, sizeof(float) * 2 * m));
     NET_HIP(hipMalloc(&nb.pw, sizeof(float) * kPairs * m));
     NET_HIP(hipMalloc(&nb.pd, sizeof(float) * kPairs * m));
-    nb.wparts = kWeightParts;
-    NET_HIP(hipMalloc(&nb.wpart, sizeof(float) * kWeightParts * kLayerStride));
-    NET_HIP(hipMalloc(&nb.rpart, sizeof(float) * row_blocks(n) * kReadout));
-    NET_HIP(hipMalloc(&nb.loss_part, sizeof(double) * row_blocks(n)));
+    NET_HIP(hipMalloc(&nb.wpart, sizeof(float) * (kLayers + 1) * kWeightParts * kLayerStride));
+    NET_HIP(hipMalloc(&nb.rpart, sizeof(float) * kReadoutParts * kReadout));
+    NET_HIP(hipMalloc(&nb.loss_part, sizeof(double) * pair_blocks(n)));
     nb.cap = n;
     return NPBCG_OK;
 }
@@ -151,16 +149,16 @@ int evaluate(npbcg_net *net, npbcg_ctx *ctx, bool grad, bool base, bool relative
         NET_HIP(launch_feature_stats(sys.feat, sys.n, net->norm, st));
         net->norm_set = true;
     }
-    const int rb = row_blocks(sys.n);
+    const int parts = pair_blocks(sys.n);
     if (base) {
         NetBuffers b0 = nb;
         b0.gh = const_cast<float *>(npbcg_detail::ctx_zero_gh(ctx));
         NET_HIP(launch_pair_loss(b0, sys, ps, 0, st));
-        NET_HIP(launch_sum(nb.loss_part, rb, net->d_loss + 1, st));
+        NET_HIP(launch_sum(nb.loss_part, parts, net->d_loss + 1, st));
     }
     NET_HIP(launch_net_forward(nb, sys, net->params, net->wb, kGmax, st));
     NET_HIP(launch_pair_loss(nb, sys, ps, grad ? 1 : 0, st));
-    NET_HIP(launch_sum(nb.loss_part, rb, net->d_loss, st));
+    NET_HIP(launch_sum(nb.loss_part, parts, net->d_loss, st));
     if (grad) {
         NET_HIP(launch_net_backward(nb, sys, net->params, net->wb, kGmax, net->grad, st));
         if (relative) NET_HIP(launch_scale_inverse(net->grad, kParams, net->d_loss + 1, st));
