@@ -1709,17 +1709,11 @@ int ensure_mixed(npbcg_ctx *c) {
     return NPBCG_OK;
 }
 
-// One or two sets of device scalars, once the stream has run what it holds.
-int read_scalars_from(npbcg_ctx *c, const Scalars *dev, Scalars *out,
-                      const Scalars *dev2 = nullptr, Scalars *out2 = nullptr) {
-    Scalars *stage = reinterpret_cast<Scalars *>(c->h_stage);
-    NPBCG_HIP(hipMemcpyAsync(stage, dev, sizeof(Scalars), hipMemcpyDeviceToHost, c->stream));
-    if (dev2)
-        NPBCG_HIP(hipMemcpyAsync(stage + 1, dev2, sizeof(Scalars), hipMemcpyDeviceToHost,
-                                 c->stream));
+int read_scalars_from(npbcg_ctx *c, const Scalars *dev, Scalars *out) {
+    NPBCG_HIP(hipMemcpyAsync(c->h_stage, dev, sizeof(Scalars), hipMemcpyDeviceToHost,
+                             c->stream));
     NPBCG_HIP(hipStreamSynchronize(c->stream));
-    std::memcpy(out, stage, sizeof(Scalars));
-    if (dev2) std::memcpy(out2, stage + 1, sizeof(Scalars));
+    std::memcpy(out, c->h_stage, sizeof(Scalars));
     return NPBCG_OK;
 }
 
@@ -2241,53 +2235,39 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
         if (relres <= rtol) bud[0] = std::min(batch0, sc.steps + 1);
     } else {
         const npbcg_dev::MixedProblem &mp = c->mp;
-        Fp64Problem inner = pbs;  // same launch shapes, inner scalars
-        inner.sc = mp.sc;
-        // Sweeps are decided on the device (launch_sweep_prepare), so two are
+        // Sweeps are decided on the device (resid_finish_kernel), so two are
         // enqueued before the first host synchronisation (FP32 holds about
         // 1e-6 per sweep, so two reach 1e-10 from x = 0 on well-conditioned
         // systems); later ones go one at a time.  maxit is checked per sweep.
         int *bud = c->budget[1][c->active_precond];
         const int b1 = bud[0] > 0 ? bud[0] : batch0 - 2;
         const int b2 = bud[1] > 0 ? bud[1] : batch0 / 2 + 1;
+        const npbcg_dev::NextSweep next{mp.d, mp.r,       mp.p,        mp.minv, mp.part_xx,
+                                        mp.sc, c->rhs_norm, rtol, maxit};
         auto sweep = [&](int index) -> hipError_t {
             const int steps = index == 0 ? b1 : index == 1 ? b2 : batch0 / 2 + 1;
-            hipError_t e = npbcg_dev::launch_sweep_prepare(pbs.sc, mp.sc, c->rhs_norm, rtol,
-                                                           maxit, index == 0 ? 1 : 0, c->stream);
-            if (e == hipSuccess)
-                e = npbcg_dev::enqueue_inner32(pbs, mp, index == 0 ? 1 : 0, steps, c->stream);
+            hipError_t e = npbcg_dev::enqueue_inner32(pbs, mp, steps, c->stream);
             if (e == hipSuccess) e = npbcg_dev::launch_refine(pbs, mp, c->stream);
-            if (e == hipSuccess) e = npbcg_dev::launch_resid(pbs, 0, c->stream);
-            return e;
-        };
-        auto first_two = [&]() -> hipError_t {
-            hipError_t e = npbcg_dev::launch_reset_scalars(pbs, 0.0, c->stream, rtol, 0);
-            if (e == hipSuccess) e = npbcg_dev::launch_reset_scalars(inner, 0.0, c->stream, 1e-6, 1);
-            if (e == hipSuccess)
-                e = npbcg_dev::launch_fill(pbs.z, c->n + 1, 0.0, c->pb.vec_blocks, c->stream);
-            if (e == hipSuccess) e = sweep(0);
-            if (e == hipSuccess) e = sweep(1);
+            if (e == hipSuccess) e = npbcg_dev::launch_resid(pbs, 0, c->stream, next);
             return e;
         };
         NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
-        NPBCG_HIP(first_two());
-        int enqueued = 2, inner_steps = 0, si_last_steps = 0;
-        for (bool first = true;; first = false) {
-            if (!first) NPBCG_HIP(sweep(enqueued++));
+        NPBCG_HIP(npbcg_dev::launch_begin32(pbs, mp, rtol, c->stream));
+        NPBCG_HIP(sweep(0));
+        int enqueued = 1;
+        do {
+            NPBCG_HIP(sweep(enqueued++));
             NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
-            Scalars si{};
-            int rc = read_scalars_from(c, pbs.sc, &sc, mp.sc, &si);
+            int rc = read_scalars_from(c, pbs.sc, &sc);
             if (rc != NPBCG_OK) return rc;
-            inner_steps = sc.inner_total + si.steps;
-            si_last_steps = si.steps;
             relres = sc.rnorm / c->rhs_norm;
-            if (relres <= rtol || inner_steps >= maxit || enqueued >= 1000) break;
-        }
-        s.sweeps = sc.sweeps;
+        } while (!(relres <= rtol) && sc.inner_total < maxit && enqueued < 1000);
+        const int inner_steps = sc.inner_total;
+        s.sweeps = std::min(sc.sweeps, enqueued);  // (one more may be decided on, not run)
         s.iterations = inner_steps;
         if (relres <= rtol && s.sweeps == 2) {  // the common case: learn both budgets
             bud[0] = std::min(batch0 - 2, std::max(2, sc.sweep1_steps + 1));
-            bud[1] = std::min(batch0 / 2 + 1, std::max(2, si_last_steps + 1));
+            bud[1] = std::min(batch0 / 2 + 1, std::max(2, sc.sweep2_steps + 1));
         } else if (relres <= rtol && s.sweeps == 1) {
             bud[0] = std::min(batch0 - 2, std::max(2, sc.sweep1_steps + 1));
         } else if (relres <= rtol) {  // needed more sweeps: back to the defaults

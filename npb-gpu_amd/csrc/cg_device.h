@@ -183,6 +183,33 @@ struct Scalars {
     double cg_alpha[2];
 };
 
+// Next sweep of a mixed solve whose relative residual is rel: its inner stop level
+// max(1e-6, rtol / (2 rel))^2, or nothing to do (stop).
+__device__ __forceinline__ void start_sweep(Scalars *outer, Scalars *inner, double rel,
+                                            double rtol, bool stop) {
+    const double t = fmax(1e-6, 0.5 * rtol / fmax(rel, 1e-300));
+    inner->rtol2 = t * t;
+    inner->tol2 = 0.0;
+    inner->stop_enabled = 1;
+    inner->steps = 0;
+    inner->done = stop ? 1 : 0;
+    outer->skip_resid = stop ? 1 : 0;
+    if (!stop) outer->sweeps += 1;
+}
+
+// Row j of an inner solve's start from the residual v: d = 0, r = v, p = M^-1 r in
+// FP32; returns r.p.
+__device__ __forceinline__ double start32(double v, int j, float *__restrict__ d,
+                                          float *__restrict__ r, float *__restrict__ p,
+                                          const float *__restrict__ minv) {
+    const float rj = (float)v;
+    const float sj = minv ? minv[j] * rj : rj;
+    d[j] = 0.0f;
+    r[j] = rj;
+    p[j] = sj;
+    return (double)rj * (double)sj;
+}
+
 // Sum of this workgroup's per-thread values, written to part[blockIdx.x]
 // (one store per workgroup; fixed order: DPP tree per wave, waves in order).
 template <int BLOCK>

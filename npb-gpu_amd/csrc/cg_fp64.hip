@@ -294,13 +294,15 @@ __global__ __launch_bounds__(kBlock) void combine_rows_kernel(
 }
 
 // r = sum over blocks of the residual SpMV's row partials, with partials of
-// ||x - r||^2, x.z and z.z (stride gridDim.x).
+// ||x - r||^2, x.z and z.z (stride gridDim.x).  In a mixed solve (next.d given) also
+// the start of the next sweep's inner solve on x - r, so that it needs no pass of
+// its own.
 __global__ __launch_bounds__(kBlock) void resid_combine_kernel(
     const double *__restrict__ rows_part, const int *__restrict__ row_slot, int nblk,
     const double *__restrict__ x, const double *__restrict__ z, double *__restrict__ r, int n,
-    double *__restrict__ res, const Scalars *__restrict__ sc) {
+    double *__restrict__ res, const Scalars *__restrict__ sc, NextSweep next) {
     if (sc->skip_resid) return;
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0;
+    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
     for (int j = xcd_chunk(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; j < n;
          j += gridDim.x * kBlock) {
         double rj = rows_part[row_slot[j]];
@@ -312,6 +314,11 @@ __global__ __launch_bounds__(kBlock) void resid_combine_kernel(
         a0 += dlt * dlt;
         a1 += xv * zv;
         a2 += zv * zv;
+        if (next.d) a3 += start32(dlt, j, next.d, next.r, next.p, next.minv);
+    }
+    if (next.d) {
+        store_block_partial<kBlock>(a3, next.rr);
+        __syncthreads();
     }
     store_block_partial<kBlock>(a0, res);
     __syncthreads();
@@ -608,12 +615,14 @@ __global__ __launch_bounds__(kBlock) void cg_init_kernel(
 
 // One workgroup: reduce the residual SpMV's partials and form
 // rnorm = ||x - A z|| (cg.cu:795-800), norm_temp1 = x.z, norm_temp2 =
-// 1/sqrt(z.z) and zeta = shift + 1/(x.z) (:505-514).
+// 1/sqrt(z.z) and zeta = shift + 1/(x.z) (:505-514).  In a mixed solve
+// (next.inner given) then the decision on the next sweep: stop when rtol is met or
+// maxit inner steps are used up.
 __global__ __launch_bounds__(kBlock) void resid_finish_kernel(
     const double *__restrict__ res, int count, Scalars *sc,
     double *__restrict__ zeta_hist, double *__restrict__ rnorm_hist, int hist_cap,
-    int record) {
-    if (sc->skip_resid) return;
+    int record, NextSweep next) {
+    if (sc->skip_resid) return;  // nothing changed since the decision to stop
     const double s0 = reduce_partials<kBlock>(res, count);
     const double s1 = reduce_partials<kBlock>(res + count, count);
     const double s2 = reduce_partials<kBlock>(res + 2 * count, count);
@@ -632,6 +641,15 @@ __global__ __launch_bounds__(kBlock) void resid_finish_kernel(
                 rnorm_hist[it] = rnorm;
             }
             sc->iter = it + 1;
+        }
+        if (next.inner) {
+            const int steps = next.inner->steps;
+            sc->inner_total += steps;
+            if (sc->sweeps == 1) sc->sweep1_steps = steps;
+            if (sc->sweeps == 2) sc->sweep2_steps = steps;
+            const double rel = rnorm / next.rhs_norm;
+            start_sweep(sc, next.inner, rel, next.rtol,
+                        rel <= next.rtol || sc->inner_total >= next.maxit);
         }
     }
 }
@@ -915,19 +933,19 @@ hipError_t launch_spmv_kernel(const Fp64Problem &pb, int step, hipEvent_t e0, hi
     return launch_spmv<0>(pb, st, e0, e1, step);
 }
 
-hipError_t launch_resid(const Fp64Problem &pb, int record, hipStream_t st) {
+hipError_t launch_resid(const Fp64Problem &pb, int record, hipStream_t st, const NextSweep &next) {
     hipError_t e = launch_spmv<1>(pb, st);
     if (e != hipSuccess) return e;
     if (pb.spmv_variant == kSpmvTiled) {
         resid_combine_kernel<<<pb.vec_blocks, kBlock, 0, st>>>(
             pb.sell.rows_part, pb.sell.row_slot, pb.sell.nblk, pb.x, pb.z, pb.r, pb.n,
-            pb.part.res, pb.sc);
+            pb.part.res, pb.sc, next);
         e = noted(pb, hipGetLastError(), "resid_combine_kernel", kBlock, st);
         if (e != hipSuccess) return e;
     }
     resid_finish_kernel<<<1, kBlock, 0, st>>>(pb.part.res, resid_partials(pb), pb.sc,
                                               pb.zeta_hist, pb.rnorm_hist, pb.hist_cap,
-                                              record);
+                                              record, next);
     return noted(pb, hipGetLastError(), "resid_finish_kernel", kBlock, st);
 }
 

@@ -148,7 +148,18 @@ hipError_t launch_spmv_kernel(const Fp64Problem &pb, int step, hipEvent_t e0, hi
                               hipStream_t st);
 // r = A z (partials ||x - r||^2, x.z, z.z), then a one-workgroup finish that
 // forms rnorm, zeta, xscale and, with record != 0, appends to the history.
-hipError_t launch_resid(const Fp64Problem &pb, int record, hipStream_t st);
+// `next` (mixed solves): the start of the next sweep, decided on the device, so that
+// several sweeps are enqueued with one host synchronisation.
+struct NextSweep {
+    float *d = nullptr, *r = nullptr, *p = nullptr;  // inner vectors to start
+    const float *minv = nullptr;
+    double *rr = nullptr;       // r.p partials [vec_blocks]
+    Scalars *inner = nullptr;
+    double rhs_norm = 0.0, rtol = 0.0;
+    int maxit = 0;
+};
+hipError_t launch_resid(const Fp64Problem &pb, int record, hipStream_t st,
+                        const NextSweep &next = NextSweep{});
 hipError_t launch_cg_init(const Fp64Problem &pb, int scale_x, hipStream_t st);
 // CG step `step` of a sequence; with sets_tol, step 0 also fixes the solve's
 // stop level from its r0.r0.
@@ -212,10 +223,14 @@ hipError_t prepare_mixed_kernels(int lds_bytes);
 hipError_t launch_spmv32_kernel(const Fp64Problem &pb, const MixedProblem &mp, int step,
                                 hipEvent_t e0, hipEvent_t e1, hipStream_t st);
 hipError_t launch_to_fp32(const double *src, float *dst, long long count, hipStream_t st);
-// Inner FP32 CG on A d = b - A x (or b on the first sweep): init and `steps`
-// steps; pb is the solve view (x holds b, z the FP64 iterate, r = A z).
-hipError_t enqueue_inner32(const Fp64Problem &pb, const MixedProblem &mp, int first_sweep,
-                           int steps, hipStream_t st);
+// Start of a mixed solve: x = 0 (pb is the solve view: x holds b, z the FP64
+// iterate), both levels' scalars, the first inner solve's vectors.
+hipError_t launch_begin32(const Fp64Problem &pb, const MixedProblem &mp, double rtol,
+                          hipStream_t st);
+// Inner FP32 CG on A d = r (the FP64 residual), `steps` steps from the vectors that
+// launch_begin32 or the last residual pass (NextSweep) started.
+hipError_t enqueue_inner32(const Fp64Problem &pb, const MixedProblem &mp, int steps,
+                           hipStream_t st);
 // z += d (the FP64 iterate takes the FP32 correction).
 hipError_t launch_refine(const Fp64Problem &pb, const MixedProblem &mp, hipStream_t st);
 // r = b - r (r held A z), p = r, r.r partials into part.xx.
@@ -224,14 +239,6 @@ hipError_t launch_residual_restart(const Fp64Problem &pb, hipStream_t st);
 hipError_t launch_narrow(const double *in, float *out, int n, int blocks, hipStream_t st);
 // minv = 1/diag(A) from the CSR.
 hipError_t launch_jacobi(const Fp64Problem &pb, double *minv, hipStream_t st);
-
-// Start of a refinement sweep of the mixed solve, decided on the device from
-// the FP64 true residual of the previous sweep (outer->rnorm): if it met rtol
-// (or maxit inner steps are used up) the inner solve and this sweep's residual
-// pass are skipped; else the inner stop level max(1e-6, rtol/(2 relres))^2 is
-// set.  Lets several sweeps be enqueued with one host synchronisation.
-hipError_t launch_sweep_prepare(Scalars *outer, Scalars *inner, double rhs_norm, double rtol,
-                                int maxit, int first, hipStream_t st);
 
 size_t scalars_bytes();
 

@@ -38,11 +38,14 @@ __global__ __launch_bounds__(kBlock) void to_fp32_kernel(const double *__restric
 // sort window, so storing them straight away writes 4 bytes into each of up
 // to 64 cache lines.  stage_rows = 0 stores them directly (ranges whose rows
 // do not fit in the LDS beside the vector block).
-// PUPD: the previous step's p update is done here.  beta = (r.r) / (old r.r)
-// from the partials and the stop test on r.r (one workgroup records it; all
-// workgroups reach the same decision and return); else p = r + beta p_old is
+// PUPD: the previous step's p update is done here.  beta = (r.z) / (old r.z)
+// from the partials (r is z without a preconditioner) and the stop test on r.z, or
+// on stop_part's r.r when that is given (one workgroup records it; all
+// workgroups reach the same decision and return); else p = z + beta p_old is
 // formed while the vector block is staged, and the workgroups of row range 0
-// store their block of it in p_new (p_old and p_new are different buffers).
+// store their block of it in p_new (p_old and p_new are different buffers).  z is
+// r, or minv r when minv is given.  (A launch of its own for the p update took
+// 3.3 us and a launch boundary of each step with a preconditioner.)
 template <int BLOCK, int UNR, bool PUPD>
 __global__ __launch_bounds__(BLOCK) void spmv_sell32_kernel(
     const int *__restrict__ wg_slice, const int *__restrict__ slice_off,
@@ -51,13 +54,15 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell32_kernel(
     float *__restrict__ rows_part, double *__restrict__ dot_part, int n, int W, int nrange,
     Scalars *sc, const float *__restrict__ r, float *__restrict__ p_new,
     const double *__restrict__ rr_part, const double *__restrict__ rho_part, int n_vec,
-    int rev, int stage_rows) {
+    int rev, int stage_rows, const float *__restrict__ minv,
+    const double *__restrict__ stop_part) {
     if (sc->done) return;
     float b32 = 0.0f;
     if constexpr (PUPD) {
         double rho, rho0;
         reduce_partials2<BLOCK>(rr_part, n_vec, rho_part, n_vec, rho, rho0);
-        const bool stop = fabs(rho) <= sc->tol2;
+        const double level = stop_part ? reduce_partials<BLOCK>(stop_part, n_vec) : rho;
+        const bool stop = fabs(level) <= sc->tol2;
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             sc->rho = rho;
             sc->beta = rho / rho0;
@@ -111,17 +116,29 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell32_kernel(
         float2 *o2 = reinterpret_cast<float2 *>(p_new + c0);
         float2 *l2 = reinterpret_cast<float2 *>(vblk);
         const bool store = (wg % nrange) == 0;
+        auto form = [&](auto z2) {
 #pragma unroll 4
-        for (int i = threadIdx.x; i < wb / 2; i += BLOCK) {
-            const float2 pv = v2[i], rv = r2[i];
-            float2 nv;
-            nv.x = fmaf(b32, pv.x, rv.x);
-            nv.y = fmaf(b32, pv.y, rv.y);
-            l2[i] = nv;
-            if (store) o2[i] = nv;
+            for (int i = threadIdx.x; i < wb / 2; i += BLOCK) {
+                const float2 pv = v2[i], zv = z2(i);
+                float2 nv;
+                nv.x = fmaf(b32, pv.x, zv.x);
+                nv.y = fmaf(b32, pv.y, zv.y);
+                l2[i] = nv;
+                if (store) o2[i] = nv;
+            }
+        };
+        if (minv) {
+            const float2 *m2 = reinterpret_cast<const float2 *>(minv + c0);
+            form([&](int i) {
+                const float2 rv = r2[i], mv = m2[i];
+                return make_float2(mv.x * rv.x, mv.y * rv.y);
+            });
+        } else {
+            form([&](int i) { return r2[i]; });
         }
         if ((wb & 1) && threadIdx.x == 0) {
-            const float nv = fmaf(b32, v[c0 + wb - 1], r[c0 + wb - 1]);
+            const int at = c0 + wb - 1;
+            const float nv = fmaf(b32, v[at], minv ? minv[at] * r[at] : r[at]);
             vblk[wb - 1] = nv;
             if (store) p_new[c0 + wb - 1] = nv;
         }
@@ -144,7 +161,8 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell32_kernel(
         }
         // p of the lane's row for p.q, loaded while the slice streams
         float pr = 0.0f;
-        if (row >= 0) pr = PUPD ? fmaf(b32, v[row], r[row]) : v[row];
+        if (row >= 0)
+            pr = PUPD ? fmaf(b32, v[row], minv ? minv[row] * r[row] : r[row]) : v[row];
         float acc = 0.0f;
         const int nch = (width + UNR - 1) / UNR;
         for (int ch = 0; ch < nch; ch++) {
@@ -192,20 +210,35 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell32_kernel(
     store_block_partial<BLOCK>(dot, dot_part);
 }
 
-// Start of an inner solve: d = 0, r = p = fp32(b - Ax) (or fp32(b) on the
-// first sweep, x = 0), FP64 partials of r.r.
-__global__ __launch_bounds__(kBlock) void init32_kernel(
-    const double *__restrict__ b, const double *__restrict__ ax, int first, int n,
-    float *__restrict__ d, float *__restrict__ r, float *__restrict__ p,
-    double *__restrict__ rr_out, const float *__restrict__ minv) {
+// Start of a mixed solve: z = 0, the scalars of both levels, and the
+// first inner solve's d = 0, r = fp32(b), p = M^-1 r with FP64 partials of r.p
+// (later sweeps start in resid_combine_kernel).
+__global__ __launch_bounds__(kBlock) void begin32_kernel(
+    const double *__restrict__ b, double *__restrict__ z, int n, float *__restrict__ d,
+    float *__restrict__ r, float *__restrict__ p, double *__restrict__ rr_out,
+    const float *__restrict__ minv, Scalars *outer, Scalars *inner, double rtol) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        z[n] = 0.0;
+        for (Scalars *sc : {outer, inner}) {
+            sc->iter = 0;
+            sc->shift = 0.0;
+            sc->tol2 = 0.0;
+            sc->done = 0;
+            sc->steps = 0;
+            sc->skip_resid = 0;
+            sc->sweeps = 0;
+            sc->inner_total = 0;
+            sc->sweep1_steps = 0;
+            sc->sweep2_steps = 0;
+        }
+        outer->rtol2 = rtol * rtol;
+        outer->stop_enabled = 0;
+        start_sweep(outer, inner, 1.0, rtol, false);
+    }
     double acc = 0.0;
     for (int j = blockIdx.x * kBlock + threadIdx.x; j < n; j += gridDim.x * kBlock) {
-        const float rj = (float)(first ? b[j] : b[j] - ax[j]);
-        const float sj = minv ? minv[j] * rj : rj;  // s = M^-1 r
-        d[j] = 0.0f;
-        r[j] = rj;
-        p[j] = sj;
-        acc += (double)rj * (double)sj;
+        z[j] = 0.0;
+        acc += start32(b[j], j, d, r, p, minv);
     }
     store_block_partial<kBlock>(acc, rr_out);
 }
@@ -281,72 +314,12 @@ __global__ __launch_bounds__(kBlock) void update_zr32_kernel(
     store_block_partial<kBlock>(acc, rr_out);
 }
 
-// beta = (new r.r) / (old r.r) in FP64; p = r + beta p; stop test (on
-// stop_part, the r.r of a sparse-preconditioned solve, when given).
-__global__ __launch_bounds__(kBlock) void update_p32_kernel(
-    const float *__restrict__ r, float *__restrict__ p, int n,
-    const double *__restrict__ rr_part, const double *__restrict__ rho_part, Scalars *sc,
-    const float *__restrict__ minv, const double *__restrict__ stop_part) {
-    if (sc->done) return;
-    // first row loaded ahead of the reductions (as in update_zr32_kernel)
-    const int j0 = blockIdx.x * kBlock + threadIdx.x;
-    float r0 = 0.0f, p0 = 0.0f, m0 = 0.0f;
-    if (j0 < n) {
-        r0 = r[j0];
-        p0 = p[j0];
-        if (minv) m0 = minv[j0];
-    }
-    double rho, rho0;
-    reduce_partials2<kBlock>(rr_part, gridDim.x, rho_part, gridDim.x, rho, rho0);
-    const double beta = rho / rho0;
-    const double level = stop_part ? reduce_partials<kBlock>(stop_part, gridDim.x) : rho;
-    const bool stop = fabs(level) <= sc->tol2;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        sc->rho = rho;
-        sc->beta = beta;
-        if (stop) sc->done = 1;
-    }
-    if (stop) return;
-    const float b32 = (float)beta;
-    if (j0 < n) p[j0] = minv ? fmaf(b32, p0, m0 * r0) : fmaf(b32, p0, r0);
-    if (minv) {
-        for (int j = j0 + gridDim.x * kBlock; j < n; j += gridDim.x * kBlock)
-            p[j] = fmaf(b32, p[j], minv[j] * r[j]);
-    } else {
-        for (int j = j0 + gridDim.x * kBlock; j < n; j += gridDim.x * kBlock)
-            p[j] = fmaf(b32, p[j], r[j]);
-    }
-}
-
-__global__ void sweep_prepare_kernel(Scalars *outer, Scalars *inner, double rhs_norm,
-                                     double rtol, int maxit, int first) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        if (first) {
-            outer->inner_total = 0;
-            outer->sweeps = 0;
-            outer->sweep1_steps = 0;
-            outer->sweep2_steps = 0;
-        } else {
-            outer->inner_total += inner->steps;
-            if (outer->sweeps == 1) outer->sweep1_steps = inner->steps;
-            if (outer->sweeps == 2) outer->sweep2_steps = inner->steps;
-        }
-        const double rel = first ? 1.0 : outer->rnorm / rhs_norm;
-        const bool stop = (!first && rel <= rtol) || outer->inner_total >= maxit;
-        const double t = fmax(1e-6, 0.5 * rtol / fmax(rel, 1e-300));
-        inner->rtol2 = t * t;
-        inner->tol2 = 0.0;
-        inner->stop_enabled = 1;
-        inner->steps = 0;
-        inner->done = stop ? 1 : 0;
-        outer->skip_resid = stop ? 1 : 0;
-        if (!stop) outer->sweeps += 1;
-    }
-}
-
-// x += d (FP64 accumulation of the FP32 correction).
+// x += d (FP64 accumulation of the FP32 correction), unless the sweep is not
+// needed (d is then the last one's).
 __global__ __launch_bounds__(kBlock) void refine_kernel(double *__restrict__ x,
-                                                       const float *__restrict__ d, int n) {
+                                                       const float *__restrict__ d, int n,
+                                                       const Scalars *__restrict__ sc) {
+    if (sc->skip_resid) return;
     for (int j = blockIdx.x * kBlock + threadIdx.x; j < n; j += gridDim.x * kBlock)
         x[j] += (double)d[j];
 }
@@ -404,18 +377,19 @@ hipError_t prepare_mixed_kernels(int lds_bytes) {
 template <bool PUPD>
 static hipError_t launch_spmv32(const Fp64Problem &pb, const MixedProblem &mp, const float *v,
                                 float *p_new, const double *rr_part, const double *rho_part,
-                                int rev, hipStream_t st) {
+                                const double *stop_part, int rev, hipStream_t st) {
     const SellDev &sd = pb.sell;
+    const float *z = mp.pop ? mp.pz : mp.r;
     if (sd.block == 512)
         spmv_sell32_kernel<512, kSellUnr32, PUPD><<<sd.grid, 512, mp.lds_bytes, st>>>(
             sd.wg_slice, sd.slice_off, sd.slice_row, mp.val, sd.col, v, mp.rows_part, mp.part_pq,
-            pb.n, sd.W, sd.nrange, mp.sc, mp.r, p_new, rr_part, rho_part, pb.vec_blocks, rev,
-            mp.stage_rows);
+            pb.n, sd.W, sd.nrange, mp.sc, z, p_new, rr_part, rho_part, pb.vec_blocks, rev,
+            mp.stage_rows, mp.minv, stop_part);
     else
         spmv_sell32_kernel<1024, kSellUnr32, PUPD><<<sd.grid, 1024, mp.lds_bytes, st>>>(
             sd.wg_slice, sd.slice_off, sd.slice_row, mp.val, sd.col, v, mp.rows_part, mp.part_pq,
-            pb.n, sd.W, sd.nrange, mp.sc, mp.r, p_new, rr_part, rho_part, pb.vec_blocks, rev,
-            mp.stage_rows);
+            pb.n, sd.W, sd.nrange, mp.sc, z, p_new, rr_part, rho_part, pb.vec_blocks, rev,
+            mp.stage_rows, mp.minv, stop_part);
     return hipGetLastError();
 }
 
@@ -432,13 +406,13 @@ hipError_t launch_spmv32_kernel(const Fp64Problem &pb, const MixedProblem &mp, i
                               (uint32_t)mp.lds_bytes, st, e0, e1, 0u, sd.wg_slice, sd.slice_off,
                               sd.slice_row, mp.val, sd.col, v, mp.rows_part, mp.part_pq, pb.n, sd.W,
                               sd.nrange, mp.sc, r_none, p_none, d_none, d_none, pb.vec_blocks, rev,
-                              mp.stage_rows);
+                              mp.stage_rows, r_none, d_none);
     else
         hipExtLaunchKernelGGL(spmv_sell32_kernel<1024, kSellUnr32, false>, dim3(sd.grid),
                               dim3(1024), (uint32_t)mp.lds_bytes, st, e0, e1, 0u, sd.wg_slice,
                               sd.slice_off, sd.slice_row, mp.val, sd.col, v, mp.rows_part,
                               mp.part_pq, pb.n, sd.W, sd.nrange, mp.sc, r_none, p_none, d_none,
-                              d_none, pb.vec_blocks, rev, mp.stage_rows);
+                              d_none, pb.vec_blocks, rev, mp.stage_rows, r_none, d_none);
     return hipGetLastError();
 }
 
@@ -447,64 +421,49 @@ hipError_t launch_to_fp32(const double *src, float *dst, long long count, hipStr
     return hipGetLastError();
 }
 
-static const double *rho32_source(const MixedProblem &mp, int step) {
-    return step == 0 ? mp.part_xx : mp.part_rr[(step - 1) & 1];
+hipError_t launch_begin32(const Fp64Problem &pb, const MixedProblem &mp, double rtol,
+                          hipStream_t st) {
+    begin32_kernel<<<pb.vec_blocks, kBlock, 0, st>>>(pb.x, pb.z, pb.n, mp.d, mp.r, mp.p,
+                                                     mp.part_xx, mp.minv, pb.sc, mp.sc, rtol);
+    return hipGetLastError();
 }
 
-hipError_t enqueue_inner32(const Fp64Problem &pb, const MixedProblem &mp, int first_sweep,
-                           int steps, hipStream_t st) {
+hipError_t enqueue_inner32(const Fp64Problem &pb, const MixedProblem &mp, int steps,
+                           hipStream_t st) {
     const int vb = pb.vec_blocks;
-    init32_kernel<<<vb, kBlock, 0, st>>>(pb.x, pb.r, first_sweep, pb.n, mp.d, mp.r, mp.p,
-                                         mp.part_xx, mp.minv);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && mp.pop)  // p = z = M^-1 r; r0.z0 into rz[1], r0.r0 stays in xx
-        e = launch_precond_apply32(*mp.pop, mp.r, mp.pz, mp.p, mp.part_rz[1], vb, nullptr, st);
+    hipError_t e = hipSuccess;
+    if (mp.pop)  // p = z = M^-1 r; r0.z0 into rz[1], r0.r0 stays in xx
+        e = launch_precond_apply32(*mp.pop, mp.r, mp.pz, mp.p, mp.part_rz[1], vb, mp.sc, st);
     const SellDev &sd = pb.sell;
-    // Plain CG: the p update of step it-1 runs inside step it's SpMV (two
-    // launches per step), p alternating between mp.p and mp.p_alt.
-    const bool fused = !mp.pop && !mp.minv && mp.p_alt;
+    // r.z after step `step` (-1: the start's)
+    auto rz = [&](int step) -> const double * {
+        if (mp.pop) return mp.part_rz[step & 1];
+        return step < 0 ? mp.part_xx : mp.part_rr[step & 1];
+    };
+    // The p update of step it-1 runs inside step it's SpMV, p alternating
+    // between mp.p and mp.p_alt.
     float *pbuf[2] = {mp.p, mp.p_alt};
     for (int it = 0; it < steps && e == hipSuccess; it++) {
-        float *p_it = fused ? pbuf[it & 1] : mp.p;
-        if (fused && it > 0)
-            e = launch_spmv32<true>(pb, mp, pbuf[(it - 1) & 1], p_it, mp.part_rr[(it - 1) & 1],
-                                    rho32_source(mp, it - 1), it & 1, st);
-        else
-            e = launch_spmv32<false>(pb, mp, p_it, nullptr, nullptr, nullptr, it & 1, st);
+        float *p_it = pbuf[it & 1];
+        e = it > 0 ? launch_spmv32<true>(pb, mp, pbuf[(it - 1) & 1], p_it, rz(it - 1), rz(it - 2),
+                                         mp.pop ? mp.part_rr[(it - 1) & 1] : nullptr, it & 1, st)
+                   : launch_spmv32<false>(pb, mp, p_it, nullptr, nullptr, nullptr, nullptr, 0, st);
         if (e != hipSuccess) break;
-        // sparse preconditioner: alpha from the previous step's r.z (the
-        // start's in rz[1]); beta from r.z; the stop test on r.r
-        const double *rho_prev = mp.pop ? mp.part_rz[(it + 1) & 1] : rho32_source(mp, it);
-        update_zr32_kernel<<<vb, kBlock, 0, st>>>(p_it, mp.q, mp.d, mp.r, pb.n, rho_prev,
+        // sparse preconditioner: alpha from r.z, the stop level from r0.r0
+        update_zr32_kernel<<<vb, kBlock, 0, st>>>(p_it, mp.q, mp.d, mp.r, pb.n, rz(it - 1),
                                                   mp.part_pq, sd.grid, mp.part_rr[it & 1],
                                                   mp.rows_part, sd.nblk, mp.sc, it == 0 ? 1 : 0,
                                                   mp.minv, mp.pop ? mp.part_xx : nullptr);
         e = hipGetLastError();
-        if (e != hipSuccess || fused) continue;
-        if (mp.pop) {
+        if (e == hipSuccess && mp.pop && it + 1 < steps)
             e = launch_precond_apply32(*mp.pop, mp.r, mp.pz, nullptr, mp.part_rz[it & 1], vb,
                                        mp.sc, st);
-            if (e != hipSuccess) break;
-            update_p32_kernel<<<vb, kBlock, 0, st>>>(mp.pz, mp.p, pb.n, mp.part_rz[it & 1],
-                                                     rho_prev, mp.sc, nullptr,
-                                                     mp.part_rr[it & 1]);
-        } else {
-            update_p32_kernel<<<vb, kBlock, 0, st>>>(mp.r, mp.p, pb.n, mp.part_rr[it & 1],
-                                                     rho_prev, mp.sc, mp.minv, nullptr);
-        }
-        e = hipGetLastError();
     }
     return e;
 }
 
-hipError_t launch_sweep_prepare(Scalars *outer, Scalars *inner, double rhs_norm, double rtol,
-                                int maxit, int first, hipStream_t st) {
-    sweep_prepare_kernel<<<1, 64, 0, st>>>(outer, inner, rhs_norm, rtol, maxit, first);
-    return hipGetLastError();
-}
-
 hipError_t launch_refine(const Fp64Problem &pb, const MixedProblem &mp, hipStream_t st) {
-    refine_kernel<<<pb.vec_blocks, kBlock, 0, st>>>(pb.z, mp.d, pb.n);
+    refine_kernel<<<pb.vec_blocks, kBlock, 0, st>>>(pb.z, mp.d, pb.n, pb.sc);
     return hipGetLastError();
 }
 
