@@ -169,6 +169,8 @@ constexpr int kMaxSortWindow = 8192;
 // Exchange buffers of one resident launch at most (npbcg_power runs more outer
 // iterations in several launches).
 constexpr size_t kResidentWords = (size_t)8 << 20;
+// FP64 solves up to this order update p inside the SpMV (refresh_solve_view).
+constexpr int kFuseSolveRows = 49152;
 // Steps of a resident solve launch at most.
 constexpr int kResidentSolveSteps = 64;
 // Entries of a right-hand side copied and sent at a time.
@@ -226,7 +228,12 @@ void refresh_solve_view(npbcg_ctx *c) {
     c->pbs = c->pb;
     c->pbs.x = vec_ptr(c, kVecB);
     c->pbs.z = vec_ptr(c, kVecXsol);
-    c->pbs.fuse_p_update = 0;  // a solve may stop after any step; p stays in place
+    // The p update and the stop test of a step in the next one's SpMV (SELL) while
+    // a launch is worth more than staging a second vector without its loads all in
+    // flight: plain, Jacobi and Neumann solve, us, apart and fused: n = 17003 -, 187,
+    // 248 and -, 172, 231; 30011 213, 214, 278 and 199, 205, 264; 60013 308, 308, 343
+    // and 305, 314, 340; 150000 788, 792, 939 and 801, 829, 953.
+    c->pbs.fuse_p_update = c->n <= kFuseSolveRows ? 1 : 0;
     c->pbs.cg_form = 0;        // the stop test sits in the reference-order p update
 }
 
@@ -2051,7 +2058,7 @@ int npbcg_log_pairs(npbcg_ctx *c, int pairs, float *r, float *e) {
         NPBCG_HIP(npbcg_dev::launch_log_pair(lp.r, lp.z, pr.xstar, n, pr.r + (size_t)k * n,
                                              pr.e + (size_t)k * n, pr.part + (size_t)k * vb, vb,
                                              c->stream));
-        if (k + 1 < pairs) NPBCG_HIP(npbcg_dev::enqueue_solve_step(lp, k, 0, c->stream));
+        if (k + 1 < pairs) NPBCG_HIP(npbcg_dev::enqueue_solve_step(lp, k, 0, 0, c->stream));
     }
     NPBCG_HIP(npbcg_dev::launch_pair_weights(pr.part, vb, pairs, pr.omega, c->stream));
     NPBCG_HIP(hipMemcpyAsync(c->pbs.z, pr.xstar, sizeof(double) * n, hipMemcpyDeviceToDevice,

@@ -131,9 +131,12 @@ __global__ __launch_bounds__(kBlock) void spmv_csr_kernel(
 // partial of p.q = sum_b sum_rows p[row] * (block b's sum of the row).
 // ---------------------------------------------------------------------------
 
-// PUPD: the input vector is p_new = r + beta p_old, built here instead of by
-// a separate update_p launch.  beta comes from the r.r partials (rr_part new,
-// rho_part old); the workgroups of row range 0 store their block of p_new.
+// PUPD: the input vector is p_new = z + beta p_old, built here instead of by
+// a separate update_p launch.  beta comes from the r.z partials (rr_part new,
+// rho_part old); the workgroups of row range 0 store their block of p_new.  z is
+// r, or minv r when minv is given.  The stop test of a solve, on r.z or, when
+// given, stop_part's r.r, is update_p_kernel's: workgroup 0 records it and all
+// workgroups, which reach the same decision, return.
 template <int BLOCK, int UNR, int MODE, bool PUPD>
 __global__ __launch_bounds__(BLOCK) void spmv_sell_kernel(
     const int *__restrict__ wg_slice, const int *__restrict__ slice_off,
@@ -142,7 +145,8 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell_kernel(
     double *__restrict__ rows_part, double *__restrict__ dot_part, int n, int W,
     int nrange, const double *__restrict__ r, double *__restrict__ p_new,
     const double *__restrict__ rr_part, const double *__restrict__ rho_part, int n_vec,
-    const Scalars *__restrict__ sc, int rev) {
+    Scalars *sc, int rev, const double *__restrict__ minv,
+    const double *__restrict__ stop_part) {
     if (MODE == 0 && sc->done) return;  // a solve already met its tolerance
     if (MODE == 1 && sc->skip_resid) return;  // a refinement sweep that is not needed
     // Dynamic LDS: W vector entries, then one p.q slot per slice of this
@@ -160,23 +164,43 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell_kernel(
         double rr, rho;
         reduce_partials2<BLOCK>(rr_part, n_vec, rho_part, n_vec, rr, rho);
         beta = rr / rho;
+        const double level = stop_part ? reduce_partials<BLOCK>(stop_part, n_vec) : rr;
+        const bool stop = sc->stop_enabled && fabs(level) <= sc->tol2;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            sc->rho = rr;
+            sc->beta = beta;
+            if (stop) sc->done = 1;
+        }
+        if (stop) return;
     }
     if constexpr (PUPD) {
         const double2 *v2 = reinterpret_cast<const double2 *>(v + c0);
         const double2 *r2 = reinterpret_cast<const double2 *>(r + c0);
         double2 *o2 = reinterpret_cast<double2 *>(p_new + c0);
         const bool store = (wg % nrange) == 0;
+        auto form = [&](auto z2) {
 #pragma unroll 4
-        for (int i = threadIdx.x; i < wb / 2; i += BLOCK) {
-            const double2 pv = v2[i], rv = r2[i];
-            double2 nv;
-            nv.x = rv.x + beta * pv.x;
-            nv.y = rv.y + beta * pv.y;
-            lds_v2[i] = nv;
-            if (store) o2[i] = nv;
+            for (int i = threadIdx.x; i < wb / 2; i += BLOCK) {
+                const double2 pv = v2[i], zv = z2(i);
+                double2 nv;
+                nv.x = zv.x + beta * pv.x;
+                nv.y = zv.y + beta * pv.y;
+                lds_v2[i] = nv;
+                if (store) o2[i] = nv;
+            }
+        };
+        if (minv) {
+            const double2 *m2 = reinterpret_cast<const double2 *>(minv + c0);
+            form([&](int i) {
+                const double2 rv = r2[i], mv = m2[i];
+                return make_double2(mv.x * rv.x, mv.y * rv.y);
+            });
+        } else {
+            form([&](int i) { return r2[i]; });
         }
         if ((wb & 1) && threadIdx.x == 0) {
-            const double nv = r[c0 + wb - 1] + beta * v[c0 + wb - 1];
+            const int at = c0 + wb - 1;
+            const double nv = (minv ? minv[at] * r[at] : r[at]) + beta * v[at];
             vblk[wb - 1] = nv;
             if (store) p_new[c0 + wb - 1] = nv;
         }
@@ -236,7 +260,8 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell_kernel(
         // p of the lane's row for p.q, loaded while the slice streams
         double pr = 0.0;
         if constexpr (MODE == 0)
-            if (row >= 0) pr = PUPD ? r[row] + beta * v[row] : v[row];
+            if (row >= 0)
+                pr = PUPD ? (minv ? minv[row] * r[row] : r[row]) + beta * v[row] : v[row];
         double acc = 0.0;
         const int nch = (width + UNR - 1) / UNR;
         for (int ch = 0; ch < nch; ch++) {
@@ -817,6 +842,12 @@ const double *rho_source(const Fp64Problem &pb, int step) {
     return step == 0 ? pb.part.xx : pb.part.rr[(step - 1) & 1];
 }
 
+// The r.z partials feeding CG step `step`: those of the start for step 0 (with a
+// sparse preconditioner in rz[1]), else the previous step's.
+const double *rz_source(const Fp64Problem &pb, int step) {
+    return pb.pop ? pb.part.rz[(step + 1) & 1] : rho_source(pb, step);
+}
+
 // MODE 0 at `step` (q = A p): for step > 0 the kernel forms p of this step
 // from r and the previous step's p.  MODE 1: r = A z.  Slice order: forward
 // on even steps, backward on odd ones and for r = A z, which follows the odd
@@ -831,10 +862,10 @@ hipError_t launch_sell_t(const Fp64Problem &pb, int step, hipStream_t st, hipEve
                      launch_k(spmv_sell_kernel<BLOCK, kSellUnr, 0, true>, d.grid, BLOCK, d.lds_bytes,
                               st, e0, e1, d.wg_slice, d.slice_off, d.slice_row, d.val, d.col,
                               (const double *)p_of_step(pb, step - 1), d.rows_part, pb.part.pq,
-                              pb.n, d.W, d.nrange, (const double *)pb.r, p_of_step(pb, step),
-                              (const double *)pb.part.rr[(step - 1) & 1],
-                              rho_source(pb, step - 1), pb.vec_blocks, (const Scalars *)pb.sc,
-                              rev),
+                              pb.n, d.W, d.nrange, (const double *)(pb.pop ? pb.pz : pb.r),
+                              p_of_step(pb, step), rz_source(pb, step), rz_source(pb, step - 1),
+                              pb.vec_blocks, pb.sc, rev, pb.minv,
+                              (const double *)(pb.pop ? pb.part.rr[(step - 1) & 1] : nullptr)),
                      "spmv_sell_kernel (p = r + beta p; q = A p)", BLOCK, st);
     }
     if (MODE == 0 && pb.cg_form && pb.dot_apart) {  // s = A r, block sums only
@@ -843,8 +874,8 @@ hipError_t launch_sell_t(const Fp64Problem &pb, int step, hipStream_t st, hipEve
                               d.lds_bytes, st, e0, e1, d.wg_slice, d.slice_off, d.slice_row,
                               d.val, d.col, (const double *)pb.r, d.rows_part, pb.part.pq, pb.n,
                               d.W, d.nrange, (const double *)nullptr, (double *)nullptr,
-                              (const double *)nullptr, (const double *)nullptr, 0,
-                              (const Scalars *)pb.sc, step & 1),
+                              (const double *)nullptr, (const double *)nullptr, 0, pb.sc,
+                              step & 1, (const double *)nullptr, (const double *)nullptr),
                      "spmv_sell_kernel (s = A r, r.s apart)", BLOCK, st);
     }
     // one-reduction form: the CG SpMV is s = A r (its dot partials are r.s)
@@ -854,7 +885,7 @@ hipError_t launch_sell_t(const Fp64Problem &pb, int step, hipStream_t st, hipEve
                           st, e0, e1, d.wg_slice, d.slice_off, d.slice_row, d.val, d.col, v,
                           d.rows_part, pb.part.pq, pb.n, d.W, d.nrange, (const double *)nullptr,
                           (double *)nullptr, (const double *)nullptr, (const double *)nullptr,
-                          0, (const Scalars *)pb.sc, rev),
+                          0, pb.sc, rev, (const double *)nullptr, (const double *)nullptr),
                  MODE == 1    ? "spmv_sell_kernel (r = A z)"
                  : pb.cg_form ? "spmv_sell_kernel (s = A r)"
                               : "spmv_sell_kernel (q = A p)",
@@ -965,7 +996,7 @@ hipError_t launch_update_zr(const Fp64Problem &pb, int step, hipStream_t st,
     // the start's r0.z0 sits in rz[1]; the stop level comes from r0.r0 (xx)
     update_zr_kernel<<<pb.vec_blocks, kBlock, 0, st>>>(
         p_of_step(pb, step), pb.q, pb.z, pb.r, pb.n,
-        pb.pop ? pb.part.rz[(step + 1) & 1] : rho_source(pb, step), pb.vec_blocks, pb.part.pq,
+        rz_source(pb, step), pb.vec_blocks, pb.part.pq,
         spmv_grid(pb), pb.part.rr[step & 1], pb.sell.rows_part, pb.sell.row_slot,
         pb.spmv_variant == kSpmvTiled ? pb.sell.nblk : 0, pb.sc,
         (step == 0 && sets_tol) ? 1 : 0, pb.minv, pb.pop ? pb.part.xx : nullptr);
@@ -1084,13 +1115,16 @@ int conj_grad_launches(const Fp64Problem &pb, int cgitmax) {
     return 1 + 3 * cgitmax + resid;
 }
 
-hipError_t enqueue_solve_step(const Fp64Problem &pb, int it, int sets_tol, hipStream_t st) {
+hipError_t enqueue_solve_step(const Fp64Problem &pb, int it, int sets_tol, int last,
+                              hipStream_t st) {
     hipError_t e = launch_spmv<0>(pb, st, nullptr, nullptr, it);
     if (e == hipSuccess) e = launch_update_zr(pb, it, st, sets_tol);
+    // with the p update in the next SpMV nothing follows the last step's r
+    if (last && fused_p(pb)) return e;
     if (e == hipSuccess && pb.pop)  // z = M^-1 r and its r.z partials
         e = launch_precond_apply(*pb.pop, pb.r, pb.pz, nullptr, pb.part.rz[it & 1],
                                  pb.vec_blocks, pb.sc, st);
-    if (e == hipSuccess) e = launch_update_p(pb, it, st);
+    if (e == hipSuccess && !fused_p(pb)) e = launch_update_p(pb, it, st);
     return e;
 }
 
@@ -1098,7 +1132,7 @@ hipError_t enqueue_solve_steps(const Fp64Problem &pb, int steps, int sets_tol,
                                hipStream_t st) {
     hipError_t e = hipSuccess;
     for (int it = 0; it < steps && e == hipSuccess; it++)
-        e = enqueue_solve_step(pb, it, sets_tol, st);
+        e = enqueue_solve_step(pb, it, sets_tol, it + 1 == steps, st);
     return e;
 }
 

@@ -195,8 +195,10 @@ int conj_grad_launches(const Fp64Problem &pb, int cgitmax);
 
 // `steps` CG steps (SpMV, update_zr, update_p) of a solve on pb (x holds b,
 // z the iterate); the stop flag makes steps after convergence return at once.
-// Step `it` of a solve sequence (it selects the partial-sum buffers).
-hipError_t enqueue_solve_step(const Fp64Problem &pb, int it, int sets_tol, hipStream_t st);
+// Step `it` of a solve sequence (it selects the partial-sum buffers); last: no step
+// of the sequence follows.
+hipError_t enqueue_solve_step(const Fp64Problem &pb, int it, int sets_tol, int last,
+                              hipStream_t st);
 hipError_t enqueue_solve_steps(const Fp64Problem &pb, int steps, int sets_tol,
                                hipStream_t st);
 
