@@ -788,6 +788,17 @@ __global__ void fill_kernel(double *__restrict__ v, int count, double value) {
         v[j] = value;
 }
 
+// dst = src (pairs of doubles) and one set of scalars.
+__global__ __launch_bounds__(kBlock) void save_kernel(const double2 *__restrict__ src,
+                                                      double2 *__restrict__ dst, long long pairs,
+                                                      const Scalars *__restrict__ sc,
+                                                      Scalars *__restrict__ sc_out) {
+    for (long long i = blockIdx.x * (long long)kBlock + threadIdx.x; i < pairs;
+         i += (long long)gridDim.x * kBlock)
+        dst[i] = src[i];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *sc_out = *sc;
+}
+
 // ---------------------------------------------------------------------------
 // Host-side launchers
 // ---------------------------------------------------------------------------
@@ -1046,6 +1057,14 @@ hipError_t launch_copy(const void *src, void *dst, long long bytes, int blocks,
                        hipStream_t st) {
     copy_kernel<<<blocks, kBlock, 0, st>>>(static_cast<const double2 *>(src),
                                            static_cast<double2 *>(dst), bytes / 16);
+    return hipGetLastError();
+}
+
+hipError_t launch_save(const double *src, double *dst, long long bytes, const Scalars *sc,
+                       Scalars *sc_out, int blocks, hipStream_t st) {
+    save_kernel<<<blocks, kBlock, 0, st>>>(reinterpret_cast<const double2 *>(src),
+                                           reinterpret_cast<double2 *>(dst), bytes / 16, sc,
+                                           sc_out);
     return hipGetLastError();
 }
 

@@ -181,6 +181,9 @@ hipError_t launch_fill(double *v, int count, double value, int blocks, hipStream
 // Copy of bytes (a multiple of 16) from src to dst.
 hipError_t launch_copy(const void *src, void *dst, long long bytes, int blocks,
                        hipStream_t st);
+// dst = src, bytes / 16 pairs of doubles, and *sc_out = *sc.
+hipError_t launch_save(const double *src, double *dst, long long bytes, const Scalars *sc,
+                       Scalars *sc_out, int blocks, hipStream_t st);
 // Read of bytes (a multiple of 16) from src with `blocks` 1024-thread
 // workgroups; sink (one double) is written only on an impossible sum.
 hipError_t launch_read(const void *src, long long bytes, double *sink, int blocks,
