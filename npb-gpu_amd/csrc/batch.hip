@@ -58,7 +58,7 @@ struct npbcg_batch {
     int *d_rowptr = nullptr, *d_col = nullptr;
     double *d_val = nullptr;
     float *d_val32 = nullptr;
-    int *d_tiles = nullptr;          // tile_sys | tile_row | sys_tile
+    int *d_tiles = nullptr;          // tiles (BatchTile) | sys_tile
     int tiles_cap = 0;
     int *d_block_tile = nullptr;     // workgroup -> tile of the gathering kernels
     size_t block_tile_cap = 0;
@@ -90,33 +90,35 @@ struct npbcg_batch {
     int *d_res_sys = nullptr;        // sys_item
     int *d_res_block_item = nullptr;
     int res_item_blocks = 0;
+    // what the host reads between launches, in one piece: sc | |res|^2 | |b|^2 | done
+    // of every solve, and its pinned copy
+    char *d_state = nullptr, *h_state = nullptr;
     int *d_flags = nullptr;          // done
     BatchScalars *d_sc = nullptr;
     double *d_b = nullptr, *d_x = nullptr, *d_res = nullptr;   // [rows][nr]
     void *d_inner = nullptr;         // d, r, p, q in the inner type
     double *d_part = nullptr;        // 4 * part_cap * nr (init, pq, rr0, rr1)
     int part_cap = 0;                // max(tiles, items) at the smallest tile
-    double *d_sysout = nullptr;      // nsys * nr
+    double *d_sysout = nullptr, *d_bb = nullptr;  // nsys * nr
     BatchDev bd;
 };
 
 namespace {
 
 // Cuts every system into tiles of `rt` rows (a system's last tile is shorter).
-void make_tiles(const npbcg_batch *b, int rt, std::vector<int> &tile_sys, std::vector<int> &tile_row,
-                std::vector<int> &sys_tile) {
-    tile_sys.clear();
-    tile_row.clear();
-    sys_tile.assign(b->nsys + 1, 0);
+// sys_item: first SpMM item of each system (layouts 2 and 3).
+std::vector<BatchTile> make_tiles(const npbcg_batch *b, int rt, const std::vector<int> &sys_item,
+                                  std::vector<int> *sys_tile) {
+    std::vector<BatchTile> tiles;
+    sys_tile->assign(b->nsys + 1, 0);
     for (int s = 0; s < b->nsys; s++) {
-        sys_tile[s] = (int)tile_sys.size();
-        for (int r = 0; r < b->n[s]; r += rt) {
-            tile_sys.push_back(s);
-            tile_row.push_back(b->row_off[s] + r);
-        }
+        const int t0 = (int)tiles.size(), t1 = t0 + (b->n[s] + rt - 1) / rt;
+        for (int r = 0; r < b->n[s]; r += rt)
+            tiles.push_back({s, b->row_off[s] + r, b->row_off[s] + std::min(b->n[s], r + rt), t0,
+                             t1, sys_item[s], sys_item[s + 1], 0});
+        (*sys_tile)[s + 1] = t1;
     }
-    sys_tile[b->nsys] = (int)tile_sys.size();
-    tile_row.push_back(b->rows);
+    return tiles;
 }
 
 int max_tiles(const npbcg_batch *b, int rt) {
@@ -345,11 +347,11 @@ void use_plan(BatchDev *bd, const int *plan, int blocks) {
 int apply_shape(npbcg_batch *b, int lpr, int rt, int layout) {
     if (layout == 3 && !b->sell_ok)
         return set_error(NPBCG_ERR_CAPACITY, "batch: no SELL copy (more than 2^31 stored entries)");
-    std::vector<int> ts, tr, st;
-    make_tiles(b, layout == 3 ? kSellTileRows : rt, ts, tr, st);
+    const int tile_rows = layout == 3 ? kSellTileRows : rt;
+    std::vector<int> sys_item(b->nsys + 1, 0);
     if (layout == 3) {  // items: one sorting window each, in system order
         rt = kSellWindow;
-        std::vector<int> sys_item, plan;
+        std::vector<int> plan;
         int blocks = 0;
         sell_plan(b, b->sell_h, b->opts.mode == NPBCG_SOLVE_MIXED ? 4 : 8, &sys_item, &plan, &blocks);
         B_HIP(hipMemcpyAsync(b->d_sysinfo, sys_item.data(), sizeof(int) * (b->nsys + 1),
@@ -362,7 +364,7 @@ int apply_shape(npbcg_batch *b, int lpr, int rt, int layout) {
         use_plan(&b->bd, b->d_block_item, blocks);
     }
     if (layout == 2) {  // items: (system, column block, row range) in system order
-        std::vector<int> items, sys_item(b->nsys + 1, 0);
+        std::vector<int> items;
         for (int s = 0; s < b->nsys; s++) {
             sys_item[s] = (int)(items.size() / 4);
             for (int blk = 0; blk < b->sys_nb[s]; blk++)
@@ -386,14 +388,14 @@ int apply_shape(npbcg_batch *b, int lpr, int rt, int layout) {
     b->bd.cb = layout >= 2 ? 1 : 0;
     b->bd.sell = layout == 3 ? 1 : 0;
     b->opts.layout = layout;
-    const int tiles = (int)ts.size();
+    std::vector<int> st;
+    const std::vector<BatchTile> tile = make_tiles(b, tile_rows, sys_item, &st);
+    const int tiles = (int)tile.size();
     if (tiles > b->tiles_cap) return set_error(NPBCG_ERR_INTERNAL, "batch: tile capacity");
-    std::vector<int> all;
-    all.reserve(2 * tiles + 1 + b->nsys + 1);
-    all.insert(all.end(), ts.begin(), ts.end());
-    all.insert(all.end(), tr.begin(), tr.end());
-    all.insert(all.end(), st.begin(), st.end());
-    B_HIP(hipMemcpyAsync(b->d_tiles, all.data(), sizeof(int) * all.size(), hipMemcpyHostToDevice,
+    int *d_sys_tile = b->d_tiles + (size_t)tiles * (sizeof(BatchTile) / sizeof(int));
+    B_HIP(hipMemcpyAsync(b->d_tiles, tile.data(), sizeof(BatchTile) * tile.size(),
+                         hipMemcpyHostToDevice, b->stream));
+    B_HIP(hipMemcpyAsync(d_sys_tile, st.data(), sizeof(int) * st.size(), hipMemcpyHostToDevice,
                          b->stream));
     B_HIP(hipStreamSynchronize(b->stream));
     const std::vector<int> bt = xcd_order(b, st, b->sys_nnz);
@@ -402,9 +404,8 @@ int apply_shape(npbcg_batch *b, int lpr, int rt, int layout) {
     b->bd.blocks = (int)bt.size();
     b->bd.block_tile = b->d_block_tile;
     b->bd.tiles = tiles;
-    b->bd.tile_sys = b->d_tiles;
-    b->bd.tile_row = b->d_tiles + tiles;
-    b->bd.sys_tile = b->d_tiles + 2 * tiles + 1;
+    b->bd.tile = reinterpret_cast<const BatchTile *>(b->d_tiles);
+    b->bd.sys_tile = d_sys_tile;
     b->bd.lpr = lpr;
     b->opts.lanes_per_row = lpr;
     b->opts.rows_per_tile = rt;
@@ -516,14 +517,37 @@ BatchDev resid_dev(const npbcg_batch *b) {
     return d;
 }
 
-// res = b - A x (FP64), |res|^2 per solve into d_sysout.
-int true_residual(npbcg_batch *b) {
+// Bytes of the state of `solves` solves (npbcg_batch::d_state).
+size_t state_bytes(size_t solves) {
+    return solves * (sizeof(BatchScalars) + 2 * sizeof(double) + sizeof(int));
+}
+
+// The state on the host, once the stream has run what it holds.
+struct BatchState {
+    const BatchScalars *sc;
+    const double *rr, *bb;
+    const int *done;
+};
+int read_state(npbcg_batch *b, BatchState *out) {
+    const size_t solves = (size_t)b->nsys * b->nr;
+    B_HIP(hipMemcpyAsync(b->h_state, b->d_state, state_bytes(solves), hipMemcpyDeviceToHost,
+                         b->stream));
+    B_HIP(hipStreamSynchronize(b->stream));
+    out->sc = reinterpret_cast<const BatchScalars *>(b->h_state);
+    out->rr = reinterpret_cast<const double *>(out->sc + solves);
+    out->bb = out->rr + solves;
+    out->done = reinterpret_cast<const int *>(out->bb + solves);
+    return NPBCG_OK;
+}
+
+// res = b - A x (FP64), |res|^2 per solve into d_sysout, and what follows from it.
+int true_residual(npbcg_batch *b, const BatchDecide &decide) {
     if (b->res_ok)
         B_HIP(batch_residual_sell(resid_dev(b), b->d_res_val, b->d_b, b->d_x, b->d_res, b->d_part,
-                                  b->d_sysout, b->stream));
+                                  b->d_sysout, decide, b->stream));
     else
         B_HIP(batch_residual(b->bd, b->d_val, b->d_b, b->d_x, b->d_res, b->d_part, b->d_sysout,
-                             b->stream));
+                             decide, b->stream));
     return NPBCG_OK;
 }
 
@@ -590,34 +614,41 @@ void default_shape(const npbcg_batch *b, int *lpr, int *rt) {
     *rt = 256;
 }
 
+// Steps from r.r = from to r.r = to at `rate` (natural log of r.r a step), at most 8:
+// a step past the end costs three launches that do nothing.
+int predicted_steps(double from, double to, double rate) {
+    if (!(rate > 0.0)) return 8;
+    const double steps = std::log(from / to) / rate;
+    return steps <= 1.0 ? 1 : steps <= 8.0 ? (int)std::ceil(steps) : 8;
+}
+
+// An inner solve of every unfinished system.  rate[i]: how fast solve i's r.r fell in
+// the last one (0: unknown), which the first chunk is sized by; updated.
 template <typename T>
-int run_inner(npbcg_batch *b, int maxsteps) {
+int run_inner(npbcg_batch *b, int maxsteps, const BatchState &state, std::vector<double> *rate) {
     const BatchVecs<T> v = inner_vecs<T>(b);
+    const size_t solves = rate->size();
+    int chunk = 1;
+    for (size_t i = 0; i < solves; i++)
+        if (!state.done[i])
+            chunk = std::max(chunk, predicted_steps(1.0, state.sc[i].rtol2, (*rate)[i]));
     B_HIP(batch_init<T>(b->bd, v, b->d_res, b->stream));
-    std::vector<int> done(b->nsys * b->nr);
-    std::vector<BatchScalars> sc(done.size());
-    int chunk = 8;
+    BatchState now;
     for (int step = 0; step < maxsteps;) {
         const int end = std::min(maxsteps, step + chunk);
         for (; step < end; step++) B_HIP(batch_cg_step<T>(b->bd, v, step, step == 0, b->stream));
-        // stop early when every solve has finished
-        B_HIP(hipMemcpyAsync(done.data(), b->bd.done, sizeof(int) * done.size(),
-                             hipMemcpyDeviceToHost, b->stream));
-        B_HIP(hipMemcpyAsync(sc.data(), b->d_sc, sizeof(BatchScalars) * sc.size(),
-                             hipMemcpyDeviceToHost, b->stream));
-        B_HIP(hipStreamSynchronize(b->stream));
-        // The next chunk: the steps the slowest solve still needs at the rate
-        // it went so far (rho is the r.r of the step before the last), at most
-        // 8; a step past the end costs three launches that do nothing.
+        int rc = read_state(b, &now);
+        if (rc != NPBCG_OK) return rc;
+        // stop early when every solve has finished; else the steps the slowest
+        // still needs at the rate it went so far (rho is the r.r of the step
+        // before the last)
         chunk = 0;
-        for (size_t i = 0; i < done.size(); i++) {
-            if (done[i]) continue;
-            const double start = sc[i].tol2 / sc[i].rtol2;
-            const double rate = std::log(start / sc[i].rho) / (sc[i].sweep_steps - 1);
-            const double left = std::log(sc[i].rho / sc[i].tol2) / rate - 1.0;
-            chunk = std::max(chunk, left >= 1.0 && left <= 8.0 ? (int)std::ceil(left)
-                                    : left < 1.0               ? 1
-                                                               : 8);
+        for (size_t i = 0; i < solves; i++) {
+            const BatchScalars &sc = now.sc[i];
+            if (sc.sweep_steps > 1)
+                (*rate)[i] = std::log(sc.tol2 / sc.rtol2 / sc.rho) / (sc.sweep_steps - 1);
+            if (!now.done[i])
+                chunk = std::max({chunk, 1, predicted_steps(sc.rho, sc.tol2, (*rate)[i]) - 1});
         }
         if (chunk == 0) break;
     }
@@ -650,10 +681,10 @@ void npbcg_batch_destroy(npbcg_batch *b) {
                     (void *)b->d_items, (void *)b->d_sysinfo, (void *)b->d_sys64, (void *)b->d_seg,
                     b->d_rows_part, (void *)b->d_rowptr, (void *)b->d_col, (void *)b->d_val,
                     (void *)b->d_val32,
-                    (void *)b->d_tiles, (void *)b->d_block_tile, (void *)b->d_flags, (void *)b->d_sc, (void *)b->d_b,
-                    (void *)b->d_x, (void *)b->d_res, b->d_inner, (void *)b->d_part,
-                    (void *)b->d_sysout})
+                    (void *)b->d_tiles, (void *)b->d_block_tile, (void *)b->d_state, (void *)b->d_b,
+                    (void *)b->d_x, (void *)b->d_res, b->d_inner, (void *)b->d_part})
         (void)hipFree(p);
+    if (b->h_state) (void)hipHostFree(b->h_state);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -810,9 +841,14 @@ int npbcg_batch_create(npbcg_batch **out, int nsys, const int *n, const int *con
     TRY(hipMalloc(&b->d_val, sizeof(double) * std::max<long long>(nnz, 1)));
     if (o.mode == NPBCG_SOLVE_MIXED)
         TRY(hipMalloc(&b->d_val32, sizeof(float) * std::max<long long>(nnz, 1)));
-    TRY(hipMalloc(&b->d_tiles, sizeof(int) * (2 * (size_t)b->tiles_cap + nsys + 2)));
-    TRY(hipMalloc(&b->d_flags, sizeof(int) * nsys * b->nr));
-    TRY(hipMalloc(&b->d_sc, sizeof(BatchScalars) * nsys * b->nr));
+    TRY(hipMalloc(&b->d_tiles, sizeof(BatchTile) * (size_t)b->tiles_cap + sizeof(int) * (nsys + 1)));
+    const size_t solves = (size_t)nsys * b->nr;
+    TRY(hipMalloc(&b->d_state, state_bytes(solves)));
+    TRY(hipHostMalloc(&b->h_state, state_bytes(solves)));
+    b->d_sc = reinterpret_cast<BatchScalars *>(b->d_state);
+    b->d_sysout = reinterpret_cast<double *>(b->d_sc + solves);
+    b->d_bb = b->d_sysout + solves;
+    b->d_flags = reinterpret_cast<int *>(b->d_bb + solves);
     TRY(hipMalloc(&b->d_b, sizeof(double) * m));
     TRY(hipMalloc(&b->d_x, sizeof(double) * m));
     TRY(hipMalloc(&b->d_res, sizeof(double) * m));
@@ -830,7 +866,6 @@ int npbcg_batch_create(npbcg_batch **out, int nsys, const int *n, const int *con
                        hipMemcpyHostToDevice, b->stream));
     TRY(hipMemcpyAsync(b->d_seg, seg.data(), sizeof(int) * seg_total, hipMemcpyHostToDevice,
                        b->stream));
-    TRY(hipMalloc(&b->d_sysout, sizeof(double) * nsys * b->nr));
     if (b->sell_ok) {
         const size_t stored = scol.size();
         const size_t vbytes = o.mode == NPBCG_SOLVE_MIXED ? sizeof(float) * stored
@@ -894,8 +929,7 @@ int npbcg_batch_create(npbcg_batch **out, int nsys, const int *n, const int *con
                            b->stream));
     TRY(hipMemsetAsync(b->d_x, 0, sizeof(double) * m, b->stream));
     TRY(hipMemsetAsync(b->d_inner, 0, inner_elem * 4 * m, b->stream));
-    TRY(hipMemsetAsync(b->d_flags, 0, sizeof(int) * nsys * b->nr, b->stream));
-    TRY(hipMemsetAsync(b->d_sc, 0, sizeof(BatchScalars) * nsys * b->nr, b->stream));
+    TRY(hipMemsetAsync(b->d_state, 0, state_bytes(solves), b->stream));
     TRY(hipStreamSynchronize(b->stream));  // host staging goes out of scope
 #undef TRY
     b->bd.nsys = nsys;
@@ -1009,52 +1043,26 @@ int npbcg_batch_solve(npbcg_batch *b, double rtol, int maxit, npbcg_batch_stats 
     const int ns = b->nsys * b->nr;
     const bool mixed = b->opts.mode == NPBCG_SOLVE_MIXED;
     const int inner_max = b->opts.inner_steps > 0 ? b->opts.inner_steps : 60;
-    std::vector<BatchScalars> sc(ns);
-    std::vector<int> done(ns, 0);
-    std::vector<double> bb(ns), rr(ns);
+    const BatchDecide decide{b->d_bb, rtol, maxit, mixed ? 1 : 0};
     // |b|^2 per solve: the residual of x = 0
     B_HIP(hipMemsetAsync(b->d_x, 0, sizeof(double) * (size_t)b->rows * b->nr, b->stream));
-    B_HIP(hipMemsetAsync(b->d_sc, 0, sizeof(BatchScalars) * ns, b->stream));
     B_HIP(hipEventRecord(b->ev0, b->stream));
-    B_HIP(batch_residual_zero(b->bd, b->d_b, b->d_res, b->d_part, b->d_sysout, b->stream));
-    B_HIP(hipMemcpyAsync(bb.data(), b->d_sysout, sizeof(double) * ns, hipMemcpyDeviceToHost,
-                         b->stream));
-    B_HIP(hipStreamSynchronize(b->stream));
-    rr = bb;
+    B_HIP(batch_residual_zero(b->bd, b->d_b, b->d_res, b->d_part, b->d_sysout, decide, b->stream));
+    std::vector<double> rate(ns, 0.0);
+    BatchState state;
     int sweeps = 1;
-    for (;;) {
-        B_HIP(hipMemcpyAsync(sc.data(), b->d_sc, sizeof(BatchScalars) * ns, hipMemcpyDeviceToHost,
-                             b->stream));
-        B_HIP(hipStreamSynchronize(b->stream));
-        bool any = false;
+    for (;; sweeps++) {
+        int rc = read_state(b, &state);
+        if (rc != NPBCG_OK) return rc;
         int budget = 0;
-        for (int i = 0; i < ns; i++) {
-            const double rel = bb[i] > 0.0 ? std::sqrt(rr[i] / bb[i]) : 0.0;
-            done[i] = (rel <= rtol || sc[i].steps >= maxit) ? 1 : 0;
-            // inner target relative to this sweep's residual; FP32 holds about 1e-6 of it
-            const double t = mixed ? std::max(1e-6, 0.5 * rtol / std::max(rel, 1e-300)) : 0.5 * rtol / std::max(rel, 1e-300);
-            sc[i].rtol2 = t * t;
-            sc[i].tol2 = 0.0;
-            sc[i].sweep_steps = 0;
-            if (!done[i]) {
-                any = true;
-                budget = std::max(budget, maxit - sc[i].steps);
-            }
-        }
-        if (!any) break;
+        for (int i = 0; i < ns; i++)
+            if (!state.done[i]) budget = std::max(budget, maxit - state.sc[i].steps);
+        if (budget == 0) break;  // all done
         b->bd.maxit = mixed ? std::min(inner_max, budget) : budget;
-        B_HIP(hipMemcpyAsync(b->d_sc, sc.data(), sizeof(BatchScalars) * ns, hipMemcpyHostToDevice,
-                             b->stream));
-        B_HIP(hipMemcpyAsync(b->bd.done, done.data(), sizeof(int) * ns, hipMemcpyHostToDevice,
-                             b->stream));
-        int rc = mixed ? run_inner<float>(b, b->bd.maxit) : run_inner<double>(b, b->bd.maxit);
+        rc = mixed ? run_inner<float>(b, b->bd.maxit, state, &rate)
+                   : run_inner<double>(b, b->bd.maxit, state, &rate);
+        if (rc == NPBCG_OK) rc = true_residual(b, decide);
         if (rc != NPBCG_OK) return rc;
-        rc = true_residual(b);
-        if (rc != NPBCG_OK) return rc;
-        B_HIP(hipMemcpyAsync(rr.data(), b->d_sysout, sizeof(double) * ns, hipMemcpyDeviceToHost,
-                             b->stream));
-        B_HIP(hipStreamSynchronize(b->stream));
-        sweeps++;
     }
     B_HIP(hipEventRecord(b->ev1, b->stream));
     B_HIP(hipEventSynchronize(b->ev1));
@@ -1068,11 +1076,11 @@ int npbcg_batch_solve(npbcg_batch *b, double rtol, int maxit, npbcg_batch_stats 
     st.layout = b->opts.layout;
     st.time_ms = ms;
     for (int i = 0; i < ns; i++) {
-        const double rel = bb[i] > 0.0 ? std::sqrt(rr[i] / bb[i]) : 0.0;
+        const double rel = state.bb[i] > 0.0 ? std::sqrt(state.rr[i] / state.bb[i]) : 0.0;
         if (rel <= rtol) st.converged++;
         st.max_relres = std::max(st.max_relres, rel);
-        st.max_steps = std::max(st.max_steps, sc[i].steps);
-        if (steps_out) steps_out[i] = sc[i].steps;
+        st.max_steps = std::max(st.max_steps, state.sc[i].steps);
+        if (steps_out) steps_out[i] = state.sc[i].steps;
         if (relres_out) relres_out[i] = rel;
     }
     if (stats) *stats = st;

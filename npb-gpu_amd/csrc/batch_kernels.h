@@ -24,13 +24,29 @@ struct SellItem {
     int first, stride;
 };
 
+// One tile of the vector kernels, likewise in one load: its system, rows
+// [row, end) (global), and where the system's partials lie, [t0, t1) per tile and
+// [i0, i1) per item of the SpMM.
+struct BatchTile {
+    int sys, row, end, t0, t1, i0, i1, pad;
+};
+
 // Per (system, right-hand side) scalars of the inner CG.
 struct BatchScalars {
-    double rtol2;     // inner stop level relative to the start r.r (set by the host)
+    double rtol2;     // inner stop level relative to the start r.r (decide_sweep)
     double tol2;      // rtol2 * r0.r0, set by the first step
     double rho;       // r.r of the last step
     int steps;        // inner CG steps, all sweeps
     int sweep_steps;  // inner CG steps of this sweep
+};
+
+// What the device decides for every solve from a sweep's true residual: done, and
+// the next sweep's inner stop level.
+struct BatchDecide {
+    double *bb;     // |b|^2, set by the first residual (of x = 0)
+    double rtol;
+    int maxit;      // inner steps in all
+    int mixed;
 };
 
 // The concatenated batch (device pointers) and its launch shape.
@@ -46,8 +62,7 @@ struct BatchDev {
                                       // Workgroup b runs on XCD b % 8, so the tiles of one
                                       // system are placed on one XCD and its vector stays
                                       // in that XCD's L2.
-    const int *tile_sys = nullptr;  // [tiles]
-    const int *tile_row = nullptr;  // [tiles + 1] first row of each tile
+    const BatchTile *tile = nullptr;  // [tiles]
     const int *sys_tile = nullptr;  // [nsys + 1] first tile of each system
     const int *rowptr = nullptr;    // [rows + 1]
     const int *col = nullptr;       // global column indices
@@ -122,18 +137,20 @@ hipError_t batch_init(const BatchDev &bd, const BatchVecs<T> &v, const double *r
                       hipStream_t st);
 template <typename T>
 hipError_t batch_refine(const BatchDev &bd, double *x, const T *d, hipStream_t st);
-// res = b - A x (FP64) and |res|^2 per (system, rhs) into sys_out[nsys * nr].
+// res = b - A x (FP64), |res|^2 per (system, rhs) into sys_out[nsys * nr], and the
+// decision on the next sweep.
 hipError_t batch_residual(const BatchDev &bd, const double *val, const double *b, const double *x,
-                          double *res, double *part, double *sys_out, hipStream_t st);
+                          double *res, double *part, double *sys_out, const BatchDecide &decide,
+                          hipStream_t st);
 // The same from an FP64 SELL copy described by bd (its window items and
 // column blocks): one SELL SpMM writes res and the |res|^2 partials of its
 // items, then the per-system sums.
 hipError_t batch_residual_sell(const BatchDev &bd, const double *sval, const double *b,
                                const double *x, double *res, double *part, double *sys_out,
-                               hipStream_t st);
-// Residual of x = 0 (res = b).
+                               const BatchDecide &decide, hipStream_t st);
+// Residual of x = 0 (res = b): the start of a solve.
 hipError_t batch_residual_zero(const BatchDev &bd, const double *b, double *res, double *part,
-                               double *sys_out, hipStream_t st);
+                               double *sys_out, const BatchDecide &decide, hipStream_t st);
 hipError_t batch_narrow(const double *in, float *out, long long count, hipStream_t st);
 
 }  // namespace npbcg_dev
