@@ -147,8 +147,11 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell_kernel(
     const double *__restrict__ rr_part, const double *__restrict__ rho_part, int n_vec,
     Scalars *sc, int rev, const double *__restrict__ minv,
     const double *__restrict__ stop_part) {
-    if (MODE == 0 && sc->done) return;  // a solve already met its tolerance
-    if (MODE == 1 && sc->skip_resid) return;  // a refinement sweep that is not needed
+    // a solve that already met its tolerance, a refinement sweep that is not needed:
+    // tested once the first loads are on their way (a test before them held every
+    // launch up by a round trip: CG step at n = 30011 15.46 us, now 15.11, at 75000
+    // 32.05 and 31.80)
+    const int skip = MODE == 0 ? sc->done : sc->skip_resid;
     // Dynamic LDS: W vector entries, then one p.q slot per slice of this
     // workgroup (the p.q partial is summed in slice order).
     extern __shared__ double2 lds_v2[];  // 16-byte aligned
@@ -160,51 +163,6 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell_kernel(
     const int c0 = b * W;
     const int wb = min(W, n - c0);
     double beta = 0.0;
-    if constexpr (PUPD) {
-        double rr, rho;
-        reduce_partials2<BLOCK>(rr_part, n_vec, rho_part, n_vec, rr, rho);
-        beta = rr / rho;
-        const double level = stop_part ? reduce_partials<BLOCK>(stop_part, n_vec) : rr;
-        const bool stop = sc->stop_enabled && fabs(level) <= sc->tol2;
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            sc->rho = rr;
-            sc->beta = beta;
-            if (stop) sc->done = 1;
-        }
-        if (stop) return;
-    }
-    if constexpr (PUPD) {
-        const double2 *v2 = reinterpret_cast<const double2 *>(v + c0);
-        const double2 *r2 = reinterpret_cast<const double2 *>(r + c0);
-        double2 *o2 = reinterpret_cast<double2 *>(p_new + c0);
-        const bool store = (wg % nrange) == 0;
-        auto form = [&](auto z2) {
-#pragma unroll 4
-            for (int i = threadIdx.x; i < wb / 2; i += BLOCK) {
-                const double2 pv = v2[i], zv = z2(i);
-                double2 nv;
-                nv.x = zv.x + beta * pv.x;
-                nv.y = zv.y + beta * pv.y;
-                lds_v2[i] = nv;
-                if (store) o2[i] = nv;
-            }
-        };
-        if (minv) {
-            const double2 *m2 = reinterpret_cast<const double2 *>(minv + c0);
-            form([&](int i) {
-                const double2 rv = r2[i], mv = m2[i];
-                return make_double2(mv.x * rv.x, mv.y * rv.y);
-            });
-        } else {
-            form([&](int i) { return r2[i]; });
-        }
-        if ((wb & 1) && threadIdx.x == 0) {
-            const int at = c0 + wb - 1;
-            const double nv = (minv ? minv[at] * r[at] : r[at]) + beta * v[at];
-            vblk[wb - 1] = nv;
-            if (store) p_new[c0 + wb - 1] = nv;
-        }
-    }
     const int lane = threadIdx.x & (kWave - 1);
     // Wave-uniform indices (readfirstlane): every branch below that depends on
     // them is a scalar branch, so the wavefront stays converged around the
@@ -242,7 +200,76 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell_kernel(
         nrow = slice_row[(size_t)(s0 + cur) * kWave + lane];
         if (cwidth > 0) sell_chunk<double, UNR>(val, col, cbase, cwidth, 0, lane, na, nc);
     }
-    if constexpr (!PUPD) {
+    if constexpr (PUPD) {
+        // The thread's first pairs of p_old and z, like the chunk, are loaded ahead
+        // of the sums that beta needs: in the order sums, vectors, chunk, a launch
+        // spent two more memory round trips (plain solve at n = 30011 200 us, now
+        // 195; Neumann 266, now 257).  1024 threads have no registers for more.
+        constexpr int kPre = BLOCK == 512 ? 6 : 1;
+        const double2 *v2 = reinterpret_cast<const double2 *>(v + c0);
+        const double2 *r2 = reinterpret_cast<const double2 *>(r + c0);
+        const double2 *m2 = reinterpret_cast<const double2 *>(minv + c0);
+        double2 *o2 = reinterpret_cast<double2 *>(p_new + c0);
+        const int pairs = wb / 2;
+        const bool store = (wg % nrange) == 0;
+        double2 pv[kPre], zv[kPre];
+        if (pairs > 0) {
+#pragma unroll
+            for (int u = 0; u < kPre; u++) {
+                const int i = min((int)threadIdx.x + u * BLOCK, pairs - 1);
+                pv[u] = v2[i];
+                zv[u] = r2[i];
+            }
+            if (minv)
+#pragma unroll
+                for (int u = 0; u < kPre; u++) {
+                    const double2 mv = m2[min((int)threadIdx.x + u * BLOCK, pairs - 1)];
+                    zv[u].x *= mv.x;
+                    zv[u].y *= mv.y;
+                }
+        }
+        asm volatile("" ::: "memory");  // the loads stay ahead
+        if (skip) return;
+        double rr, rho;
+        reduce_partials2<BLOCK>(rr_part, n_vec, rho_part, n_vec, rr, rho);
+        beta = rr / rho;
+        const double level = stop_part ? reduce_partials<BLOCK>(stop_part, n_vec) : rr;
+        const bool stop = sc->stop_enabled && fabs(level) <= sc->tol2;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            sc->rho = rr;
+            sc->beta = beta;
+            if (stop) sc->done = 1;
+        }
+        if (stop) return;
+        auto form = [&](int i, const double2 &p2, const double2 &z2) {
+            double2 nv;
+            nv.x = z2.x + beta * p2.x;
+            nv.y = z2.y + beta * p2.y;
+            lds_v2[i] = nv;
+            if (store) o2[i] = nv;
+        };
+#pragma unroll
+        for (int u = 0; u < kPre; u++)
+            if ((int)threadIdx.x + u * BLOCK < pairs) form(threadIdx.x + u * BLOCK, pv[u], zv[u]);
+#pragma unroll 4
+        for (int i = threadIdx.x + kPre * BLOCK; i < pairs; i += BLOCK) {
+            double2 z2 = r2[i];
+            if (minv) {
+                const double2 mv = m2[i];
+                z2.x *= mv.x;
+                z2.y *= mv.y;
+            }
+            form(i, v2[i], z2);
+        }
+        if ((wb & 1) && threadIdx.x == 0) {
+            const int at = c0 + wb - 1;
+            const double nv = (minv ? minv[at] * r[at] : r[at]) + beta * v[at];
+            vblk[wb - 1] = nv;
+            if (store) p_new[c0 + wb - 1] = nv;
+        }
+    } else {
+        asm volatile("" ::: "memory");
+        if (skip) return;
         // a block of up to 20,480 doubles: 10 (or 20) 16-byte loads per thread
         stage_block<BLOCK, 10240 / BLOCK>(reinterpret_cast<const double2 *>(v + c0), lds_v2,
                                           wb / 2);
