@@ -155,7 +155,7 @@ struct npbcg_ctx {
     // residual/correction pairs (lazy)
     struct Pairs {
         int count = 0;
-        float *r = nullptr, *e = nullptr, *omega = nullptr;
+        float *r = nullptr, *rt = nullptr, *e = nullptr, *omega = nullptr;
         double *part = nullptr, *xstar = nullptr;
     } pairs;
 };
@@ -1069,7 +1069,7 @@ void npbcg_destroy(npbcg_ctx *c) {
                     (void *)c->g.tval, (void *)c->g.cnt, (void *)c->g.op_off, (void *)c->g.op_col,
                     (void *)c->g.op_src, (void *)c->g.op_val, (void *)c->g.op_val32,
                     (void *)c->g.gh_zero, (void *)c->g.gh_learned, (void *)c->g.pz,
-                    (void *)c->g.pz32, (void *)c->pairs.r, (void *)c->pairs.e,
+                    (void *)c->g.pz32, (void *)c->pairs.r, (void *)c->pairs.rt, (void *)c->pairs.e,
                     (void *)c->pairs.omega, (void *)c->pairs.part, (void *)c->pairs.xstar})
         (void)hipFree(p);
     (void)hipFree(c->d_vec32);
@@ -1942,6 +1942,7 @@ int ensure_pairs(npbcg_ctx *c) {
     if (pr.r) return NPBCG_OK;
     const size_t pn = (size_t)NPBCG_MAX_PAIRS * c->n;
     NPBCG_HIP(hipMalloc(&pr.r, sizeof(float) * pn));
+    NPBCG_HIP(hipMalloc(&pr.rt, sizeof(float) * pn));
     NPBCG_HIP(hipMalloc(&pr.e, sizeof(float) * pn));
     NPBCG_HIP(hipMalloc(&pr.omega, sizeof(float) * NPBCG_MAX_PAIRS));
     NPBCG_HIP(hipMalloc(&pr.part, sizeof(double) * NPBCG_MAX_PAIRS * c->pb.vec_blocks));
@@ -1979,7 +1980,7 @@ int ctx_net_system(npbcg_ctx *c, npbcg_dev::NetSystem *sys) {
 npbcg_dev::PairSet ctx_pairs(const npbcg_ctx *c) {
     npbcg_dev::PairSet ps;
     ps.count = c->pairs.count;
-    ps.r = c->pairs.r;
+    ps.rt = c->pairs.rt;
     ps.e = c->pairs.e;
     ps.omega = c->pairs.omega;
     return ps;
@@ -2114,6 +2115,7 @@ int npbcg_log_pairs(npbcg_ctx *c, int pairs, float *r, float *e) {
     NPBCG_HIP(npbcg_dev::launch_pair_weights(pr.part, vb, pairs, pr.omega, c->stream));
     NPBCG_HIP(hipMemcpyAsync(c->pbs.z, pr.xstar, sizeof(double) * n, hipMemcpyDeviceToDevice,
                              c->stream));  // npbcg_get_solution returns x*
+    NPBCG_HIP(npbcg_dev::launch_interleave_pairs(pr.r, pairs, n, pr.rt, c->stream));
     pr.count = pairs;
     if (r)
         NPBCG_HIP(hipMemcpyAsync(r, pr.r, sizeof(float) * pairs * (size_t)n,
@@ -2142,6 +2144,7 @@ int npbcg_set_pairs(npbcg_ctx *c, int pairs, const float *r, const float *e) {
     auto &pr = c->pairs;
     NPBCG_HIP(hipMemcpyAsync(pr.r, r, sizeof(float) * pairs * (size_t)n, hipMemcpyHostToDevice,
                              c->stream));
+    NPBCG_HIP(npbcg_dev::launch_interleave_pairs(pr.r, pairs, n, pr.rt, c->stream));
     NPBCG_HIP(hipMemcpyAsync(pr.e, e, sizeof(float) * pairs * (size_t)n, hipMemcpyHostToDevice,
                              c->stream));
     NPBCG_HIP(hipMemcpyAsync(pr.omega, omega.data(), sizeof(float) * pairs,

@@ -55,11 +55,11 @@ struct NetSystem {
     const float *tval = nullptr;     // its N value (N_src,node)
 };
 
-// Residual/correction pairs of one system: r_p, e_p = x* - x_p (FP32, [p][n])
+// Residual/correction pairs of one system: r_p, e_p = x* - x_p (FP32, e [p][n])
 // and their loss weights 1 / (P |e_p|^2).
 struct PairSet {
     int count = 0;
-    const float *r = nullptr;
+    const float *rt = nullptr;  // the r_p as [n][kPairs]
     const float *e = nullptr;
     const float *omega = nullptr;
 };
@@ -105,15 +105,17 @@ hipError_t launch_log_pair(const double *r, const double *z, const double *xstar
                            float *r_out, float *e_out, double *part, int blocks,
                            hipStream_t st);
 // omega_p = 1 / (P * sum of the |e_p|^2 partials of pair p).
+hipError_t launch_interleave_pairs(const float *r, int pairs, int n, float *rt, hipStream_t st);
 hipError_t launch_pair_weights(const double *part, int parts, int pairs, float *omega,
                                hipStream_t st);
 hipError_t launch_random_rhs(double *b, int n, unsigned long long seed, hipStream_t st);
 int row_blocks(int n);   // workgroups of the 16-lanes-per-row kernels
 int pair_blocks(int n);  // workgroups of the pair-loss kernels
 
-// Forward through the readout: gh = (g, h).
+// Forward through the readout: gh = (g, h).  keep: the aggregated halves of nb.x are
+// stored too, as the backward pass reads them.
 hipError_t launch_net_forward(const NetBuffers &nb, const NetSystem &sys, const float *params,
-                              const __bf16 *wb, float gmax, hipStream_t st);
+                              const __bf16 *wb, float gmax, int keep, hipStream_t st);
 // Loss of the pairs under the preconditioner of gh; loss_part, pw, pd; then
 // dL/dg, dL/dh into dgh when want_grad.
 hipError_t launch_pair_loss(const NetBuffers &nb, const NetSystem &sys, const PairSet &ps,

@@ -414,7 +414,7 @@ __global__ __launch_bounds__(kBlock) void build_x0_kernel(const float *__restric
 }
 
 // Y[n x 64] = ReLU(X[n x K] W + b): a wavefront computes the four 16x16
-// output blocks of kFwdTiles consecutive 16-row tiles, K in steps of 32.  Wt
+// output blocks of TILES consecutive 16-row tiles, K in steps of 32.  Wt
 // is W transposed (64 x K, BF16); the wavefront loads its B fragments (and
 // the bias) once and keeps them in registers for all its tiles, so the
 // weights are read once per wavefront rather than once per tile (at K = 128
@@ -422,18 +422,54 @@ __global__ __launch_bounds__(kBlock) void build_x0_kernel(const float *__restric
 // are loaded before the current tile's products.  Lane l supplies
 // A[l%16][8(l/16)..+7] and B[8(l/16)..+7][l%16] and receives
 // D[4(l/16)..+3][l%16] of each 16x16x32 product.
-constexpr int kFwdTiles = 4;
-template <int K>
-__global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(const __bf16 *__restrict__ x, int ldx,
-                                                          int n, const __bf16 *__restrict__ wt,
+//
+// AGG (K = 128, a message-passing layer): columns 64.. of X are formed here,
+// X[j, 64:128] = sum_t w[j,t] X[nbr[j,t], 0:64] in FP32, rounded to BF16, each lane
+// its 16 columns of its row (the four lanes of a row read whole lines of the
+// neighbours), and stored for the backward pass when `keep`.  As a kernel of its own
+// before the product: 5.8 + 8.6 us and a launch boundary at n = 40009; now 13.3 (network
+// and readout at 17003 71 us, now 60).  TILES = 2: 4 leave too few wavefronts (77 us at
+// 17003), 1 reads the weights twice as often (97 against 93 us at 75000).
+template <int K, int TILES, bool AGG>
+__global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(__bf16 *x, int ldx, int n,
+                                                          const __bf16 *__restrict__ wt,
                                                           const float *__restrict__ bias,
-                                                          __bf16 *__restrict__ y, int ldy) {
+                                                          __bf16 *__restrict__ y, int ldy,
+                                                          const int *__restrict__ nbr,
+                                                          const float *__restrict__ wgt,
+                                                          int keep) {
     constexpr int KS = K / 32;
+    constexpr int KL = AGG ? KS / 2 : KS;  // fragments that are loaded
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
-    const int tile0 = (blockIdx.x * kWavesPerBlock + wave) * kFwdTiles;
+    const int tile0 = (blockIdx.x * kWavesPerBlock + wave) * TILES;
     if (tile0 * 16 >= n) return;
     const int kq = 8 * (lane >> 4);
+    bf16x8 av[KL], hv[AGG ? kNbr : 1][AGG ? KL : 1];
+    float wv[kNbr];
+    auto load_a = [&](int row0) {
+        const int ar = row0 + (lane & 15);
+        if constexpr (AGG) {
+            const int j = min(ar, n - 1);
+            int k[kNbr];
+#pragma unroll
+            for (int t = 0; t < kNbr; t++) {
+                k[t] = nbr[(size_t)j * kNbr + t];
+                wv[t] = wgt[(size_t)j * kNbr + t];
+            }
+#pragma unroll
+            for (int t = 0; t < kNbr; t++)
+#pragma unroll
+                for (int q = 0; q < KL; q++)
+                    hv[t][q] = *reinterpret_cast<const bf16x8 *>(x + (size_t)k[t] * ldx + 32 * q + kq);
+        }
+#pragma unroll
+        for (int q = 0; q < KL; q++) {
+            av[q] = bf16x8{};
+            if (ar < n) av[q] = *reinterpret_cast<const bf16x8 *>(x + (size_t)ar * ldx + 32 * q + kq);
+        }
+    };
+    load_a(tile0 * 16);
     bf16x8 bw[KS][4];
     float bj[4];
 #pragma unroll
@@ -444,23 +480,31 @@ __global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(const __bf16 *__restri
                 wt + (size_t)(jb * 16 + (lane & 15)) * K + 32 * k + kq);
         bj[jb] = bias[jb * 16 + (lane & 15)];
     }
-    auto load_a = [&](int row0, bf16x8 (&av)[KS]) {
-        const int ar = row0 + (lane & 15);
-#pragma unroll
-        for (int k = 0; k < KS; k++) {
-            av[k] = bf16x8{};
-            if (ar < n) av[k] = *reinterpret_cast<const bf16x8 *>(x + (size_t)ar * ldx + 32 * k + kq);
-        }
-    };
-    bf16x8 av[KS];
-    load_a(tile0 * 16, av);
-    for (int t = 0; t < kFwdTiles; t++) {
+    for (int t = 0; t < TILES; t++) {
         const int row0 = (tile0 + t) * 16;
         if (row0 >= n) break;  // the same for the whole wavefront
         bf16x8 cur[KS];
 #pragma unroll
-        for (int k = 0; k < KS; k++) cur[k] = av[k];
-        if (t + 1 < kFwdTiles) load_a(row0 + 16, av);
+        for (int k = 0; k < KL; k++) cur[k] = av[k];
+        if constexpr (AGG) {
+            const int ar = row0 + (lane & 15);
+#pragma unroll
+            for (int q = 0; q < KL; q++) {
+                bf16x8 o;
+#pragma unroll
+                for (int c = 0; c < 8; c++) {
+                    float acc = 0.f;
+#pragma unroll
+                    for (int u = 0; u < kNbr; u++) acc = fmaf(wv[u], (float)hv[u][q][c], acc);
+                    o[c] = (__bf16)acc;
+                }
+                if (ar >= n) o = bf16x8{};
+                cur[KL + q] = o;
+                if (keep && ar < n)
+                    *reinterpret_cast<bf16x8 *>(x + (size_t)ar * ldx + kHid + 32 * q + kq) = o;
+            }
+        }
+        if (t + 1 < TILES) load_a(row0 + 16);
         f32x4 acc[4] = {};
 #pragma unroll
         for (int k = 0; k < KS; k++)
@@ -477,29 +521,6 @@ __global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(const __bf16 *__restri
             }
         }
     }
-}
-
-// X[:, 64:128] = sum_t w[j,t] X[nbr[j,t], 0:64]: 16 lanes per row, 4 columns each.
-__global__ __launch_bounds__(kBlock) void aggregate_kernel(__bf16 *__restrict__ x,
-                                                           const int *__restrict__ nbr,
-                                                           const float *__restrict__ wgt,
-                                                           int n) {
-    const long long gid = blockIdx.x * (long long)kBlock + threadIdx.x;
-    const int j = (int)(gid / 16), f = (int)(gid % 16) * 4;
-    if (j >= n) return;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < kNbr; t++) {
-        const int k = nbr[(size_t)j * kNbr + t];
-        const float w = wgt[(size_t)j * kNbr + t];
-        const bf16x4 h = *reinterpret_cast<const bf16x4 *>(x + (size_t)k * kXW + f);
-#pragma unroll
-        for (int c = 0; c < 4; c++) acc[c] = fmaf(w, (float)h[c], acc[c]);
-    }
-    bf16x4 o;
-#pragma unroll
-    for (int c = 0; c < 4; c++) o[c] = (__bf16)acc[c];
-    *reinterpret_cast<bf16x4 *>(x + (size_t)j * kXW + kHid + f) = o;
 }
 
 // The readout's sums ug . H3 + cg and uh . H3 + ch of kReadRows rows from j0 for a
@@ -566,7 +587,7 @@ __global__ __launch_bounds__(kBlock) void readout_fwd_kernel(const __bf16 *__res
 
 // Eight lanes per row, one per pair: 40009 rows are 5000 wavefronts that gather
 // at the same time, where a thread per row left 2.4 of them on a CU, each with 64
-// gathers of its own in turn (forward and backward 56 and 55 us; now 19 and 10).
+// gathers of its own in turn (forward and backward 56 and 55 us; now 10 and 10).
 static_assert(kPairs == 8, "a row's lanes");
 
 // Sum over the symmetric pattern of row j of C_jk q_k v_k for the lane's pair,
@@ -622,12 +643,12 @@ __global__ __launch_bounds__(kBlock) void pair_loss_fwd_kernel(NetSystem sys,
     double acc = 0.0;
     if (j < n) {
         const size_t column = (size_t)min(p, ps.count - 1) * n;
-        const float w = gather_sym(sys, gh, n, j, ps.r + column, 1);
+        const float w = gather_sym(sys, gh, n, j, ps.rt + min(p, ps.count - 1), kPairs);
         if (p < ps.count) {
             const float g = gh[j], h = gh[n + j];
             const float s2 = (float)(exp(2.0 * g) / sys.adiag[j]);
             const float q = expf(g + h);
-            const float y = s2 * ps.r[column + j] - q * w;
+            const float y = s2 * ps.rt[gid] - q * w;
             const float diff = y - ps.e[column + j];
             acc = (double)ps.omega[p] * (double)diff * (double)diff;
             pw[gid] = w;
@@ -651,7 +672,7 @@ __global__ __launch_bounds__(kBlock) void pair_loss_bwd_kernel(NetSystem sys,
     if (j >= n) return;
     const float phi = gather_sym(sys, gh, n, j, pd + p, kPairs);
     const size_t at = (size_t)j * kPairs + p;
-    const float d = pd[at], r = ps.r[(size_t)p * n + j];
+    const float d = pd[at], r = ps.rt[at];
     const float term = d * pw[at] + r * phi;
     float dq = 0.0f, ds = 0.0f;
     for (int t = 0; t < ps.count; t++) {
@@ -1158,6 +1179,20 @@ hipError_t launch_log_pair(const double *r, const double *z, const double *xstar
     return hipGetLastError();
 }
 
+// rt[j][p] = r[p][j], so that a row's lanes read the pairs of a neighbour as one run.
+__global__ __launch_bounds__(kBlock) void interleave_pairs_kernel(const float *__restrict__ r,
+                                                                  int pairs, int n,
+                                                                  float *__restrict__ rt) {
+    const long long gid = blockIdx.x * (long long)kBlock + threadIdx.x;
+    const int j = (int)(gid / kPairs), p = (int)(gid % kPairs);
+    if (j < n) rt[gid] = p < pairs ? r[(size_t)p * n + j] : 0.0f;
+}
+
+hipError_t launch_interleave_pairs(const float *r, int pairs, int n, float *rt, hipStream_t st) {
+    interleave_pairs_kernel<<<pair_blocks(n), kBlock, 0, st>>>(r, pairs, n, rt);
+    return hipGetLastError();
+}
+
 hipError_t launch_pair_weights(const double *part, int parts, int pairs, float *omega,
                                hipStream_t st) {
     pair_weights_kernel<<<1, kBlock, 0, st>>>(part, parts, pairs, omega);
@@ -1175,24 +1210,22 @@ hipError_t launch_sum(const double *part, int count, double *out, hipStream_t st
 }
 
 hipError_t launch_net_forward(const NetBuffers &nb, const NetSystem &sys, const float *params,
-                              const __bf16 *wb, float gmax, hipStream_t st) {
+                              const __bf16 *wb, float gmax, int keep, hipStream_t st) {
     const int n = sys.n;
     hipError_t e;
     build_x0_kernel<<<blocks_for((long long)n * kK0), kBlock, 0, st>>>(sys.feat, nb.norm, n,
                                                                       nb.x0);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    const int gb = exact_blocks(n, 16 * kFwdTiles * kWavesPerBlock);
-    gemm_fwd_kernel<kK0><<<gb, kBlock, 0, st>>>(nb.x0, kK0, n, wb + kWtTransposed,
-                                                params + kOffB0, nb.x[0], kXW);
+    constexpr int kT0 = 4, kT = 2;
+    gemm_fwd_kernel<kK0, kT0, false><<<exact_blocks(n, 16 * kT0 * kWavesPerBlock), kBlock, 0, st>>>(
+        nb.x0, kK0, n, wb + kWtTransposed, params + kOffB0, nb.x[0], kXW, nullptr, nullptr, 0);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     for (int l = 0; l < kLayers; l++) {
-        aggregate_kernel<<<row_blocks(n), kBlock, 0, st>>>(nb.x[l], sys.nbr, sys.wgt, n);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
         __bf16 *out = l + 1 < kLayers ? nb.x[l + 1] : nb.h3;
         const int ldy = l + 1 < kLayers ? kXW : kHid;
-        gemm_fwd_kernel<kXW><<<gb, kBlock, 0, st>>>(
+        gemm_fwd_kernel<kXW, kT, true><<<exact_blocks(n, 16 * kT * kWavesPerBlock), kBlock, 0, st>>>(
             nb.x[l], kXW, n, wb + kWtTransposed + kK0 * kHid + l * kXW * kHid,
-            params + kOffB1 + l * kLayerStride, out, ldy);
+            params + kOffB1 + l * kLayerStride, out, ldy, sys.nbr, sys.wgt, keep);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     readout_fwd_kernel<<<exact_blocks((long long)n * 16, kBlock * kReadRows), kBlock, 0, st>>>(nb.h3, params + kOffR, gmax, n, nb.gh);

@@ -156,7 +156,7 @@ int evaluate(npbcg_net *net, npbcg_ctx *ctx, bool grad, bool base, bool relative
         NET_HIP(launch_pair_loss(b0, sys, ps, 0, st));
         NET_HIP(launch_sum(nb.loss_part, parts, net->d_loss + 1, st));
     }
-    NET_HIP(launch_net_forward(nb, sys, net->params, net->wb, kGmax, st));
+    NET_HIP(launch_net_forward(nb, sys, net->params, net->wb, kGmax, grad ? 1 : 0, st));
     NET_HIP(launch_pair_loss(nb, sys, ps, grad ? 1 : 0, st));
     NET_HIP(launch_sum(nb.loss_part, parts, net->d_loss, st));
     if (grad) {
@@ -402,7 +402,7 @@ int npbcg_net_apply(npbcg_net *net, npbcg_ctx *ctx, double *ms) {
         NET_HIP(launch_feature_stats(sys.feat, sys.n, net->norm, st));
         net->norm_set = true;
     }
-    NET_HIP(launch_net_forward(net->nb, sys, net->params, net->wb, kGmax, st));
+    NET_HIP(launch_net_forward(net->nb, sys, net->params, net->wb, kGmax, 0, st));
     NET_HIP(hipEventRecord(net->ev1, st));
     rc = npbcg_detail::ctx_install_learned(ctx, net->nb.gh);
     if (rc != NPBCG_OK) return rc;
