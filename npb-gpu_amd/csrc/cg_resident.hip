@@ -450,7 +450,13 @@ __global__ __launch_bounds__(kResBlock) void resident_fill_kernel(
 
 // Kernels by words per thread, smallest first.  Few words a thread go with
 // many lanes per row: the fewer rows a workgroup has, the more lanes each
-// gets, and all of them still find a place in one pass.
+// gets, and all of them still find a place in one pass.  A step grows with the
+// words a thread reads in the exchange, whether they are rows or not, by
+// 0.06 to 0.15 us a word, so there is a kernel for every second word
+// count and every one up to 8; as many entries are held as leave no spills.  With
+// 4, 8, 16, 32 and 38 words only, and now, us a step: n = 1400 2.02 and 1.94, 2000
+// 2.50 and 2.16, 4500 3.45 and 2.81, 8100 6.48 and 4.52, 10000 6.91 and 5.26, 14000
+// 6.72 and 6.35, 17000 9.44 and 8.55.
 struct ResKernel {
     int lpr, per, chunk, chunks;  // as the kernel's template
     const void *fn;
@@ -461,9 +467,17 @@ ResKernel res_kernel() {
             reinterpret_cast<const void *>(&cg_resident_kernel<LPR, PER, C, CH, HELD>)};
 }
 const ResKernel kResKernels[] = {
-    res_kernel<32, 4, 16, 1, 8>(),   res_kernel<32, 8, 16, 1, 12>(),
-    res_kernel<16, 16, 32, 1, 24>(), res_kernel<8, 32, 64, 1, 16>(),
-    res_kernel<4, 38, 64, 2, 8>(),
+    res_kernel<32, 2, 16, 1, 8>(),   res_kernel<32, 3, 16, 1, 8>(),
+    res_kernel<32, 4, 16, 1, 8>(),   res_kernel<32, 5, 16, 1, 12>(),
+    res_kernel<32, 6, 16, 1, 12>(),  res_kernel<32, 7, 16, 1, 12>(),
+    res_kernel<32, 8, 16, 1, 12>(),  res_kernel<16, 10, 32, 1, 24>(),
+    res_kernel<16, 12, 32, 1, 24>(), res_kernel<16, 14, 32, 1, 24>(),
+    res_kernel<16, 16, 32, 1, 24>(), res_kernel<8, 18, 64, 1, 24>(),
+    res_kernel<8, 20, 64, 1, 24>(),  res_kernel<8, 22, 64, 1, 24>(),
+    res_kernel<8, 24, 64, 1, 24>(),  res_kernel<8, 26, 64, 1, 20>(),
+    res_kernel<8, 28, 64, 1, 20>(),  res_kernel<8, 30, 64, 1, 16>(),
+    res_kernel<8, 32, 64, 1, 16>(),  res_kernel<4, 34, 64, 2, 8>(),
+    res_kernel<4, 36, 64, 2, 8>(),   res_kernel<4, 38, 64, 2, 8>(),
 };
 
 }  // namespace
