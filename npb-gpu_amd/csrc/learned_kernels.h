@@ -70,8 +70,7 @@ struct NetBuffers {
     __bf16 *x0 = nullptr;        // [cap][kK0]
     __bf16 *x[kLayers] = {};     // [cap][kXW]: [H_l | agg H_l]
     __bf16 *h3 = nullptr;        // [cap][kHid]
-    __bf16 *dz = nullptr;        // [cap][kHid]
-    float *dx = nullptr;         // [cap][kXW]
+    __bf16 *dz[kLayers + 1] = {};  // [cap][kHid] per layer, the embedding's first
     float *gh = nullptr;         // g [cap], h [cap]
     float *dgh = nullptr;        // dL/dg [cap], dL/dh [cap]
     float *pw = nullptr;         // loss forward: (N + N^T) Q r_p per pair [cap][kPairs]

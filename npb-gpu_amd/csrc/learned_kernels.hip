@@ -759,77 +759,129 @@ __global__ __launch_bounds__(kBlock) void readout_bwd_kernel(const __bf16 *__res
     }
 }
 
-// dX[n x 128] = dZ[n x 64] W^T with W row-major [128 x 64] (BF16); FP32 out.
-__global__ __launch_bounds__(kBlock) void gemm_bwd_data_kernel(const __bf16 *__restrict__ dz,
-                                                               int n,
-                                                               const __bf16 *__restrict__ w,
-                                                               float *__restrict__ dx) {
+// The top 16 bits of eight floats as BF16 (truncated); v keeps what is left over.
+// Three of them hold all 24 bits of a float, so a product over the three is one
+// over the FP32 value.  A value without a remainder (infinity, NaN) leaves 0.
+__device__ __forceinline__ bf16x8 take_bf16(float *v) {
+    union {
+        unsigned short h[8];
+        bf16x8 b;
+    } o;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        const unsigned bits = __float_as_uint(v[c]);
+        o.h[c] = (unsigned short)(bits >> 16);
+        const float rest = v[c] - __uint_as_float(bits & 0xffff0000u);
+        v[c] = fabsf(v[c]) < INFINITY ? rest : 0.f;
+    }
+    return o.b;
+}
+
+// Data gradient of a message-passing layer, W row-major [128 x 64] (BF16):
+//   dH[k] = dZ[k] W[0:64]^T + (sum over in-edges (j -> k) of w dZ[j]) W[64:128]^T
+//   dZprev = dH * (Hprev > 0) in BF16, Hprev = X[:, 0:64] of the layer's input.
+// The sum over the in-edges is taken in FP32 before the product, where a row is 128
+// bytes of BF16, not of the product's FP32 result; as three BF16 terms (take_bf16) it
+// enters the matrix units whole.  A wavefront owns 16 rows, four lanes a row, each the
+// 16 columns its A fragments need; four edges a round, the next round's edges loaded
+// ahead.  W sits in LDS, read once a workgroup.  Bound by the chain row pointer ->
+// edges -> gathers and the longest in-edge list of 16 rows.
+// As a product to FP32 rows in memory and an aggregation kernel, 11.0 + 12.3 us and a
+// launch boundary at n = 40009; now 16.6 (eight edges a round: the step is 3 % slower at
+// 17003 and 75000).
+constexpr int kWPad = kHid + 8;
+__global__ __launch_bounds__(kBlock) void layer_bwd_kernel(
+    const __bf16 *__restrict__ dz, const int *__restrict__ tptr, const int *__restrict__ tsrc,
+    const float *__restrict__ tw, const __bf16 *__restrict__ w, const __bf16 *__restrict__ x,
+    int n, __bf16 *__restrict__ dzprev) {
+    __shared__ __bf16 ws[kXW][kWPad];
+    constexpr int WV = kXW * kHid / 8 / kBlock;  // vectors of W a thread loads
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const int row0 = (blockIdx.x * kWavesPerBlock + wave) * 16;
-    if (row0 >= n) return;
     const int ar = row0 + (lane & 15);
     const int kq = 8 * (lane >> 4);
-    bf16x8 av[2] = {};
+    int e0 = 0, e1 = 0;
+    bf16x8 own[2] = {};
     if (ar < n) {
-        av[0] = *reinterpret_cast<const bf16x8 *>(dz + (size_t)ar * kHid + kq);
-        av[1] = *reinterpret_cast<const bf16x8 *>(dz + (size_t)ar * kHid + 32 + kq);
-    }
+        e0 = tptr[ar];
+        e1 = tptr[ar + 1];
 #pragma unroll
-    for (int jb = 0; jb < kXW / 16; jb++) {
+        for (int q = 0; q < 2; q++)
+            own[q] = *reinterpret_cast<const bf16x8 *>(dz + (size_t)ar * kHid + 32 * q + kq);
+    }
+    bf16x8 wv[WV];
+#pragma unroll
+    for (int u = 0; u < WV; u++)
+        wv[u] = *reinterpret_cast<const bf16x8 *>(w + (size_t)(threadIdx.x + u * kBlock) * 8);
+    int src[4];
+    float wt[4];
+    auto edges = [&](int b) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int e = min(b + u, e1 - 1);
+            src[u] = tsrc[e];
+            wt[u] = tw[e];
+        }
+    };
+    if (e0 < e1) edges(e0);
+#pragma unroll
+    for (int u = 0; u < WV; u++) {
+        const int i = (threadIdx.x + u * kBlock) * 8;
+        *reinterpret_cast<bf16x8 *>(&ws[i / kHid][i % kHid]) = wv[u];
+    }
+    __bf16 h[kHid / 16][4];
+#pragma unroll
+    for (int jb = 0; jb < kHid / 16; jb++)
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            h[jb][t] = x[(size_t)min(row0 + 4 * (lane >> 4) + t, n - 1) * kXW + jb * 16 + (lane & 15)];
+    float s[2][8] = {};
+    for (int b = e0; b < e1; b += 4) {
+        bf16x8 g[4][2];
+        float cur[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            cur[u] = wt[u];
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+                g[u][q] = *reinterpret_cast<const bf16x8 *>(dz + (size_t)src[u] * kHid + 32 * q + kq);
+        }
+        if (b + 4 < e1) edges(b + 4);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (b + u < e1)
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+#pragma unroll
+                    for (int c = 0; c < 8; c++) s[q][c] = fmaf(cur[u], (float)g[u][q][c], s[q][c]);
+    }
+    bf16x8 agg[3][2];
+#pragma unroll
+    for (int t = 0; t < 3; t++)
+#pragma unroll
+        for (int q = 0; q < 2; q++) agg[t][q] = take_bf16(s[q]);
+    __syncthreads();
+#pragma unroll
+    for (int jb = 0; jb < kHid / 16; jb++) {
+        const int j = jb * 16 + (lane & 15);
         f32x4 acc = {};
 #pragma unroll
-        for (int ks = 0; ks < 2; ks++) {
-            const bf16x8 bv = *reinterpret_cast<const bf16x8 *>(
-                w + (size_t)(jb * 16 + (lane & 15)) * kHid + ks * 32 + kq);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[ks], bv, acc, 0, 0, 0);
+        for (int q = 0; q < 2; q++) {
+            const bf16x8 b1 = *reinterpret_cast<const bf16x8 *>(&ws[j][32 * q + kq]);
+            const bf16x8 b2 = *reinterpret_cast<const bf16x8 *>(&ws[kHid + j][32 * q + kq]);
+#pragma unroll
+            for (int t = 2; t >= 0; t--)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(agg[t][q], b2, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(own[q], b1, acc, 0, 0, 0);
         }
-        const int jcol = jb * 16 + (lane & 15);
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             const int row = row0 + 4 * (lane >> 4) + t;
-            if (row < n) dx[(size_t)row * kXW + jcol] = acc[t];
+            if (row < n)
+                dzprev[(size_t)row * kHid + j] = (__bf16)((float)h[jb][t] > 0.f ? acc[t] : 0.f);
         }
     }
-}
-
-// dH[k] = dX[k, 0:64] + sum over in-edges (j -> k) of w dX[j, 64:128];
-// dZprev = dH * (Hprev > 0) in BF16, Hprev = X[:, 0:64] of this layer's input.
-__global__ __launch_bounds__(kBlock) void aggregate_bwd_kernel(
-    const float *__restrict__ dx, const int *__restrict__ tptr, const int *__restrict__ tsrc,
-    const float *__restrict__ tw, const __bf16 *__restrict__ x, int n,
-    __bf16 *__restrict__ dzprev) {
-    const long long gid = blockIdx.x * (long long)kBlock + threadIdx.x;
-    const int k = (int)(gid / 16), f = (int)(gid % 16) * 4;
-    if (k >= n) return;
-    const int e0 = tptr[k], e1 = tptr[k + 1];
-    const f32x4 own = *reinterpret_cast<const f32x4 *>(dx + (size_t)k * kXW + f);
-    float acc[4] = {own[0], own[1], own[2], own[3]};
-    for (int b = e0; b < e1; b += 16) {  // the row's lanes load the next 16 edges
-        const int mine = min(b + (int)(threadIdx.x & 15), e1 - 1);
-        const int src = tsrc[mine];
-        const float w = tw[mine];
-        for (int t = 0; t < 16 && b + t < e1; t += 4) {  // four gathers in flight
-            f32x4 g[4];
-            float wt[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                g[u] = *reinterpret_cast<const f32x4 *>(
-                    dx + (size_t)__shfl(src, t + u, 16) * kXW + kHid + f);
-                wt[u] = __shfl(w, t + u, 16);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-                if (b + t + u < e1)
-#pragma unroll
-                    for (int c = 0; c < 4; c++) acc[c] = fmaf(wt[u], g[u][c], acc[c]);
-        }
-    }
-    const bf16x4 hv = *reinterpret_cast<const bf16x4 *>(x + (size_t)k * kXW + f);
-    bf16x4 o;
-#pragma unroll
-    for (int c = 0; c < 4; c++) o[c] = (__bf16)((float)hv[c] > 0.f ? acc[c] : 0.f);
-    *reinterpret_cast<bf16x4 *>(dzprev + (size_t)k * kHid + f) = o;
 }
 
 // Per-workgroup partial dW[K x 64] = X^T dZ and db[64] = column sums of dZ
@@ -838,21 +890,30 @@ __global__ __launch_bounds__(kBlock) void aggregate_bwd_kernel(
 // eight rows of a fragment are one 16-byte read, and the next chunk's loads are
 // on their way while this one is multiplied.  Eight wavefronts, one 16-row block
 // of dW each (K = 128).  part holds K*64 + 64 floats per workgroup; 256 of them
-// (one a CU) instead of 512 halve what the reduction reads.  (32-row chunks read
-// from LDS two bytes at a time, 10.3 us at n = 40009, K = 128; now 7.4.)
+// a gradient instead of 512 halve what the reduction reads.  All four gradients are one
+// launch (blockIdx.y), after the data gradients, which keep every layer's dZ: a launch
+// per layer took 7.4 us at n = 40009 (K = 128; 10.3 with 32-row chunks read from LDS two
+// bytes at a time), 4 x and their boundaries; now 13.6 for the four.
 constexpr int kWgBlock = 512;
 constexpr int kWgRows = 64;
+struct WeightSet {
+    const __bf16 *x, *dz;  // the layer's input [n][K] and dZ [n][kHid]
+    float *part;
+};
+struct WeightSets {
+    WeightSet set[kLayers + 1];  // layers 1 to 3 (K = kXW), then the embedding (K = kK0)
+};
+
 template <int K>
-__global__ __launch_bounds__(kWgBlock) void gemm_bwd_weight_kernel(const __bf16 *__restrict__ x,
-                                                                   int ldx, int n,
-                                                                   const __bf16 *__restrict__ dz,
-                                                                   float *__restrict__ part) {
+__device__ __forceinline__ void weight_gradient(const __bf16 *__restrict__ x, int n,
+                                                const __bf16 *__restrict__ dz,
+                                                float *__restrict__ part,
+                                                __bf16 (*xs)[kWgRows + 8],
+                                                __bf16 (*gs)[kWgRows + 8]) {
     constexpr int RB = K / 16;                               // 16-row blocks of dW
     constexpr int XV = kWgRows * K / 8 / kWgBlock;           // vectors of X a thread loads
     constexpr int XT = XV > 0 ? XV : 1;
     static_assert(RB <= kWgBlock / kWave && kWgRows * kHid / 8 == kWgBlock, "chunk shape");
-    __shared__ __bf16 xs[K][kWgRows + 8];
-    __shared__ __bf16 gs[kHid][kWgRows + 8];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const int rr = lane;  // a wavefront loads 8 columns of the chunk's 64 rows
@@ -866,7 +927,7 @@ __global__ __launch_bounds__(kWgBlock) void gemm_bwd_weight_kernel(const __bf16 
             const int cc = (wave + u * (kWgBlock / kWave)) * 8;
             xv[u] = bf16x8{};
             if (row < n && cc < K)
-                xv[u] = *reinterpret_cast<const bf16x8 *>(x + (size_t)row * ldx + cc);
+                xv[u] = *reinterpret_cast<const bf16x8 *>(x + (size_t)row * K + cc);
         }
         gv = bf16x8{};
         if (row < n) gv = *reinterpret_cast<const bf16x8 *>(dz + (size_t)row * kHid + wave * 8);
@@ -918,6 +979,16 @@ __global__ __launch_bounds__(kWgBlock) void gemm_bwd_weight_kernel(const __bf16 
                     acc[jb][t];
     }
     if (threadIdx.x < kHid) out[K * kHid + threadIdx.x] = db;
+}
+
+__global__ __launch_bounds__(kWgBlock) void gemm_bwd_weight_kernel(WeightSets sets, int n) {
+    __shared__ __bf16 xs[kXW][kWgRows + 8];
+    __shared__ __bf16 gs[kHid][kWgRows + 8];
+    const WeightSet ws = sets.set[blockIdx.y];
+    if (blockIdx.y < kLayers)
+        weight_gradient<kXW>(ws.x, n, ws.dz, ws.part, xs, gs);
+    else
+        weight_gradient<kK0>(ws.x, n, ws.dz, ws.part, xs, gs);
 }
 
 // out[i] = sum over p of part[p * stride + i], i < count, p in increasing
@@ -1247,8 +1318,8 @@ hipError_t launch_net_backward(const NetBuffers &nb, const NetSystem &sys, const
     const int n = sys.n;
     hipError_t e;
     const int rb = std::min(kReadoutParts, exact_blocks((long long)n * 16, kBlock * kReadRows));
-    readout_bwd_kernel<<<rb, kBlock, 0, st>>>(nb.h3, params + kOffR, gmax, n, nb.dgh, nb.dz,
-                                              nb.rpart);
+    readout_bwd_kernel<<<rb, kBlock, 0, st>>>(nb.h3, params + kOffR, gmax, n, nb.dgh,
+                                              nb.dz[kLayers], nb.rpart);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     RedSets sets;
     int blocks = 0, used = 0;
@@ -1259,22 +1330,21 @@ hipError_t launch_net_backward(const NetBuffers &nb, const NetSystem &sys, const
     reduce(nb.rpart, rb, kReadout, grad + kOffR);
     const int gb = exact_blocks(n, 16 * kWavesPerBlock);  // one 16-row tile per wavefront
     const int wgb = std::min(kWeightParts, exact_blocks(n, kWgRows));
+    WeightSets ws;
     for (int l = kLayers - 1; l >= 0; l--) {
+        layer_bwd_kernel<<<gb, kBlock, 0, st>>>(
+            nb.dz[l + 1], sys.tptr, sys.tsrc, sys.tw,
+            wb + kWtRowMajor + kK0 * kHid + l * kXW * kHid, nb.x[l], n, nb.dz[l]);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
         float *part = nb.wpart + (size_t)l * kWeightParts * kLayerStride;
-        gemm_bwd_weight_kernel<kXW><<<wgb, kWgBlock, 0, st>>>(nb.x[l], kXW, n, nb.dz, part);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        ws.set[l] = {nb.x[l], nb.dz[l + 1], part};
         reduce(part, wgb, kLayerStride, grad + kOffW1 + l * kLayerStride);
-        gemm_bwd_data_kernel<<<gb, kBlock, 0, st>>>(
-            nb.dz, n, wb + kWtRowMajor + kK0 * kHid + l * kXW * kHid, nb.dx);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        aggregate_bwd_kernel<<<row_blocks(n), kBlock, 0, st>>>(nb.dx, sys.tptr, sys.tsrc, sys.tw,
-                                                               nb.x[l], n, nb.dz);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     float *part = nb.wpart + (size_t)kLayers * kWeightParts * kLayerStride;
-    gemm_bwd_weight_kernel<kK0><<<wgb, kWgBlock, 0, st>>>(nb.x0, kK0, n, nb.dz, part);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    ws.set[kLayers] = {nb.x0, nb.dz[0], part};
     reduce(part, wgb, kK0 * kHid + kHid, grad + kOffW0);
+    gemm_bwd_weight_kernel<<<dim3(wgb, kLayers + 1), kWgBlock, 0, st>>>(ws, n);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
     reduce_parts_kernel<<<blocks, kRedWaves * kWave, 0, st>>>(sets);
     return hipGetLastError();
 }

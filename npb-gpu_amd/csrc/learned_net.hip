@@ -83,8 +83,9 @@ namespace {
 
 void free_buffers(NetBuffers &nb) {
     for (void *p : {(void *)nb.x0, (void *)nb.x[0], (void *)nb.x[1], (void *)nb.x[2],
-                    (void *)nb.h3, (void *)nb.dz, (void *)nb.dx, (void *)nb.gh, (void *)nb.dgh,
-                    (void *)nb.pw, (void *)nb.pd, (void *)nb.wpart, (void *)nb.rpart,
+                    (void *)nb.dz[0], (void *)nb.dz[1], (void *)nb.dz[2], (void *)nb.dz[3],
+                    (void *)nb.h3, (void *)nb.gh, (void *)nb.dgh, (void *)nb.pw,
+                    (void *)nb.pd, (void *)nb.wpart, (void *)nb.rpart,
                     (void *)nb.loss_part})
         (void)hipFree(p);
     const float *norm = nb.norm;
@@ -100,8 +101,7 @@ int ensure_buffers(npbcg_net *net, int n) {
     NET_HIP(hipMalloc(&nb.x0, sizeof(__bf16) * m * kK0));
     for (int l = 0; l < kLayers; l++) NET_HIP(hipMalloc(&nb.x[l], sizeof(__bf16) * m * kXW));
     NET_HIP(hipMalloc(&nb.h3, sizeof(__bf16) * m * kHid));
-    NET_HIP(hipMalloc(&nb.dz, sizeof(__bf16) * m * kHid));
-    NET_HIP(hipMalloc(&nb.dx, sizeof(float) * m * kXW));
+    for (int l = 0; l <= kLayers; l++) NET_HIP(hipMalloc(&nb.dz[l], sizeof(__bf16) * m * kHid));
     NET_HIP(hipMalloc(&nb.gh, sizeof(float) * 2 * m));
     NET_HIP(hipMalloc(&nb.dgh, sizeof(float) * 2 * m));
     NET_HIP(hipMalloc(&nb.pw, sizeof(float) * kPairs * m));
