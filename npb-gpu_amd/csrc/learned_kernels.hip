@@ -399,20 +399,6 @@ __global__ __launch_bounds__(kBlock) void sum_kernel(const double *__restrict__ 
 // Network forward
 // ---------------------------------------------------------------------------
 
-// X0 = standardised features, zero-padded to kK0 columns (BF16).
-__global__ __launch_bounds__(kBlock) void build_x0_kernel(const float *__restrict__ feat,
-                                                          const float *__restrict__ norm, int n,
-                                                          __bf16 *__restrict__ x0) {
-    const long long m = (long long)n * kK0;
-    for (long long i = blockIdx.x * (long long)kBlock + threadIdx.x; i < m;
-         i += (long long)gridDim.x * kBlock) {
-        const int j = (int)(i / kK0), c = (int)(i % kK0);
-        float v = 0.0f;
-        if (c < kFeat) v = (feat[(size_t)j * kFeat + c] - norm[c]) / norm[kFeat + c];
-        x0[i] = (__bf16)v;
-    }
-}
-
 // Y[n x 64] = ReLU(X[n x K] W + b): a wavefront computes the four 16x16
 // output blocks of TILES consecutive 16-row tiles, K in steps of 32.  Wt
 // is W transposed (64 x K, BF16); the wavefront loads its B fragments (and
@@ -423,21 +409,38 @@ __global__ __launch_bounds__(kBlock) void build_x0_kernel(const float *__restric
 // A[l%16][8(l/16)..+7] and B[8(l/16)..+7][l%16] and receives
 // D[4(l/16)..+3][l%16] of each 16x16x32 product.
 //
-// AGG (K = 128, a message-passing layer): columns 64.. of X are formed here,
+// Layer kinds.  kEmbed (K = 32): X is formed here, the eight standardised features
+// zero-padded to 32 columns (BF16), by the 16 lanes whose columns they are, and stored for
+// the backward pass when `keep` (a kernel of its own: 4.5 us and a launch boundary).
+// TILES = 1: the weights are 4 KB (4 tiles: network 51, 82 us at 17003, 75000, now 49, 80).
+// kMessage and kLast (K = 128, message passing): columns 64.. of X are formed here,
 // X[j, 64:128] = sum_t w[j,t] X[nbr[j,t], 0:64] in FP32, rounded to BF16, each lane
 // its 16 columns of its row (the four lanes of a row read whole lines of the
 // neighbours), and stored for the backward pass when `keep`.  As a kernel of its own
 // before the product: 5.8 + 8.6 us and a launch boundary at n = 40009; now 13.3 (network
-// and readout at 17003 71 us, now 60).  TILES = 2: 4 leave too few wavefronts (77 us at
+// and readout at 17003 71 us, then 60).  TILES = 2: 4 leave too few wavefronts (77 us at
 // 17003), 1 reads the weights twice as often (97 against 93 us at 75000).
-template <int K, int TILES, bool AGG>
+// kLast also computes the readout g = G tanh(ug . H3 + cg), h = G tanh(uh . H3 + ch) from
+// its rounded outputs, FP64 sums as in readout_sums: a lane's four columns, then the eight
+// sums (four rows, g and h) over 16 lanes, every step handing half of them on, so that
+// each pair of lanes ends with one sum and the tile needs one tanh; H3 itself is stored
+// for the backward pass alone.  A kernel of its own read H3 back: 5.7 us and a launch
+// boundary at n = 40009; here it adds 2.7.  (Network, with both kernels apart and now: 60
+// and 49 us at 17003, 73 and 65 at 40009, 92 and 80 at 75000.)
+enum LayerKind { kEmbed, kMessage, kLast };
+template <int K, int TILES, LayerKind KIND>
 __global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(__bf16 *x, int ldx, int n,
                                                           const __bf16 *__restrict__ wt,
                                                           const float *__restrict__ bias,
                                                           __bf16 *__restrict__ y, int ldy,
                                                           const int *__restrict__ nbr,
                                                           const float *__restrict__ wgt,
+                                                          const float *__restrict__ feat,
+                                                          const float *__restrict__ norm,
+                                                          const float *__restrict__ ro,
+                                                          float gmax, float *__restrict__ gh,
                                                           int keep) {
+    constexpr bool AGG = KIND != kEmbed;
     constexpr int KS = K / 32;
     constexpr int KL = AGG ? KS / 2 : KS;  // fragments that are loaded
     const int lane = threadIdx.x & (kWave - 1);
@@ -447,8 +450,22 @@ __global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(__bf16 *x, int ldx, in
     const int kq = 8 * (lane >> 4);
     bf16x8 av[KL], hv[AGG ? kNbr : 1][AGG ? KL : 1];
     float wv[kNbr];
+    f32x4 fv[2], mean[2], dev[2];
+    if constexpr (KIND == kEmbed) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            mean[q] = *reinterpret_cast<const f32x4 *>(norm + 4 * q);
+            dev[q] = *reinterpret_cast<const f32x4 *>(norm + kFeat + 4 * q);
+        }
+    }
     auto load_a = [&](int row0) {
         const int ar = row0 + (lane & 15);
+        if constexpr (KIND == kEmbed) {
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+                fv[q] = *reinterpret_cast<const f32x4 *>(feat + (size_t)min(ar, n - 1) * kFeat + 4 * q);
+            return;
+        }
         if constexpr (AGG) {
             const int j = min(ar, n - 1);
             int k[kNbr];
@@ -471,7 +488,7 @@ __global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(__bf16 *x, int ldx, in
     };
     load_a(tile0 * 16);
     bf16x8 bw[KS][4];
-    float bj[4];
+    float bj[4], ug[4], uh[4];
 #pragma unroll
     for (int jb = 0; jb < 4; jb++) {
 #pragma unroll
@@ -479,6 +496,10 @@ __global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(__bf16 *x, int ldx, in
             bw[k][jb] = *reinterpret_cast<const bf16x8 *>(
                 wt + (size_t)(jb * 16 + (lane & 15)) * K + 32 * k + kq);
         bj[jb] = bias[jb * 16 + (lane & 15)];
+        if constexpr (KIND == kLast) {
+            ug[jb] = ro[jb * 16 + (lane & 15)];
+            uh[jb] = ro[kHid + 1 + jb * 16 + (lane & 15)];
+        }
     }
     for (int t = 0; t < TILES; t++) {
         const int row0 = (tile0 + t) * 16;
@@ -486,6 +507,15 @@ __global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(__bf16 *x, int ldx, in
         bf16x8 cur[KS];
 #pragma unroll
         for (int k = 0; k < KL; k++) cur[k] = av[k];
+        if constexpr (KIND == kEmbed) {
+            const int ar = row0 + (lane & 15);
+            cur[0] = bf16x8{};
+            if (kq == 0 && ar < n)
+#pragma unroll
+                for (int c = 0; c < kFeat; c++)
+                    cur[0][c] = (__bf16)((fv[c / 4][c % 4] - mean[c / 4][c % 4]) / dev[c / 4][c % 4]);
+            if (keep && ar < n) *reinterpret_cast<bf16x8 *>(x + (size_t)ar * ldx + kq) = cur[0];
+        }
         if constexpr (AGG) {
             const int ar = row0 + (lane & 15);
 #pragma unroll
@@ -511,14 +541,39 @@ __global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(__bf16 *x, int ldx, in
 #pragma unroll
             for (int jb = 0; jb < 4; jb++)
                 acc[jb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur[k], bw[k][jb], acc[jb], 0, 0, 0);
+        double sums[8] = {};  // g of the lane's four rows, then h
 #pragma unroll
         for (int jb = 0; jb < 4; jb++) {
             const int j = jb * 16 + (lane & 15);
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 const int row = row0 + 4 * (lane >> 4) + q;
-                if (row < n) y[(size_t)row * ldy + j] = (__bf16)fmaxf(acc[jb][q] + bj[jb], 0.0f);
+                const __bf16 v = (__bf16)fmaxf(acc[jb][q] + bj[jb], 0.0f);
+                if (row < n && (KIND != kLast || keep)) y[(size_t)row * ldy + j] = v;
+                if constexpr (KIND == kLast) {
+                    sums[q] += (double)((float)v * ug[jb]);
+                    sums[4 + q] += (double)((float)v * uh[jb]);
+                }
             }
+        }
+        if constexpr (KIND == kLast) {
+            // sum i of the eight ends in the lanes with bits 3, 2, 1 of the lane = bits 2, 1, 0 of i
+#pragma unroll
+            for (int half = 4; half >= 1; half /= 2) {
+                const bool up = (lane & (2 * half)) != 0;
+#pragma unroll
+                for (int i = 0; i < half; i++) {
+                    const double give = up ? sums[i] : sums[i + half];
+                    const double mine = up ? sums[i + half] : sums[i];
+                    sums[i] = mine + __shfl_xor(give, 2 * half, 16);
+                }
+            }
+            sums[0] += __shfl_xor(sums[0], 1, 16);
+            const int i = (lane & 15) >> 1;
+            const int row = row0 + 4 * (lane >> 4) + (i & 3);
+            const double at = sums[0] + (double)(i < 4 ? ro[kHid] : ro[2 * kHid + 1]);
+            const float v = (float)(gmax * tanh(at));
+            if ((lane & 1) == 0 && row < n) gh[(i < 4 ? 0 : n) + row] = v;
         }
     }
 }
@@ -527,8 +582,7 @@ __global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(__bf16 *x, int ldx, in
 // group of 16 lanes, four columns a lane: lane t of the group keeps row j0 + t's
 // sums (lanes past kReadRows: the last row's), so that one tanh serves kReadRows
 // rows; hv holds the lane's columns of every row.  FP64 tanh is most of the
-// readout kernels (a row per group: 11.0 us forward, 11.1 backward at n = 40009; now
-// 5.7 and 7.5).
+// readout's backward kernel (a row per group: 11.1 us at n = 40009, now 7.5).
 constexpr int kReadRows = 4;
 __device__ __forceinline__ void readout_sums(const __bf16 *__restrict__ h3,
                                              const float (&ug)[4], const float (&uh)[4],
@@ -556,28 +610,6 @@ __device__ __forceinline__ void readout_sums(const __bf16 *__restrict__ h3,
             sg = a;
             sh = b;
         }
-    }
-}
-
-// g = G tanh(ug . H3 + cg), h = G tanh(uh . H3 + ch).
-__global__ __launch_bounds__(kBlock) void readout_fwd_kernel(const __bf16 *__restrict__ h3,
-                                                             const float *__restrict__ ro,
-                                                             float gmax, int n,
-                                                             float *__restrict__ gh) {
-    const long long j0 = (blockIdx.x * (long long)kBlock + threadIdx.x) / 16 * kReadRows;
-    const int sub = threadIdx.x & 15, f = sub * 4;
-    float ug[4], uh[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        ug[q] = ro[f + q];
-        uh[q] = ro[kHid + 1 + f + q];
-    }
-    bf16x4 hv[kReadRows];
-    double sg, sh;
-    readout_sums(h3, ug, uh, ro[kHid], ro[2 * kHid + 1], j0, n, hv, sg, sh);
-    if (sub < kReadRows && j0 + sub < n) {
-        gh[j0 + sub] = (float)(gmax * tanh(sg));
-        gh[n + j0 + sub] = (float)(gmax * tanh(sh));
     }
 }
 
@@ -1284,23 +1316,22 @@ hipError_t launch_net_forward(const NetBuffers &nb, const NetSystem &sys, const 
                               const __bf16 *wb, float gmax, int keep, hipStream_t st) {
     const int n = sys.n;
     hipError_t e;
-    build_x0_kernel<<<blocks_for((long long)n * kK0), kBlock, 0, st>>>(sys.feat, nb.norm, n,
-                                                                      nb.x0);
+    constexpr int kT0 = 1, kT = 2;
+    gemm_fwd_kernel<kK0, kT0, kEmbed><<<exact_blocks(n, 16 * kT0 * kWavesPerBlock), kBlock, 0, st>>>(
+        nb.x0, kK0, n, wb + kWtTransposed, params + kOffB0, nb.x[0], kXW, nullptr, nullptr, sys.feat,
+        nb.norm, nullptr, 0.f, nullptr, keep);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    constexpr int kT0 = 4, kT = 2;
-    gemm_fwd_kernel<kK0, kT0, false><<<exact_blocks(n, 16 * kT0 * kWavesPerBlock), kBlock, 0, st>>>(
-        nb.x0, kK0, n, wb + kWtTransposed, params + kOffB0, nb.x[0], kXW, nullptr, nullptr, 0);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    const int blocks = exact_blocks(n, 16 * kT * kWavesPerBlock);
     for (int l = 0; l < kLayers; l++) {
-        __bf16 *out = l + 1 < kLayers ? nb.x[l + 1] : nb.h3;
-        const int ldy = l + 1 < kLayers ? kXW : kHid;
-        gemm_fwd_kernel<kXW, kT, true><<<exact_blocks(n, 16 * kT * kWavesPerBlock), kBlock, 0, st>>>(
+        const bool last = l + 1 == kLayers;
+        const auto kernel = last ? gemm_fwd_kernel<kXW, kT, kLast> : gemm_fwd_kernel<kXW, kT, kMessage>;
+        kernel<<<blocks, kBlock, 0, st>>>(
             nb.x[l], kXW, n, wb + kWtTransposed + kK0 * kHid + l * kXW * kHid,
-            params + kOffB1 + l * kLayerStride, out, ldy, sys.nbr, sys.wgt, keep);
+            params + kOffB1 + l * kLayerStride, last ? nb.h3 : nb.x[l + 1], last ? kHid : kXW,
+            sys.nbr, sys.wgt, nullptr, nullptr, params + kOffR, gmax, nb.gh, keep);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    readout_fwd_kernel<<<exact_blocks((long long)n * 16, kBlock * kReadRows), kBlock, 0, st>>>(nb.h3, params + kOffR, gmax, n, nb.gh);
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 hipError_t launch_pair_loss(const NetBuffers &nb, const NetSystem &sys, const PairSet &ps,
