@@ -400,35 +400,31 @@ __global__ __launch_bounds__(kBlock) void sum_kernel(const double *__restrict__ 
 // ---------------------------------------------------------------------------
 
 // Y[n x 64] = ReLU(X[n x K] W + b): a wavefront computes the four 16x16
-// output blocks of TILES consecutive 16-row tiles, K in steps of 32.  Wt
-// is W transposed (64 x K, BF16); the wavefront loads its B fragments (and
-// the bias) once and keeps them in registers for all its tiles, so the
-// weights are read once per wavefront rather than once per tile (at K = 128
-// they are 16 KB against the tile's 4 KB of X).  The next tile's A fragments
-// are loaded before the current tile's products.  Lane l supplies
+// output blocks of a 16-row tile, K in steps of 32.  Wt is W transposed (64 x K,
+// BF16), which the workgroup's four wavefronts share in LDS.  Lane l supplies
 // A[l%16][8(l/16)..+7] and B[8(l/16)..+7][l%16] and receives
-// D[4(l/16)..+3][l%16] of each 16x16x32 product.
+// D[4(l/16)..+3][l%16] of each 16x16x32 product.  Bound by the chain neighbours ->
+// their rows -> products -> stores with few wavefronts to cover it (2.4 a SIMD at
+// n = 40009): W in registers, 64 of them a lane, and two tiles a wavefront to read it
+// half as often took the network 33, 50 and 66 us at 10007, 40009 and 75000; LDS and
+// one tile take 24, 36 and 48 (two tiles: 29, 42, 53).
 //
 // Layer kinds.  kEmbed (K = 32): X is formed here, the eight standardised features
 // zero-padded to 32 columns (BF16), by the 16 lanes whose columns they are, and stored for
 // the backward pass when `keep` (a kernel of its own: 4.5 us and a launch boundary).
-// TILES = 1: the weights are 4 KB (4 tiles: network 51, 82 us at 17003, 75000, now 49, 80).
 // kMessage and kLast (K = 128, message passing): columns 64.. of X are formed here,
 // X[j, 64:128] = sum_t w[j,t] X[nbr[j,t], 0:64] in FP32, rounded to BF16, each lane
 // its 16 columns of its row (the four lanes of a row read whole lines of the
-// neighbours), and stored for the backward pass when `keep`.  As a kernel of its own
-// before the product: 5.8 + 8.6 us and a launch boundary at n = 40009; now 13.3 (network
-// and readout at 17003 71 us, then 60).  TILES = 2: 4 leave too few wavefronts (77 us at
-// 17003), 1 reads the weights twice as often (97 against 93 us at 75000).
+// neighbours), and stored for the backward pass when `keep`.  (As a kernel of its own
+// before the product 5.8 us at n = 40009 and a launch boundary.)
 // kLast also computes the readout g = G tanh(ug . H3 + cg), h = G tanh(uh . H3 + ch) from
 // its rounded outputs, FP64 sums as in readout_sums: a lane's four columns, then the eight
 // sums (four rows, g and h) over 16 lanes, every step handing half of them on, so that
 // each pair of lanes ends with one sum and the tile needs one tanh; H3 itself is stored
-// for the backward pass alone.  A kernel of its own read H3 back: 5.7 us and a launch
-// boundary at n = 40009; here it adds 2.7.  (Network, with both kernels apart and now: 60
-// and 49 us at 17003, 73 and 65 at 40009, 92 and 80 at 75000.)
+// for the backward pass alone.  (A kernel of its own read H3 back: 5.7 us at n = 40009
+// and a launch boundary; here 2.7.)
 enum LayerKind { kEmbed, kMessage, kLast };
-template <int K, int TILES, LayerKind KIND>
+template <int K, LayerKind KIND>
 __global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(__bf16 *x, int ldx, int n,
                                                           const __bf16 *__restrict__ wt,
                                                           const float *__restrict__ bias,
@@ -442,139 +438,123 @@ __global__ __launch_bounds__(kBlock) void gemm_fwd_kernel(__bf16 *x, int ldx, in
                                                           int keep) {
     constexpr bool AGG = KIND != kEmbed;
     constexpr int KS = K / 32;
-    constexpr int KL = AGG ? KS / 2 : KS;  // fragments that are loaded
+    constexpr int KL = AGG ? KS / 2 : KS;        // fragments that are loaded
+    constexpr int WV = K * kHid / 8 / kBlock;    // vectors of W^T a thread loads
+    __shared__ __bf16 ws[kHid][K + 8];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
-    const int tile0 = (blockIdx.x * kWavesPerBlock + wave) * TILES;
-    if (tile0 * 16 >= n) return;
+    const int row0 = (blockIdx.x * kWavesPerBlock + wave) * 16;
+    const int ar = row0 + (lane & 15);
+    const int at = min(ar, n - 1);  // every wavefront reaches the barrier
     const int kq = 8 * (lane >> 4);
-    bf16x8 av[KL], hv[AGG ? kNbr : 1][AGG ? KL : 1];
+    int k[kNbr];
     float wv[kNbr];
-    f32x4 fv[2], mean[2], dev[2];
-    if constexpr (KIND == kEmbed) {
+    if constexpr (AGG)
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            mean[q] = *reinterpret_cast<const f32x4 *>(norm + 4 * q);
-            dev[q] = *reinterpret_cast<const f32x4 *>(norm + kFeat + 4 * q);
+        for (int t = 0; t < kNbr; t++) {
+            k[t] = nbr[(size_t)at * kNbr + t];
+            wv[t] = wgt[(size_t)at * kNbr + t];
         }
-    }
-    auto load_a = [&](int row0) {
-        const int ar = row0 + (lane & 15);
-        if constexpr (KIND == kEmbed) {
+    bf16x8 wl[WV];
 #pragma unroll
-            for (int q = 0; q < 2; q++)
-                fv[q] = *reinterpret_cast<const f32x4 *>(feat + (size_t)min(ar, n - 1) * kFeat + 4 * q);
-            return;
-        }
-        if constexpr (AGG) {
-            const int j = min(ar, n - 1);
-            int k[kNbr];
-#pragma unroll
-            for (int t = 0; t < kNbr; t++) {
-                k[t] = nbr[(size_t)j * kNbr + t];
-                wv[t] = wgt[(size_t)j * kNbr + t];
-            }
-#pragma unroll
-            for (int t = 0; t < kNbr; t++)
-#pragma unroll
-                for (int q = 0; q < KL; q++)
-                    hv[t][q] = *reinterpret_cast<const bf16x8 *>(x + (size_t)k[t] * ldx + 32 * q + kq);
-        }
+    for (int u = 0; u < WV; u++)
+        wl[u] = *reinterpret_cast<const bf16x8 *>(wt + (size_t)(threadIdx.x + u * kBlock) * 8);
+    bf16x8 cur[KS], hv[AGG ? kNbr : 1][KL];
+    if constexpr (AGG) {
 #pragma unroll
         for (int q = 0; q < KL; q++) {
-            av[q] = bf16x8{};
-            if (ar < n) av[q] = *reinterpret_cast<const bf16x8 *>(x + (size_t)ar * ldx + 32 * q + kq);
+            cur[q] = *reinterpret_cast<const bf16x8 *>(x + (size_t)at * ldx + 32 * q + kq);
+            if (ar >= n) cur[q] = bf16x8{};
         }
-    };
-    load_a(tile0 * 16);
-    bf16x8 bw[KS][4];
+#pragma unroll
+        for (int t = 0; t < kNbr; t++)
+#pragma unroll
+            for (int q = 0; q < KL; q++)
+                hv[t][q] = *reinterpret_cast<const bf16x8 *>(x + (size_t)k[t] * ldx + 32 * q + kq);
+    } else {
+        float f[kFeat];
+#pragma unroll
+        for (int c = 0; c < kFeat; c++) f[c] = (feat[(size_t)at * kFeat + c] - norm[c]) / norm[kFeat + c];
+        cur[0] = bf16x8{};
+        if (kq == 0 && ar < n)
+#pragma unroll
+            for (int c = 0; c < kFeat; c++) cur[0][c] = (__bf16)f[c];
+        if (keep && ar < n) *reinterpret_cast<bf16x8 *>(x + (size_t)ar * ldx + kq) = cur[0];
+    }
     float bj[4], ug[4], uh[4];
 #pragma unroll
     for (int jb = 0; jb < 4; jb++) {
-#pragma unroll
-        for (int k = 0; k < KS; k++)
-            bw[k][jb] = *reinterpret_cast<const bf16x8 *>(
-                wt + (size_t)(jb * 16 + (lane & 15)) * K + 32 * k + kq);
         bj[jb] = bias[jb * 16 + (lane & 15)];
         if constexpr (KIND == kLast) {
             ug[jb] = ro[jb * 16 + (lane & 15)];
             uh[jb] = ro[kHid + 1 + jb * 16 + (lane & 15)];
         }
     }
-    for (int t = 0; t < TILES; t++) {
-        const int row0 = (tile0 + t) * 16;
-        if (row0 >= n) break;  // the same for the whole wavefront
-        bf16x8 cur[KS];
 #pragma unroll
-        for (int k = 0; k < KL; k++) cur[k] = av[k];
-        if constexpr (KIND == kEmbed) {
-            const int ar = row0 + (lane & 15);
-            cur[0] = bf16x8{};
-            if (kq == 0 && ar < n)
+    for (int u = 0; u < WV; u++) {
+        const int i = (threadIdx.x + u * kBlock) * 8;
+        *reinterpret_cast<bf16x8 *>(&ws[i / K][i % K]) = wl[u];
+    }
+    __syncthreads();
+    if (row0 >= n) return;
+    if constexpr (AGG) {
 #pragma unroll
-                for (int c = 0; c < kFeat; c++)
-                    cur[0][c] = (__bf16)((fv[c / 4][c % 4] - mean[c / 4][c % 4]) / dev[c / 4][c % 4]);
-            if (keep && ar < n) *reinterpret_cast<bf16x8 *>(x + (size_t)ar * ldx + kq) = cur[0];
-        }
-        if constexpr (AGG) {
-            const int ar = row0 + (lane & 15);
+        for (int q = 0; q < KL; q++) {
+            bf16x8 o;
 #pragma unroll
-            for (int q = 0; q < KL; q++) {
-                bf16x8 o;
+            for (int c = 0; c < 8; c++) {
+                float acc = 0.f;
 #pragma unroll
-                for (int c = 0; c < 8; c++) {
-                    float acc = 0.f;
-#pragma unroll
-                    for (int u = 0; u < kNbr; u++) acc = fmaf(wv[u], (float)hv[u][q][c], acc);
-                    o[c] = (__bf16)acc;
-                }
-                if (ar >= n) o = bf16x8{};
-                cur[KL + q] = o;
-                if (keep && ar < n)
-                    *reinterpret_cast<bf16x8 *>(x + (size_t)ar * ldx + kHid + 32 * q + kq) = o;
+                for (int t = 0; t < kNbr; t++) acc = fmaf(wv[t], (float)hv[t][q][c], acc);
+                o[c] = (__bf16)acc;
             }
+            if (ar >= n) o = bf16x8{};
+            cur[KL + q] = o;
+            if (keep && ar < n)
+                *reinterpret_cast<bf16x8 *>(x + (size_t)ar * ldx + kHid + 32 * q + kq) = o;
         }
-        if (t + 1 < TILES) load_a(row0 + 16);
-        f32x4 acc[4] = {};
+    }
+    f32x4 acc[4] = {};
 #pragma unroll
-        for (int k = 0; k < KS; k++)
-#pragma unroll
-            for (int jb = 0; jb < 4; jb++)
-                acc[jb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur[k], bw[k][jb], acc[jb], 0, 0, 0);
-        double sums[8] = {};  // g of the lane's four rows, then h
+    for (int q = 0; q < KS; q++)
 #pragma unroll
         for (int jb = 0; jb < 4; jb++) {
-            const int j = jb * 16 + (lane & 15);
+            const bf16x8 bv = *reinterpret_cast<const bf16x8 *>(&ws[jb * 16 + (lane & 15)][32 * q + kq]);
+            acc[jb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur[q], bv, acc[jb], 0, 0, 0);
+        }
+    double sums[8] = {};  // g of the lane's four rows, then h
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int row = row0 + 4 * (lane >> 4) + q;
-                const __bf16 v = (__bf16)fmaxf(acc[jb][q] + bj[jb], 0.0f);
-                if (row < n && (KIND != kLast || keep)) y[(size_t)row * ldy + j] = v;
-                if constexpr (KIND == kLast) {
-                    sums[q] += (double)((float)v * ug[jb]);
-                    sums[4 + q] += (double)((float)v * uh[jb]);
-                }
+    for (int jb = 0; jb < 4; jb++) {
+        const int j = jb * 16 + (lane & 15);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int row = row0 + 4 * (lane >> 4) + q;
+            const __bf16 v = (__bf16)fmaxf(acc[jb][q] + bj[jb], 0.0f);
+            if (row < n && (KIND != kLast || keep)) y[(size_t)row * ldy + j] = v;
+            if constexpr (KIND == kLast) {
+                sums[q] += (double)((float)v * ug[jb]);
+                sums[4 + q] += (double)((float)v * uh[jb]);
             }
         }
-        if constexpr (KIND == kLast) {
-            // sum i of the eight ends in the lanes with bits 3, 2, 1 of the lane = bits 2, 1, 0 of i
+    }
+    if constexpr (KIND == kLast) {
+        // sum i of the eight ends in the lanes with bits 3, 2, 1 of the lane = bits 2, 1, 0 of i
 #pragma unroll
-            for (int half = 4; half >= 1; half /= 2) {
-                const bool up = (lane & (2 * half)) != 0;
+        for (int half = 4; half >= 1; half /= 2) {
+            const bool up = (lane & (2 * half)) != 0;
 #pragma unroll
-                for (int i = 0; i < half; i++) {
-                    const double give = up ? sums[i] : sums[i + half];
-                    const double mine = up ? sums[i + half] : sums[i];
-                    sums[i] = mine + __shfl_xor(give, 2 * half, 16);
-                }
+            for (int i = 0; i < half; i++) {
+                const double give = up ? sums[i] : sums[i + half];
+                const double mine = up ? sums[i + half] : sums[i];
+                sums[i] = mine + __shfl_xor(give, 2 * half, 16);
             }
-            sums[0] += __shfl_xor(sums[0], 1, 16);
-            const int i = (lane & 15) >> 1;
-            const int row = row0 + 4 * (lane >> 4) + (i & 3);
-            const double at = sums[0] + (double)(i < 4 ? ro[kHid] : ro[2 * kHid + 1]);
-            const float v = (float)(gmax * tanh(at));
-            if ((lane & 1) == 0 && row < n) gh[(i < 4 ? 0 : n) + row] = v;
         }
+        sums[0] += __shfl_xor(sums[0], 1, 16);
+        const int i = (lane & 15) >> 1;
+        const int row = row0 + 4 * (lane >> 4) + (i & 3);
+        const double sum = sums[0] + (double)(i < 4 ? ro[kHid] : ro[2 * kHid + 1]);
+        const float v = (float)(gmax * tanh(sum));
+        if ((lane & 1) == 0 && row < n) gh[(i < 4 ? 0 : n) + row] = v;
     }
 }
 
@@ -1316,15 +1296,14 @@ hipError_t launch_net_forward(const NetBuffers &nb, const NetSystem &sys, const 
                               const __bf16 *wb, float gmax, int keep, hipStream_t st) {
     const int n = sys.n;
     hipError_t e;
-    constexpr int kT0 = 1, kT = 2;
-    gemm_fwd_kernel<kK0, kT0, kEmbed><<<exact_blocks(n, 16 * kT0 * kWavesPerBlock), kBlock, 0, st>>>(
+    const int blocks = exact_blocks(n, 16 * kWavesPerBlock);  // one 16-row tile per wavefront
+    gemm_fwd_kernel<kK0, kEmbed><<<blocks, kBlock, 0, st>>>(
         nb.x0, kK0, n, wb + kWtTransposed, params + kOffB0, nb.x[0], kXW, nullptr, nullptr, sys.feat,
         nb.norm, nullptr, 0.f, nullptr, keep);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    const int blocks = exact_blocks(n, 16 * kT * kWavesPerBlock);
     for (int l = 0; l < kLayers; l++) {
         const bool last = l + 1 == kLayers;
-        const auto kernel = last ? gemm_fwd_kernel<kXW, kT, kLast> : gemm_fwd_kernel<kXW, kT, kMessage>;
+        const auto kernel = last ? gemm_fwd_kernel<kXW, kLast> : gemm_fwd_kernel<kXW, kMessage>;
         kernel<<<blocks, kBlock, 0, st>>>(
             nb.x[l], kXW, n, wb + kWtTransposed + kK0 * kHid + l * kXW * kHid,
             params + kOffB1 + l * kLayerStride, last ? nb.h3 : nb.x[l + 1], last ? kHid : kXW,
