@@ -794,38 +794,51 @@ __device__ __forceinline__ bf16x8 take_bf16(float *v) {
 //   dZprev = dH * (Hprev > 0) in BF16, Hprev = X[:, 0:64] of the layer's input.
 // The sum over the in-edges is taken in FP32 before the product, where a row is 128
 // bytes of BF16, not of the product's FP32 result; as three BF16 terms (take_bf16) it
-// enters the matrix units whole.  A wavefront owns 16 rows, four lanes a row, each the
-// 16 columns its A fragments need; four edges a round, the next round's edges loaded
-// ahead.  W sits in LDS, read once a workgroup.  Bound by the chain row pointer ->
-// edges -> gathers and the longest in-edge list of 16 rows.
+// enters the matrix units whole.  A workgroup owns 64 rows: eight lanes a row gather, 8
+// columns each, four edges a round with the next round's edges loaded ahead, and leave the
+// terms in LDS beside W; then each of the eight wavefronts makes half of a 16-row
+// tile's output.  Bound by the chain row pointer -> edges -> gathers and the longest
+// in-edge list of a wavefront's rows.
 // As a product to FP32 rows in memory and an aggregation kernel, 11.0 + 12.3 us and a
-// launch boundary at n = 40009; now 16.6 (eight edges a round: the step is 3 % slower at
-// 17003 and 75000).
+// launch boundary at n = 40009; with a tile and its gathers (four lanes a row) to a
+// wavefront 15.3; now 13.9 (loss and gradient at 17003 170 us, now 163; at 40009 210 and
+// 207).
 constexpr int kWPad = kHid + 8;
-__global__ __launch_bounds__(kBlock) void layer_bwd_kernel(
+constexpr int kBwdBlock = 512, kBwdRows = kBwdBlock / 8;
+__global__ __launch_bounds__(kBwdBlock) void layer_bwd_kernel(
     const __bf16 *__restrict__ dz, const int *__restrict__ tptr, const int *__restrict__ tsrc,
     const float *__restrict__ tw, const __bf16 *__restrict__ w, const __bf16 *__restrict__ x,
     int n, __bf16 *__restrict__ dzprev) {
     __shared__ __bf16 ws[kXW][kWPad];
-    constexpr int WV = kXW * kHid / 8 / kBlock;  // vectors of W a thread loads
+    __shared__ __bf16 terms[3][kBwdRows][kWPad];
+    constexpr int WV = kXW * kHid / 8 / kBwdBlock;  // vectors of W a thread loads
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
-    const int row0 = (blockIdx.x * kWavesPerBlock + wave) * 16;
-    const int ar = row0 + (lane & 15);
-    const int kq = 8 * (lane >> 4);
+    const int block0 = blockIdx.x * kBwdRows;
+    const int local = threadIdx.x / 8, col = 8 * (threadIdx.x & 7);
     int e0 = 0, e1 = 0;
-    bf16x8 own[2] = {};
-    if (ar < n) {
-        e0 = tptr[ar];
-        e1 = tptr[ar + 1];
-#pragma unroll
-        for (int q = 0; q < 2; q++)
-            own[q] = *reinterpret_cast<const bf16x8 *>(dz + (size_t)ar * kHid + 32 * q + kq);
+    if (block0 + local < n) {
+        e0 = tptr[block0 + local];
+        e1 = tptr[block0 + local + 1];
     }
     bf16x8 wv[WV];
 #pragma unroll
     for (int u = 0; u < WV; u++)
-        wv[u] = *reinterpret_cast<const bf16x8 *>(w + (size_t)(threadIdx.x + u * kBlock) * 8);
+        wv[u] = *reinterpret_cast<const bf16x8 *>(w + (size_t)(threadIdx.x + u * kBwdBlock) * 8);
+    // the wavefront's part of the output: tile wave / 2, columns 32 (wave % 2) ..
+    const int tile = 16 * (wave / 2), row0 = block0 + tile, j0 = 32 * (wave & 1);
+    const int kq = 8 * (lane >> 4);
+    bf16x8 own[2];
+    __bf16 h[2][4];
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+        own[q] = *reinterpret_cast<const bf16x8 *>(
+            dz + (size_t)min(row0 + (lane & 15), n - 1) * kHid + 32 * q + kq);
+#pragma unroll
+    for (int jb = 0; jb < 2; jb++)
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            h[jb][t] = x[(size_t)min(row0 + 4 * (lane >> 4) + t, n - 1) * kXW + j0 + jb * 16 + (lane & 15)];
     int src[4];
     float wt[4];
     auto edges = [&](int b) {
@@ -837,54 +850,45 @@ __global__ __launch_bounds__(kBlock) void layer_bwd_kernel(
         }
     };
     if (e0 < e1) edges(e0);
-#pragma unroll
-    for (int u = 0; u < WV; u++) {
-        const int i = (threadIdx.x + u * kBlock) * 8;
-        *reinterpret_cast<bf16x8 *>(&ws[i / kHid][i % kHid]) = wv[u];
-    }
-    __bf16 h[kHid / 16][4];
-#pragma unroll
-    for (int jb = 0; jb < kHid / 16; jb++)
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-            h[jb][t] = x[(size_t)min(row0 + 4 * (lane >> 4) + t, n - 1) * kXW + jb * 16 + (lane & 15)];
-    float s[2][8] = {};
+    float s[8] = {};
     for (int b = e0; b < e1; b += 4) {
-        bf16x8 g[4][2];
+        bf16x8 g[4];
         float cur[4];
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             cur[u] = wt[u];
-#pragma unroll
-            for (int q = 0; q < 2; q++)
-                g[u][q] = *reinterpret_cast<const bf16x8 *>(dz + (size_t)src[u] * kHid + 32 * q + kq);
+            g[u] = *reinterpret_cast<const bf16x8 *>(dz + (size_t)src[u] * kHid + col);
         }
         if (b + 4 < e1) edges(b + 4);
 #pragma unroll
         for (int u = 0; u < 4; u++)
             if (b + u < e1)
 #pragma unroll
-                for (int q = 0; q < 2; q++)
-#pragma unroll
-                    for (int c = 0; c < 8; c++) s[q][c] = fmaf(cur[u], (float)g[u][q][c], s[q][c]);
+                for (int c = 0; c < 8; c++) s[c] = fmaf(cur[u], (float)g[u][c], s[c]);
     }
-    bf16x8 agg[3][2];
 #pragma unroll
     for (int t = 0; t < 3; t++)
+        *reinterpret_cast<bf16x8 *>(&terms[t][local][col]) = take_bf16(s);
 #pragma unroll
-        for (int q = 0; q < 2; q++) agg[t][q] = take_bf16(s[q]);
+    for (int u = 0; u < WV; u++) {
+        const int i = (threadIdx.x + u * kBwdBlock) * 8;
+        *reinterpret_cast<bf16x8 *>(&ws[i / kHid][i % kHid]) = wv[u];
+    }
     __syncthreads();
 #pragma unroll
-    for (int jb = 0; jb < kHid / 16; jb++) {
-        const int j = jb * 16 + (lane & 15);
+    for (int jb = 0; jb < 2; jb++) {
+        const int j = j0 + jb * 16 + (lane & 15);
         f32x4 acc = {};
 #pragma unroll
         for (int q = 0; q < 2; q++) {
             const bf16x8 b1 = *reinterpret_cast<const bf16x8 *>(&ws[j][32 * q + kq]);
             const bf16x8 b2 = *reinterpret_cast<const bf16x8 *>(&ws[kHid + j][32 * q + kq]);
 #pragma unroll
-            for (int t = 2; t >= 0; t--)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(agg[t][q], b2, acc, 0, 0, 0);
+            for (int t = 2; t >= 0; t--) {
+                const bf16x8 at =
+                    *reinterpret_cast<const bf16x8 *>(&terms[t][tile + (lane & 15)][32 * q + kq]);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at, b2, acc, 0, 0, 0);
+            }
             acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(own[q], b1, acc, 0, 0, 0);
         }
 #pragma unroll
@@ -1338,11 +1342,10 @@ hipError_t launch_net_backward(const NetBuffers &nb, const NetSystem &sys, const
         blocks += (columns + kWave - 1) / kWave;
     };
     reduce(nb.rpart, rb, kReadout, grad + kOffR);
-    const int gb = exact_blocks(n, 16 * kWavesPerBlock);  // one 16-row tile per wavefront
     const int wgb = std::min(kWeightParts, exact_blocks(n, kWgRows));
     WeightSets ws;
     for (int l = kLayers - 1; l >= 0; l--) {
-        layer_bwd_kernel<<<gb, kBlock, 0, st>>>(
+        layer_bwd_kernel<<<exact_blocks(n, kBwdRows), kBwdBlock, 0, st>>>(
             nb.dz[l + 1], sys.tptr, sys.tsrc, sys.tw,
             wb + kWtRowMajor + kK0 * kHid + l * kXW * kHid, nb.x[l], n, nb.dz[l]);
         if ((e = hipGetLastError()) != hipSuccess) return e;
