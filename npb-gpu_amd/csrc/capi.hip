@@ -476,7 +476,7 @@ int ensure_resident(npbcg_ctx *c, int steps, int niter) {
         NPBCG_HIP(hipMalloc(&rs.wave_off, sizeof(int) * maps.size()));
         rs.word_row = rs.wave_off + sh.wave_off.size();
         rs.row_word = rs.word_row + sh.word_row.size();
-        NPBCG_HIP(hipMalloc(&rs.abort_word, sizeof(unsigned)));
+        NPBCG_HIP(hipMalloc(&rs.abort_word, 2 * sizeof(unsigned)));
         NPBCG_HIP(hipMalloc(&rs.col, sizeof(uint16_t) * entries));
         NPBCG_HIP(hipMalloc(&rs.val, sizeof(double) * entries));
         NPBCG_HIP(hipMemcpyAsync(rs.wave_off, maps.data(), sizeof(int) * maps.size(),
@@ -1156,6 +1156,15 @@ int save_state(npbcg_ctx *c, bool back) {
 }
 
 }  // namespace
+
+int npbcg_test_resident_give_up(npbcg_ctx *c, int iteration) {
+    if (!c || c->rshape.grid < 1 || c->rshape.words >= c->rshape.stride)
+        return set_error(NPBCG_ERR_INVALID,
+                         "npbcg_test_resident_give_up: no resident engine with a spare word");
+    c->rstate.give_up_at = iteration;
+    clear_error();
+    return NPBCG_OK;
+}
 
 int npbcg_conj_grad_device(npbcg_ctx *c, double *rnorm) {
     npbcg_detail::TraceRange trace("npbcg_conj_grad");

@@ -296,8 +296,9 @@ struct ResidentState {
     size_t xchg_words = 0;
     double *part = nullptr;        // resident_partials(shape, niter) doubles
     size_t part_words = 0;
-    unsigned *abort_word = nullptr;
+    unsigned *abort_word = nullptr;  // two words
     long long spin_limit = 0;      // wall-clock ticks one exchange may wait
+    int give_up_at = -1;           // tests: the launch with this history entry gives up
 };
 // The shape for order n on `cus` CUs with lds_cap bytes of LDS per workgroup;
 // false where the engine does not apply (the vector does not fit the LDS, or
@@ -309,10 +310,11 @@ size_t resident_partials(const ResidentShape &s, int niter);
 hipError_t launch_resident_fill(const Fp64Problem &pb, const ResidentShape &s,
                                 const ResidentState &rs, hipStream_t st);
 // niter outer iterations {conj_grad of `steps` steps; rnorm, zeta, xscale} from
-// pb.x (scale_first: from xscale z of the previous call), recorded as history
-// entries first, first + 1, ... with `record`; pb.x is not written.  With
-// `solve` (niter 1) pb.x is the right-hand side and the steps stop once
-// r.r <= rtol^2 r0.r0.  sc->aborted is set if a wait ran out.
+// pb.x (scale_first: from xscale z of the previous launch), recorded as history
+// entries first, first + 1, ... with `record`; pb.x is not written.  first = 0
+// begins a call.  With `solve` (niter 1) pb.x is the right-hand side and the
+// steps stop once r.r <= rtol^2 r0.r0.  sc->aborted is set if a wait ran out in
+// this launch or in one before it of the same call, and cleared else.
 hipError_t launch_resident(const Fp64Problem &pb, const ResidentShape &s, const ResidentState &rs,
                            int steps, int niter, int scale_first, int first, int record,
                            int solve, double rtol, hipStream_t st);

@@ -33,8 +33,10 @@
 // cooperative queue to one process at a time, and a second process on the GPU
 // would be refused.  Where another process's kernels keep workgroups from
 // starting, every wait is bounded: one longer than spin_limit wall-clock ticks
-// sets the abort word, after which no read waits, so the grid always drains;
-// the host sees the word and runs the multi-kernel engine from the untouched x.
+// sets the abort word, after which no read waits, so the grid always drains.
+// The word is cleared once a call: the later launches of a power loop whose
+// results start from that one's do nothing, and the host sees the word and
+// runs the multi-kernel engine from the untouched x.
 //
 // Words: the exchange buffers and the LDS vector are cut into chunks of C
 // words, C - 1 rows and the chunk's partial.  One wavefront owns a chunk and
@@ -65,7 +67,7 @@ struct ResArgs {
     const int *word_row;   // [words] row of a word; -1: a partial, or past the rows
     int n, words, stride;  // words in use; words of one exchange buffer
     u64 *xchg;
-    unsigned *abort_word;
+    unsigned *abort_word;  // set by a wait that ran out; [1] by one of an earlier launch
     long long spin_limit;
     double *x, *z, *p, *q, *r;
     double *part;          // [niter][2][chunks]: ||x - A z||^2 and x.z
@@ -151,6 +153,7 @@ __global__ __launch_bounds__(kResBlock) void cg_resident_kernel(ResArgs a) {
     static_assert(kResBlock % C == 0 && (CH == 1 || C == kWave), "a wavefront per chunk");
     static_assert(HELD % 2 == 0, "columns are held in pairs");
     constexpr int kAhead = 8;
+    if (a.abort_word[1]) return;  // written between launches only: the same for every thread
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     // threads 0 .. CH * C - 1 own the workgroup's words; the last word of a
@@ -375,11 +378,13 @@ __global__ __launch_bounds__(kResBlock) void cg_resident_kernel(ResArgs a) {
     }
 }
 
-// Before a launch: every word that will be stored empty, the others zero, the
-// abort word clear. 
+// Before a launch: every word that will be stored empty, the others zero; the
+// abort words clear before the first launch of a call, else what the launches
+// before left.  hole: a word of the first buffer left empty though nobody stores
+// it, so that the launch gives up (-1: none).
 __global__ __launch_bounds__(kBlock) void resident_arm_kernel(
     u64 *xchg, const int *__restrict__ word_row, int words, int chunk, int stride, int buffers,
-    unsigned *abort_word) {
+    int hole, int clear, unsigned *abort_word) {
     const int per = stride / 2;  // 16-byte pairs of a buffer
     ulonglong2 *x2 = reinterpret_cast<ulonglong2 *>(xchg);
     auto first = [&](int w) {  // a row, or the partial of a chunk
@@ -387,9 +392,13 @@ __global__ __launch_bounds__(kBlock) void resident_arm_kernel(
     };
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < per; i += gridDim.x * kBlock) {
         const ulonglong2 v = make_ulonglong2(first(2 * i), first(2 * i + 1));
-        for (int b = blockIdx.y; b < buffers; b += gridDim.y) x2[(size_t)b * per + i] = v;
+        for (int b = blockIdx.y; b < buffers; b += gridDim.y)
+            x2[(size_t)b * per + i] = b == 0 && i == hole >> 1 ? make_ulonglong2(kEmpty, kEmpty) : v;
     }
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) abort_word[0] = 0u;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+        if (clear) abort_word[0] = 0u;
+        abort_word[1] = abort_word[0];
+    }
 }
 
 // After a launch, one workgroup per outer iteration: rnorm = ||x - A z||,
@@ -402,6 +411,10 @@ __global__ __launch_bounds__(kBlock) void resident_finish_kernel(
     double *__restrict__ z, double *__restrict__ p, double *__restrict__ q,
     double *__restrict__ r, int n) {
     const int it = blockIdx.x;
+    if (abort_word[0]) {  // of this launch or an earlier one: nothing here is valid
+        if (it == 0 && threadIdx.x == 0) sc->aborted = 1;
+        return;
+    }
     const double *pt = part + (size_t)it * 2 * count;
     double s0, s1;
     reduce_partials2<kBlock>(pt, count, pt + count, count, s0, s1);
@@ -419,7 +432,7 @@ __global__ __launch_bounds__(kBlock) void resident_finish_kernel(
     sc->xscale = 1.0 / sqrt(zz[it]);
     sc->zeta = zeta;
     if (record) sc->iter = first + niter;
-    sc->aborted = (int)abort_word[0];
+    sc->aborted = 0;
     const double xn = x[n];
     q[n] = 0.0;
     z[n] = 0.0;
@@ -590,9 +603,14 @@ hipError_t launch_resident(const Fp64Problem &pb, const ResidentShape &s, const 
     a.solve = solve;
     a.rtol2 = rtol * rtol;
     const int buffers = niter * (steps + 1);
+    int hole = -1;
+    if (rs.give_up_at >= first && rs.give_up_at < first + niter) {  // (tests)
+        hole = s.words;
+        a.spin_limit = rs.spin_limit / 1000;
+    }
     resident_arm_kernel<<<dim3(std::min(8, s.stride / (2 * kBlock)), std::min(buffers, 256)),
                           kBlock, 0, st>>>(a.xchg, rs.word_row, s.words, s.chunk, s.stride,
-                                           buffers, rs.abort_word);
+                                           buffers, hole, first == 0 ? 1 : 0, rs.abort_word);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (pb.marks) pb.marks->note("resident_arm_kernel", kBlock, st);
