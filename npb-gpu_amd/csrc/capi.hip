@@ -152,6 +152,14 @@ struct npbcg_ctx {
     // batch; mixed inner steps of sweeps 1, 2
     int budget[2][4][2] = {};
 
+    // captured first stretches of FP64 solves by step count (run_solve_sequence)
+    struct SolveGraph {
+        hipGraph_t g = nullptr;
+        hipGraphExec_t ex = nullptr;
+        int kind = -1, batch = 0, seen = 0;
+        double rtol = 0.0;
+    } solve_graph[16];
+
     // residual/correction pairs (lazy)
     struct Pairs {
         int count = 0;
@@ -173,6 +181,10 @@ constexpr int kMaxSortWindow = 8192;
 constexpr size_t kResidentWords = (size_t)8 << 20;
 // FP64 solves up to this order update p inside the SpMV (refresh_solve_view).
 constexpr int kFuseSolveRows = 49152;
+// Below this order repeated solves on the CSR kernels replay a graph, from this sight on
+// (run_solve_sequence).
+constexpr int kGraphSolveRows = 16384;
+constexpr int kGraphSolveSights = 4;
 // Steps of a resident solve launch at most.
 constexpr int kResidentSolveSteps = 64;
 // Entries of a right-hand side copied and sent at a time.
@@ -246,6 +258,12 @@ void drop_graph(npbcg_ctx *c) {
         c->outer_graph[i] = nullptr;
         c->outer_graph_src[i] = nullptr;
     }
+}
+
+void drop_solve_graph(npbcg_ctx::SolveGraph &sg) {
+    if (sg.ex) (void)hipGraphExecDestroy(sg.ex);
+    if (sg.g) (void)hipGraphDestroy(sg.g);
+    sg = npbcg_ctx::SolveGraph{};
 }
 
 int check_rowstr(int n, const int *rowstr, long long *nnz_out) {
@@ -1050,6 +1068,7 @@ void npbcg_destroy(npbcg_ctx *c) {
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     drop_graph(c);
+    for (auto &sg : c->solve_graph) drop_solve_graph(sg);
     for (auto e : c->probe_start) (void)hipEventDestroy(e);
     for (auto e : c->probe_stop) (void)hipEventDestroy(e);
     if (c->ev_start) (void)hipEventDestroy(c->ev_start);
@@ -2210,6 +2229,51 @@ int npbcg_solve(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stat
 
 namespace {
 
+// Runs the first stretch of an FP64 solve: reset, init, `batch` steps, residual.
+//
+// Small orders on the CSR kernels are bound by their launches (three of 2 to 4 us a
+// step), so a sequence that comes again (same preconditioner in effect, rtol and step
+// count, whatever the right-hand side) replays a captured graph: Jacobi solve at
+// n = 1400 164 us launched and 125 replayed, 4001 166 and 132, 9001 174 and 159, 15001
+// 189 and 179 (a faster host: 128 and 124 at 1400).  From about there on the two are
+// equal (17003: 194 and 191, 150000: 645 and 653).  A capture costs about 150 us, what
+// four solves lose to their launches, so it is made when a sequence is seen for the
+// fourth time.  The buffers that the kernels read are the context's own and stay
+// where they are.
+int run_solve_sequence(npbcg_ctx *c, double rtol, int batch,
+                       const std::function<hipError_t()> &enqueue) {
+    auto &sg = c->solve_graph[batch % 16];
+    if (!c->opts.use_graph || c->pb.spmv_variant == npbcg_dev::kSpmvTiled ||
+        c->n >= kGraphSolveRows) {
+        NPBCG_HIP(enqueue());
+        return NPBCG_OK;
+    }
+    if (sg.kind != c->active_precond || sg.rtol != rtol || sg.batch != batch) {
+        drop_solve_graph(sg);
+        sg.kind = c->active_precond;
+        sg.rtol = rtol;
+        sg.batch = batch;
+    }
+    if (!sg.ex && ++sg.seen < kGraphSolveSights) {
+        NPBCG_HIP(enqueue());
+        return NPBCG_OK;
+    }
+    if (!sg.ex) {
+        NPBCG_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+        hipError_t e = enqueue();
+        hipError_t e2 = hipStreamEndCapture(c->stream, &sg.g);
+        if (e == hipSuccess) e = e2;
+        if (e == hipSuccess) e = hipGraphInstantiate(&sg.ex, sg.g, nullptr, nullptr, 0);
+        if (e != hipSuccess) {
+            drop_solve_graph(sg);
+            return set_error(NPBCG_ERR_DEVICE,
+                             std::string("solve graph capture failed: ") + hipGetErrorString(e));
+        }
+    }
+    NPBCG_HIP(hipGraphLaunch(sg.ex, c->stream));
+    return NPBCG_OK;
+}
+
 int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats *st) {
     if (!c || !(rtol > 0.0) || maxit < 1 ||
         (mode != NPBCG_SOLVE_FP64 && mode != NPBCG_SOLVE_MIXED))
@@ -2249,9 +2313,6 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
         const int res_steps = std::min(maxit, kResidentSolveSteps);
         const bool resident = c->active_precond == NPBCG_PRECOND_NONE &&
                               c->opts.solve_batch <= 0 && use_resident(c, res_steps);
-        // First batch: reset, init, `batch` steps, residual.  Launched as they
-        // are: a captured graph of them replays no faster (n = 150000: 653
-        // against 645 us, 17003: 191 against 194) and costs 150 us to make.
         auto first_batch = [&]() -> hipError_t {
             hipError_t e = npbcg_dev::launch_reset_scalars(pbs, 0.0, c->stream, rtol, 1);
             if (e == hipSuccess) e = npbcg_dev::launch_cg_init(pbs, 0, c->stream);
@@ -2270,7 +2331,8 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
             NPBCG_HIP(npbcg_dev::launch_resident(pbs, c->rshape, c->rstate, res_steps, 1, 0, 0, 0,
                                                  1, rtol, c->stream));
         } else {
-            NPBCG_HIP(first_batch());
+            int rc = run_solve_sequence(c, rtol, batch, first_batch);
+            if (rc != NPBCG_OK) return rc;
         }
         for (;;) {
             if (!first) {
