@@ -601,15 +601,18 @@ __global__ __launch_bounds__(kBlock) void batch_pupdate_kernel(BatchDev bd,
         p0 = load_vec<T, NR>(p + (size_t)first * NR);
         r0 = load_vec<T, NR>(r + (size_t)first * NR);
     }
-    if (system_done<NR>(bd.done, s)) return;
+    // the system's first tile may be setting the flags: one read of them for the workgroup
+    __shared__ int done[NR];
+    if (threadIdx.x < NR) done[threadIdx.x] = bd.done[s * NR + threadIdx.x];
     double rr[NR], rho[NR];
-    system_sums<NR>(rr_part, tile.t0, tile.t1, rho_part, tile.t0, tile.t1, rr, rho);
+    system_sums<NR>(rr_part, tile.t0, tile.t1, rho_part, tile.t0, tile.t1, rr, rho);  // (a barrier)
+    if (system_done<NR>(done, 0)) return;
     T beta[NR];
     bool run[NR];
 #pragma unroll
     for (int k = 0; k < NR; k++) {
         const BatchScalars &sc = bd.sc[s * NR + k];
-        const bool act = bd.done[s * NR + k] == 0;
+        const bool act = done[k] == 0;
         const bool stop = act && (fabs(rr[k]) <= sc.tol2 || sc.sweep_steps >= bd.maxit);
         run[k] = act && !stop;
         beta[k] = run[k] && rho[k] != 0.0 ? (T)(rr[k] / rho[k]) : T(0);
@@ -617,7 +620,7 @@ __global__ __launch_bounds__(kBlock) void batch_pupdate_kernel(BatchDev bd,
     if ((int)blockIdx.x == tile.t0)
 #pragma unroll
         for (int k = 0; k < NR; k++)
-            if (threadIdx.x == k && bd.done[s * NR + k] == 0 && !run[k]) bd.done[s * NR + k] = 1;
+            if (threadIdx.x == k && done[k] == 0 && !run[k]) bd.done[s * NR + k] = 1;
     auto update = [&](int row, VecT<T, NR> pv, const VecT<T, NR> &rv) {
 #pragma unroll
         for (int k = 0; k < NR; k++)

@@ -136,7 +136,8 @@ __global__ __launch_bounds__(kBlock) void spmv_csr_kernel(
 // rho_part old); the workgroups of row range 0 store their block of p_new.  z is
 // r, or minv r when minv is given.  The stop test of a solve, on r.z or, when
 // given, stop_part's r.r, is update_p_kernel's: workgroup 0 records it and all
-// workgroups, which reach the same decision, return.
+// workgroups, which reach the same decision, return.  One that starts late may find
+// the flag set already; a single thread's read of it holds for the workgroup.
 template <int BLOCK, int UNR, int MODE, bool PUPD>
 __global__ __launch_bounds__(BLOCK) void spmv_sell_kernel(
     const int *__restrict__ wg_slice, const int *__restrict__ slice_off,
@@ -229,9 +230,11 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell_kernel(
                 }
         }
         asm volatile("" ::: "memory");  // the loads stay ahead
-        if (skip) return;
+        __shared__ int skip_all;
+        if (threadIdx.x == 0) skip_all = skip;
         double rr, rho;
-        reduce_partials2<BLOCK>(rr_part, n_vec, rho_part, n_vec, rr, rho);
+        reduce_partials2<BLOCK>(rr_part, n_vec, rho_part, n_vec, rr, rho);  // (barriers)
+        if (skip_all) return;
         beta = rr / rho;
         const double level = stop_part ? reduce_partials<BLOCK>(stop_part, n_vec) : rr;
         const bool stop = sc->stop_enabled && fabs(level) <= sc->tol2;
@@ -482,7 +485,9 @@ __global__ __launch_bounds__(kBlock) void update_p_kernel(
     const double *__restrict__ r, const double *p_in, double *p_out, int n,
     const double *__restrict__ rr_part, const double *__restrict__ rho_part, int n_vec,
     Scalars *sc, const double *__restrict__ minv, const double *__restrict__ stop_part) {
-    if (sc->done) return;
+    // workgroup 0 may be setting the flag: one thread's read holds for the workgroup
+    __shared__ int done;
+    if (threadIdx.x == 0) done = sc->done;
     // first row loaded ahead of the reductions (as in update_zr_kernel)
     const int j0 = blockIdx.x * kBlock + threadIdx.x;
     double r0 = 0.0, p0 = 0.0, m0 = 0.0;
@@ -492,7 +497,8 @@ __global__ __launch_bounds__(kBlock) void update_p_kernel(
         if (minv) m0 = minv[j0];
     }
     double rho, rho0;
-    reduce_partials2<kBlock>(rr_part, n_vec, rho_part, n_vec, rho, rho0);
+    reduce_partials2<kBlock>(rr_part, n_vec, rho_part, n_vec, rho, rho0);  // (barriers)
+    if (done) return;
     const double beta = rho / rho0;
     const double level = stop_part ? reduce_partials<kBlock>(stop_part, n_vec) : rho;
     const bool stop = sc->stop_enabled && fabs(level) <= sc->tol2;

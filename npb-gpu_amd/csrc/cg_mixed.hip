@@ -56,11 +56,16 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell32_kernel(
     const double *__restrict__ rr_part, const double *__restrict__ rho_part, int n_vec,
     int rev, int stage_rows, const float *__restrict__ minv,
     const double *__restrict__ stop_part) {
-    if (sc->done) return;
     float b32 = 0.0f;
-    if constexpr (PUPD) {
+    if constexpr (!PUPD) {
+        if (sc->done) return;
+    } else {
+        // workgroup 0 may be setting the flag: one thread's read holds for the workgroup
+        __shared__ int done;
+        if (threadIdx.x == 0) done = sc->done;
         double rho, rho0;
-        reduce_partials2<BLOCK>(rr_part, n_vec, rho_part, n_vec, rho, rho0);
+        reduce_partials2<BLOCK>(rr_part, n_vec, rho_part, n_vec, rho, rho0);  // (barriers)
+        if (done) return;
         const double level = stop_part ? reduce_partials<BLOCK>(stop_part, n_vec) : rho;
         const bool stop = fabs(level) <= sc->tol2;
         if (blockIdx.x == 0 && threadIdx.x == 0) {
