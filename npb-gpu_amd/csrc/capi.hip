@@ -519,16 +519,34 @@ int ensure_resident(npbcg_ctx *c, int steps, int niter) {
     return NPBCG_OK;
 }
 
-// Held from a resident launch until its results are on the host: the
-// workgroups of two such launches could each take part of the CUs and wait for
-// the rest.
-std::mutex &resident_turn(int device) {
-    static std::mutex turn[64];
-    return turn[device & 63];
+// Resident launches of a device run one after another: the workgroups of two
+// could each take part of the CUs and wait for the rest.  The order is the
+// GPU's (a launch waits for the event behind the last one of another context),
+// so the lock is held while a call enqueues and not while it waits or hashes.
+struct ResidentDevice {
+    std::mutex mu;
+    npbcg_ctx *last = nullptr;  // its ev_stop lies behind the last launch
+};
+ResidentDevice &resident_device(int device) {
+    static ResidentDevice dev[64];
+    return dev[device & 63];
+}
+
+// enqueue() between the last resident launch and the next one; ev_stop is
+// recorded behind what it enqueued.
+template <class F>
+int in_resident_order(npbcg_ctx *c, const F &enqueue) {
+    ResidentDevice &d = resident_device(c->device);
+    std::lock_guard<std::mutex> lk(d.mu);
+    if (d.last && d.last != c) NPBCG_HIP(hipStreamWaitEvent(c->stream, d.last->ev_stop, 0));
+    const int rc = enqueue();
+    NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
+    d.last = c;
+    return rc;
 }
 
 // niter outer iterations on the resident engine, in launches whose exchange
-// buffers fit the workspace; the caller holds resident_turn.
+// buffers fit the workspace; inside in_resident_order.
 int run_resident(npbcg_ctx *c, const Fp64Problem &pb, int niter, int record, int *launches) {
     const size_t per = (size_t)(c->cgitmax + 1) * c->rshape.stride;
     const int chunk = std::min(niter, (int)std::max<size_t>(1, kResidentWords / per));
@@ -1067,6 +1085,11 @@ void npbcg_destroy(npbcg_ctx *c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
+    {
+        ResidentDevice &d = resident_device(c->device);
+        std::lock_guard<std::mutex> lk(d.mu);
+        if (d.last == c) d.last = nullptr;
+    }
     drop_graph(c);
     for (auto &sg : c->solve_graph) drop_solve_graph(sg);
     for (auto e : c->probe_start) (void)hipEventDestroy(e);
@@ -1120,21 +1143,24 @@ namespace {
 // the launches and the wait for them.
 int conj_grad_run(npbcg_ctx *c, double *rnorm, const std::function<void()> &meanwhile) {
     NPBCG_HIP(hipSetDevice(c->device));
-    NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
     bool resident = use_resident(c, c->cgitmax);
     int launches = 0;
-    std::unique_lock<std::mutex> turn;
     if (resident) {
-        turn = std::unique_lock<std::mutex>(resident_turn(c->device));
-        int rc = run_resident(c, c->pb, 1, 0, &launches);
-        if (rc != NPBCG_OK) return rc;
-    } else if (c->engine == NPBCG_ENGINE_PERSISTENT) {
-        int rc = run_persistent(c, 1, 0, 0, 0);
+        int rc = in_resident_order(c, [&]() -> int {
+            NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
+            return run_resident(c, c->pb, 1, 0, &launches);
+        });
         if (rc != NPBCG_OK) return rc;
     } else {
-        NPBCG_HIP(npbcg_dev::enqueue_conj_grad(c->pb, c->cgitmax, 0, 0, c->stream, nullptr));
+        NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
+        if (c->engine == NPBCG_ENGINE_PERSISTENT) {
+            int rc = run_persistent(c, 1, 0, 0, 0);
+            if (rc != NPBCG_OK) return rc;
+        } else {
+            NPBCG_HIP(npbcg_dev::enqueue_conj_grad(c->pb, c->cgitmax, 0, 0, c->stream, nullptr));
+        }
+        NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
     }
-    NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
     if (meanwhile) meanwhile();
     Scalars s;
     int rc = read_scalars(c, &s);
@@ -1142,7 +1168,6 @@ int conj_grad_run(npbcg_ctx *c, double *rnorm, const std::function<void()> &mean
     if (resident && s.aborted) {  // x is untouched: the multi-kernel engine takes over
         c->rshape.grid = 0;
         resident = false;
-        turn.unlock();
         NPBCG_HIP(npbcg_dev::enqueue_conj_grad(c->pb, c->cgitmax, 0, 0, c->stream, nullptr));
         NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
         rc = read_scalars(c, &s);
@@ -1300,15 +1325,14 @@ int npbcg_power(npbcg_ctx *c, int niter, double shift, double *zeta_out,
     c->device_calls++;
     if (niter > 0 && !sample && use_resident(c, c->cgitmax)) {
         int launches = 2;
-        std::unique_lock<std::mutex> turn(resident_turn(c->device));
-        NPBCG_HIP(npbcg_dev::launch_reset_scalars(c->pb, shift, c->stream));
-        NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
-        rc = run_resident(c, c->pb, niter, 1, &launches);
+        rc = in_resident_order(c, [&]() -> int {
+            NPBCG_HIP(npbcg_dev::launch_reset_scalars(c->pb, shift, c->stream));
+            NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
+            return run_resident(c, c->pb, niter, 1, &launches);
+        });
         if (rc != NPBCG_OK) return rc;
-        NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
         Scalars s;
         rc = read_scalars(c, &s);
-        turn.unlock();
         if (rc != NPBCG_OK) return rc;
         if (!s.aborted) {
             NPBCG_HIP(npbcg_dev::launch_scale_x(c->pb, 0.0, 1, c->stream));
@@ -1411,8 +1435,7 @@ int npbcg_profile_kernels(npbcg_ctx *c, int niter, double shift, double *zeta_ou
     bool resident = use_resident(c, c->cgitmax);
     if (resident) {
         int launches = 0;
-        std::unique_lock<std::mutex> turn(resident_turn(c->device));
-        rc = run_resident(c, pb, niter, 1, &launches);
+        rc = in_resident_order(c, [&]() { return run_resident(c, pb, niter, 1, &launches); });
         Scalars s;
         if (rc == NPBCG_OK) rc = read_scalars(c, &s);
         if (rc != NPBCG_OK) return rc;
@@ -2320,28 +2343,31 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
             if (e == hipSuccess) e = npbcg_dev::launch_resid(pbs, 0, c->stream);
             return e;
         };
-        NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
         bool first = true;
-        std::unique_lock<std::mutex> turn;
         if (resident) {
-            turn = std::unique_lock<std::mutex>(resident_turn(c->device));
-            int rc = ensure_resident(c, res_steps, 1);
+            int rc = in_resident_order(c, [&]() -> int {
+                NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
+                int rc2 = ensure_resident(c, res_steps, 1);
+                if (rc2 != NPBCG_OK) return rc2;
+                NPBCG_HIP(npbcg_dev::launch_reset_scalars(pbs, 0.0, c->stream, rtol, 1));
+                NPBCG_HIP(npbcg_dev::launch_resident(pbs, c->rshape, c->rstate, res_steps, 1, 0, 0,
+                                                     0, 1, rtol, c->stream));
+                return NPBCG_OK;
+            });
             if (rc != NPBCG_OK) return rc;
-            NPBCG_HIP(npbcg_dev::launch_reset_scalars(pbs, 0.0, c->stream, rtol, 1));
-            NPBCG_HIP(npbcg_dev::launch_resident(pbs, c->rshape, c->rstate, res_steps, 1, 0, 0, 0,
-                                                 1, rtol, c->stream));
         } else {
+            NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
             int rc = run_solve_sequence(c, rtol, batch, first_batch);
             if (rc != NPBCG_OK) return rc;
+            NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
         }
         for (;;) {
             if (!first) {
                 NPBCG_HIP(npbcg_dev::enqueue_solve_steps(pbs, batch, 0, c->stream));
                 NPBCG_HIP(npbcg_dev::launch_resid(pbs, 0, c->stream));
+                NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
             }
-            NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
             int rc = read_scalars_from(c, pbs.sc, &sc);
-            if (turn.owns_lock()) turn.unlock();
             if (rc != NPBCG_OK) return rc;
             if (first && resident && sc.aborted) {  // b is untouched: start over without it
                 c->rshape.grid = 0;

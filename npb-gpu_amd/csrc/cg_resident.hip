@@ -28,8 +28,8 @@
 // alone): 1.4 us at n = 1400, 2.3 at 7000, 3.5 at 14000; a flag per workgroup
 // followed by plain loads takes 3.1, 5.7 and 6.9 us.
 // The grid fits the GPU at one workgroup per CU, and the host lets one such
-// launch run at a time on a device (run_resident), so the workgroups wait for
-// each other only.  It is not a cooperative launch: the runtime gives its
+// launch run at a time on a device (in_resident_order), so the workgroups wait
+// for each other only.  It is not a cooperative launch: the runtime gives its
 // cooperative queue to one process at a time, and a second process on the GPU
 // would be refused.  Where another process's kernels keep workgroups from
 // starting, every wait is bounded: one longer than spin_limit wall-clock ticks
