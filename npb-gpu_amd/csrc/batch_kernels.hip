@@ -593,7 +593,8 @@ __global__ __launch_bounds__(kBlock) void batch_pupdate_kernel(BatchDev bd,
                                                                const T *__restrict__ r,
                                                                T *__restrict__ p,
                                                                const double *__restrict__ rr_part,
-                                                               const double *__restrict__ rho_part) {
+                                                               const double *__restrict__ rho_part,
+                                                               int tag) {
     const BatchTile tile = bd.tile[blockIdx.x];
     const int s = tile.sys, first = tile.row + threadIdx.x;
     VecT<T, NR> p0{}, r0{};  // the first row, ahead of the sums
@@ -601,26 +602,28 @@ __global__ __launch_bounds__(kBlock) void batch_pupdate_kernel(BatchDev bd,
         p0 = load_vec<T, NR>(p + (size_t)first * NR);
         r0 = load_vec<T, NR>(r + (size_t)first * NR);
     }
-    // the system's first tile may be setting the flags: one read of them for the workgroup
-    __shared__ int done[NR];
-    if (threadIdx.x < NR) done[threadIdx.x] = bd.done[s * NR + threadIdx.x];
+    bool act[NR], any = false;  // (the system's first tile may be setting the flags)
+#pragma unroll
+    for (int k = 0; k < NR; k++) {
+        act[k] = !stopped_before(bd.done[s * NR + k], tag);
+        any = any || act[k];
+    }
+    if (!any) return;
     double rr[NR], rho[NR];
-    system_sums<NR>(rr_part, tile.t0, tile.t1, rho_part, tile.t0, tile.t1, rr, rho);  // (a barrier)
-    if (system_done<NR>(done, 0)) return;
+    system_sums<NR>(rr_part, tile.t0, tile.t1, rho_part, tile.t0, tile.t1, rr, rho);
     T beta[NR];
     bool run[NR];
 #pragma unroll
     for (int k = 0; k < NR; k++) {
         const BatchScalars &sc = bd.sc[s * NR + k];
-        const bool act = done[k] == 0;
-        const bool stop = act && (fabs(rr[k]) <= sc.tol2 || sc.sweep_steps >= bd.maxit);
-        run[k] = act && !stop;
+        const bool stop = act[k] && (fabs(rr[k]) <= sc.tol2 || sc.sweep_steps >= bd.maxit);
+        run[k] = act[k] && !stop;
         beta[k] = run[k] && rho[k] != 0.0 ? (T)(rr[k] / rho[k]) : T(0);
     }
     if ((int)blockIdx.x == tile.t0)
 #pragma unroll
         for (int k = 0; k < NR; k++)
-            if (threadIdx.x == k && done[k] == 0 && !run[k]) bd.done[s * NR + k] = 1;
+            if (threadIdx.x == k && act[k] && !run[k]) bd.done[s * NR + k] = tag;
     auto update = [&](int row, VecT<T, NR> pv, const VecT<T, NR> &rv) {
 #pragma unroll
         for (int k = 0; k < NR; k++)
@@ -828,7 +831,8 @@ hipError_t batch_cg_step(const BatchDev &bd, const BatchVecs<T> &v, int step, in
                                                              rho, v.part_pq, rr, first);
         hipError_t e2 = hipGetLastError();
         if (e2 != hipSuccess) return e2;
-        batch_pupdate_kernel<T, NR><<<tiles, kBlock, 0, st>>>(bd, v.r, v.p, rr, rho);
+        // (1 is batch_decide_kernel's)
+        batch_pupdate_kernel<T, NR><<<tiles, kBlock, 0, st>>>(bd, v.r, v.p, rr, rho, step + 2);
         return hipGetLastError();
     });
     return e;

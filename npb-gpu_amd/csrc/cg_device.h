@@ -169,7 +169,8 @@ struct Scalars {
     double bb;       // solve: r0.r0 of the step that set tol2 (b.b for x0 = 0)
     int iter;        // outer iterations recorded so far in the history
     int stop_enabled;  // solve mode: CG steps stop once r.r <= tol2
-    int done;        // set when the stop test passed; later CG steps return at once
+    int done;        // not 0 once the stop test passed (stopped_before); later CG steps
+                     // return at once
     int steps;       // CG steps executed since the last reset
     int skip_resid;  // mixed solve: the residual pass of a sweep that is not needed
     int sweeps;      // mixed solve: refinement sweeps run
@@ -182,6 +183,14 @@ struct Scalars {
     double cg_rho[2];
     double cg_alpha[2];
 };
+
+// Whether a solve (a right-hand side of a batch) had stopped when a launch began that
+// makes the stop test itself and then records it as `tag`.  A workgroup that
+// starts late may find this launch's own tag or the 0 before it, one wavefront the
+// one and one the other; both say no, and the test's sums decide.
+__device__ __forceinline__ bool stopped_before(int done, int tag) {
+    return done != 0 && done != tag;
+}
 
 // Next sweep of a mixed solve whose relative residual is rel: its inner stop level
 // max(1e-6, rtol / (2 rel))^2, or nothing to do (stop).

@@ -135,9 +135,8 @@ __global__ __launch_bounds__(kBlock) void spmv_csr_kernel(
 // a separate update_p launch.  beta comes from the r.z partials (rr_part new,
 // rho_part old); the workgroups of row range 0 store their block of p_new.  z is
 // r, or minv r when minv is given.  The stop test of a solve, on r.z or, when
-// given, stop_part's r.r, is update_p_kernel's: workgroup 0 records it and all
-// workgroups, which reach the same decision, return.  One that starts late may find
-// the flag set already; a single thread's read of it holds for the workgroup.
+// given, stop_part's r.r, is update_p_kernel's: workgroup 0 records it (as tag, see
+// stopped_before) and all workgroups, which reach the same decision, return.
 template <int BLOCK, int UNR, int MODE, bool PUPD>
 __global__ __launch_bounds__(BLOCK) void spmv_sell_kernel(
     const int *__restrict__ wg_slice, const int *__restrict__ slice_off,
@@ -147,7 +146,7 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell_kernel(
     int nrange, const double *__restrict__ r, double *__restrict__ p_new,
     const double *__restrict__ rr_part, const double *__restrict__ rho_part, int n_vec,
     Scalars *sc, int rev, const double *__restrict__ minv,
-    const double *__restrict__ stop_part) {
+    const double *__restrict__ stop_part, int tag) {
     // a solve that already met its tolerance, a refinement sweep that is not needed:
     // tested once the first loads are on their way (a test before them held every
     // launch up by a round trip: CG step at n = 30011 15.46 us, now 15.11, at 75000
@@ -230,18 +229,16 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell_kernel(
                 }
         }
         asm volatile("" ::: "memory");  // the loads stay ahead
-        __shared__ int skip_all;
-        if (threadIdx.x == 0) skip_all = skip;
+        if (stopped_before(skip, tag)) return;
         double rr, rho;
-        reduce_partials2<BLOCK>(rr_part, n_vec, rho_part, n_vec, rr, rho);  // (barriers)
-        if (skip_all) return;
+        reduce_partials2<BLOCK>(rr_part, n_vec, rho_part, n_vec, rr, rho);
         beta = rr / rho;
         const double level = stop_part ? reduce_partials<BLOCK>(stop_part, n_vec) : rr;
         const bool stop = sc->stop_enabled && fabs(level) <= sc->tol2;
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             sc->rho = rr;
             sc->beta = beta;
-            if (stop) sc->done = 1;
+            if (stop) sc->done = tag;
         }
         if (stop) return;
         auto form = [&](int i, const double2 &p2, const double2 &z2) {
@@ -484,10 +481,8 @@ __global__ __launch_bounds__(kBlock) void update_zr_kernel(
 __global__ __launch_bounds__(kBlock) void update_p_kernel(
     const double *__restrict__ r, const double *p_in, double *p_out, int n,
     const double *__restrict__ rr_part, const double *__restrict__ rho_part, int n_vec,
-    Scalars *sc, const double *__restrict__ minv, const double *__restrict__ stop_part) {
-    // workgroup 0 may be setting the flag: one thread's read holds for the workgroup
-    __shared__ int done;
-    if (threadIdx.x == 0) done = sc->done;
+    Scalars *sc, const double *__restrict__ minv, const double *__restrict__ stop_part, int tag) {
+    if (stopped_before(sc->done, tag)) return;
     // first row loaded ahead of the reductions (as in update_zr_kernel)
     const int j0 = blockIdx.x * kBlock + threadIdx.x;
     double r0 = 0.0, p0 = 0.0, m0 = 0.0;
@@ -497,8 +492,7 @@ __global__ __launch_bounds__(kBlock) void update_p_kernel(
         if (minv) m0 = minv[j0];
     }
     double rho, rho0;
-    reduce_partials2<kBlock>(rr_part, n_vec, rho_part, n_vec, rho, rho0);  // (barriers)
-    if (done) return;
+    reduce_partials2<kBlock>(rr_part, n_vec, rho_part, n_vec, rho, rho0);
     const double beta = rho / rho0;
     const double level = stop_part ? reduce_partials<kBlock>(stop_part, n_vec) : rho;
     const bool stop = sc->stop_enabled && fabs(level) <= sc->tol2;
@@ -508,7 +502,7 @@ __global__ __launch_bounds__(kBlock) void update_p_kernel(
         // Solve mode: the recursive residual met the tolerance; the remaining
         // steps of the launched sequence return at entry.  p is left as is
         // (the solution z is final).
-        if (stop) sc->done = 1;
+        if (stop) sc->done = tag;
     }
     if (stop) return;
     if (j0 < n) p_out[j0] = minv ? m0 * r0 + beta * p0 : r0 + beta * p0;
@@ -909,7 +903,8 @@ hipError_t launch_sell_t(const Fp64Problem &pb, int step, hipStream_t st, hipEve
                               pb.n, d.W, d.nrange, (const double *)(pb.pop ? pb.pz : pb.r),
                               p_of_step(pb, step), rz_source(pb, step), rz_source(pb, step - 1),
                               pb.vec_blocks, pb.sc, rev, pb.minv,
-                              (const double *)(pb.pop ? pb.part.rr[(step - 1) & 1] : nullptr)),
+                              (const double *)(pb.pop ? pb.part.rr[(step - 1) & 1] : nullptr),
+                              step + 1),
                      "spmv_sell_kernel (p = r + beta p; q = A p)", BLOCK, st);
     }
     if (MODE == 0 && pb.cg_form && pb.dot_apart) {  // s = A r, block sums only
@@ -919,7 +914,7 @@ hipError_t launch_sell_t(const Fp64Problem &pb, int step, hipStream_t st, hipEve
                               d.val, d.col, (const double *)pb.r, d.rows_part, pb.part.pq, pb.n,
                               d.W, d.nrange, (const double *)nullptr, (double *)nullptr,
                               (const double *)nullptr, (const double *)nullptr, 0, pb.sc,
-                              step & 1, (const double *)nullptr, (const double *)nullptr),
+                              step & 1, (const double *)nullptr, (const double *)nullptr, 0),
                      "spmv_sell_kernel (s = A r, r.s apart)", BLOCK, st);
     }
     // one-reduction form: the CG SpMV is s = A r (its dot partials are r.s)
@@ -929,7 +924,7 @@ hipError_t launch_sell_t(const Fp64Problem &pb, int step, hipStream_t st, hipEve
                           st, e0, e1, d.wg_slice, d.slice_off, d.slice_row, d.val, d.col, v,
                           d.rows_part, pb.part.pq, pb.n, d.W, d.nrange, (const double *)nullptr,
                           (double *)nullptr, (const double *)nullptr, (const double *)nullptr,
-                          0, pb.sc, rev, (const double *)nullptr, (const double *)nullptr),
+                          0, pb.sc, rev, (const double *)nullptr, (const double *)nullptr, 0),
                  MODE == 1    ? "spmv_sell_kernel (r = A z)"
                  : pb.cg_form ? "spmv_sell_kernel (s = A r)"
                               : "spmv_sell_kernel (q = A p)",
@@ -1052,11 +1047,12 @@ hipError_t launch_update_p(const Fp64Problem &pb, int step, hipStream_t st) {
     if (pb.pop)  // beta from r.z; stop test on r.r
         update_p_kernel<<<pb.vec_blocks, kBlock, 0, st>>>(
             pb.pz, p_of_step(pb, step), pb.p, pb.n, pb.part.rz[step & 1],
-            pb.part.rz[(step + 1) & 1], pb.vec_blocks, pb.sc, nullptr, pb.part.rr[step & 1]);
+            pb.part.rz[(step + 1) & 1], pb.vec_blocks, pb.sc, nullptr, pb.part.rr[step & 1],
+            step + 1);
     else
         update_p_kernel<<<pb.vec_blocks, kBlock, 0, st>>>(
             pb.r, p_of_step(pb, step), pb.p, pb.n, pb.part.rr[step & 1], rho_source(pb, step),
-            pb.vec_blocks, pb.sc, pb.minv, nullptr);
+            pb.vec_blocks, pb.sc, pb.minv, nullptr, step + 1);
     return noted(pb, hipGetLastError(), "update_p_kernel", kBlock, st);
 }
 

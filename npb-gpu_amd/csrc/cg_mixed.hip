@@ -55,23 +55,18 @@ __global__ __launch_bounds__(BLOCK) void spmv_sell32_kernel(
     Scalars *sc, const float *__restrict__ r, float *__restrict__ p_new,
     const double *__restrict__ rr_part, const double *__restrict__ rho_part, int n_vec,
     int rev, int stage_rows, const float *__restrict__ minv,
-    const double *__restrict__ stop_part) {
+    const double *__restrict__ stop_part, int tag) {
     float b32 = 0.0f;
-    if constexpr (!PUPD) {
-        if (sc->done) return;
-    } else {
-        // workgroup 0 may be setting the flag: one thread's read holds for the workgroup
-        __shared__ int done;
-        if (threadIdx.x == 0) done = sc->done;
+    if (PUPD ? stopped_before(sc->done, tag) : sc->done != 0) return;
+    if constexpr (PUPD) {
         double rho, rho0;
-        reduce_partials2<BLOCK>(rr_part, n_vec, rho_part, n_vec, rho, rho0);  // (barriers)
-        if (done) return;
+        reduce_partials2<BLOCK>(rr_part, n_vec, rho_part, n_vec, rho, rho0);
         const double level = stop_part ? reduce_partials<BLOCK>(stop_part, n_vec) : rho;
         const bool stop = fabs(level) <= sc->tol2;
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             sc->rho = rho;
             sc->beta = rho / rho0;
-            if (stop) sc->done = 1;
+            if (stop) sc->done = tag;
         }
         if (stop) return;
         b32 = (float)(rho / rho0);
@@ -382,19 +377,19 @@ hipError_t prepare_mixed_kernels(int lds_bytes) {
 template <bool PUPD>
 static hipError_t launch_spmv32(const Fp64Problem &pb, const MixedProblem &mp, const float *v,
                                 float *p_new, const double *rr_part, const double *rho_part,
-                                const double *stop_part, int rev, hipStream_t st) {
+                                const double *stop_part, int rev, int tag, hipStream_t st) {
     const SellDev &sd = pb.sell;
     const float *z = mp.pop ? mp.pz : mp.r;
     if (sd.block == 512)
         spmv_sell32_kernel<512, kSellUnr32, PUPD><<<sd.grid, 512, mp.lds_bytes, st>>>(
             sd.wg_slice, sd.slice_off, sd.slice_row, mp.val, sd.col, v, mp.rows_part, mp.part_pq,
             pb.n, sd.W, sd.nrange, mp.sc, z, p_new, rr_part, rho_part, pb.vec_blocks, rev,
-            mp.stage_rows, mp.minv, stop_part);
+            mp.stage_rows, mp.minv, stop_part, tag);
     else
         spmv_sell32_kernel<1024, kSellUnr32, PUPD><<<sd.grid, 1024, mp.lds_bytes, st>>>(
             sd.wg_slice, sd.slice_off, sd.slice_row, mp.val, sd.col, v, mp.rows_part, mp.part_pq,
             pb.n, sd.W, sd.nrange, mp.sc, z, p_new, rr_part, rho_part, pb.vec_blocks, rev,
-            mp.stage_rows, mp.minv, stop_part);
+            mp.stage_rows, mp.minv, stop_part, tag);
     return hipGetLastError();
 }
 
@@ -411,13 +406,13 @@ hipError_t launch_spmv32_kernel(const Fp64Problem &pb, const MixedProblem &mp, i
                               (uint32_t)mp.lds_bytes, st, e0, e1, 0u, sd.wg_slice, sd.slice_off,
                               sd.slice_row, mp.val, sd.col, v, mp.rows_part, mp.part_pq, pb.n, sd.W,
                               sd.nrange, mp.sc, r_none, p_none, d_none, d_none, pb.vec_blocks, rev,
-                              mp.stage_rows, r_none, d_none);
+                              mp.stage_rows, r_none, d_none, 0);
     else
         hipExtLaunchKernelGGL(spmv_sell32_kernel<1024, kSellUnr32, false>, dim3(sd.grid),
                               dim3(1024), (uint32_t)mp.lds_bytes, st, e0, e1, 0u, sd.wg_slice,
                               sd.slice_off, sd.slice_row, mp.val, sd.col, v, mp.rows_part,
                               mp.part_pq, pb.n, sd.W, sd.nrange, mp.sc, r_none, p_none, d_none,
-                              d_none, pb.vec_blocks, rev, mp.stage_rows, r_none, d_none);
+                              d_none, pb.vec_blocks, rev, mp.stage_rows, r_none, d_none, 0);
     return hipGetLastError();
 }
 
@@ -451,8 +446,10 @@ hipError_t enqueue_inner32(const Fp64Problem &pb, const MixedProblem &mp, int st
     for (int it = 0; it < steps && e == hipSuccess; it++) {
         float *p_it = pbuf[it & 1];
         e = it > 0 ? launch_spmv32<true>(pb, mp, pbuf[(it - 1) & 1], p_it, rz(it - 1), rz(it - 2),
-                                         mp.pop ? mp.part_rr[(it - 1) & 1] : nullptr, it & 1, st)
-                   : launch_spmv32<false>(pb, mp, p_it, nullptr, nullptr, nullptr, nullptr, 0, st);
+                                         mp.pop ? mp.part_rr[(it - 1) & 1] : nullptr, it & 1,
+                                         it + 1, st)
+                   : launch_spmv32<false>(pb, mp, p_it, nullptr, nullptr, nullptr, nullptr, 0, 0,
+                                          st);
         if (e != hipSuccess) break;
         // sparse preconditioner: alpha from r.z, the stop level from r0.r0
         update_zr32_kernel<<<vb, kBlock, 0, st>>>(p_it, mp.q, mp.d, mp.r, pb.n, rz(it - 1),
