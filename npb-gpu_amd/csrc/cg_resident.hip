@@ -153,7 +153,8 @@ __global__ __launch_bounds__(kResBlock) void cg_resident_kernel(ResArgs a) {
     static_assert(kResBlock % C == 0 && (CH == 1 || C == kWave), "a wavefront per chunk");
     static_assert(HELD % 2 == 0, "columns are held in pairs");
     constexpr int kAhead = 8;
-    if (a.abort_word[1]) return;  // written between launches only: the same for every thread
+    const unsigned gave_up = a.abort_word[1];  // written between launches only: the same for
+                                               // every thread
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     // threads 0 .. CH * C - 1 own the workgroup's words; the last word of a
@@ -234,6 +235,8 @@ __global__ __launch_bounds__(kResBlock) void cg_resident_kernel(ResArgs a) {
         rr += v * v;
     }
     if (own) xo = xscale * src[row];
+    asm volatile("" ::: "memory");  // the loads are on their way
+    if (gave_up) return;
     int k = 0;
     double rho = 0.0, rho0 = 0.0;
     for (int it = 0; it < a.niter; it++) {
