@@ -43,7 +43,14 @@ enum {
                                      vectors and matrix on chip (plain FP64 solves with
                                      solve_batch 0 too).  Else KERNELS (8.5 ms against
                                      14.6 ms of PERSISTENT for 10 outer iterations at
-                                     n = 75000) */
+                                     n = 75000).  A resident launch needs all its
+                                     workgroups on the GPU at once.  The launches of one
+                                     process take turns; where another process's
+                                     launches of this kind, or kernels that do not let
+                                     go of their CUs, keep some from starting, the
+                                     launch gives up after 0.1 s, its call runs on the
+                                     KERNELS engine, and so do the process's calls on
+                                     that device in the next 10 s */
     NPBCG_ENGINE_KERNELS = 1,     /* fused per-phase kernels (two a CG step), replayed
                                      from a captured HIP graph per outer iteration */
     NPBCG_ENGINE_PERSISTENT = 2   /* one cooperative kernel runs whole outer iterations

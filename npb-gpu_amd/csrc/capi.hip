@@ -2,6 +2,8 @@
 // device-resident inverse-power loop.  Declarations and reference citations
 // are in include/npbcg.h.
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -475,11 +477,44 @@ int run_persistent(npbcg_ctx *c, int niter, int scale_first, int record, int fin
     return NPBCG_OK;
 }
 
-// Whether calls of this context run on the resident engine; one outer
+// Resident launches of a device run one after another: the workgroups of two
+// could each take part of the CUs and wait for the rest.  The order is the
+// GPU's (a launch waits for the event behind the last one of another context),
+// so the lock is held while a call enqueues and not while it waits or hashes.
+//
+// Another process's launches are not in that order, nor are other kernels that
+// hold CUs for long: a launch that waited kResidentWaitMs in vain gave up, and
+// its call ran again on the kernels.  The device then rests for kResidentRestMs,
+// in which no context of the process tries again, so such waits are at most
+// 1 % of the time.
+struct ResidentDevice {
+    std::mutex mu;
+    npbcg_ctx *last = nullptr;  // its ev_stop lies behind the last launch
+    std::atomic<long long> rest_until{0};  // steady_clock, ms
+};
+constexpr long long kResidentWaitMs = 100, kResidentRestMs = 10000;
+ResidentDevice &resident_device(int device) {
+    static ResidentDevice dev[64];
+    return dev[device & 63];
+}
+
+long long now_ms() {
+    return std::chrono::duration_cast<std::chrono::milliseconds>(
+               std::chrono::steady_clock::now().time_since_epoch())
+        .count();
+}
+
+void rest_resident(const npbcg_ctx *c) {
+    resident_device(c->device).rest_until = now_ms() + kResidentRestMs;
+}
+
+// Whether a call of this context runs on the resident engine now; one outer
 // iteration of `steps` CG steps has to fit the exchange workspace.
 bool use_resident(const npbcg_ctx *c, int steps) {
-    return c->rshape.grid > 0 &&
-           (size_t)(steps + 1) * (size_t)c->rshape.stride <= kResidentWords;
+    if (c->rshape.grid < 1 || (size_t)(steps + 1) * (size_t)c->rshape.stride > kResidentWords)
+        return false;
+    const long long rest = resident_device(c->device).rest_until;
+    return rest == 0 || now_ms() >= rest;
 }
 
 // Buffers of a resident launch of niter outer iterations of `steps` steps.
@@ -517,19 +552,6 @@ int ensure_resident(npbcg_ctx *c, int steps, int niter) {
         rs.part_words = part;
     }
     return NPBCG_OK;
-}
-
-// Resident launches of a device run one after another: the workgroups of two
-// could each take part of the CUs and wait for the rest.  The order is the
-// GPU's (a launch waits for the event behind the last one of another context),
-// so the lock is held while a call enqueues and not while it waits or hashes.
-struct ResidentDevice {
-    std::mutex mu;
-    npbcg_ctx *last = nullptr;  // its ev_stop lies behind the last launch
-};
-ResidentDevice &resident_device(int device) {
-    static ResidentDevice dev[64];
-    return dev[device & 63];
 }
 
 // enqueue() between the last resident launch and the next one; ev_stop is
@@ -1059,8 +1081,9 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
             CREATE_HIP(npbcg_dev::resident_capacity(c->rshape, &per_cu));
             CREATE_HIP(hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate,
                                              c->device));
-            // a read that waits 1 s has lost a workgroup: the launch gives up
-            c->rstate.spin_limit = (long long)std::max(clock_khz, 1000) * 1000;
+            // an exchange takes microseconds: one this long waits for a workgroup
+            // that has no CU, and the launch gives up
+            c->rstate.spin_limit = (long long)std::max(clock_khz, 1000) * kResidentWaitMs;
         }
         if (per_cu < 1) c->rshape = npbcg_dev::ResidentShape{};
     }
@@ -1166,7 +1189,7 @@ int conj_grad_run(npbcg_ctx *c, double *rnorm, const std::function<void()> &mean
     int rc = read_scalars(c, &s);
     if (rc != NPBCG_OK) return rc;
     if (resident && s.aborted) {  // x is untouched: the multi-kernel engine takes over
-        c->rshape.grid = 0;
+        rest_resident(c);
         resident = false;
         NPBCG_HIP(npbcg_dev::enqueue_conj_grad(c->pb, c->cgitmax, 0, 0, c->stream, nullptr));
         NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
@@ -1206,6 +1229,7 @@ int npbcg_test_resident_give_up(npbcg_ctx *c, int iteration) {
         return set_error(NPBCG_ERR_INVALID,
                          "npbcg_test_resident_give_up: no resident engine with a spare word");
     c->rstate.give_up_at = iteration;
+    resident_device(c->device).rest_until = 0;
     clear_error();
     return NPBCG_OK;
 }
@@ -1355,7 +1379,7 @@ int npbcg_power(npbcg_ctx *c, int niter, double shift, double *zeta_out,
             clear_error();
             return NPBCG_OK;
         }
-        c->rshape.grid = 0;  // x is untouched: the multi-kernel engine takes over
+        rest_resident(c);  // x is untouched: the multi-kernel engine takes over
     }
     const bool use_graph = c->opts.use_graph != 0;
     if (use_graph) {
@@ -1440,7 +1464,7 @@ int npbcg_profile_kernels(npbcg_ctx *c, int niter, double shift, double *zeta_ou
         if (rc == NPBCG_OK) rc = read_scalars(c, &s);
         if (rc != NPBCG_OK) return rc;
         if (s.aborted) {
-            c->rshape.grid = 0;
+            rest_resident(c);
             return npbcg_profile_kernels(c, niter, shift, zeta_out, out, max_kinds, nkinds,
                                          total_ms);
         }
@@ -2370,7 +2394,7 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
             int rc = read_scalars_from(c, pbs.sc, &sc);
             if (rc != NPBCG_OK) return rc;
             if (first && resident && sc.aborted) {  // b is untouched: start over without it
-                c->rshape.grid = 0;
+                rest_resident(c);
                 NPBCG_HIP(first_batch());
                 NPBCG_HIP(hipEventRecord(c->ev_stop, c->stream));
                 rc = read_scalars_from(c, pbs.sc, &sc);

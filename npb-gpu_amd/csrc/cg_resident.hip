@@ -609,7 +609,7 @@ hipError_t launch_resident(const Fp64Problem &pb, const ResidentShape &s, const 
     int hole = -1;
     if (rs.give_up_at >= first && rs.give_up_at < first + niter) {  // (tests)
         hole = s.words;
-        a.spin_limit = rs.spin_limit / 1000;
+        a.spin_limit = rs.spin_limit / 100;
     }
     resident_arm_kernel<<<dim3(std::min(8, s.stride / (2 * kBlock)), std::min(buffers, 256)),
                           kBlock, 0, st>>>(a.xchg, rs.word_row, s.words, s.chunk, s.stride,

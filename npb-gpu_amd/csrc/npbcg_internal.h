@@ -20,10 +20,11 @@ struct npbcg_ctx;
 
 // For tests of the resident engine's fallback: in the calls that follow, the
 // launch that holds outer iteration `iteration` (0: conj_grad, a solve) waits
-// for a word that nobody stores until its bounded wait runs out, a thousandth
+// for a word that nobody stores until its bounded wait runs out, a hundredth
 // of the limit other launches have, and then ends as any launch does.  -1:
-// none.  NPBCG_ERR_INVALID where the context does not run on that engine, or
-// its order leaves no word of the exchange buffers unused.
+// none.  Also ends the device's rest after a launch that gave up.
+// NPBCG_ERR_INVALID where the context does not run on that engine, or its order
+// leaves no word of the exchange buffers unused.
 extern "C" int npbcg_test_resident_give_up(npbcg_ctx *c, int iteration);
 
 #endif

@@ -1,6 +1,6 @@
 """A launch of the resident engine that gives up waiting: whichever launch of a call it is,
 the call's results are bit for bit those of the kernels engine, from the x it was given, and
-the context goes on with that engine."""
+for a while no context of the process tries that engine again."""
 import numpy as np
 import pytest
 
@@ -11,6 +11,13 @@ RESIDENT, KERNELS = 2, 1   # npbcg_timing.engine
 
 def _give_up(gpu, ctx, iteration):
     assert gpu.LIB.npbcg_test_resident_give_up(ctx._h, iteration) == 0, gpu.last_error()
+
+
+@pytest.fixture(autouse=True)
+def _rested(gpu):
+    yield
+    with gpu.Context(gpu.makea(1400, 7, 10.0, 271.0)) as ctx:
+        _give_up(gpu, ctx, -1)   # the tests that follow use the engine again
 
 
 @pytest.mark.parametrize("iteration", [0, 17, 33])   # launches of 16, 16 and 2 iterations
@@ -68,3 +75,23 @@ def test_conj_grad_and_solve(gpu):
         got_solve = solve(ctx)
     for u, v in zip(got + got_solve, want + want_solve):
         assert np.array_equal(u, v)
+
+
+def test_other_contexts_do_not_wait_too(gpu):
+    m = gpu.makea(1400, 7, 10.0, 271.0)
+    x = np.random.default_rng(3).uniform(-1, 1, m.n + 1)
+    with gpu.Context(m) as first, gpu.Context(m) as second:
+        want = second.conj_grad(x)
+        assert second.timing().engine == RESIDENT
+        _give_up(gpu, first, 0)
+        first.conj_grad(x)
+        with gpu.Context(m) as third:
+            for ctx in (first, second, third):
+                ctx.conj_grad(x)
+                assert ctx.timing().engine == KERNELS
+            _give_up(gpu, first, -1)   # the rest is over
+            for ctx in (first, second, third):
+                got = ctx.conj_grad(x)
+                assert ctx.timing().engine == RESIDENT
+                for u, v in zip(got, want):
+                    assert np.array_equal(u, v)
