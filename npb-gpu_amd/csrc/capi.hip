@@ -537,21 +537,21 @@ int ensure_resident(npbcg_ctx *c, int steps, int niter) {
         NPBCG_HIP(hipStreamSynchronize(c->stream));  // maps goes out of scope
         NPBCG_HIP(npbcg_dev::launch_resident_fill(c->pb, sh, rs, c->stream));
     }
-    const size_t words = (size_t)niter * (steps + 1) * sh.stride;
-    const size_t part = npbcg_dev::resident_partials(sh, niter);
-    if (words > rs.xchg_words || part > rs.part_words) {
+    // each buffer grows by itself: a solve has more exchanges than an outer
+    // iteration and one set of partials, a power loop the other way round
+    auto grow = [&](double *&buf, size_t &have, size_t need) -> int {
+        if (need <= have) return NPBCG_OK;
         NPBCG_HIP(hipStreamSynchronize(c->stream));
-        (void)hipFree(rs.xchg);
-        (void)hipFree(rs.part);
-        rs.xchg = nullptr;
-        rs.part = nullptr;
-        rs.xchg_words = rs.part_words = 0;
-        NPBCG_HIP(hipMalloc(&rs.xchg, sizeof(double) * words));
-        NPBCG_HIP(hipMalloc(&rs.part, sizeof(double) * part));
-        rs.xchg_words = words;
-        rs.part_words = part;
-    }
-    return NPBCG_OK;
+        (void)hipFree(buf);
+        buf = nullptr;
+        have = 0;
+        NPBCG_HIP(hipMalloc(&buf, sizeof(double) * need));
+        have = need;
+        return NPBCG_OK;
+    };
+    int rc = grow(rs.xchg, rs.xchg_words, (size_t)niter * (steps + 1) * sh.stride);
+    if (rc == NPBCG_OK) rc = grow(rs.part, rs.part_words, npbcg_dev::resident_partials(sh, niter));
+    return rc;
 }
 
 // enqueue() between the last resident launch and the next one; ev_stop is
