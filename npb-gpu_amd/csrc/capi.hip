@@ -88,6 +88,7 @@ struct npbcg_ctx {
     // buffers, allocated by the first call that runs on it
     npbcg_dev::ResidentShape rshape;
     npbcg_dev::ResidentState rstate;
+    bool no_memory = false;  // tests: buffers that a call can do without are refused
 
     // Captured outer iterations: [0] first (x used as is), [1] later ones
     // (x = z/||z|| of the previous iteration applied first).
@@ -517,50 +518,81 @@ void rest_resident(const npbcg_ctx *c) {
     resident_device(c->device).rest_until = now_ms() + kResidentRestMs;
 }
 
-// Whether a call of this context runs on the resident engine now; one outer
-// iteration of `steps` CG steps has to fit the exchange workspace.
-bool use_resident(const npbcg_ctx *c, int steps) {
-    if (c->rshape.grid < 1 || (size_t)(steps + 1) * (size_t)c->rshape.stride > kResidentWords)
-        return false;
-    const long long rest = resident_device(c->device).rest_until;
-    return rest == 0 || now_ms() >= rest;
+// A device buffer that a call can do without: false when there is no memory.
+template <class T>
+bool try_malloc(const npbcg_ctx *c, T **p, size_t bytes) {
+    if (!c->no_memory && hipMalloc(p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();  // (a later launch would report it)
+    *p = nullptr;
+    return false;
+}
+
+// The matrix and row maps of the resident engine.
+bool ensure_resident_matrix(npbcg_ctx *c) {
+    auto &rs = c->rstate;
+    const auto &sh = c->rshape;
+    if (rs.val) return true;
+    const size_t entries = (size_t)std::max(1, sh.wave_off.back()) * npbcg_dev::kWave;
+    std::vector<int> maps(sh.wave_off);
+    maps.insert(maps.end(), sh.word_row.begin(), sh.word_row.end());
+    maps.insert(maps.end(), sh.row_word.begin(), sh.row_word.end());
+    if (try_malloc(c, &rs.wave_off, sizeof(int) * maps.size()) &&
+        try_malloc(c, &rs.abort_word, 2 * sizeof(unsigned)) &&
+        try_malloc(c, &rs.col, sizeof(uint16_t) * entries) &&
+        try_malloc(c, &rs.val, sizeof(double) * entries)) {
+        rs.word_row = rs.wave_off + sh.wave_off.size();
+        rs.row_word = rs.word_row + sh.word_row.size();
+        hipError_t e = hipMemcpyAsync(rs.wave_off, maps.data(), sizeof(int) * maps.size(),
+                                      hipMemcpyHostToDevice, c->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);  // maps goes out of scope
+        if (e == hipSuccess) e = npbcg_dev::launch_resident_fill(c->pb, sh, rs, c->stream);
+        if (e == hipSuccess) return true;
+    }
+    for (void *p : {(void *)rs.wave_off, (void *)rs.abort_word, (void *)rs.col, (void *)rs.val})
+        (void)hipFree(p);
+    rs.wave_off = rs.word_row = rs.row_word = nullptr;
+    rs.abort_word = nullptr;
+    rs.col = nullptr;
+    rs.val = nullptr;
+    return false;
 }
 
 // Buffers of a resident launch of niter outer iterations of `steps` steps.
-int ensure_resident(npbcg_ctx *c, int steps, int niter) {
+bool ensure_resident(npbcg_ctx *c, int steps, int niter) {
     auto &rs = c->rstate;
-    const auto &sh = c->rshape;
-    if (!rs.val) {
-        const size_t entries = (size_t)std::max(1, sh.wave_off.back()) * npbcg_dev::kWave;
-        std::vector<int> maps(sh.wave_off);
-        maps.insert(maps.end(), sh.word_row.begin(), sh.word_row.end());
-        maps.insert(maps.end(), sh.row_word.begin(), sh.row_word.end());
-        NPBCG_HIP(hipMalloc(&rs.wave_off, sizeof(int) * maps.size()));
-        rs.word_row = rs.wave_off + sh.wave_off.size();
-        rs.row_word = rs.word_row + sh.word_row.size();
-        NPBCG_HIP(hipMalloc(&rs.abort_word, 2 * sizeof(unsigned)));
-        NPBCG_HIP(hipMalloc(&rs.col, sizeof(uint16_t) * entries));
-        NPBCG_HIP(hipMalloc(&rs.val, sizeof(double) * entries));
-        NPBCG_HIP(hipMemcpyAsync(rs.wave_off, maps.data(), sizeof(int) * maps.size(),
-                                 hipMemcpyHostToDevice, c->stream));
-        NPBCG_HIP(hipStreamSynchronize(c->stream));  // maps goes out of scope
-        NPBCG_HIP(npbcg_dev::launch_resident_fill(c->pb, sh, rs, c->stream));
-    }
     // each buffer grows by itself: a solve has more exchanges than an outer
     // iteration and one set of partials, a power loop the other way round
-    auto grow = [&](double *&buf, size_t &have, size_t need) -> int {
-        if (need <= have) return NPBCG_OK;
-        NPBCG_HIP(hipStreamSynchronize(c->stream));
+    auto grow = [&](double *&buf, size_t &have, size_t need) {
+        if (need <= have) return true;
+        if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
         (void)hipFree(buf);
-        buf = nullptr;
         have = 0;
-        NPBCG_HIP(hipMalloc(&buf, sizeof(double) * need));
+        if (!try_malloc(c, &buf, sizeof(double) * need)) return false;
         have = need;
-        return NPBCG_OK;
+        return true;
     };
-    int rc = grow(rs.xchg, rs.xchg_words, (size_t)niter * (steps + 1) * sh.stride);
-    if (rc == NPBCG_OK) rc = grow(rs.part, rs.part_words, npbcg_dev::resident_partials(sh, niter));
-    return rc;
+    return ensure_resident_matrix(c) &&
+           grow(rs.xchg, rs.xchg_words, (size_t)niter * (steps + 1) * c->rshape.stride) &&
+           grow(rs.part, rs.part_words, npbcg_dev::resident_partials(c->rshape, niter));
+}
+
+// Outer iterations of `steps` steps that one resident launch runs of niter: its
+// exchange buffers fit the workspace.
+int resident_chunk(const npbcg_ctx *c, int steps, int niter) {
+    const size_t per = (size_t)(steps + 1) * c->rshape.stride;
+    return std::min(niter, (int)(kResidentWords / per));
+}
+
+// Whether a call of niter outer iterations of `steps` CG steps runs on the
+// resident engine now: an iteration fits the exchange workspace, the device does
+// not rest and there is memory for the buffers (up to 64 MB more than the
+// kernels engine has, which runs the call otherwise).
+bool use_resident(npbcg_ctx *c, int steps, int niter) {
+    if (c->rshape.grid < 1 || (size_t)(steps + 1) * (size_t)c->rshape.stride > kResidentWords)
+        return false;
+    const long long rest = resident_device(c->device).rest_until;
+    if (rest != 0 && now_ms() < rest) return false;
+    return ensure_resident(c, steps, resident_chunk(c, steps, niter));
 }
 
 // enqueue() between the last resident launch and the next one; ev_stop is
@@ -576,13 +608,10 @@ int in_resident_order(npbcg_ctx *c, const F &enqueue) {
     return rc;
 }
 
-// niter outer iterations on the resident engine, in launches whose exchange
-// buffers fit the workspace; inside in_resident_order.
+// niter outer iterations on the resident engine (use_resident said yes), inside
+// in_resident_order.
 int run_resident(npbcg_ctx *c, const Fp64Problem &pb, int niter, int record, int *launches) {
-    const size_t per = (size_t)(c->cgitmax + 1) * c->rshape.stride;
-    const int chunk = std::min(niter, (int)std::max<size_t>(1, kResidentWords / per));
-    int rc = ensure_resident(c, c->cgitmax, chunk);
-    if (rc != NPBCG_OK) return rc;
+    const int chunk = resident_chunk(c, c->cgitmax, niter);
     for (int done = 0; done < niter; done += chunk) {
         NPBCG_HIP(npbcg_dev::launch_resident(pb, c->rshape, c->rstate, c->cgitmax,
                                              std::min(chunk, niter - done), done > 0, done,
@@ -1183,7 +1212,7 @@ namespace {
 // the launches and the wait for them.
 int conj_grad_run(npbcg_ctx *c, double *rnorm, const std::function<void()> &meanwhile) {
     NPBCG_HIP(hipSetDevice(c->device));
-    bool resident = use_resident(c, c->cgitmax);
+    bool resident = use_resident(c, c->cgitmax, 1);
     int launches = 0;
     if (resident) {
         int rc = in_resident_order(c, [&]() -> int {
@@ -1247,6 +1276,13 @@ int npbcg_test_resident_give_up(npbcg_ctx *c, int iteration) {
                          "npbcg_test_resident_give_up: no resident engine with a spare word");
     c->rstate.give_up_at = iteration;
     resident_device(c->device).rest_until = 0;
+    clear_error();
+    return NPBCG_OK;
+}
+
+int npbcg_test_no_memory(npbcg_ctx *c, int on) {
+    if (!c) return set_error(NPBCG_ERR_INVALID, "npbcg_test_no_memory: NULL context");
+    c->no_memory = on != 0;
     clear_error();
     return NPBCG_OK;
 }
@@ -1365,7 +1401,7 @@ int npbcg_power(npbcg_ctx *c, int niter, double shift, double *zeta_out,
     }
     const bool sample = c->sample_every > 0 && (c->device_calls % c->sample_every) == 0;
     c->device_calls++;
-    if (niter > 0 && !sample && use_resident(c, c->cgitmax)) {
+    if (niter > 0 && !sample && use_resident(c, c->cgitmax, niter)) {
         int launches = 2;
         rc = in_resident_order(c, [&]() -> int {
             NPBCG_HIP(npbcg_dev::launch_reset_scalars(c->pb, shift, c->stream));
@@ -1474,7 +1510,7 @@ int npbcg_profile_kernels(npbcg_ctx *c, int niter, double shift, double *zeta_ou
     pb.marks = &marks;
     marks.stamp(c->stream);
     hipError_t e = marks.err;
-    bool resident = use_resident(c, c->cgitmax);
+    bool resident = use_resident(c, c->cgitmax, niter);
     if (resident) {
         int launches = 0;
         rc = in_resident_order(c, [&]() { return run_resident(c, pb, niter, 1, &launches); });
@@ -2377,7 +2413,7 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
         // test passes; a solve it leaves unfinished goes on below
         const int res_steps = std::min(maxit, kResidentSolveSteps);
         const bool resident = c->active_precond == NPBCG_PRECOND_NONE &&
-                              c->opts.solve_batch <= 0 && use_resident(c, res_steps);
+                              c->opts.solve_batch <= 0 && use_resident(c, res_steps, 1);
         auto first_batch = [&]() -> hipError_t {
             hipError_t e = npbcg_dev::launch_reset_scalars(pbs, 0.0, c->stream, rtol, 1);
             if (e == hipSuccess) e = npbcg_dev::launch_cg_init(pbs, 0, c->stream);
@@ -2389,8 +2425,6 @@ int solve_once(npbcg_ctx *c, int mode, double rtol, int maxit, npbcg_solve_stats
         if (resident) {
             int rc = in_resident_order(c, [&]() -> int {
                 NPBCG_HIP(hipEventRecord(c->ev_start, c->stream));
-                int rc2 = ensure_resident(c, res_steps, 1);
-                if (rc2 != NPBCG_OK) return rc2;
                 NPBCG_HIP(npbcg_dev::launch_reset_scalars(pbs, 0.0, c->stream, rtol, 1));
                 NPBCG_HIP(npbcg_dev::launch_resident(pbs, c->rshape, c->rstate, res_steps, 1, 0, 0,
                                                      0, 1, rtol, c->stream));

@@ -27,4 +27,8 @@ struct npbcg_ctx;
 // leaves no word of the exchange buffers unused.
 extern "C" int npbcg_test_resident_give_up(npbcg_ctx *c, int iteration);
 
+// For tests: while on, device buffers that a call of this context would add to
+// run faster cannot be had, as on a full device.
+extern "C" int npbcg_test_no_memory(npbcg_ctx *c, int on);
+
 #endif
