@@ -1257,10 +1257,15 @@ int conj_grad_run(npbcg_ctx *c, double *rnorm, const std::function<void()> &mean
     return NPBCG_OK;
 }
 
+// Room for save_state.
+bool ensure_saved(npbcg_ctx *c) {
+    return c->d_saved ||
+           try_malloc(c, &c->d_saved, sizeof(double) * 5 * c->vstride + sizeof(Scalars));
+}
+
 // Keeps (or with `back` puts back) x, z, p, q, r and the scalars of the context.
 int save_state(npbcg_ctx *c, bool back) {
     const size_t vectors = sizeof(double) * 5 * c->vstride;
-    if (!c->d_saved) NPBCG_HIP(hipMalloc(&c->d_saved, vectors + sizeof(Scalars)));
     Scalars *scalars = reinterpret_cast<Scalars *>(c->d_saved + 5 * c->vstride);
     NPBCG_HIP(npbcg_dev::launch_save(back ? c->d_saved : c->d_vec, back ? c->d_vec : c->d_saved,
                                      (long long)vectors, back ? scalars : c->d_sc,
@@ -1302,16 +1307,20 @@ int npbcg_conj_grad(npbcg_ctx *c, int colidx[], int rowstr[], double x[], double
     // work, so the two run at the same time; when the arrays turn out to differ, the
     // context is put back as it was.  n = 30011: 960 us a call with the digest first,
     // now 730.  Another matrix altogether shows in the samples, before any work.
-    const bool digest = c->opts.matrix_check == NPBCG_CHECK_FULL;
+    // Without memory to keep the state in, the digest comes first.
+    const bool full = c->opts.matrix_check == NPBCG_CHECK_FULL;
     auto differs = [&]() {
         return set_error(NPBCG_ERR_MISMATCH,
                          "npbcg_conj_grad: rowstr/colidx/a differ from the context's matrix");
     };
-    const bool same_arrays = !digest && colidx == c->h_colidx_ptr && a == c->h_a_ptr;
+    auto same_digest = [&]() { return matrix_digest(colidx, a, c->nnz) == c->matrix_digest; };
+    const bool same_arrays = !full && colidx == c->h_colidx_ptr && a == c->h_a_ptr;
     if (!same_rows(c, rowstr) || !(same_arrays || same_samples(c, colidx, a))) return differs();
     NPBCG_HIP(hipSetDevice(c->device));
     const npbcg_timing timing = c->timing;
-    if (digest) {
+    const bool beside = full && ensure_saved(c);
+    if (full && !beside && !same_digest()) return differs();
+    if (beside) {
         int rc = save_state(c, false);
         if (rc != NPBCG_OK) return rc;
     }
@@ -1321,7 +1330,7 @@ int npbcg_conj_grad(npbcg_ctx *c, int colidx[], int rowstr[], double x[], double
     double rn = 0.0;
     bool same = true;
     int rc = conj_grad_run(c, &rn, [&]() {
-        if (digest) same = matrix_digest(colidx, a, c->nnz) == c->matrix_digest;
+        if (beside) same = same_digest();
     });
     if (!same) {
         c->timing = timing;
