@@ -69,6 +69,7 @@ struct npbcg_ctx {
     uint16_t *d_sell_col = nullptr;
     double *d_rows_part = nullptr; // nblk * n per-block row sums
     bool cols_sorted = true;
+    size_t sell_idx_cap = 0, rows_part_cap = 0;  // elements allocated
     long long sell_stored = 0;     // SELL entries, padding included
     int sort_window = 0;           // rows sorted together per column block
     double *d_vec = nullptr;   // x, z, p, q, r, p_alt, b, xsol back to back, stride vstride
@@ -252,7 +253,11 @@ void refresh_solve_view(npbcg_ctx *c) {
     // flight: plain, Jacobi and Neumann solve, us, apart and fused: n = 17003 -, 187,
     // 248 and -, 172, 231; 30011 213, 214, 278 and 199, 205, 264; 60013 308, 308, 343
     // and 305, 314, 340; 150000 788, 792, 939 and 801, 829, 953.
-    c->pbs.fuse_p_update = c->n <= kFuseSolveRows ? 1 : 0;
+    // With wider blocks than six of that order (fewer_blocks, tile_width) the second
+    // vector costs more: Jacobi, band of 41, one block at n = 18000 133 apart and 151
+    // fused, two at 36000 149 and 162.
+    c->pbs.fuse_p_update =
+        c->n <= kFuseSolveRows && c->pb.sell.W <= (kFuseSolveRows + 5) / 6 ? 1 : 0;
     c->pbs.cg_form = 0;        // the stop test sits in the reference-order p update
 }
 
@@ -629,17 +634,28 @@ int read_scalars(npbcg_ctx *c, Scalars *out) {
     return NPBCG_OK;
 }
 
+void drop_sell(npbcg_ctx *c) {
+    (void)hipFree(c->d_sell_idx);
+    (void)hipFree(c->d_rows_part);
+    c->d_sell_idx = nullptr;
+    c->d_rows_part = nullptr;
+}
+
 // Device arrays of a SELL copy: wg_slice | slice_off | slice_row | row_slot in
 // one allocation (with room for `extra` more ints), and the block sums.
 hipError_t alloc_sell(npbcg_ctx *c, npbcg_dev::SellDev *sd, int slices, size_t extra) {
     const size_t nwg1 = (size_t)sd->grid + 1, nsl1 = (size_t)slices + 1;
     const size_t nrow = (size_t)slices * npbcg_detail::kSliceRows;
-    hipError_t e = hipMalloc(&c->d_sell_idx,
-                             sizeof(int) * (nwg1 + nsl1 + nrow + (size_t)sd->nblk * c->n + extra));
-    // one block sum per slot (64 per slice), stored by slot
-    if (e == hipSuccess)
-        e = hipMalloc(&c->d_rows_part, sizeof(double) * std::max<size_t>(1, nrow));
-    if (e != hipSuccess) return e;
+    const size_t idx = nwg1 + nsl1 + nrow + (size_t)sd->nblk * c->n + extra;
+    const size_t sums = std::max<size_t>(1, nrow);  // one block sum per slot, stored by slot
+    if (c->d_sell_idx && (idx > c->sell_idx_cap || sums > c->rows_part_cap)) drop_sell(c);
+    if (!c->d_sell_idx) {  // (else those of a shape that was not taken)
+        hipError_t e = hipMalloc(&c->d_sell_idx, sizeof(int) * idx);
+        if (e == hipSuccess) e = hipMalloc(&c->d_rows_part, sizeof(double) * sums);
+        if (e != hipSuccess) return e;
+        c->sell_idx_cap = idx;
+        c->rows_part_cap = sums;
+    }
     sd->wg_slice = c->d_sell_idx;
     sd->slice_off = c->d_sell_idx + nwg1;
     sd->slice_row = c->d_sell_idx + nwg1 + nsl1;
@@ -664,55 +680,131 @@ int alloc_error(hipError_t e, const char *what) {
                      std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// The SELL copy of shape *sd from the context's device CSR; sm->wg_slice is
-// set.  *ok = false if it does not fit 32-bit offsets.
-int build_sell_device(npbcg_ctx *c, npbcg_detail::SellBlocks<double> *sm,
-                      npbcg_dev::SellDev *sd, int window, int waves, bool *ok) {
-    const int n = c->n, slices = sm->wg_slice.back();
+// A shape of the SELL copy: what follows from the sizes, before the matrix is looked at.
+struct SellShape {
+    npbcg_dev::SellDev sd;
+    std::vector<int> wg_slice;  // first slice of each workgroup, and the end
+    int window = 0;             // rows sorted together
+};
+
+// Orders the rows of every sort window of the shape and fetches the slices' widths
+// (longest row of each, in sorted order).  sb->order, seg and width and wg_slice are
+// device scratch.
+int order_sell(npbcg_ctx *c, const SellShape &sh, int *wg_slice, npbcg_dev::SellBuild *sb,
+               std::vector<int> *width) {
+    const int slice = npbcg_detail::kSliceRows;
+    sb->n = c->n;
+    sb->W = sh.sd.W;
+    sb->nblk = sh.sd.nblk;
+    sb->R = sh.sd.R;
+    sb->nrange = sh.sd.nrange;
+    sb->window = std::min(sh.window, (sh.sd.R + slice - 1) / slice * slice);
+    sb->rowstr = c->d_rowstr;
+    sb->colidx = c->d_colidx;
+    sb->a = c->d_a;
+    sb->wg_slice = wg_slice;
+    width->resize((size_t)sh.wg_slice.back());
+    NPBCG_HIP(hipMemcpyAsync(wg_slice, sh.wg_slice.data(), sizeof(int) * sh.wg_slice.size(),
+                             hipMemcpyHostToDevice, c->stream));
+    NPBCG_HIP(npbcg_dev::launch_sell_order(*sb, c->stream));
+    NPBCG_HIP(hipMemcpyAsync(width->data(), sb->width, sizeof(int) * width->size(),
+                             hipMemcpyDeviceToHost, c->stream));
+    NPBCG_HIP(hipStreamSynchronize(c->stream));
+    return NPBCG_OK;
+}
+
+// Microseconds of a CG step of the power loop on a SELL copy, fitted to 284 copies of 142
+// matrices (orders 16500 to 115000, 16 to 240 entries a row: makea's, bands, stencils,
+// random and evenly spread rows, six blocks and the widest; 3 % RMS error): the heaviest
+// workgroup and wavefront (entries), all entries stored, and the partial sums.
+double sell_step_us(const npbcg_detail::SellLoad &l, double partial_sums) {
+    return 8.14 + 0.876e-4 * l.workgroup + 4.965e-4 * l.wavefront + 0.901e-6 * l.stored +
+           0.904e-5 * partial_sums;
+}
+
+// Whether `few` (the widest column blocks) is to be taken instead of six blocks, whose
+// load is given.  Six even out makea's rows, which are anywhere in a row; where a row's
+// entries lie in one or two blocks (bands, stencils) a sixth of the workgroups has all of
+// them, and short rows of like length gain nothing for six partial sums a row.  us a CG
+// step, widest blocks and six: band of 81 at n = 25000 15.1 and 21.4, 48000 19.4 and 29.9,
+// 97000 38.1 and 43.5; stencil of 27 at 48000 12.9 and 17.0; 40 evenly spread entries at
+// 48000 12.3 and 14.2; makea with 57 entries a row at 16500 15.9 and 11.3, 40000 14.7 and
+// 14.0, 60000 17.8 and 16.8.  The estimate has to be 7 % less, its error: in the matrices
+// it was fitted to six blocks then stay wherever they are faster, and the widest are
+// missed where they are up to 8 % faster.
+int fewer_blocks(npbcg_ctx *c, const SellShape &few, const npbcg_detail::SellLoad &six_load,
+                 double six_sums, bool *take) {
+    constexpr double kLess = 0.93;
+    const npbcg_dev::SellDev &sd = few.sd;
+    const double limit = kLess * sell_step_us(six_load, six_sums);
+    const double sums = (double)sd.nblk * c->n;
+    const int waves = sd.block / npbcg_dev::kWave;
+    *take = false;
+    // the least it can be: no padding, and the entries spread over all wavefronts with a slice
+    const int slices = few.wg_slice[1] - few.wg_slice[0];
+    npbcg_detail::SellLoad load;
+    load.stored = c->nnz;
+    load.workgroup = c->nnz / sd.grid;
+    load.wavefront = load.workgroup / std::min(waves, slices);
+    if (sell_step_us(load, sums) >= limit) return NPBCG_OK;
+    const size_t rows = (size_t)sd.nblk * c->n, head = few.wg_slice.size();
+    if (head + 2 * rows + (size_t)few.wg_slice.back() > 2 * kNumVectors * c->vstride)
+        return NPBCG_OK;
+    int *scratch = reinterpret_cast<int *>(c->d_vec);  // (cleared later)
+    npbcg_dev::SellBuild sb;
+    sb.order = scratch + head;
+    sb.seg = sb.order + rows;
+    sb.width = sb.seg + rows;
+    std::vector<int> width;
+    int rc = order_sell(c, few, scratch, &sb, &width);
+    if (rc != NPBCG_OK) return rc;
+    load = npbcg_detail::sell_load(few.wg_slice, width.data(), nullptr, waves);
+    *take = sell_step_us(load, sums) < limit;
+    return NPBCG_OK;
+}
+
+// The SELL copy of *sh from the context's device CSR, or of *few, when that is given and
+// the better one (*sh is it then).  *ok = false if it does not fit 32-bit offsets.
+int build_sell_device(npbcg_ctx *c, SellShape *sh, const SellShape *few, bool *ok) {
+    npbcg_dev::SellDev *const sd = &sh->sd;
+    const int n = c->n, slices = sh->wg_slice.back(), waves = sd->block / npbcg_dev::kWave;
     const size_t rows = (size_t)sd->nblk * n;
     hipError_t e = alloc_sell(c, sd, slices, (size_t)slices);
     if (e != hipSuccess) return alloc_error(e, "npbcg_create: SELL index");
     int *const idx = c->d_sell_idx;
     int *const slice_off = idx + (sd->slice_off - idx), *const slice_row = idx + (sd->slice_row - idx);
     int *const row_slot = idx + (sd->row_slot - idx), *const src = row_slot + rows;
-    npbcg_dev::SellBuild sb;
-    sb.n = n;
-    sb.W = sd->W;
-    sb.nblk = sd->nblk;
-    sb.R = sd->R;
-    sb.nrange = sd->nrange;
-    sb.window = std::min(window, (sd->R + npbcg_detail::kSliceRows - 1) /
-                                     npbcg_detail::kSliceRows * npbcg_detail::kSliceRows);
-    sb.rowstr = c->d_rowstr;
-    sb.colidx = c->d_colidx;
-    sb.a = c->d_a;
-    sb.wg_slice = sd->wg_slice;
     // scratch in arrays that are written last: 2 nblk - 1 ints a row fit the
     // block sums' 2 nblk, the widths the lane rows they turn into
+    npbcg_dev::SellBuild sb;
     sb.order = reinterpret_cast<int *>(c->d_rows_part);
     sb.seg = sb.order + rows;
     sb.width = slice_row;
-    NPBCG_HIP(hipMemcpyAsync(idx, sm->wg_slice.data(), sizeof(int) * sm->wg_slice.size(),
-                             hipMemcpyHostToDevice, c->stream));
-    NPBCG_HIP(npbcg_dev::launch_sell_order(sb, c->stream));
-    std::vector<int> width((size_t)slices), place, off;
-    NPBCG_HIP(hipMemcpyAsync(width.data(), sb.width, sizeof(int) * (size_t)slices,
-                             hipMemcpyDeviceToHost, c->stream));
-    NPBCG_HIP(hipStreamSynchronize(c->stream));
+    std::vector<int> width, place, off;
+    int rc = order_sell(c, *sh, idx, &sb, &width);
+    if (rc != NPBCG_OK) return rc;
     const long long stored =
-        npbcg_detail::place_sell_slices(sm->wg_slice, width.data(), waves, &place, &off);
+        npbcg_detail::place_sell_slices(sh->wg_slice, width.data(), waves, &place, &off);
     if (stored < 0) {
-        (void)hipFree(c->d_sell_idx);
-        (void)hipFree(c->d_rows_part);
-        c->d_sell_idx = nullptr;
-        c->d_rows_part = nullptr;
+        drop_sell(c);
         *ok = false;
         return NPBCG_OK;
     }
+    if (few) {
+        bool take = false;
+        const auto load =
+            npbcg_detail::sell_load(sh->wg_slice, width.data(), place.data(), waves);
+        rc = fewer_blocks(c, *few, load, (double)rows, &take);
+        if (rc != NPBCG_OK) return rc;
+        if (take) {
+            *sh = *few;
+            return build_sell_device(c, sh, nullptr, ok);
+        }
+    }
     // sorted slice i of a workgroup -> its first row's place in `order`
     for (int wg = 0; wg < sd->grid; wg++) {
-        const int s0 = sm->wg_slice[wg], b = wg / sd->nrange, r0 = wg % sd->nrange * sd->R;
-        for (int s = s0; s < sm->wg_slice[wg + 1]; s++)
+        const int s0 = sh->wg_slice[wg], b = wg / sd->nrange, r0 = wg % sd->nrange * sd->R;
+        for (int s = s0; s < sh->wg_slice[wg + 1]; s++)
             place[s] = b * n + r0 + (place[s] - s0) * npbcg_detail::kSliceRows;
     }
     e = alloc_sell_entries(c, sd, stored);
@@ -907,11 +999,14 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
     // narrow that they fit twice, two of 512 threads.  Row ranges spread the
     // nblk * nrange workgroups evenly over the CUs.
     //
-    // Up to 6 of the widest blocks (n <= 121344 with 160 KB) 6 blocks are
+    // Up to 6 of the widest blocks (n <= 121068 with 160 KB; six of the very
+    // widest leave the LDS no room for the slices' slots) 6 blocks are
     // taken all the same, and ranges of whole 64-row slices, one workgroup per
     // CU: fewer blocks mean shorter ranges, whose last slice is mostly padding
     // (1.99 entries stored per nonzero in 79-row ranges at n = 20000), and a
-    // longer block for every workgroup to stage.  FP64 step of the power loop /
+    // longer block for every workgroup to stage.  From 16 entries a row on, where
+    // this layout is the library's own choice, the matrix decides (fewer_blocks).
+    // FP64 step of the power loop /
     // FP32 product, us, before and with 6 blocks: n = 8009 25.7 / 20.0 and
     // 11.3 / 7.0, 20000 27.0 / 22.0 and 15.4 / 8.2, 30011 19.1 / 10.7 and 15.3 /
     // 7.9, 60013 26.4 / 15.9 and 25.1 / 13.1, 75000 32.0 / 17.9 and 31.9 / 16.5;
@@ -921,6 +1016,8 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
     // wavefronts share the rest better (21.5 against 22.5 us at 45000).
     npbcg_detail::SellBlocks<double> sm;
     npbcg_dev::SellDev sd;
+    c->vstride = ((size_t)n + 2 + 63) & ~(size_t)63;
+    CREATE_HIP(hipMalloc(&c->d_vec, sizeof(double) * kNumVectors * c->vstride));
     if (variant == npbcg_dev::kSpmvTiled) {
         int lds_cap = 0;
         if (hipDeviceGetAttribute(&lds_cap, hipDeviceAttributeSharedMemPerBlockOptin,
@@ -928,134 +1025,136 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
             lds_cap = 64 * 1024;
         const int lds_budget = lds_cap - 2048;  // static LDS of the reduction epilogue
         constexpr int kMidBlocks = 6;
-        int W;
-        bool mid = false;
-        if (c->opts.tile_width > 0) {
-            W = c->opts.tile_width;
-        } else {
-            const int wmax = std::min(65536, lds_budget / 8);
-            int nblk = (n + wmax - 1) / wmax;
-            mid = nblk <= kMidBlocks && c->opts.tile_rows <= 0 && cus >= kMidBlocks;
-            if (mid) nblk = kMidBlocks;
-            W = (n + nblk - 1) / nblk;
-        }
-        W = std::max(2, (W + 1) & ~1);
-        if (W > n) W = (n + 1) & ~1;
-        int block = (W * 8 <= lds_budget / 2 - 1024) ? 512 : 1024;
-        int nblk = (n + W - 1) / W;
-        auto default_rows = [&]() {
-            const int slots = cus * (block == 512 ? 2 : 1);
-            const int nrange = std::max(1, slots / nblk);
-            return (int)(((long long)n + nrange - 1) / nrange);
-        };
-        int R = c->opts.tile_rows > 0 ? c->opts.tile_rows : default_rows();
         const int kSlice = npbcg_detail::kSliceRows;
-        if (mid) {
-            const int nrange = cus / kMidBlocks;
-            const int slices = ((n + nrange - 1) / nrange + kSlice - 1) / kSlice;
-            R = slices * kSlice;
-            block = slices <= 16 ? 512 : 1024;
-        }
-        // The per-slice p.q slots (one double per 64-row slice of a workgroup)
-        // share the LDS with the vector block.  When the range's slices do not
-        // fit beside the block (large n: few ranges of many rows), the block
-        // is narrowed to 7/8 of the LDS and the range capped at the slices
-        // the rest holds: more, shorter workgroups instead of the CSR kernel.
-        if ((long long)(W + (R + kSlice - 1) / kSlice) * 8 > lds_budget) {
-            if (c->opts.tile_width <= 0) {
-                const int wcap = (lds_budget / 8) * 7 / 8;
-                if (W > wcap) {
-                    const int nb = (n + wcap - 1) / wcap;
-                    W = std::max(2, ((n + nb - 1) / nb + 1) & ~1);
-                    block = (W * 8 <= lds_budget / 2 - 1024) ? 512 : 1024;
-                    nblk = (n + W - 1) / W;
-                    if (c->opts.tile_rows <= 0) R = default_rows();
-                }
+        const int wmax = std::min(65536, lds_budget / 8), widest = (n + wmax - 1) / wmax;
+        // The shape in column blocks as wide as fit or, with mid, in six; false if the
+        // LDS does not hold it or the slices are too many.
+        auto shape_of = [&](bool mid, SellShape *out) {
+            int W;
+            if (c->opts.tile_width > 0) {
+                W = c->opts.tile_width;
+            } else {
+                const int nblk = mid ? kMidBlocks : widest;
+                W = (n + nblk - 1) / nblk;
             }
-            if (c->opts.tile_rows <= 0) {
-                const int rmax = kSlice * (lds_budget / 8 - W - 1);
-                if (rmax >= kSlice && R > rmax) {
-                    // The capped ranges give nblk * nrange workgroups for
-                    // `slots` CU slots; of the range counts from the least
-                    // the cap allows up to twice that, take the one whose
-                    // last round of workgroups fills the most slots (equal
-                    // workgroups: a part-filled round leaves CUs idle).  At
-                    // 1.5 M rows: 85 blocks x 12 ranges = 3.98 rounds of 256
-                    // instead of 85 x 10 = 3.32.
-                    const int slots = cus * (block == 512 ? 2 : 1);
-                    const int nr0 = (n + rmax - 1) / rmax;
-                    int best = nr0;
-                    double best_idle = 2.0;
-                    for (int nr = nr0; nr <= 2 * nr0; nr++) {
-                        const double rounds = (double)nblk * nr / slots;
-                        const double idle = (std::ceil(rounds) - rounds) / std::ceil(rounds);
-                        if (idle < best_idle - 1e-9) {
-                            best_idle = idle;
-                            best = nr;
-                        }
+            W = std::max(2, (W + 1) & ~1);
+            if (W > n) W = (n + 1) & ~1;
+            int block = (W * 8 <= lds_budget / 2 - 1024) ? 512 : 1024;
+            int nblk = (n + W - 1) / W;
+            auto default_rows = [&]() {
+                const int slots = cus * (block == 512 ? 2 : 1);
+                const int nrange = std::max(1, slots / nblk);
+                return (int)(((long long)n + nrange - 1) / nrange);
+            };
+            int R = c->opts.tile_rows > 0 ? c->opts.tile_rows : default_rows();
+            if (mid) {
+                const int nrange = cus / kMidBlocks;
+                const int slices = ((n + nrange - 1) / nrange + kSlice - 1) / kSlice;
+                R = slices * kSlice;
+                block = slices <= 16 ? 512 : 1024;
+            }
+            // The per-slice p.q slots (one double per 64-row slice of a workgroup)
+            // share the LDS with the vector block.  When the range's slices do not
+            // fit beside the block (large n: few ranges of many rows), the block
+            // is narrowed to 7/8 of the LDS and the range capped at the slices
+            // the rest holds: more, shorter workgroups instead of the CSR kernel.
+            if ((long long)(W + (R + kSlice - 1) / kSlice) * 8 > lds_budget) {
+                if (c->opts.tile_width <= 0) {
+                    const int wcap = (lds_budget / 8) * 7 / 8;
+                    if (W > wcap) {
+                        const int nb = (n + wcap - 1) / wcap;
+                        W = std::max(2, ((n + nb - 1) / nb + 1) & ~1);
+                        block = (W * 8 <= lds_budget / 2 - 1024) ? 512 : 1024;
+                        nblk = (n + W - 1) / W;
+                        if (c->opts.tile_rows <= 0) R = default_rows();
                     }
-                    R = (int)(((long long)n + best - 1) / best);
+                }
+                if (c->opts.tile_rows <= 0) {
+                    const int rmax = kSlice * (lds_budget / 8 - W - 1);
+                    if (rmax >= kSlice && R > rmax) {
+                        // The capped ranges give nblk * nrange workgroups for
+                        // `slots` CU slots; of the range counts from the least
+                        // the cap allows up to twice that, take the one whose
+                        // last round of workgroups fills the most slots (equal
+                        // workgroups: a part-filled round leaves CUs idle).  At
+                        // 1.5 M rows: 85 blocks x 12 ranges = 3.98 rounds of 256
+                        // instead of 85 x 10 = 3.32.
+                        const int slots = cus * (block == 512 ? 2 : 1);
+                        const int nr0 = (n + rmax - 1) / rmax;
+                        int best = nr0;
+                        double best_idle = 2.0;
+                        for (int nr = nr0; nr <= 2 * nr0; nr++) {
+                            const double rounds = (double)nblk * nr / slots;
+                            const double idle = (std::ceil(rounds) - rounds) / std::ceil(rounds);
+                            if (idle < best_idle - 1e-9) {
+                                best_idle = idle;
+                                best = nr;
+                            }
+                        }
+                        R = (int)(((long long)n + best - 1) / best);
+                    }
                 }
             }
-        }
-        // Rows are sorted by their length in a block over the whole range,
-        // from 2048 up to 8192 rows: at n = 150000 (ranges of 4688 rows) that
-        // stores 1.019 entries per nonzero instead of 1.048 with 2048-row
-        // windows, at 1.5 M rows 1.016 instead of 1.058.
-        const int window =
-            c->opts.sort_window > 0
-                ? c->opts.sort_window
-                : std::min(kMaxSortWindow, std::max(npbcg_detail::kSortWindow,
-                                                    (R + kSlice - 1) / kSlice * kSlice));
-        const int kept_blocks = (n + W - 1) / W, kept_ranges = (n + R - 1) / R;
-        // windows the device's sort takes (in range of its keys); wider ones,
-        // which only sort_window asks for, are built on the host
-        const bool on_device = std::min(window, R) <= npbcg_dev::kSellSortRows;
-        bool built = W * 8 <= lds_budget && W <= 65536 && sorted;
-        if (built && on_device) {
+            // Rows are sorted by their length in a block over the whole range,
+            // from 2048 up to 8192 rows: at n = 150000 (ranges of 4688 rows) that
+            // stores 1.019 entries per nonzero instead of 1.048 with 2048-row
+            // windows, at 1.5 M rows 1.016 instead of 1.058.
+            const int window =
+                c->opts.sort_window > 0
+                    ? c->opts.sort_window
+                    : std::min(kMaxSortWindow, std::max(npbcg_detail::kSortWindow,
+                                                        (R + kSlice - 1) / kSlice * kSlice));
+            npbcg_dev::SellDev &d = out->sd;
+            out->window = window;
+            d.W = W;
+            d.R = R;
+            d.nblk = (n + W - 1) / W;
+            d.nrange = (n + R - 1) / R;
+            d.block = block;
+            const int slices = (std::min(n, R) + kSlice - 1) / kSlice;  // of a whole range
+            d.lds_bytes = (W + slices) * 8;
+            if (W > 65536 || d.lds_bytes > lds_budget) return false;
             // slices of every workgroup follow from the sizes
-            const long long slices_ll = (long long)kept_blocks *
-                                        ((long long)(kept_ranges - 1) * ((R + kSlice - 1) / kSlice) +
-                                         (n - (long long)(kept_ranges - 1) * R + kSlice - 1) / kSlice);
-            built = slices_ll * kSlice <= (long long)INT32_MAX;
-            if (built) {
-                sm.wg_slice.assign((size_t)kept_blocks * kept_ranges + 1, 0);
-                for (int wg = 0; wg < kept_blocks * kept_ranges; wg++) {
-                    const int r0 = wg % kept_ranges * R, rows = std::min(n, r0 + R) - r0;
-                    sm.wg_slice[wg + 1] = sm.wg_slice[wg] + (rows + kSlice - 1) / kSlice;
-                }
+            const long long last = n - (d.nrange - 1) * (long long)R;  // rows
+            const long long all =
+                d.nblk * ((d.nrange - 1ll) * slices + (last + kSlice - 1) / kSlice);
+            if (all * kSlice > (long long)INT32_MAX) return false;
+            d.grid = d.nblk * d.nrange;
+            out->wg_slice.assign((size_t)d.grid + 1, 0);
+            for (int wg = 0; wg < d.grid; wg++) {
+                const int r0 = wg % d.nrange * R, rows = std::min(n, r0 + R) - r0;
+                out->wg_slice[wg + 1] = out->wg_slice[wg] + (rows + kSlice - 1) / kSlice;
             }
-        } else if (built) {
-            built = npbcg_detail::build_sell_blocks(n, rowstr, colidx, a, W, R, &sm, window,
-                                                    block / 64);
+            return true;
+        };
+        const bool mid = c->opts.tile_width <= 0 && c->opts.tile_rows <= 0 &&
+                         widest <= kMidBlocks && cus >= kMidBlocks;
+        SellShape shape, few;
+        bool built = sorted && shape_of(mid, &shape);
+        if (built) {
+            // windows the device's sort takes (in range of its keys); wider ones,
+            // which only sort_window asks for, are built on the host
+            if (std::min(shape.window, shape.sd.R) <= npbcg_dev::kSellSortRows) {
+                const bool compare = mid && widest < kMidBlocks && nnz >= 16ll * n &&
+                                     shape.sd.nblk == kMidBlocks && shape_of(false, &few) &&
+                                     std::min(few.window, few.sd.R) <= npbcg_dev::kSellSortRows;
+                rc = build_sell_device(c, &shape, compare ? &few : nullptr, &built);
+                if (rc != NPBCG_OK) return fail(rc);
+            } else {
+                built = npbcg_detail::build_sell_blocks(n, rowstr, colidx, a, shape.sd.W,
+                                                        shape.sd.R, &sm, shape.window,
+                                                        shape.sd.block / npbcg_dev::kWave);
+            }
         }
         if (built) {
-            c->sort_window = window;
-            sd.W = W;
-            sd.nblk = kept_blocks;
-            sd.R = R;
-            sd.nrange = kept_ranges;
-            sd.grid = kept_blocks * kept_ranges;
-            sd.block = block;
-            int max_slices = 0;
-            for (size_t w = 0; w + 1 < sm.wg_slice.size(); w++)
-                max_slices = std::max(max_slices, sm.wg_slice[w + 1] - sm.wg_slice[w]);
-            sd.lds_bytes = (W + max_slices) * 8;
-            built = sd.lds_bytes <= lds_budget;
-        }
-        if (built && on_device) {
-            rc = build_sell_device(c, &sm, &sd, window, block / 64, &built);
-            if (rc != NPBCG_OK) return fail(rc);
-        }
-        if (!built) {
+            sd = shape.sd;
+            c->sort_window = shape.window;
+        } else {
             variant = pick_variant(npbcg_dev::kSpmvSeg64, n, nnz, false);
-            sd = npbcg_dev::SellDev{};
             sm = npbcg_detail::SellBlocks<double>{};
         }
     }
 
-    c->vstride = ((size_t)n + 2 + 63) & ~(size_t)63;
-    CREATE_HIP(hipMalloc(&c->d_vec, sizeof(double) * kNumVectors * c->vstride));
     c->part_vec = vec_blocks;
     c->part_spmv = variant == npbcg_dev::kSpmvTiled ? std::max(sd.grid, vec_blocks)
                                                     : spmv_blocks;

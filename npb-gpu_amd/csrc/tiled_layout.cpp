@@ -129,6 +129,28 @@ long long place_sell_slices(const std::vector<int> &wg_slice, const int *width, 
     return off;
 }
 
+SellLoad sell_load(const std::vector<int> &wg_slice, const int *width, const int *src,
+                   int waves) {
+    SellLoad l;
+    std::vector<long long> load((size_t)waves);
+    for (size_t wg = 0; wg + 1 < wg_slice.size(); wg++) {
+        std::fill(load.begin(), load.end(), 0);
+        for (int s = wg_slice[wg]; s < wg_slice[wg + 1]; s++) {
+            const int k = s - wg_slice[wg], rd = k / waves, i = k % waves;
+            load[(size_t)((rd & 1) ? waves - 1 - i : i)] +=
+                (long long)kSliceRows * width[src ? src[s] : s];
+        }
+        long long sum = 0;
+        for (long long v : load) {
+            sum += v;
+            l.wavefront = std::max(l.wavefront, v);
+        }
+        l.workgroup = std::max(l.workgroup, sum);
+        l.stored += sum;
+    }
+    return l;
+}
+
 namespace {
 
 template <class V>

@@ -66,6 +66,14 @@ bool build_sell_blocks(int n, const int *rowstr, const int *colidx, const double
 long long place_sell_slices(const std::vector<int> &wg_slice, const int *width, int waves,
                             std::vector<int> *src, std::vector<int> *slice_off);
 
+// Entries, padding included, of a copy placed so (src null: slices in sorted order): of
+// the heaviest workgroup, of the heaviest wavefront, and of all.
+struct SellLoad {
+    long long workgroup = 0, wavefront = 0, stored = 0;
+};
+SellLoad sell_load(const std::vector<int> &wg_slice, const int *width, const int *src,
+                   int waves);
+
 }  // namespace npbcg_detail
 
 #endif
