@@ -185,9 +185,9 @@ constexpr int kMaxSortWindow = 8192;
 constexpr size_t kResidentWords = (size_t)8 << 20;
 // FP64 solves up to this order update p inside the SpMV (refresh_solve_view).
 constexpr int kFuseSolveRows = 49152;
-// Below this order repeated solves on the CSR kernels replay a graph, from this sight on
-// (run_solve_sequence).
-constexpr int kGraphSolveRows = 16384;
+// Below these orders repeated solves on the CSR kernels and on the SELL copy replay a
+// graph, from this sight on (run_solve_sequence).
+constexpr int kGraphSolveCsr = 131072, kGraphSolveSell = 32768;
 constexpr int kGraphSolveSights = 4;
 // Steps of a resident solve launch at most.
 constexpr int kResidentSolveSteps = 64;
@@ -2440,20 +2440,23 @@ namespace {
 
 // Runs the first stretch of an FP64 solve: reset, init, `batch` steps, residual.
 //
-// Small orders on the CSR kernels are bound by their launches (three of 2 to 4 us a
-// step), so a sequence that comes again (same preconditioner in effect, rtol and step
-// count, whatever the right-hand side) replays a captured graph: Jacobi solve at
-// n = 1400 164 us launched and 125 replayed, 4001 166 and 132, 9001 174 and 159, 15001
-// 189 and 179 (a faster host: 128 and 124 at 1400).  From about there on the two are
-// equal (17003: 194 and 191, 150000: 645 and 653).  A capture costs about 150 us, what
-// four solves lose to their launches, so it is made when a sequence is seen for the
-// fourth time.  The buffers that the kernels read are the context's own and stay
-// where they are.
+// The launches of small steps (three of 2 to 5 us) cost the host as much as the GPU, so
+// a sequence that comes again (same preconditioner in effect, rtol and step count,
+// whatever the right-hand side) replays a captured graph.  Launched and replayed, us,
+// Jacobi, one right-hand side: on the CSR kernels n = 1400 164 and 125, 4001 166 and 132,
+// 9001 174 and 159, 15001 189 and 179 (a faster host: 128 and 124 at 1400); band of 5
+// 17000 264 and 231, 30000 266 and 244, 100000 344 and 337, and with 9 entries a row
+// 150000 444 and 441, three right-hand sides in turn 439 and 443.  On the SELL copy a
+// step has fewer or longer launches: band of 41 at 18000 178 and 160, of 81 at 30000 194
+// and 187, makea 18000 172 and 165, 40000 210 and 212, in turn 204 and 208.  A capture
+// costs about 150 us, what four solves lose to their launches, so it is made when a
+// sequence is seen for the fourth time.  The buffers that the kernels read are the
+// context's own and stay where they are.
 int run_solve_sequence(npbcg_ctx *c, double rtol, int batch,
                        const std::function<hipError_t()> &enqueue) {
     auto &sg = c->solve_graph[batch % 16];
-    if (!c->opts.use_graph || c->pb.spmv_variant == npbcg_dev::kSpmvTiled ||
-        c->n >= kGraphSolveRows) {
+    const bool sell = c->pb.spmv_variant == npbcg_dev::kSpmvTiled;
+    if (!c->opts.use_graph || c->n >= (sell ? kGraphSolveSell : kGraphSolveCsr)) {
         NPBCG_HIP(enqueue());
         return NPBCG_OK;
     }
