@@ -38,10 +38,13 @@ enum {
     NPBCG_ENGINE_AUTO = 0,        /* up to n = 19152, with the layout and step form left
                                      to the library too (spmv_variant, cg_form,
                                      dot_pass, fuse_p_update, tile and sort options 0)
-                                     and no row of more than some thousand entries: the
+                                     and no row of more than 4096 entries (n <= 3840),
+                                     2048 (n <= 7936), 1024 (n <= 16128) or 512: the
                                      resident engine, one launch per call that keeps
                                      vectors and matrix on chip (plain FP64 solves with
-                                     solve_batch 0 too).  Else KERNELS (8.5 ms against
+                                     solve_batch 0 too) and up to 64 MB of exchange
+                                     buffers a context; without memory for those the
+                                     call runs on KERNELS.  Else KERNELS (8.5 ms against
                                      14.6 ms of PERSISTENT for 10 outer iterations at
                                      n = 75000).  A resident launch needs all its
                                      workgroups on the GPU at once.  The launches of one

@@ -1213,8 +1213,11 @@ int npbcg_create(npbcg_ctx **out, int n, const int *rowstr, const int *colidx,
     // Resident engine: the engine, layout and step form all left to the
     // library, and an order its kernels take.  Microseconds a CG step, resident
     // against the kernels this context would launch (CSR below n = 16384,
-    // LDS-staged above): 2.2 / 8.8 at n = 1400, 3.8 / 10.9 at 7000, 7.1 / 16.2
-    // at 14000, 7.2 / 17.8 at 16000, 11.9 / 27.5 at 19000, where the LDS ends.
+    // LDS-staged above): 1.9 / 8.9 at n = 1400, 3.5 / 11.1 at 7000, 6.4 / 16.4
+    // at 14000, 7.0 / 18.4 at 16000, 9.0 / 12.4 at 19000, where the LDS ends.
+    // Rows that are read from memory in every step, too: 200 entries a row 8.3 /
+    // 13.6 (LDS-staged) at 16000 and 12.1 / 15.6 at 19000, 500 a row 17.1 / 21.7
+    // and 25.2 / 24.3; one row of 1024 10.2 / 16.0 at 16000.
     if (c->opts.engine == NPBCG_ENGINE_AUTO && c->opts.spmv_variant == 0 &&
         c->opts.cg_form == 0 && c->opts.dot_pass == 0 && !c->opts.fuse_p_update &&
         c->opts.tile_rows <= 0 && c->opts.tile_width <= 0 && c->opts.sort_window == 0) {

@@ -16,7 +16,8 @@
 // and beta, and take the same branches.  The reference's order with the same
 // exchange (p in LDS; rho, beta and p = r + beta p before the next product)
 // took 2.8, 5.0 and 8.3 us a step at n = 1400, 7000 and 14000 against 2.2,
-// 3.8 and 7.0.
+// 3.8 and 7.0 (both with kernels for five word counts; with those below 1.9,
+// 3.5 and 6.4).
 //
 // Exchange: a value is its own flag.  Each exchange of a launch has its own
 // buffer, filled with the all-ones NaN before the launch (resident_arm_kernel,
