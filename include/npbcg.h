@@ -77,7 +77,8 @@ typedef struct npbcg_opts {
     int engine;       /* NPBCG_ENGINE_* */
     int spmv_variant; /* 0 = auto; 1-4 CSR row kernels (64/32/16 lanes per row,
                          64 with 2 loads in flight); 5 = LDS-staged column blocks */
-    int use_graph;    /* nonzero: replay each outer iteration as a captured HIP graph */
+    int use_graph;    /* nonzero: replay each outer iteration, and FP64 solves of small
+                         systems that come again, as a captured HIP graph */
     int tile_rows;    /* LDS-staged SpMV: rows per tile, 0 = auto */
     int tile_width;   /* LDS-staged SpMV: vector entries per LDS block, 0 = auto */
     int fuse_p_update;/* LDS-staged SpMV: form p = r + beta p inside the next SpMV
