@@ -1394,6 +1394,12 @@ int npbcg_test_no_memory(npbcg_ctx *c, int on) {
     return NPBCG_OK;
 }
 
+int npbcg_test_solve_graphs(npbcg_ctx *c) {
+    int count = 0;
+    for (const auto &sg : c->solve_graph) count += sg.ex != nullptr;
+    return count;
+}
+
 int npbcg_conj_grad_device(npbcg_ctx *c, double *rnorm) {
     npbcg_detail::TraceRange trace("npbcg_conj_grad");
     if (!c) return set_error(NPBCG_ERR_INVALID, "npbcg_conj_grad_device: NULL context");

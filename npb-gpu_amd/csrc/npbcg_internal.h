@@ -31,4 +31,7 @@ extern "C" int npbcg_test_resident_give_up(npbcg_ctx *c, int iteration);
 // run faster cannot be had, as on a full device.
 extern "C" int npbcg_test_no_memory(npbcg_ctx *c, int on);
 
+// For tests: the solve sequences that the context has captured as graphs.
+extern "C" int npbcg_test_solve_graphs(npbcg_ctx *c);
+
 #endif
